@@ -3,65 +3,28 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "attention_plain.hpp"
 #include "lm.hpp"
 
 namespace {
 
-// Any size, either element type: one workgroup per (row, head).  256 keys at a time: a thread's score is its key's dot product, then the threads change over to latent columns
-// (up to 8 each) for the weighted sum; online softmax across chunks.
-template <typename T>
-__global__ __launch_bounds__(256) void latent_attn_plain_kernel(const LatentAttnParams p) {
-    extern __shared__ float sm[];
-    __shared__ float red[8];
-    float* q = sm;                   // [Rp]
-    float* w = sm + p.Rp;            // [256]
-    const int row = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
+// Any size, either element type: one workgroup per (row, head), the cached row as key and value (attention_plain.hpp).
+template <typename T, int TPB>
+__global__ __launch_bounds__(TPB) void latent_attn_plain_kernel(const LatentAttnParams p) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    __shared__ float red[2 * TPB / 64];
+    const int row = blockIdx.x, head = blockIdx.y;
     const int seq = p.ix.row_seq ? p.ix.row_seq[row] : p.ix.seqs[row];
     const int n = (p.ix.row_pos ? p.ix.row_pos[row] : p.ix.lens[seq]) + 1;
-    const T* Q = (const T*)p.Q + ((int64_t)row * p.H + head) * p.Rp;
     const T* C = (const T*)p.C + (int64_t)seq * p.max_tokens * p.Rp;
-    for (int i = tid; i < p.Rp; i += 256) q[i] = (float)Q[i];
-    float acc[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.f;
-    for (int k0 = 0; k0 < n; k0 += 256) {
-        __syncthreads();
-        const int key = k0 + tid;
-        float s = -INFINITY;
-        if (key < n) {
-            const T* c = C + (int64_t)key * p.Rp;
-            float d0 = 0.f, d1 = 0.f, d2 = 0.f, d3 = 0.f;
-            for (int i = 0; i < p.Rp; i += 4) { d0 += q[i] * (float)c[i]; d1 += q[i + 1] * (float)c[i + 1]; d2 += q[i + 2] * (float)c[i + 2]; d3 += q[i + 3] * (float)c[i + 3]; }
-            s = ((d0 + d1) + (d2 + d3)) * p.scale;
-        }
-        float mx = wave_max(s);
-        if ((tid & 63) == 0) red[tid >> 6] = mx;
-        __syncthreads();
-        const float m_new = fmaxf(m_run, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-        const float e = key < n ? expf(s - m_new) : 0.f;
-        w[tid] = e;
-        const float sum = wave_sum(e);
-        if ((tid & 63) == 0) red[4 + (tid >> 6)] = sum;
-        __syncthreads();
-        const float alpha = expf(m_run - m_new);
-        l_run = l_run * alpha + (red[4] + red[5] + red[6] + red[7]);
-        m_run = m_new;
-        const int nk = min(256, n - k0);
-#pragma unroll
-        for (int j = 0; j < 8; j++) {
-            const int i = tid + 256 * j;
-            if (i >= p.Rp) break;
-            float a = acc[j] * alpha;
-            const T* c = C + (int64_t)k0 * p.Rp + i;
-            for (int k = 0; k < nk; k++) a += w[k] * (float)c[(int64_t)k * p.Rp];
-            acc[j] = a;
-        }
-    }
-    T* O = (T*)p.O + ((int64_t)row * p.H + head) * p.Rp;
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const int i = tid + 256 * j;
-        if (i < p.Rp) O[i] = (T)(acc[j] / l_run);
-    }
+    const int64_t at = ((int64_t)row * p.H + head) * p.Rp;
+    T* O = (T*)p.O + at;
+    plain_attend<T, TPB>((const T*)p.Q + at, C, p.Rp, C, p.Rp, n, p.Rp, p.Rp, p.scale, 0.f, sm, red, [&](int i, float v) { O[i] = (T)v; });
+}
+template <typename T>
+void launch_plain_t(const LatentAttnParams& p, hipStream_t st) {
+    if ((int64_t)p.M * p.H <= 1024) hipLaunchKernelGGL((latent_attn_plain_kernel<T, 1024>), dim3(p.M, p.H), dim3(1024), plain_lds_floats(p.Rp, 1024) * 4, st, p);
+    else hipLaunchKernelGGL((latent_attn_plain_kernel<T, 256>), dim3(p.M, p.H), dim3(256), plain_lds_floats(p.Rp, 256) * 4, st, p);
 }
 
 // ---- bf16 decode --------------------------------------------------------------------------------------------------------
@@ -424,11 +387,9 @@ int launch_latent_decode(const LatentDecodeParams& p, hipStream_t st) {
 }
 
 int launch_latent_attn_plain(bool f32, const LatentAttnParams& p, hipStream_t st) {
-    if (p.M <= 0 || p.H <= 0 || p.Rp <= 0 || p.Rp % 4 || p.Rp > 2048) return cr_fail(CR_ERR_ARG, "latent attention: rows %d, heads %d, latent %d", p.M, p.H, p.Rp);
-    const dim3 grid(p.M, p.H), block(256);
-    const size_t lds = (size_t)(p.Rp + 256) * 4;
-    if (f32) hipLaunchKernelGGL(latent_attn_plain_kernel<float>, grid, block, lds, st, p);
-    else hipLaunchKernelGGL(latent_attn_plain_kernel<bf16>, grid, block, lds, st, p);
+    if (p.M <= 0 || p.H <= 0 || p.Rp <= 0 || p.Rp % 64 || p.Rp > PLAIN_MAX_COLS) return cr_fail(CR_ERR_ARG, "latent attention: rows %d, heads %d, latent %d", p.M, p.H, p.Rp);
+    if (f32) launch_plain_t<float>(p, st);
+    else launch_plain_t<bf16>(p, st);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }

@@ -274,8 +274,13 @@ GemmParams slice_params(const void* A, int64_t lda, const void* W, const bf16* d
     return p;
 }
 bool one_slice(int M, int N, int K) { return gemm_stream_supported(EPI_F32, slice_params(nullptr, K, nullptr, nullptr, nullptr, M, N, K), 1); }
-int slices_of(const Lm& lm, int M, int N, int K, bool decode) { return lm.f32 || !decode || M > 64 ? 0 : one_slice(M, N, K) ? 1 : gemm_partial_splits(N, K); }
+int slices_of(const Lm& lm, int M, int N, int K, bool decode) { return !decode || M > 64 ? 0 : lm.f32 ? lm_rows_slices(N, K) : one_slice(M, N, K) ? 1 : gemm_partial_splits(N, K); }
 int sliced(cr_ctx* c, const void* A, int64_t lda, const void* W, const bf16* dl, float* C, int M, int N, int K, hipStream_t st) {
+    if (c->lm->f32) {
+        LmGemmParams g{};
+        g.A = A; g.lda = lda; g.W = W; g.ldw = K; g.C = C; g.ldc = N; g.M = M; g.N = N; g.K = K; g.stream = 1; g.slices = lm_rows_slices(N, K);
+        return launch_lm_gemm(true, LM_RAW32, g, st);
+    }
     GemmParams p = slice_params(A, lda, W, dl, C, M, N, K);
     if (!one_slice(M, N, K)) return ctx_gemm(c, EPI_PARTIAL, p, st);
     p.raw32 = 1;
@@ -288,9 +293,9 @@ int side_slices(int K) { return K % 256 == 0 ? 4 : K % 128 == 0 ? 2 : 1; }
 Buffers carve(const Lm& lm, Arena& ar, const Step& sp) {
     const size_t es = lm.esz();
     const int M = sp.M, Wp = lm.Wp;
-    const bool decode = sp.decode, sliced = decode && !lm.f32 && M <= 64;
+    const bool decode = sp.decode, sliced = decode && M <= 64;
     size_t Na = 0, Qp = 0, Rp = 0, Gp = 0, qn = 0, kvn = 0, hr = 0, Ep = 0, top = 0, act = 0, tiles = 0, part = 0, sl = 0, kvh = 0, r32 = 0, r16 = 0, raw = 0, snap = 0;
-    auto slices = [&](int N, int K) { if (sliced) sl = std::max(sl, (size_t)M * std::max(1, gemm_partial_splits(N, K)) * N); };
+    auto slices = [&](int N, int K) { if (sliced) sl = std::max(sl, (size_t)M * std::max(1, lm.f32 ? lm_rows_slices(N, K) : gemm_partial_splits(N, K)) * N); };
     for (const LmLayer& L : lm.layers) {
         Na = std::max<size_t>(Na, L.Na); Gp = std::max<size_t>(Gp, L.Gp);
         slices(L.Na, Wp); slices(Wp, L.Gp);
@@ -347,7 +352,7 @@ int dense(cr_ctx* c, const Lm& lm, const void* A, int64_t lda, const void* W, vo
           bool relu2 = false) {
     if (lm.f32) {
         LmGemmParams p{};
-        p.A = A; p.lda = lda; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K;
+        p.A = A; p.lda = lda; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.stream = !prompt && M <= LM_ROWS_MAX;
         return launch_lm_gemm(true, relu2 ? LM_RELU2 : LM_STORE, p, st);
     }
     GemmParams p{};
@@ -356,8 +361,8 @@ int dense(cr_ctx* c, const Lm& lm, const void* A, int64_t lda, const void* W, vo
     if (!prompt && M <= 64 && dl) { p.W = dl; p.wsw = 1; }
     return ctx_gemm(c, relu2 ? EPI_RELU2 : EPI_STORE, p, st);
 }
-// the same product left in fp32 (router scores, logits, the looped span's entry)
-int raw32(cr_ctx* c, const Lm& lm, const void* A, const void* W, float* C, int64_t ldc, int M, int N, int K, float softcap, hipStream_t st, const bf16* dl = nullptr) {
+// the same product left in fp32 (router scores, logits, the looped span's entry); few: rows that fp32 streams the weights for (decode steps, logits)
+int raw32(cr_ctx* c, const Lm& lm, const void* A, const void* W, float* C, int64_t ldc, int M, int N, int K, float softcap, hipStream_t st, bool few, const bf16* dl = nullptr) {
     if (!lm.f32) {
         GemmParams p{};
         p.A = (const bf16*)A; p.lda = K; p.W = (const bf16*)W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.raw32 = 1; p.softcap = softcap;
@@ -365,7 +370,7 @@ int raw32(cr_ctx* c, const Lm& lm, const void* A, const void* W, float* C, int64
         return ctx_gemm(c, EPI_F32, p, st);
     }
     LmGemmParams p{};
-    p.A = A; p.lda = K; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.softcap = softcap;
+    p.A = A; p.lda = K; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.softcap = softcap; p.stream = few && M <= LM_ROWS_MAX;
     return launch_lm_gemm(lm.f32, LM_RAW32, p, st);
 }
 
@@ -380,7 +385,7 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
     if (s_a) CR_TRY(sliced(c, b.h, Wp, L.wa, L.wa_dl, b.sl, M, L.Na, Wp, st));
     else CR_TRY(dense(c, lm, b.h, Wp, L.wa, b.a, L.Na, M, L.Na, Wp, st, !sp.decode, L.wa_dl));
     CR_TRY(launch_lm_latents(lm.f32, lm, L, M, b.a, s_a ? b.sl : nullptr, s_a, b.cq, sp.decode ? nullptr : b.c, cache, kv->max_tokens, sp.ix, b.ao, st));
-    const int s_q = L.Ap <= 512 ? slices_of(lm, M, H * L.Ap, L.Qp, sp.decode) : 0;
+    const int s_q = !lm.f32 && L.Ap <= 512 ? slices_of(lm, M, H * L.Ap, L.Qp, sp.decode) : 0;
     if (s_q) CR_TRY(sliced(c, b.cq, L.Qp, L.wuq, L.wuq_dl, b.sl, M, H * L.Ap, L.Qp, st));
     else CR_TRY(dense(c, lm, b.cq, L.Qp, L.wuq, b.q, (int64_t)H * L.Ap, M, H * L.Ap, L.Qp, st, !sp.decode, L.wuq_dl));
     const void* gate = (const char*)b.a + (size_t)L.off_g * es;
@@ -400,7 +405,7 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
     } else {
         LmGemmParams g{};
         g.A = b.q; g.lda = (int64_t)H * L.Ap; g.W = L.wukT; g.ldw = L.Ap; g.C = b.qp; g.ldc = (int64_t)H * L.Rp; g.M = M; g.N = L.Rp; g.K = L.Ap;
-        g.batch = H; g.a_bs = L.Ap; g.w_bs = (int64_t)L.Rp * L.Ap; g.c_bs = L.Rp;
+        g.batch = H; g.a_bs = L.Ap; g.w_bs = (int64_t)L.Rp * L.Ap; g.c_bs = L.Rp; g.stream = lm.f32 && sp.decode && M <= LM_ROWS_MAX;
         if (s_q) CR_TRY(launch_latent_absorb(L, M, b.sl, s_q, b.qp, st));
         else CR_TRY(launch_lm_gemm(lm.f32, LM_STORE, g, st));
         LatentAttnParams ap{};
@@ -415,6 +420,7 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
         g = LmGemmParams{};
         g.A = b.ol; g.lda = (int64_t)H * L.Rp; g.W = (const char*)L.wkv + (size_t)H * L.Ap * L.Rp * es; g.ldw = L.Rp; g.C = b.ao; g.ldc = L.Gp; g.M = M; g.N = s.vdim; g.K = L.Rp;
         g.batch = H; g.a_bs = L.Rp; g.w_bs = (int64_t)L.Ap * L.Rp; g.c_bs = s.vdim; g.gate = gate; g.ldg = L.Na; g.g_bs = s.vdim;
+        g.stream = lm.f32 && sp.decode && M <= LM_ROWS_MAX;
         CR_TRY(launch_lm_gemm(lm.f32, LM_GATE, g, st));
         }
     }
@@ -489,7 +495,7 @@ int expert_mixture(cr_ctx* c, const Step& sp, Buffers& b, const LmLayer& L, hipS
     const int M = sp.M, Wp = lm.Wp;
     if (!lm.f32 && lm_router_supported(L)) CR_TRY(launch_lm_router(lm, L, M, b.h, b.idx, b.wt, b.z, st));
     else {
-        CR_TRY(raw32(c, lm, b.h, L.router, b.z, L.Ep, M, s.experts, Wp, 0.f, st));
+        CR_TRY(raw32(c, lm, b.h, L.router, b.z, L.Ep, M, s.experts, Wp, 0.f, st, sp.decode));
         CR_TRY(launch_lm_route(L, M, b.z, L.Ep, 1, b.idx, b.wt, st));
     }
     if (!lm.f32) {
@@ -513,6 +519,7 @@ int expert_mixture(cr_ctx* c, const Step& sp, Buffers& b, const LmLayer& L, hipS
     LmGemmParams g{};
     g.A = b.h; g.lda = Wp; g.W = L.wgu; g.ldw = Wp; g.w_bs = (int64_t)2 * L.ffp * Wp; g.C = b.act; g.ldc = L.ffp; g.N = 2 * L.ffp; g.K = Wp;
     g.tiles = b.tiles; g.n_tiles = b.n_tiles; g.max_tiles = lm_max_tiles(M * s.top, s.experts, LM_TILE_M); g.perm = b.perm; g.gather_div = s.top; g.limit = s.limit;
+    g.M = M; g.stream = sp.decode && M <= LM_ROWS_MAX;                      // (a row chooses an expert once: at most M rows each)
     CR_TRY(launch_lm_gemm(lm.f32, LM_GLU, g, st));
     g.A = b.act; g.lda = L.ffp; g.W = L.wdn; g.ldw = L.ffp; g.w_bs = (int64_t)Wp * L.ffp; g.C = b.ye; g.ldc = Wp; g.N = Wp; g.K = L.ffp; g.gather_div = 0; g.scatter = 1;
     CR_TRY(launch_lm_gemm(lm.f32, LM_STORE, g, st));
@@ -554,7 +561,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
                 CR_TRY(sliced(c, b.cat, 2 * Wp, lm.loop_in, lm.loop_dl, b.sl, M, Wp, 2 * Wp, st));
                 CR_TRY(launch_lm_post(lm.f32, lm, M, LmPostIn{b.sl, Wp, n, nullptr, 0}, b.x, nullptr, true, to, st));
             } else {
-                CR_TRY(raw32(c, lm, b.cat, lm.loop_in, b.x, Wp, M, Wp, 2 * Wp, 0.f, st, sp.decode ? lm.loop_dl : nullptr));
+                CR_TRY(raw32(c, lm, b.cat, lm.loop_in, b.x, Wp, M, Wp, 2 * Wp, 0.f, st, sp.decode, sp.decode ? lm.loop_dl : nullptr));
                 CR_TRY(launch_lm_pick_rows(lm.f32, lm, M, b.x, nullptr, b.h, L.n1, st));
             }
         }
@@ -576,7 +583,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
             bool projected = false;
             if (lm.f32) {
                 LmGemmParams g{};
-                g.A = b.h; g.lda = Wp; g.W = L.sgate; g.ldw = Wp; g.C = b.z2; g.ldc = lm.Sp; g.M = M; g.N = lm.Sp; g.K = Wp; g.gate = side; g.ldg = lds; g.tok = b.tok;
+                g.A = b.h; g.lda = Wp; g.W = L.sgate; g.ldw = Wp; g.C = b.z2; g.ldc = lm.Sp; g.M = M; g.N = lm.Sp; g.K = Wp; g.gate = side; g.ldg = lds; g.tok = b.tok; g.stream = sp.decode && M <= LM_ROWS_MAX;
                 CR_TRY(launch_lm_gemm(true, LM_SIDE, g, st));
             } else {
                 // few columns: K-slices keep the chip busy, and the kernel that adds them applies the activation and the token's row
@@ -605,7 +612,7 @@ int lm_head(cr_ctx* c, const Lm& lm, const float* x, const int32_t* rows, int n,
     for (int i = 0; i < n; i += piece) {
         const int m = std::min(piece, n - i);
         CR_TRY(launch_lm_pick_rows(lm.f32, lm, m, x, rows + i, hl, lm.fin, st));
-        CR_TRY(raw32(c, lm, hl, lm.head, out + (size_t)i * lm.d.vocab, lm.d.vocab, m, lm.d.vocab, lm.Wp, lm.d.softcap, st));
+        CR_TRY(raw32(c, lm, hl, lm.head, out + (size_t)i * lm.d.vocab, lm.d.vocab, m, lm.d.vocab, lm.Wp, lm.d.softcap, st, true));
     }
     return CR_OK;
 }
@@ -698,7 +705,7 @@ int lm_decode_step(cr_ctx* c, cr_kv* kv, int n, const int64_t* force_tokens, flo
     void* hl = ar.take<char>((size_t)n * lm.Wp * lm.esz());
     float* lg = ar.take<float>((size_t)n * lm.d.vocab);
     CR_TRY(run_passes(c, kv, sp, b, hl, st));
-    CR_TRY(raw32(c, lm, hl, lm.head, lg, lm.d.vocab, n, lm.d.vocab, lm.Wp, lm.d.softcap, st, lm.head_dl));
+    CR_TRY(raw32(c, lm, hl, lm.head, lg, lm.d.vocab, n, lm.d.vocab, lm.Wp, lm.d.softcap, st, true, lm.head_dl));
     if (logits) CR_HIP(hipMemcpyAsync(logits, lg, (size_t)n * lm.d.vocab * 4, hipMemcpyDeviceToDevice, st));
     return launch_pick(lg, lm.d.vocab, lm.d.vocab, penalty, n, kv->d_seqs, kv, 1, st);
 }

@@ -4,6 +4,7 @@
 // Row kernel: a wave holds 512 columns, eight per lane.  A head's padded size is a power of two (64 .. 512) and regions are laid out widest first, so a head is a run of lanes of
 // one wave: its norm is a lane reduction, its rotation partner (half a rotation away, at any distance) comes through 2 KiB of the wave's own LDS.  Angles are fp32 and are
 // computed once per row.
+#include "attention_plain.hpp"
 #include "lm.hpp"
 
 namespace {
@@ -165,58 +166,25 @@ __global__ __launch_bounds__(256) void lm_prefix_kernel(const int32_t* __restric
     }
 }
 
-template <typename T>
-__global__ __launch_bounds__(256) void heads_attn_plain_kernel(const HeadsAttnParams p) {
-    __shared__ float q[LM_MAX_HEAD], w[256], red[8];
-    const int row = blockIdx.x, head = blockIdx.y, tid = threadIdx.x;
+template <typename T, int TPB>
+__global__ __launch_bounds__(TPB) void heads_attn_plain_kernel(const HeadsAttnParams p) {
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    __shared__ float red[2 * TPB / 64];
+    const int row = blockIdx.x, head = blockIdx.y;
     const int g = head / (p.H / p.G);
     const int seq = p.ix.row_seq ? p.ix.row_seq[row] : p.ix.seqs[row];
     const int n = (p.ix.row_pos ? p.ix.row_pos[row] : p.ix.lens[seq]) % p.chunk + 1;
     const int64_t base = p.row_key ? (int64_t)(p.row_key[row] - n + 1) * p.k_rs + g * p.k_hs : ((int64_t)seq * p.G + g) * p.ring * p.Ap;
-    const T *Q = (const T*)p.Q + ((int64_t)row * p.H + head) * p.Ap, *K = (const T*)p.K + base, *V = (const T*)p.V + base;
-    for (int i = tid; i < p.Ap; i += 256) q[i] = (float)Q[i];
-    float acc[LM_MAX_HEAD / 256] = {0.f, 0.f};
-    float m_run = -INFINITY, l_run = 0.f;
-    for (int k0 = 0; k0 < n; k0 += 256) {
-        __syncthreads();
-        const int key = k0 + tid;
-        float s = -INFINITY;
-        if (key < n) {
-            const T* c = K + (int64_t)key * p.k_rs;
-            float d0 = 0.f, d1 = 0.f, d2 = 0.f, d3 = 0.f;
-            for (int i = 0; i < p.Ap; i += 4) { d0 += q[i] * (float)c[i]; d1 += q[i + 1] * (float)c[i + 1]; d2 += q[i + 2] * (float)c[i + 2]; d3 += q[i + 3] * (float)c[i + 3]; }
-            s = ((d0 + d1) + (d2 + d3)) * p.scale;
-            if (p.softcap > 0.f) s = p.softcap * tanhf(s / p.softcap);
-        }
-        const float mx = wave_max(s);
-        if ((tid & 63) == 0) red[tid >> 6] = mx;
-        __syncthreads();
-        const float m_new = fmaxf(m_run, fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3])));
-        const float e = key < n ? expf(s - m_new) : 0.f;
-        w[tid] = e;
-        const float sum = wave_sum(e);
-        if ((tid & 63) == 0) red[4 + (tid >> 6)] = sum;
-        __syncthreads();
-        const float alpha = expf(m_run - m_new);
-        l_run = l_run * alpha + (red[4] + red[5] + red[6] + red[7]);
-        m_run = m_new;
-        const int nk = min(256, n - k0);
-#pragma unroll
-        for (int j = 0; j < LM_MAX_HEAD / 256; j++) {
-            const int i = tid + 256 * j;
-            if (i >= p.vdim) break;
-            float a = acc[j] * alpha;
-            const T* c = V + (int64_t)k0 * p.k_rs + i;
-            for (int k = 0; k < nk; k++) a += w[k] * (float)c[(int64_t)k * p.k_rs];
-            acc[j] = a;
-        }
-    }
     T* O = (T*)p.O + (int64_t)row * p.ldo + (int64_t)head * p.vdim;
-#pragma unroll
-    for (int j = 0; j < LM_MAX_HEAD / 256; j++) {
-        const int i = tid + 256 * j;
-        if (i < p.vdim) O[i] = (T)(acc[j] * (p.out_scale / l_run));
-    }
+    plain_attend<T, TPB>((const T*)p.Q + ((int64_t)row * p.H + head) * p.Ap, (const T*)p.K + base, p.k_rs, (const T*)p.V + base, p.k_rs, n, p.Ap, p.vdim, p.scale, p.softcap, sm, red,
+                         [&](int i, float v) { O[i] = (T)(v * p.out_scale); });
+}
+
+template <typename T>
+void launch_plain_t(const HeadsAttnParams& p, hipStream_t st) {
+    // few workgroups: sixteen waves each (a row's chain of loads is what counts); many: four, and the chip is full
+    if ((int64_t)p.M * p.H <= 1024) hipLaunchKernelGGL((heads_attn_plain_kernel<T, 1024>), dim3(p.M, p.H), dim3(1024), plain_lds_floats(p.Ap, 1024) * 4, st, p);
+    else hipLaunchKernelGGL((heads_attn_plain_kernel<T, 256>), dim3(p.M, p.H), dim3(256), plain_lds_floats(p.Ap, 256) * 4, st, p);
 }
 
 }  // namespace
@@ -252,8 +220,8 @@ int launch_lm_prefix(bool f32, const LmLayer& L, int n, const int32_t* key_rows,
 int launch_heads_attn_plain(bool f32, const HeadsAttnParams& p, hipStream_t st) {
     if (p.M <= 0 || p.H <= 0 || p.G <= 0 || p.H % p.G || p.Ap <= 0 || p.Ap > LM_MAX_HEAD || p.vdim > p.Ap || p.chunk <= 0)
         return cr_fail(CR_ERR_ARG, "attention over heads: rows %d, heads %d / %d, size %d / %d", p.M, p.H, p.G, p.Ap, p.vdim);
-    if (f32) hipLaunchKernelGGL(heads_attn_plain_kernel<float>, dim3(p.M, p.H), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(heads_attn_plain_kernel<bf16>, dim3(p.M, p.H), dim3(256), 0, st, p);
+    if (f32) launch_plain_t<float>(p, st);
+    else launch_plain_t<bf16>(p, st);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }
