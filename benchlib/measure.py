@@ -105,10 +105,8 @@ def measure_traffic(pages=16):
             vals = []
             for row in csv.DictReader(open(files[0])):
                 k = row['Kernel_Name']
-                if row['Counter_Name'] != counter or not ('gemm256_kernel' in k or 'gemm128_kernel' in k):
+                if row['Counter_Name'] != counter or 'gemm256_kernel' not in k:      # (gemm_mid_kernel's launches here are nearly all of M < 1024: not in the roofline class)
                     continue
-                if 'gemm128' in k and int(row['Grid_Size']) < 8 * 8 * 256:
-                    continue                                  # M < 1024: not in the roofline class
                 vals.append(float(row['Counter_Value']))
             if not vals:
                 return None, f'no tiled-GEMM rows in the {counter} pass'

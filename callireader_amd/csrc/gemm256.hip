@@ -62,7 +62,7 @@
 // (K = 8192 lowest), so the matrix peak actually on offer is ~1.9-2.0 PFLOP/s, not the 2.5 of the 2.4 GHz figure.
 #include <stdlib.h>
 
-#include "gemm_epilogue.hpp"
+#include "common.hpp"
 #include "diag.hpp"
 
 namespace {
@@ -855,16 +855,12 @@ int launch_t(const GemmParams& p, hipStream_t stream) {
 
 }  // namespace
 
-bool gemm256_supported(int epi, const GemmParams& p) {
-    if (p.M < 2048 || p.N < 512 || (p.K % 128) != 0 || p.raw32) return false;
-    // wave-quantisation model (calibrated on the measured shapes): a round of 256x256 tiles on
-    // 256 CUs costs 1; a round of 512 co-resident 128x128 tiles covers half the output at ~0.65 of this kernel's rate
-    // (ViT shapes: 0.50-0.82 vs 0.78-1.23 PFLOP/s), i.e. 0.75; pick the kernel with the cheaper schedule
-    const long t256 = (long)((p.M + 255) / 256) * ((p.N + 255) / 256);
-    const long t128 = (long)((p.M + 127) / 128) * ((p.N + 127) / 128);
-    const double c256 = (double)((t256 + 255) / 256);
-    const double c128 = 0.75 * (double)((t128 + 511) / 512);
-    return c256 <= c128;
+bool gemm256_supported(int epi, const GemmParams& p) { return epi != EPI_PARTIAL && p.N >= 64 && p.K % 128 == 0 && !p.raw32; }
+
+// us of a launch, on the scale of gemm_mid_cost: rounds of one tile per CU, a K-tile 1.15 us of operand bytes (512 rows; 700 x 4096 x 14336 takes 244 us, 8200 x 1024 x 4096 75)
+double gemm256_cost(int epi, const GemmParams& p) {
+    const long tiles = (long)((p.M + BM2 - 1) / BM2) * ((p.N + BN2 - 1) / BN2), cus = cr_device_cus();
+    return 3.5 + (double)((tiles + cus - 1) / cus) * (p.K / BK2 * 1.12 + 3.0);
 }
 
 int launch_gemm256_grouped(int epi, const GemmParams& p, hipStream_t stream) {

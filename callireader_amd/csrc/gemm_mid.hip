@@ -1,0 +1,420 @@
+// bf16 MFMA GEMM for the row counts between decode (gemm_skinny.hip) and the persistent 256x256 kernel (gemm256.hip):  C = epi(A[M,K] . W[N,K]^T),  K % 64 == 0.
+//
+// What bounds these shapes is not arithmetic but how many bytes are under way: a 128x128 grid over M = 1025, N = 1024 is 72 workgroups, and a K loop that waits for each K-tile's
+// loads before it asks for the next-but-one pays a memory round trip per 64 of K.  So (a) the tile shape is a template and picked by the grid it gives (mid_pick below), down to
+// 16 x 16 for a single wave, and (b) NBUF K-tiles live in LDS and NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles.
+//   * one global_load_lds_dwordx4 brings eight rows x 64 k, whole 128-byte lines (pieces of 16 rows x 32 k reach 56 of the 69 GB/s per CU that these do on cold weights);
+//     LDS rows of 128 bytes, the 16-byte chunk XORed with (row >> 1) & 7 on both sides: a fragment's ds_read_b128 is free of bank conflicts;
+//   * step t: wait until K-tile t + 1 has landed (this wave's pieces), barrier (everybody's have, and everybody holds tile t in registers), ask for tile t + NBUF into the buffer
+//     tile t leaves, read the fragments of t + 1, multiply t: the LDS reads' latency runs under the MFMAs;
+//   * the weights are the MFMA's A operand: a lane's accumulator holds four consecutive columns of one row, and the epilogue works there, without a stage in LDS;
+//   * a row tile's fragments past M are neither read nor multiplied (M = 1025: the last row costs a sixteenth of a tile, not a tile);
+//   * a row's sum runs over K in ascending 32-steps of the same MFMA as in gemm256, whatever the tile: the same bits from every kernel and every shape here.
+#include <algorithm>
+#include <type_traits>
+
+#include "common.hpp"
+
+namespace {
+
+template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// ... with `behind` <= R K-tiles of PER instructions left under way
+template <int R, int PER> __device__ __forceinline__ void wait_tail(int behind) {
+    if (behind >= R) wait_vm<R * PER>();
+    else if constexpr (R > 0) wait_tail<R - 1, PER>(behind);
+}
+
+// ---- epilogue of four consecutive columns gn .. gn + 3 (gn % 4 == 0) of row gm: the reference's bf16 rounding sequence ----
+template <int EPI>
+__device__ __forceinline__ void put1(const GemmParams& p, int gm, int gn, float v) {
+    const float sum = v + (p.bias ? bf2f(p.bias[gn]) : 0.0f);
+    if (EPI == EPI_F32) { ((float*)p.C)[(int64_t)gm * p.ldc + gn] = f32_out(p, sum); return; }
+    float x = EPI == EPI_RELU2 ? relu2(sum) : EPI == EPI_STORE ? sum : rbf(sum);
+    int64_t orow = gm;
+    if (EPI == EPI_GELU) x = gelu_erf(x);
+    else if (EPI == EPI_LS_RES) x = bf2f(p.res[(int64_t)gm * p.ldr + gn]) + rbf(x * bf2f(p.scale[gn]));
+    else if (EPI == EPI_RES) x = bf2f(p.res[(int64_t)gm * p.ldr + gn]) + x;
+    else if (EPI == EPI_PATCH) {
+        const int t = gm / p.group, pi = gm - t * p.group;
+        orow = (int64_t)t * (p.group + 1) + 1 + pi;
+        x = x + bf2f(p.res[(int64_t)(1 + pi) * p.ldr + gn]);
+    }
+    ((bf16*)p.C)[orow * p.ldc + gn] = f2bf(x);
+}
+template <int EPI>
+__device__ __forceinline__ void put4(const GemmParams& p, int gm, int gn, f32x4 v) {
+    constexpr bool ROUND = EPI != EPI_STORE && EPI != EPI_F32 && EPI != EPI_RELU2;
+    float x[4];
+#pragma unroll
+    for (int e = 0; e < 4; e++) x[e] = v[e];
+    if (p.bias) {
+        const bf16x4 b = *(const bf16x4*)(p.bias + gn);
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] += bf2f(b[e]);
+    }
+    if (EPI == EPI_F32) {
+        *(f32x4*)((float*)p.C + (int64_t)gm * p.ldc + gn) = f32x4{f32_out(p, x[0]), f32_out(p, x[1]), f32_out(p, x[2]), f32_out(p, x[3])};
+        return;
+    }
+    if (ROUND) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = rbf(x[e]);
+    }
+    int64_t orow = gm;
+    if (EPI == EPI_RELU2) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = relu2(x[e]);
+    } else if (EPI == EPI_GELU) {
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = gelu_erf(x[e]);
+    } else if (EPI == EPI_LS_RES) {
+        const bf16x4 s = *(const bf16x4*)(p.scale + gn), r = *(const bf16x4*)(p.res + (int64_t)gm * p.ldr + gn);
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = bf2f(r[e]) + rbf(x[e] * bf2f(s[e]));
+    } else if (EPI == EPI_RES) {
+        const bf16x4 r = *(const bf16x4*)(p.res + (int64_t)gm * p.ldr + gn);
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = bf2f(r[e]) + x[e];
+    } else if (EPI == EPI_PATCH) {
+        const int t = gm / p.group, pi = gm - t * p.group;
+        orow = (int64_t)t * (p.group + 1) + 1 + pi;
+        const bf16x4 r = *(const bf16x4*)(p.res + (int64_t)(1 + pi) * p.ldr + gn);
+#pragma unroll
+        for (int e = 0; e < 4; e++) x[e] = x[e] + bf2f(r[e]);
+    }
+    *(bf16x4*)((bf16*)p.C + orow * p.ldc + gn) = bf16x4{f2bf(x[0]), f2bf(x[1]), f2bf(x[2]), f2bf(x[3])};
+}
+
+// what a column can do by itself, in the accumulator layout: the linear output with its bias, then GELU / LayerScale / squared relu, each on its rounded input
+template <int EPI>
+__device__ __forceinline__ bf16x4 by_column(f32x4 v, const float (&bias)[4], const float (&scale)[4]) {
+    bf16x4 o;
+#pragma unroll
+    for (int e = 0; e < 4; e++) {
+        float x = v[e] + bias[e];                             // -0.0f where there is no bias: x + -0 = x, bit for bit
+        if (EPI == EPI_RELU2) x = relu2(x);
+        if (EPI == EPI_GELU) x = gelu_erf(rbf(x));
+        if (EPI == EPI_LS_RES) x = rbf(x) * scale[e];
+        o[e] = f2bf(x);
+    }
+    return o;
+}
+
+// bf16 results of a wave's columns, all inside the matrix: 16 rows at a time through 16 x (FN * 16) of the wave's own LDS, so that memory is read and written in whole 16-byte chunks of
+// a row by neighbouring lanes (straight from the accumulators every lane writes eight bytes of a row of its own: 5 us a launch more on 128 x 256 tiles).  Rows of FN * 32 + 16 bytes:
+// sixteen rows start at sixteen different bank groups.
+template <int EPI, int FM, int FN>
+__device__ __forceinline__ void epilogue_staged(const GemmParams& p, const f32x4 (&acc)[FM][FN], char* stg, int row0, int live, int col0, int lane) {
+    constexpr int LD = FN * 32 + 16, CPR = EPI == EPI_SWIGLU ? FN : 2 * FN, RPP = 64 / CPR < 16 ? 64 / CPR : 16;      // bytes a row, chunks of a row that leave, rows a pass
+    float bias[FN][4], scale[FN][4];
+#pragma unroll
+    for (int j = 0; j < FN; j++) {
+        const int gn = col0 + j * 16 + 4 * (lane >> 4);
+#pragma unroll
+        for (int e = 0; e < 4; e++) {
+            bias[j][e] = p.bias ? bf2f(p.bias[gn + e]) : -0.0f;
+            scale[j][e] = EPI == EPI_LS_RES ? bf2f(p.scale[gn + e]) : 1.f;
+        }
+    }
+    const int rin = lane / CPR, c = lane % CPR;
+#pragma unroll
+    for (int i = 0; i < FM; i++) {
+        if (i >= live) break;
+        char* buf = stg + (i & 1) * 16 * LD;
+#pragma unroll
+        for (int j = 0; j < FN; j++) *(bf16x4*)(buf + (lane & 15) * LD + j * 32 + (lane >> 4) * 8) = by_column<EPI>(acc[i][j], bias[j], scale[j]);
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+#pragma unroll
+        for (int r0 = 0; r0 < 16; r0 += RPP) {
+            const int row = r0 + rin, gm = row0 + i * 16 + row;
+            if (rin >= RPP || gm >= p.M) continue;
+            if (EPI == EPI_SWIGLU) {                          // [8 gate | 8 up]
+                const bf16x8 g = *(const bf16x8*)(buf + row * LD + c * 32), u = *(const bf16x8*)(buf + row * LD + c * 32 + 16);
+                bf16x8 o;
+#pragma unroll
+                for (int e = 0; e < 8; e++) o[e] = f2bf(rbf(silu(bf2f(g[e]))) * bf2f(u[e]));
+                *(bf16x8*)((bf16*)p.C + (int64_t)gm * p.ldc + col0 / 2 + c * 8) = o;
+                continue;
+            }
+            bf16x8 v = *(const bf16x8*)(buf + row * LD + c * 16);
+            int64_t orow = gm, rrow = gm;
+            if (EPI == EPI_PATCH) {
+                const int t = gm / p.group, pi = gm - t * p.group;
+                orow = (int64_t)t * (p.group + 1) + 1 + pi;
+                rrow = 1 + pi;
+            }
+            if (EPI == EPI_LS_RES || EPI == EPI_RES || EPI == EPI_PATCH) {
+                const bf16x8 r = *(const bf16x8*)(p.res + rrow * p.ldr + col0 + c * 8);
+#pragma unroll
+                for (int e = 0; e < 8; e++) v[e] = f2bf(bf2f(r[e]) + bf2f(v[e]));
+            }
+            *(bf16x8*)((bf16*)p.C + orow * p.ldc + col0 + c * 8) = v;
+        }
+    }
+}
+
+template <int EPI, int FM, int FN>
+__device__ __forceinline__ void epilogue(const GemmParams& p, const f32x4 (&acc)[FM][FN], char* stg, int row0, int live, int col0, int lane) {
+    if constexpr (EPI != EPI_F32 && EPI != EPI_ARGMAX) {
+        constexpr bool ROWS = EPI == EPI_LS_RES || EPI == EPI_RES || EPI == EPI_PATCH;
+        if (col0 + FN * 16 <= p.N && (p.ldc & 7) == 0 && (!ROWS || ((p.ldr & 7) == 0 && ((uintptr_t)p.res & 15) == 0))) {      // (wave-uniform; C is 16-byte aligned)
+            epilogue_staged<EPI, FM, FN>(p, acc, stg, row0, live, col0, lane);
+            return;
+        }
+    }
+    const bool vec = (p.ldc & 3) == 0;
+#pragma unroll
+    for (int i = 0; i < FM; i++) {
+        if (i >= live) break;
+        const int gm = row0 + i * 16 + (lane & 15);
+        if (EPI == EPI_ARGMAX) {                              // the wave's 64 columns: one partial per row
+            float bv = -INFINITY; int bc = 0x7fffffff;
+#pragma unroll
+            for (int j = 0; j < FN; j++)
+#pragma unroll
+                for (int e = 0; e < 4; e++) {
+                    const int n = col0 + j * 16 + 4 * (lane >> 4) + e;
+                    float v = rbf(acc[i][j][e] + (p.bias && n < p.N ? bf2f(p.bias[n]) : 0.f));
+                    v = n < p.N ? v : -INFINITY;
+                    if (v > bv) { bv = v; bc = n; }              // ascending columns inside a lane: strict > keeps the first
+                }
+#pragma unroll
+            for (int o = 16; o <= 32; o <<= 1) argmax_merge(bv, bc, __shfl_xor(bv, o, 64), __shfl_xor(bc, o, 64));
+            if (lane < 16 && gm < p.M && col0 < p.N) ((unsigned long long*)p.C)[(int64_t)gm * p.ldc + (col0 >> 6)] = argmax_pack(bv, bc);
+            continue;
+        }
+#pragma unroll
+        for (int j = 0; j < FN; j++) {
+            const int gn = col0 + j * 16 + 4 * (lane >> 4);
+            if (EPI == EPI_SWIGLU) {                          // a fragment's columns are [8 gate | 8 up]: the partner sits 32 lanes away
+                f32x4 u;
+#pragma unroll
+                for (int e = 0; e < 4; e++) u[e] = __shfl_xor(acc[i][j][e], 32, 64);
+                if (lane >= 32 || gm >= p.M || gn >= p.N) continue;
+                bf16x4 o;
+#pragma unroll
+                for (int e = 0; e < 4; e++) o[e] = f2bf(rbf(silu(rbf(acc[i][j][e]))) * rbf(u[e]));
+                bf16* c = (bf16*)p.C + (int64_t)gm * p.ldc + (col0 + j * 16) / 2 + 4 * (lane >> 4);
+                if (vec) *(bf16x4*)c = o;
+                else {
+#pragma unroll
+                    for (int e = 0; e < 4; e++) c[e] = o[e];
+                }
+                continue;
+            }
+            if (gm >= p.M || gn >= p.N) continue;
+            if (vec && gn + 4 <= p.N) put4<EPI>(p, gm, gn, acc[i][j]);
+            else
+                for (int e = 0; e < 4 && gn + e < p.N; e++) put1<EPI>(p, gm, gn + e, acc[i][j][e]);
+        }
+    }
+}
+
+// WM x WN waves of FM x FN fragments of 16 x 16
+template <int WM, int WN, int FM, int FN, int NBUF>
+struct MidGeom {
+    static constexpr int BM = WM * FM * 16, BN = WN * FN * 16, WAVES = WM * WN, PIECES = (BM + BN) / 8, PER = (PIECES + WAVES - 1) / WAVES, STAGE = PIECES * 1024, LDS = NBUF * STAGE;
+    static_assert(WAVES * 32 * (FN * 32 + 16) <= LDS, "the epilogue's stage lies in the buffers");
+    static_assert((NBUF - 2) * PER <= 63 && NBUF >= 2 && LDS <= 160 * 1024, "vmcnt is six bits wide; a CU has 160 KiB");
+};
+
+template <int WM, int WN, int FM, int FN, int NBUF>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams p, const int epi, const int ntm) {
+    typedef MidGeom<WM, WN, FM, FN, NBUF> G;
+    extern __shared__ __attribute__((aligned(16))) char smem[];
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int wm = wave / WN, wn = wave % WN;
+
+    // ---- workgroup -> tile: bijective XCD remap (an XCD's L2 gets a contiguous run of tiles), then super-groups of 8 row tiles ----
+    const int ntn = (p.N + G::BN - 1) / G::BN;
+    const int nwg = gridDim.x, orig = blockIdx.x;
+    const int nk = p.K / 64 / (int)gridDim.y;                 // K-tiles of this slice (EPI_PARTIAL: gridDim.y of them; one otherwise)
+    const int xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
+    const int pid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
+    constexpr int GM = 8;
+    const int per_group = GM * ntn, grp = pid / per_group, first_m = grp * GM, gsz = min(ntm - first_m, GM), in_g = pid - grp * per_group;
+    const int tile_m = first_m + in_g % gsz, n0 = in_g / gsz * G::BN;
+    // ---- the matrix's fragments of 16 rows dealt evenly over the row tiles (at most WM * FM each), a tile's over its wave rows ----
+    const int nf = (p.M + 15) >> 4, f0 = (int)((int64_t)tile_m * nf / ntm), fn = (int)((int64_t)(tile_m + 1) * nf / ntm) - f0;
+    const int m0 = f0 * 16, wf0 = fn * wm / WM, live = fn * (wm + 1) / WM - wf0;
+
+    // ---- this wave's pieces of a K-tile: eight rows of A or W, all 64 k (128 bytes a row); numbers past the last repeat it ----
+    // (pieces of rows past the tile's move one lane's 16 bytes: the count of instructions under way stays a constant)
+    const bf16* src[G::PER];
+    int dst[G::PER];
+    bool dead[G::PER];
+#pragma unroll
+    for (int i = 0; i < G::PER; i++) {
+        const int piece = min(wave + i * G::WAVES, G::PIECES - 1), row = piece * 8 + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
+        const bf16* at = piece * 8 < G::BM ? p.A + (int64_t)min(m0 + row, p.M - 1) * p.lda : p.W + (int64_t)min(n0 + row - G::BM, p.N - 1) * p.ldw;
+        src[i] = at + chunk * 8 + (int64_t)blockIdx.y * nk * 64;
+        dst[i] = piece * 1024;
+        dead[i] = piece * 8 < G::BM && piece >= 2 * fn;
+    }
+    auto ask = [&](int kt, int buf) {
+#pragma unroll
+        for (int i = 0; i < G::PER; i++)
+            if (!dead[i] || lane == 0) __builtin_amdgcn_global_load_lds(CR_GLB(src[i] + (int64_t)kt * 64), CR_LDS(smem + buf * G::STAGE + dst[i]), 16, 0, 0);
+    };
+
+    f32x4 acc[FM][FN];
+#pragma unroll
+    for (int i = 0; i < FM; i++)
+#pragma unroll
+        for (int j = 0; j < FN; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int swz = (lane >> 1) & 7;
+    const int c_off[2] = {((lane >> 4) ^ swz) * 16, ((4 + (lane >> 4)) ^ swz) * 16};
+    const int a_off = (wf0 * 16 + (lane & 15)) * 128, w_off = (G::BM + wn * FN * 16 + (lane & 15)) * 128;
+
+    struct Frags { bf16x8 a[2][FM], w[2][FN]; };
+    auto read = [&](Frags& f, int buf, auto count) {
+        const char* s = smem + buf * G::STAGE;
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+#pragma unroll
+            for (int j = 0; j < FN; j++) f.w[h][j] = *(const bf16x8*)(s + w_off + j * 2048 + c_off[h]);
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+                if (i < decltype(count)::value) f.a[h][i] = *(const bf16x8*)(s + a_off + i * 2048 + c_off[h]);
+        }
+    };
+    auto multiply = [&](const Frags& f, auto count) {
+#pragma unroll
+        for (int h = 0; h < 2; h++)
+#pragma unroll
+            for (int i = 0; i < FM; i++)
+                if (i < decltype(count)::value) {
+#pragma unroll
+                    for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[h][j], f.a[h][i], acc[i][j], 0, 0, 0);
+                }
+    };
+    // K-tile t has landed in every wave's pieces, and every wave holds tile t - 1 in registers
+    auto arrive = [&](int t) {
+        const int behind = nk - 1 - t;                        // tiles after t: at most NBUF - 2 of them are under way
+        if (behind >= NBUF - 2) wait_vm<(NBUF - 2) * G::PER>();
+        else if constexpr (NBUF > 2) wait_tail<NBUF - 3, G::PER>(behind);
+        __builtin_amdgcn_s_waitcnt(0xC07F);                   // lgkmcnt(0)
+        __builtin_amdgcn_sched_barrier(0);
+        if constexpr (G::WAVES > 1) __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    auto loop = [&](auto count) {
+        for (int t = 0; t < min(NBUF - 1, nk); t++) ask(t, t);
+        Frags f0, f1;
+        arrive(0);
+        if (NBUF - 1 < nk) ask(NBUF - 1, NBUF - 1);
+        read(f0, 0, count);
+        int buf = 0;                                          // buffer of tile kt
+        auto step = [&](int kt, Frags& now, Frags& next) {
+            if (kt + 1 < nk) {
+                arrive(kt + 1);
+                if (kt + NBUF < nk) ask(kt + NBUF, buf);      // the buffer that tile kt was read from
+                buf = buf + 1 == NBUF ? 0 : buf + 1;
+                read(next, buf, count);
+            }
+            multiply(now, count);
+        };
+        for (int kt = 0; kt < nk; kt += 2) {
+            step(kt, f0, f1);
+            if (kt + 1 < nk) step(kt + 1, f1, f0);
+        }
+    };
+    if (live == FM) loop(std::integral_constant<int, FM>{});
+    else if (FM > 1 && live == FM - 1) loop(std::integral_constant<int, FM - 1>{});
+    else if (FM > 2 && live == FM - 2) loop(std::integral_constant<int, (FM > 2 ? FM - 2 : 0)>{});
+    else if (FM > 3 && live == FM - 3) loop(std::integral_constant<int, (FM > 3 ? FM - 3 : 0)>{});
+    else loop(std::integral_constant<int, 0>{});
+
+    if constexpr (G::WAVES > 1) {
+        __builtin_amdgcn_s_waitcnt(0xC07F);
+        __builtin_amdgcn_s_barrier();                         // everybody has read the last K-tile: the buffers become the epilogue's stage
+    }
+    char* stg = smem + wave * (2 * 16 * (FN * 32 + 16));
+    const int row0 = m0 + wf0 * 16, col0 = n0 + wn * FN * 16;
+    switch (epi) {                                            // (uniform)
+        case EPI_STORE: epilogue<EPI_STORE, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_GELU: epilogue<EPI_GELU, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_RELU2: epilogue<EPI_RELU2, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_LS_RES: epilogue<EPI_LS_RES, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_RES: epilogue<EPI_RES, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_SWIGLU: epilogue<EPI_SWIGLU, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_PATCH: epilogue<EPI_PATCH, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_F32: epilogue<EPI_F32, FM, FN>(p, acc, stg, row0, live, col0, lane); break;
+        case EPI_PARTIAL: {
+            GemmParams s = p;
+            s.C = (float*)p.C + (int64_t)blockIdx.y * p.M * p.ldc; s.raw32 = 1; s.softcap = 0.f;
+            epilogue<EPI_F32, FM, FN>(s, acc, stg, row0, live, col0, lane);
+            break;
+        }
+        case EPI_ARGMAX:
+            if constexpr (FN == 4) epilogue<EPI_ARGMAX, FM, FN>(p, acc, stg, row0, live, col0, lane);
+            break;
+    }
+}
+
+template <int WM, int WN, int FM, int FN, int NBUF>
+int launch_t(int epi, const GemmParams& p, int rt, hipStream_t stream) {
+    typedef MidGeom<WM, WN, FM, FN, NBUF> G;
+    static std::atomic<uint64_t> attr_done{0};
+    if (!cr_dyn_lds_once(attr_done, (const void*)gemm_mid_kernel<WM, WN, FM, FN, NBUF>, G::LDS)) return CR_ERR_HIP;
+    const int ntm = std::max((p.M + G::BM - 1) / G::BM, rt), ntn = (p.N + G::BN - 1) / G::BN;
+    hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, FM, FN, NBUF>), dim3(ntm * ntn, epi == EPI_PARTIAL ? p.group : 1), dim3(64 * G::WAVES), G::LDS, stream, p, epi, ntm);
+    return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
+}
+
+}  // namespace
+
+namespace {
+
+// Tile shapes (launch_gemm_mid's `tile` = index + 1).  Eight waves where the tile is large enough to feed them: two waves a SIMD cover each other's LDS reads and barriers (64 x 64 at
+// M = 1025, N = 1024, K = 4096: four waves 27.5 us, eight 26.6; 128 x 128 at N = 3072, K = 1024: 20 and 13.4).
+struct MidShape { int bm, bn; };
+constexpr MidShape SHAPES[] = {{16, 32}, {16, 64}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {64, 128}, {96, 128}, {128, 128}, {96, 256}, {128, 256}};
+constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
+
+}  // namespace
+
+// The time a launch takes, in us, and the tile shape (and number of row tiles) that takes least.  Every shape measured here (M 1 .. 4100, N 512 .. 28672, K 512 .. 16384) follows one law:
+// a CU brings in its workgroups' operand bytes at 61 GB/s and does the rest under that, so a K-tile (64) of a workgroup costs 0.05 us + 2.1 ns per row of A or W in it; a workgroup
+// more on a CU costs its time again; launch, first fill and drain 3.5 us, the epilogue 0.1 ns an element.  (32 x 64, K 14336: 52.3 us measured, 57 by the law; 64 x 64, K 4096: 21.7 and
+// 24.1; 96 x 64, K 14336: 79.5 and 90; 128 x 128, K 4096: 43.5 and 42.5; 128 x 256, K 4096: 55.1 and 56.8.)
+double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
+    const int nf = (p.M + 15) / 16, slices = epi == EPI_PARTIAL && p.group > 0 ? p.group : 1, nk = p.K / 64 / slices, cus = cr_device_cus();
+    double best = 1e30;
+    for (int t = 0; t < N_SHAPES; t++) {
+        if (epi == EPI_ARGMAX && SHAPES[t].bn != 256) continue;          // (a wave's columns are a partial's 64)
+        const long ntn = (long)((p.N + SHAPES[t].bn - 1) / SHAPES[t].bn) * slices;
+        const int cap = SHAPES[t].bm / 16, least = (nf + cap - 1) / cap;
+        for (int per_cu = 0; per_cu <= 2; per_cu++) {                    // the fewest row tiles, or as many as make one or two workgroups per CU
+            const long want = per_cu == 0 ? least : (long)per_cu * cus / ntn;
+            if (want < least || want > nf || (per_cu && want > 2L * least)) continue;
+            const int rows = 16 * ((nf + (int)want - 1) / (int)want);
+            const double rounds = (double)((want * ntn + cus - 1) / cus);
+            const double c = 3.5 + rounds * (nk * (0.05 + 0.0021 * (rows + SHAPES[t].bn)) + 1e-4 * rows * SHAPES[t].bn);
+            if (c < best - 1e-9) { best = c; *tile = t + 1; *row_tiles = (int)want; }
+        }
+    }
+    return best;
+}
+
+int launch_gemm_mid(int epi, const GemmParams& p, hipStream_t stream) {
+    int tile = p.tile, rt = 0;
+    if (!tile) gemm_mid_cost(epi, p, &tile, &rt);
+    switch (tile) {
+        case 1: return launch_t<1, 2, 1, 1, 12>(epi, p, rt, stream);
+        case 2: return launch_t<1, 4, 1, 1, 8>(epi, p, rt, stream);
+        case 3: return launch_t<1, 4, 2, 1, 6>(epi, p, rt, stream);
+        case 4: return launch_t<2, 2, 2, 1, 6>(epi, p, rt, stream);
+        case 5: return launch_t<2, 4, 2, 1, 4>(epi, p, rt, stream);
+        case 6: return launch_t<2, 4, 3, 1, 4>(epi, p, rt, stream);
+        case 7: return launch_t<2, 4, 4, 1, 3>(epi, p, rt, stream);
+        case 8: return launch_t<2, 4, 2, 2, 3>(epi, p, rt, stream);
+        case 9: return launch_t<2, 4, 3, 2, 5>(epi, p, rt, stream);
+        case 10: return launch_t<2, 4, 4, 2, 4>(epi, p, rt, stream);
+        case 11: return launch_t<2, 4, 3, 4, 3>(epi, p, rt, stream);
+        case 12: return launch_t<2, 4, 4, 4, 3>(epi, p, rt, stream);
+    }
+    return CR_ERR_ARG;
+}

@@ -139,39 +139,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const GemmParam
         }
     }
     int ks = W8 ? ksteps : 0;
-    if (WAVES == 1 && RT == 1 && !W8) {
-        // The tail kernel (launch_gemm_tail): ONE wave walks the whole K in ascending order (the tiled kernels' order: these rows must
-        // get their bits), so its time is a chain of load round trips -- 128 k-steps at K = 4096.  Two register batches of UR k-steps:
-        // the loads of batch b + 1 are in flight while batch b is multiplied (config 2's fc2 tail: 43 us per launch before).
-        bf16x8 wa[UR], wb[UR], xa[MT][UR], xb[MT][UR];
-        auto load = [&](bf16x8* w, bf16x8 (*x)[UR], int k0) {
-#pragma unroll
-            for (int u = 0; u < UR; u++) w[u] = __builtin_nontemporal_load((const bf16x8*)(wp[0] + (k0 + u) * 32));
-#pragma unroll
-            for (int t = 0; t < MT; t++)
-#pragma unroll
-                for (int u = 0; u < UR; u++) x[t][u] = *(const bf16x8*)(xp[t] + (k0 + u) * 32);
-        };
-        auto mma = [&](const bf16x8* w, const bf16x8 (*x)[UR]) {
-#pragma unroll
-            for (int u = 0; u < UR; u++)
-#pragma unroll
-                for (int t = 0; t < MT; t++) acc[0][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u], x[t][u], acc[0][t], 0, 0, 0);
-        };
-        const int nb = ksteps / UR;
-        if (nb > 0) {
-            load(wa, xa, 0);
-            int b = 0;
-            for (; b + 2 <= nb; b += 2) {                    // (wa, xa) hold batch b
-                load(wb, xb, (b + 1) * UR);
-                mma(wa, xa);
-                if (b + 2 < nb) load(wa, xa, (b + 2) * UR);
-                mma(wb, xb);
-            }
-            if (b < nb) mma(wa, xa);
-            ks = nb * UR;
-        }
-    }
     for (; ks + UR <= ksteps; ks += UR) {
         bf16x8 w[RT][UR], x[MT][UR];
 #pragma unroll
@@ -247,8 +214,6 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const GemmParam
         const float sum = red[0][t][n][m] + (p.bias ? bf2f(p.bias[gn]) : 0.f);
         if (EPI == EPI_F32) { ((float*)p.C)[(int64_t)gm * p.ldc + gn] = f32_out(p, sum); continue; }
         float x = EPI == EPI_RELU2 ? relu2(sum) : rbf(sum);
-        if (EPI == EPI_GELU) x = gelu_erf(x);
-        if (EPI == EPI_LS_RES) x = bf2f(p.res[(int64_t)gm * p.ldr + gn]) + rbf(x * bf2f(p.scale[gn]));
         if (EPI == EPI_RES) x = bf2f(p.res[(int64_t)gm * p.ldr + gn]) + x;
         ((bf16*)p.C)[(int64_t)gm * p.ldc + gn] = f2bf(x);
     }
@@ -320,32 +285,6 @@ PartialGeom partial_geom(int N, int K) {
 }
 
 }  // namespace
-
-// The last M % 256 rows (<= 64) of a tiled GEMM whose 256x256 launch would otherwise pay a whole extra round of tiles for them
-// (gemm.hip: launch_gemm).  ONE wave per workgroup walks the whole K in ascending 32-steps with the same MFMA and the same
-// operand roles as the tiled kernels, so these rows get bit for bit what the tiled kernels would have given them
-// (tests/test_gpu_ops.py::test_gemm_tail_rows_take_the_small_kernel); eight k-steps of loads in flight hide the latency that a
-// lone 128x128 workgroup per 128 columns would expose K / 64 times over.
-bool gemm_tail_supported(int epi, const GemmParams& p) {
-    if (p.M > 64 || p.M <= 0 || p.K % 32 != 0 || p.w8 || p.a8) return false;
-    if (epi == EPI_LS_RES) return p.res && p.scale;
-    if (epi == EPI_RES) return p.res != nullptr;
-    if (epi == EPI_SWIGLU) return p.N % 16 == 0;
-    return epi == EPI_STORE || epi == EPI_GELU || epi == EPI_RELU2 || epi == EPI_F32;
-}
-
-int launch_gemm_tail(int epi, const GemmParams& p, hipStream_t stream) {
-    switch (epi) {
-        case EPI_STORE: return launch_mt8<EPI_STORE, 1, 1, false>(p, stream, 1);
-        case EPI_GELU: return launch_mt8<EPI_GELU, 1, 1, false>(p, stream, 1);
-        case EPI_RELU2: return launch_mt8<EPI_RELU2, 1, 1, false>(p, stream, 1);
-        case EPI_LS_RES: return launch_mt8<EPI_LS_RES, 1, 1, false>(p, stream, 1);
-        case EPI_RES: return launch_mt8<EPI_RES, 1, 1, false>(p, stream, 1);
-        case EPI_SWIGLU: return launch_mt8<EPI_SWIGLU, 1, 1, false>(p, stream, 1);
-        case EPI_F32: return launch_mt8<EPI_F32, 1, 1, false>(p, stream, 1);
-    }
-    return CR_ERR_ARG;
-}
 
 int gemm_partial_splits(int N, int K) { return partial_geom(N, K).splits; }
 

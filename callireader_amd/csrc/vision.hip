@@ -16,7 +16,7 @@ static constexpr int VIT_CHUNK = 255;  // 255*1025 rows = 1021 row-tiles of 256:
                                        // start, tail) spread over 4x the work of round 1's 63-tile chunks: 1.3 % on 510 tiles; operands stay < 4 GiB
 // Chunks of 16k-1 tiles (127, ..., 31, 15) put ceil(rows/256) * {4,12,16} GEMM tiles just under a whole number of
 // 256-CU rounds.  Up to 64 tiles go as ONE chunk: rows = 1024 T + T, so the T rows past the last multiple of 256 are exactly
-// what the dispatcher hands to the one-wave tail kernel (gemm.hip: launch_gemm_tail, <= 64 rows) -- 32 tiles
+// what the dispatcher hands to the small tiles (gemm_mid.hip) -- 32 tiles
 // used to run as 31 + 1, and the 1-tile chunk's 24 x 7 launches of almost nothing cost more than the 32nd tile's work.
 static int next_chunk(int remaining) {
     static const int cap = [] { const char* e = getenv("CR_VIT_CHUNK"); const int v = e ? atoi(e) : 0; return v > 0 && v < VIT_CHUNK ? v : VIT_CHUNK; }();   // tuning aid

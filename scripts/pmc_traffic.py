@@ -13,11 +13,9 @@ def load(d, counter):
         if r['Counter_Name'] != counter:
             continue
         k = r['Kernel_Name']
-        fam = 'gemm_tiled_big' if ('gemm256_kernel' in k or 'gemm128_kernel' in k) else ('gemm_skinny' if 'gemm_skinny' in k else None)
+        fam = 'gemm_tiled_big' if 'gemm256_kernel' in k else ('gemm_skinny' if 'gemm_skinny' in k else None)
         if fam is None:
             continue
-        if fam == 'gemm_tiled_big' and 'gemm128' in k and int(r['Grid_Size']) < 8 * 8 * 256:
-            continue            # small 128-tile launches (M < 1024) are not in the roofline class
         per.setdefault(fam, []).append(float(r['Counter_Value']))
     return per
 

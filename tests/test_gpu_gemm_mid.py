@@ -1,0 +1,63 @@
+"""The tile shapes of gemm_mid.hip: every epilogue of every shape at the edges of tiles, K pipelines and vector stores, against a plain fp32 expression (outputs are bf16: two ulp, 1.6e-2,
+and an absolute floor for cancellation) and, bit for bit, against each other and the 256x256 kernel: a row's sum is the same chain of MFMAs whichever kernel takes it."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+TILES = range(16, 28)                                   # cr_op_gemm's pins of gemm_mid's shapes
+# K-tiles from one to more than any shape keeps in flight; N with and without whole vectors and fragments; rows around fragments and row tiles
+SHAPES = [(1, 64, 64), (15, 200, 128), (17, 72, 704), (33, 331, 192), (65, 272, 1344), (129, 512, 256), (300, 1040, 640)]
+
+
+def rb(t):
+    return t.to(torch.bfloat16).float()
+
+
+@pytest.mark.parametrize('M,N,K', SHAPES)
+def test_every_shape_and_epilogue(M, N, K):
+    from callireader_amd import engine as E
+    g = torch.Generator().manual_seed(M * 1000 + N)
+    dev = torch.device('cuda', 0)
+    A, W = torch.randn(M, K, generator=g).bfloat16().to(dev), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(dev)
+    bias, scale, res = ((torch.randn(*s, generator=g) * 0.3).bfloat16().to(dev) for s in ((N,), (N,), (M + 8, N)))
+    acc = A.float() @ W.float().T
+    lin = rb(acc + bias.float())
+    cases = {'store': (0, dict(bias=bias), lin), 'gelu': (1, dict(bias=bias), rb(torch.nn.functional.gelu(lin))),
+             'scaled residual': (2, dict(bias=bias, scale=scale, res=res), rb(res[:M].float() + rb(lin * scale.float()))), 'residual': (3, dict(res=res), rb(res[:M].float() + rb(acc))),
+             'fp32': (6, dict(out_dtype=torch.float32), rb(acc)), 'relu2': (12, {}, rb(acc.clamp(min=0).square()))}
+    if N % 16 == 0:
+        gu = rb(acc).view(M, N // 16, 2, 8)
+        cases['swiglu'] = (4, {}, rb(rb(torch.nn.functional.silu(gu[:, :, 0])) * gu[:, :, 1]).reshape(M, N // 2))
+    for name, (epi, kw, want) in cases.items():
+        first = None
+        for tile in list(TILES) + ([2] if K % 128 == 0 else []):
+            out = E.op_gemm(epi, A, W, kernel=tile, **kw)
+            torch.cuda.synchronize()
+            if first is None:
+                first = out
+                torch.testing.assert_close(out.float(), want, rtol=1.6e-2, atol=2e-2, msg=lambda m: f'{name}: {m}')
+            assert torch.equal(out, first), (name, tile)
+
+
+def test_rows_of_patches_keys_of_the_table_and_slices():
+    """Position rows behind a class row (epi 5), first maxima of 64-column blocks (epi 8), K-slices (epi 7), an output in place of its residual."""
+    from callireader_amd import engine as E
+    g = torch.Generator().manual_seed(3)
+    dev = torch.device('cuda', 0)
+    M, N, K, group = 3 * 40, 192, 320, 40
+    A, W = torch.randint(-2, 3, (M, K), generator=g).bfloat16().to(dev), torch.randint(-2, 3, (N, K), generator=g).bfloat16().to(dev)
+    W[70] = W[66]                                        # equal keys: the first one wins
+    pos, acc = torch.randn(group + 1, N, generator=g).bfloat16().to(dev), A.float() @ W.float().T
+    for tile in TILES:
+        out = E.op_gemm(5, A, W, res=pos, group=group, kernel=tile).view(3, group + 1, N)
+        assert torch.equal(out[:, 1:].float(), rb(rb(acc).view(3, group, N) + pos[1:].float())), tile
+        x = pos[:1].repeat(M, 1).contiguous()
+        E.op_gemm(3, A, W, res=x, out=x, kernel=tile)
+        assert torch.equal(x.float(), rb(pos[:1].float() + rb(acc))), tile
+        part = E.op_gemm(7, A, W, group=5, kernel=tile).view(8, M, N)
+        assert torch.equal(part[:5].sum(0), acc) and float(part[5:].abs().max()) == 0.0, tile
+    for tile in (26, 27):
+        out = E.op_gemm(8, A, W, kernel=tile)[:, :3].cpu()
+        val = ((out >> 32) & 0xFFFFFFFF).to(torch.int32).view(torch.float32)
+        mx, at = rb(acc).cpu().view(M, 3, 64).max(-1)
+        assert torch.equal(val, mx) and torch.equal(out & 0xFFFFFFFF, at + 64 * torch.arange(3)), tile
