@@ -5,6 +5,8 @@
 
 #include "ctx.hpp"
 
+struct PickCell { unsigned long long best; unsigned arrived, pad; };      // a row's greedy pick under way (llm.hip: pick_kernel); zero between launches
+
 struct cr_kv {
     cr_ctx* ctx;
     int n_seqs, max_tokens, gen_cap, layers;
@@ -17,6 +19,7 @@ struct cr_kv {
     int32_t* d_len;      // [n_seqs] tokens cached
     int32_t* d_ngen;     // [n_seqs] ids generated
     int64_t* d_gen;      // [n_seqs][gen_cap]
+    PickCell* d_pick;    // [n_seqs]
     int32_t* d_seqs;     // [n_seqs] staging for the seqs[] of one decode call
     std::vector<int32_t> seqs_on_device;   // what d_seqs holds (decode skips the host-to-device copy of an unchanged list: a pageable copy
                                            // makes the host wait for the stream, which stops it from feeding a second stream)

@@ -156,50 +156,65 @@ __global__ __launch_bounds__(128) void rope_split_kernel(const bf16* __restrict_
 }
 
 // RepetitionPenaltyLogitsProcessor (published 4.45.2 semantics) + argmax (first max wins) + append the id.
-// One workgroup of 1024 per row.
-__global__ __launch_bounds__(1024) void pick_kernel(float* __restrict__ logits, int64_t ld, int vocab, float penalty,
-                                                    int seq0, const int32_t* __restrict__ seqs, int64_t* __restrict__ gen,
-                                                    int32_t* __restrict__ ngen, int32_t* __restrict__ lens, int gen_cap, int len_add) {
-    __shared__ float bv[1024];
-    __shared__ int bi[1024];
-    const int row = blockIdx.x, tid = threadIdx.x;
-    const int seq = seqs ? seqs[row] : seq0;
+// Bound by latency: a row of 92 553 scores is 370 KB, which one workgroup takes 30 us to walk (ninety dependent rounds of loads).  A row is therefore cut into parts of PICK_PART scores,
+// one workgroup each (sixteen loads of a thread at once; one row of 92 553 scores: 29.4 -> 4.7 us, 64 rows 31 -> 9.9, one of 32 000 11.7 -> 4.6).  A part applies the penalty to the generated ids that fall into it,
+// takes its maximum and folds it into the row's cell; the last part to arrive appends the id and leaves the cell as it found it.
+//   cell: {score ordered as an unsigned number, ~column} in one 64-bit word, so that one atomic maximum keeps the larger score and, of equal ones, the first column (-0 counts as +0;
+//   a NaN never wins); and the parts that have arrived.  Both live on atomics alone: the maximum's returned value is waited for before the count goes out.
+constexpr int PICK_PART = 4096;
+__global__ __launch_bounds__(256) void pick_kernel(float* __restrict__ logits, int64_t ld, int vocab, float penalty, const int32_t* __restrict__ seqs, int64_t* __restrict__ gen,
+                                                   int32_t* __restrict__ ngen, int32_t* __restrict__ lens, int gen_cap, int len_add, PickCell* __restrict__ cells) {
+    __shared__ unsigned long long red[4];
+    const int row = blockIdx.y, tid = threadIdx.x, c0 = blockIdx.x * PICK_PART, c1 = min(c0 + PICK_PART, vocab);
+    const int seq = seqs[row];
     float* lg = logits + (int64_t)row * ld;
     const int ng = ngen[seq];
     int64_t* g = gen + (int64_t)seq * gen_cap;
     if (penalty != 1.0f && ng > 0) {
-        // gather every score first, then scatter: duplicates of an id all see the ORIGINAL score
-        float sv[4]; int64_t si[4];
+        // gather every score first, then scatter: duplicates of an id all see the ORIGINAL score (gen_cap = 16 ids a thread)
+        float sv[16]; int si[16];
 #pragma unroll
-        for (int k = 0; k < 4; k++) {
-            const int h = tid + k * 1024;
-            si[k] = h < ng ? g[h] : -1;
+        for (int k = 0; k < 16; k++) {
+            const int h = tid + k * 256;
+            const int64_t id = h < ng ? g[h] : -1;
+            si[k] = id >= c0 && id < c1 ? (int)id : -1;
             sv[k] = si[k] >= 0 ? lg[si[k]] : 0.f;
         }
         __syncthreads();
 #pragma unroll
-        for (int k = 0; k < 4; k++)
+        for (int k = 0; k < 16; k++)
             if (si[k] >= 0) lg[si[k]] = sv[k] < 0.f ? sv[k] * penalty : sv[k] / penalty;
         __syncthreads();
     }
+    float v[PICK_PART / 256];
+#pragma unroll
+    for (int k = 0; k < PICK_PART / 256; k++) v[k] = lg[min(c0 + tid + 256 * k, c1 - 1)];
     float best = -INFINITY; int besti = 0x7fffffff;
-    for (int c = tid; c < vocab; c += 1024) {
-        const float v = lg[c];
-        if (v > best) { best = v; besti = c; }
+#pragma unroll
+    for (int k = 0; k < PICK_PART / 256; k++) {
+        const int c = c0 + tid + 256 * k;
+        if (c < c1 && v[k] > best) { best = v[k]; besti = c; }
     }
-    bv[tid] = best; bi[tid] = besti;
+    const unsigned bits = __float_as_uint(best + 0.0f);
+    unsigned long long key = best == -INFINITY ? 0ull : ((unsigned long long)(bits & 0x80000000u ? ~bits : bits | 0x80000000u) << 32) | (unsigned)~besti;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) {
+        const unsigned long long other = ((unsigned long long)__shfl_xor((unsigned)(key >> 32), o, 64) << 32) | __shfl_xor((unsigned)key, o, 64);
+        key = other > key ? other : key;
+    }
+    if ((tid & 63) == 0) red[tid >> 6] = key;
     __syncthreads();
-    for (int o = 512; o > 0; o >>= 1) {
-        if (tid < o) {
-            const float v2 = bv[tid + o]; const int i2 = bi[tid + o];
-            if (v2 > bv[tid] || (v2 == bv[tid] && i2 < bi[tid])) { bv[tid] = v2; bi[tid] = i2; }
-        }
-        __syncthreads();
-    }
-    if (tid == 0) {
-        if (ng < gen_cap) { g[ng] = bi[0]; ngen[seq] = ng + 1; }
-        lens[seq] += len_add;
-    }
+    if (tid != 0) return;
+#pragma unroll
+    for (int w = 1; w < 4; w++) key = red[w] > key ? red[w] : key;
+    PickCell* cell = cells + seq;
+    unsigned long long before = __hip_atomic_fetch_max(&cell->best, key, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    asm volatile("" : "+v"(before) : : "memory");              // (the maximum has been taken when its answer is here)
+    if (__hip_atomic_fetch_add(&cell->arrived, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1 < gridDim.x) return;
+    const unsigned long long top = __hip_atomic_exchange(&cell->best, 0ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __hip_atomic_store(&cell->arrived, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    if (ng < gen_cap) { g[ng] = top ? (int)~(unsigned)top : 0x7fffffff; ngen[seq] = ng + 1; }
+    lens[seq] += len_add;
 }
 
 // w13 rows: [16q + e] = w1[8q + e], [16q + 8 + e] = w3[8q + e]   (pairs gate/up for the SwiGLU epilogue)
@@ -517,7 +532,8 @@ size_t layers_ws(cr_ctx* c, int M, int nsplit = 0, int n_pages = 0) {
 }  // namespace
 
 int launch_pick(float* logits, int64_t ld, int vocab, float penalty, int n, const int32_t* seqs, cr_kv* kv, int len_add, hipStream_t st) {
-    hipLaunchKernelGGL(pick_kernel, dim3(n), dim3(1024), 0, st, logits, ld, vocab, penalty, 0, seqs, kv->d_gen, kv->d_ngen, kv->d_len, kv->gen_cap, len_add);
+    hipLaunchKernelGGL(pick_kernel, dim3((vocab + PICK_PART - 1) / PICK_PART, n), dim3(256), 0, st, logits, ld, vocab, penalty, seqs, kv->d_gen, kv->d_ngen, kv->d_len, kv->gen_cap, len_add,
+                       kv->d_pick);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }
@@ -766,12 +782,13 @@ int cr_kv_alloc(cr_ctx* c, int n_seqs, int max_tokens, cr_kv** out) {
     if ((bytes && (hipMalloc((void**)&kv->k, bytes) != hipSuccess || hipMalloc((void**)&kv->v, bytes) != hipSuccess)) ||
         hipMalloc((void**)&kv->d_len, n_seqs * 4) != hipSuccess || hipMalloc((void**)&kv->d_ngen, n_seqs * 4) != hipSuccess ||
         hipMalloc((void**)&kv->d_seqs, n_seqs * 4) != hipSuccess ||
-        hipMalloc((void**)&kv->d_gen, (size_t)n_seqs * kv->gen_cap * 8) != hipSuccess) {
+        hipMalloc((void**)&kv->d_gen, (size_t)n_seqs * kv->gen_cap * 8) != hipSuccess || hipMalloc((void**)&kv->d_pick, n_seqs * sizeof(PickCell)) != hipSuccess) {
         cr_kv_free(kv);
         return cr_fail(CR_ERR_NOMEM, "cr_kv_alloc: %zu bytes per K/V", bytes);
     }
     CR_HIP(hipMemset(kv->d_len, 0, n_seqs * 4));
     CR_HIP(hipMemset(kv->d_ngen, 0, n_seqs * 4));
+    CR_HIP(hipMemset(kv->d_pick, 0, n_seqs * sizeof(PickCell)));
     kv->len.assign(n_seqs, 0); kv->ngen.assign(n_seqs, 0);
     *out = kv;
     return CR_OK;
@@ -787,6 +804,7 @@ int cr_kv_free(cr_kv* kv) {
     if (kv->d_ngen) hipFree(kv->d_ngen);
     if (kv->d_seqs) hipFree(kv->d_seqs);
     if (kv->d_gen) hipFree(kv->d_gen);
+    if (kv->d_pick) hipFree(kv->d_pick);
     for (auto& e : kv->graphs) if (e.exec) hipGraphExecDestroy(e.exec);
     delete kv;
     return CR_OK;
@@ -878,9 +896,7 @@ int cr_llm_prefill_batch(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, const
         CR_TRY(rms(x + (size_t)(segs[i].row0 + segs[i].S - 1) * D, D, hl + (size_t)i * D, nw, 1, c->d.rms_eps, st));
     CR_TRY(gemm(c, EPI_F32, hl, D, ow, D, lg, V, nullptr, 0, n, V, D, st));
     if (last_logits) CR_HIP(hipMemcpyAsync(last_logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
-    hipLaunchKernelGGL(pick_kernel, dim3(n), dim3(1024), 0, st, lg, (int64_t)V, V, penalty, 0, kv->d_seqs, kv->d_gen, kv->d_ngen,
-                       kv->d_len, kv->gen_cap, 0);
-    CR_HIP(hipGetLastError());
+    CR_TRY(launch_pick(lg, V, V, penalty, n, kv->d_seqs, kv, 0, st));
     for (const Segment& sg : segs) {
         kv->len[sg.seq] += sg.S;
         if (kv->ngen[sg.seq] < kv->gen_cap) kv->ngen[sg.seq] += 1;
@@ -959,9 +975,7 @@ int cr_llm_decode(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, const int64_
         else CR_TRY(gemm(c, EPI_F32, hl, D, ow, D, lg, V, nullptr, 0, n, V, D, st, false, opt(c, "declayout.language_model.output.weight")));
         }
         if (logits) CR_HIP(hipMemcpyAsync(logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
-        hipLaunchKernelGGL(pick_kernel, dim3(n), dim3(1024), 0, st, lg, (int64_t)V, V, penalty, 0, kv->d_seqs, kv->d_gen, kv->d_ngen,
-                           kv->d_len, kv->gen_cap, 1);
-        return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
+        return launch_pick(lg, V, V, penalty, n, kv->d_seqs, kv, 1, st);
     };
     // graph path: the plain generation loop (no forced ids, no logits copy), nothing recording events on these launches
     const bool graphable = c->decode_graph && !force_tokens && !logits && !(c->prof && c->prof_mode != 2);
