@@ -224,6 +224,10 @@ __global__ __launch_bounds__(256, 2) void decode_attn_kernel(const AttnParams p)
                 a1 += w * s_o[jj][h][d0 + 1];
             }
         }
+        if (p.nsplit == 1) {                                   // nothing to merge with: attn_merge_splits' result, whose one weight is exp(0)
+            *(bf16x2*)(p.O + (int64_t)batch * p.o_bs + (int64_t)h * p.o_rs + (int64_t)head * p.o_hs + d0) = bf16x2{f2bf(a0 / L), f2bf(a1 / L)};
+            return;
+        }
         *(f32x2_t*)(p.part_o + (prow + h) * HD + d0) = f32x2_t{a0, a1};
         if ((tid & 63) == 0) { p.part_ml[(prow + h) * 2] = M; p.part_ml[(prow + h) * 2 + 1] = L; }
     }

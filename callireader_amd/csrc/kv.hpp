@@ -33,5 +33,8 @@ struct cr_kv {
     std::vector<DecodeGraph> graphs;
 };
 
+// The head may write the caller's logits itself (no copy behind it: 4.6 us a step at one row, 10 at 64): the pick reads them and, without a penalty, leaves them as they are.
+inline bool logits_in_place(const float* logits, float penalty) { return logits && penalty == 1.0f && ((uintptr_t)logits & 15) == 0; }
+
 // repetition penalty + argmax + append, one row per sequence seqs[row] (llm.hip); len_add: tokens the step added to the cache length
 int launch_pick(float* logits, int64_t ld, int vocab, float penalty, int n, const int32_t* seqs, cr_kv* kv, int len_add, hipStream_t st);

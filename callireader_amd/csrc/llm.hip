@@ -861,11 +861,14 @@ int cr_llm_prefill_batch(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, const
     hipStream_t st = (hipStream_t)stream;
     const int V = c->d.vocab;
     const size_t lw = layers_ws(c, M, 0, n);
-    CR_TRY(ws_ensure(c, lw + (size_t)M * D * 2 + (size_t)n * D * 2 + (size_t)n * V * 4 + (size_t)M * 8 + (size_t)n * 36 + 8192));
+    CR_TRY(ws_ensure(c, lw + (size_t)M * D * 2 + (size_t)n * D * 4 + (size_t)n * V * 4 + (size_t)M * 8 + (size_t)n * 36 + 8192));
     bf16* x = (bf16*)(c->ws + ((lw + 255) & ~(size_t)255));
     bf16* hl = x + (size_t)M * D;
-    float* lg = (float*)(((uintptr_t)(hl + (size_t)n * D) + 255) & ~(uintptr_t)255);
+    bf16* xlast = hl + (size_t)n * D;
+    float* lg = (float*)(((uintptr_t)(xlast + (size_t)n * D) + 255) & ~(uintptr_t)255);
     int32_t* d_row_seq = (int32_t*)(((uintptr_t)(lg + (size_t)n * V) + 255) & ~(uintptr_t)255);
+    const bool own = logits_in_place(last_logits, penalty);
+    if (own) lg = last_logits;
     int32_t* d_row_pos = d_row_seq + M;
     int32_t* d_seg = d_row_pos + M;                 // 4 per page: first row, rows, first position, cache slot (the attention launch's segments)
     int32_t* d_seg_last = d_seg + 4 * n;            // the final layer's segments: the rows that share a 32-row wave with the page's last row
@@ -892,10 +895,10 @@ int cr_llm_prefill_batch(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, const
     const bf16 *nw = W(c, "language_model.model.norm.weight"), *ow = W(c, "language_model.output.weight");
     if (!nw || !ow) return CR_ERR_STATE;
     // only each page's last row feeds the LM head (the reference computes all S rows and reads the last, :1081 + _sample)
-    for (int i = 0; i < n; i++)
-        CR_TRY(rms(x + (size_t)(segs[i].row0 + segs[i].S - 1) * D, D, hl + (size_t)i * D, nw, 1, c->d.rms_eps, st));
-    CR_TRY(gemm(c, EPI_F32, hl, D, ow, D, lg, V, nullptr, 0, n, V, D, st));
-    if (last_logits) CR_HIP(hipMemcpyAsync(last_logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
+    if (n > 1) hipLaunchKernelGGL(move_rows_kernel<true>, dim3(n), dim3(256), 0, st, x, d_last, xlast);
+    CR_TRY(rms(n > 1 ? xlast : x + (size_t)(M - 1) * D, D, hl, nw, n, c->d.rms_eps, st));
+    CR_TRY(gemm(c, EPI_F32, hl, D, ow, D, lg, V, nullptr, 0, n, V, D, st, false, opt(c, "declayout.language_model.output.weight")));
+    if (last_logits && !own) CR_HIP(hipMemcpyAsync(last_logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
     CR_TRY(launch_pick(lg, V, V, penalty, n, kv->d_seqs, kv, 0, st));
     for (const Segment& sg : segs) {
         kv->len[sg.seq] += sg.S;
@@ -952,6 +955,8 @@ int cr_llm_decode(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, const int64_
     bf16* x = (bf16*)(c->ws + ((lw + 255) & ~(size_t)255));
     bf16* hl = x + (size_t)n * D;
     float* lg = (float*)(((uintptr_t)(hl + (size_t)n * D) + 255) & ~(uintptr_t)255);
+    const bool own = logits_in_place(logits, penalty);
+    if (own) lg = logits;
     if ((int)kv->seqs_on_device.size() != n || memcmp(kv->seqs_on_device.data(), seqs, (size_t)n * 4) != 0) {      // prefill uses d_seqs too
         CR_HIP(hipMemcpyAsync(kv->d_seqs, seqs, (size_t)n * 4, hipMemcpyHostToDevice, st));
         kv->seqs_on_device.assign(seqs, seqs + n);
@@ -974,7 +979,7 @@ int cr_llm_decode(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, const int64_
         if (c->fp8_decode && n <= 64 && q_out && s_out) CR_TRY(gemm8(c, EPI_F32, hl, D, q_out, s_out, lg, V, nullptr, 0, n, V, D, st, opt(c, "fp8dl.language_model.output.weight")));
         else CR_TRY(gemm(c, EPI_F32, hl, D, ow, D, lg, V, nullptr, 0, n, V, D, st, false, opt(c, "declayout.language_model.output.weight")));
         }
-        if (logits) CR_HIP(hipMemcpyAsync(logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
+        if (logits && !own) CR_HIP(hipMemcpyAsync(logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
         return launch_pick(lg, V, V, penalty, n, kv->d_seqs, kv, 1, st);
     };
     // graph path: the plain generation loop (no forced ids, no logits copy), nothing recording events on these launches

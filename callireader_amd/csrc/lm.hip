@@ -704,9 +704,11 @@ int lm_decode_step(cr_ctx* c, cr_kv* kv, int n, const int64_t* force_tokens, flo
     Buffers b = carve(lm, ar, sp);
     void* hl = ar.take<char>((size_t)n * lm.Wp * lm.esz());
     float* lg = ar.take<float>((size_t)n * lm.d.vocab);
+    const bool own = logits_in_place(logits, penalty);
+    if (own) lg = logits;
     CR_TRY(run_passes(c, kv, sp, b, hl, st));
     CR_TRY(raw32(c, lm, hl, lm.head, lg, lm.d.vocab, n, lm.d.vocab, lm.Wp, lm.d.softcap, st, true, lm.head_dl));
-    if (logits) CR_HIP(hipMemcpyAsync(logits, lg, (size_t)n * lm.d.vocab * 4, hipMemcpyDeviceToDevice, st));
+    if (logits && !own) CR_HIP(hipMemcpyAsync(logits, lg, (size_t)n * lm.d.vocab * 4, hipMemcpyDeviceToDevice, st));
     return launch_pick(lg, lm.d.vocab, lm.d.vocab, penalty, n, kv->d_seqs, kv, 1, st);
 }
 
@@ -897,8 +899,13 @@ int cr_llm_prefill_tokens(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, cons
     }
     CR_TRY(run_passes(c, kv, sp, b, nullptr, st));
     if (n_want) CR_TRY(lm_head(c, lm, b.x, d_want, n_want, hl, piece, want_logits, st));
-    CR_TRY(lm_head(c, lm, b.x, d_last, n, hl, piece, lg, st));
-    if (last_logits) CR_HIP(hipMemcpyAsync(last_logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
+    // the rows asked for are often the last rows: their logits serve the pick too
+    const bool same = n_want == n && memcmp(h_want, h_last, (size_t)n * 4) == 0;
+    const bool own = logits_in_place(same ? want_logits : last_logits, penalty);
+    if (own) lg = same ? want_logits : last_logits;
+    if (!same) CR_TRY(lm_head(c, lm, b.x, d_last, n, hl, piece, lg, st));
+    else if (!own) CR_HIP(hipMemcpyAsync(lg, want_logits, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
+    if (last_logits && last_logits != lg) CR_HIP(hipMemcpyAsync(last_logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
     CR_TRY(launch_pick(lg, V, V, penalty, n, kv->d_seqs, kv, 0, st));
     for (const Step::Seg& sg : sp.segs) {
         kv->len[sg.seq] += sg.S;
