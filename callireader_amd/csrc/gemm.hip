@@ -15,7 +15,7 @@ int launch_gemm256(int epi, const GemmParams& p, hipStream_t stream);
 int launch_gemm256_f8(int epi, const GemmParams& p, hipStream_t stream);
 bool gemm_skinny_supported(int epi, const GemmParams& p);
 int launch_gemm_skinny(int epi, const GemmParams& p, hipStream_t stream);
-double gemm256_cost(int epi, const GemmParams& p);
+double gemm256_cost(const GemmParams& p);
 
 int launch_gemm(int epi, const GemmParams& p, hipStream_t stream) {
     if (p.M <= 0 || p.N <= 0 || p.K <= 0 || (p.K % 64) != 0) return CR_ERR_ARG;
@@ -46,7 +46,7 @@ int launch_gemm(int epi, const GemmParams& p, hipStream_t stream) {
     // three rounds for two rounds' work at N = 1024).
     int tile, rt;
     const int r = p.M % 256;
-    double whole = gemm256_cost(epi, p), mid = gemm_mid_cost(epi, p, &tile, &rt), cut = 1e30;
+    double whole = gemm256_cost(p), mid = gemm_mid_cost(epi, p, &tile, &rt), cut = 1e30;
     GemmParams a = p, b = p;
     if (r > 0 && p.M > r && epi != EPI_PATCH && epi != EPI_ARGMAX) {
         a.M = p.M - r;
@@ -54,7 +54,7 @@ int launch_gemm(int epi, const GemmParams& p, hipStream_t stream) {
         b.A = p.A + (int64_t)a.M * p.lda;
         b.C = (char*)p.C + (int64_t)a.M * p.ldc * (epi == EPI_F32 ? 4 : 2);
         if (p.res) b.res = p.res + (int64_t)a.M * p.ldr;
-        cut = gemm256_cost(epi, a) + gemm_mid_cost(epi, b, &tile, &rt);
+        cut = gemm256_cost(a) + gemm_mid_cost(epi, b, &tile, &rt);
     }
     if (mid < whole && mid < cut) return launch_gemm_mid(epi, p, stream);
     if (whole <= cut) return launch_gemm256(epi, p, stream);

@@ -1,6 +1,10 @@
 // 256x256x64 bf16 MFMA GEMM for gfx950, 8 waves, LDS-DMA kept in flight across barriers.
 //   C = epi(A[M,K] . W[N,K]^T),  K % 128 == 0  (K-tiles are processed in pairs)
 //
+// F1 = 2 makes the tile 192 rows high (quadrant row mh = 1 has two fragments instead of four, unit U3 half its sub-tiles, one DMA piece a wave: any four consecutive units are
+// 7 pieces then, so the counted waits leave 7 in flight instead of 8).  Same sums, same bits.  It costs 0.83 of a 256-row tile's time for 0.75 of its rows; tile_us() picks it
+// where the row count leaves the last round of 256-row tiles nearly empty or the card partly idle.
+//
 // Geometry: 8 waves as 2 (M) x 4 (N); a wave owns 128 x 64 of the tile = 8 x 4 accumulators of
 // v_mfma_f32_16x16x32_bf16 (128 VGPRs).  Per K-tile (64 deep) a wave runs 4 phases of 16 MFMAs, one
 // 64 x 32 quadrant (mh, nh) of its sub-tile each: (0,0) (0,1) (1,1) (1,0), so consecutive phases reuse
@@ -73,7 +77,7 @@ constexpr int KBUF = 4 * UNIT;                    // bytes per K-tile buffer
 constexpr int LDS_MAIN2 = 2 * KBUF;               // 131072
 constexpr int LDS_BYTES2 = LDS_MAIN2 + 8 * 4096;  // + one 16x64 fp32 slice per wave = 163840 (all of the CU's LDS)
 
-#define WAIT_VM6() asm volatile("s_waitcnt vmcnt(6)" ::: "memory")
+#define WAIT_VM7() asm volatile("s_waitcnt vmcnt(7)" ::: "memory")
 #include "gemm256_diag.inc"      // WAIT_VM8 / WAIT_COLD / CR_STORE_OUT / KI_VALU and the GM256_* hooks: the product's definitions, and the diagnostic builds' (diag.hpp is the door)
 #define WAIT_VM0() asm volatile("s_waitcnt vmcnt(0)" ::: "memory")
 #define WAIT_LGKM0() __builtin_amdgcn_s_waitcnt(0xC07F)   /* lgkmcnt(0); the builtin (unlike inline asm) is seen by the compiler's own wait insertion */
@@ -193,8 +197,8 @@ __device__ __forceinline__ bf16x8 read_chunk(const char* buf, int r, int c) {
     return __builtin_bit_cast(bf16x8, w);
 }
 
-template <int EPI, bool F8 = false>
-__device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (&acc)[8][4], char* stg, int row_base, int col0,
+template <int EPI, bool F8 = false, int NF = 8>
+__device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (&acc)[NF][4], char* stg, int row_base, int col0,
                                               int lane, const char* lut = nullptr, const char* pre = nullptr) {
     constexpr bool ADD_ROWS = (EPI == EPI_LS_RES || EPI == EPI_RES);
     const bool has_bias = p.bias != nullptr;
@@ -264,7 +268,7 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
         const int r = lane & 15, g = lane >> 4;
         const int64_t blk = col0 >> 6;
 #pragma unroll
-        for (int mf = 0; mf < 8; mf++) {
+        for (int mf = 0; mf < NF; mf++) {
             float bv = -INFINITY; int bc = 0x7fffffff;
 #pragma unroll
             for (int j = 0; j < 4; j++)
@@ -287,7 +291,7 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
         const int r = lane >> 2, oc = lane & 3;
         const int gno = col0 / 2 + oc * 8;
 #pragma unroll
-        for (int mf = 0; mf < 8; mf++) {
+        for (int mf = 0; mf < NF; mf++) {
             char* buf = stg + (mf & 1) * 2048;
             stage_slice<EPI, F8>(acc[mf], bias_f, scale_f, has_bias, buf, lane, dq_f, dq_row(mf));
             __builtin_amdgcn_wave_barrier();
@@ -311,12 +315,12 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
     // HBM round trip per slice (in-kernel stamps, M = 64 575, N = K = 1024: the residual epilogue 22.6 k clocks against 6.9 k for a
     // plain store) whatever the look-ahead.
     const bool fast = full_n && (EPI == EPI_F32 ? (p.ldc & 3) == 0 : (p.ldc & 7) == 0) && (!PRE || ((p.ldr & 7) == 0 && ((uintptr_t)p.res & 15) == 0));
-    if (fast && PRE && !F8 && row_base + 128 <= p.M && (EPI != EPI_PATCH || (p.group & 7) == 0)) {
+    if (fast && PRE && !F8 && row_base + NF * 16 <= p.M && (EPI != EPI_PATCH || (p.group & 7) == 0)) {
         // Rows to add (residual stream, position embedding), interior tiles.  The counter loads and stores share only orders loads
         // among loads and stores among stores, so with both in flight hipcc has to wait with vmcnt(0): the one-slice-ahead form of
         // this loop (below; still used by the last, ragged row of tiles) waited an HBM round trip per slice -- 22.6 k clocks against
         // 6.9 k for a plain store (in-kernel stamps at M = 64 575, N = K = 1024), the same with three slices ahead.  Here the rows of
-        // FOUR slices are requested together (one wave-uniform base per 8 rows + ONE per-lane offset: no address registers), the
+        // half of the sub-tile (four slices of a 256-row tile) are requested together (one wave-uniform base per 8 rows + ONE per-lane offset: no address registers), the
         // sums replace them in their registers, the first half's stores and the second half's requests go out back to back: two
         // round trips per sub-tile instead of eight.
         const uint32_t lane_off = (uint32_t)(((int64_t)rin * p.ldr + gn) * 2);
@@ -325,19 +329,20 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
             const int64_t rrow = EPI == EPI_PATCH ? 1 + gm0 % p.group : gm0;    // (EPI_PATCH: 8 | group is this path's condition, so a piece never wraps)
             return (const char*)p.res + rrow * p.ldr * 2;
         };
-        bf16x8 rr[4][2];
+        constexpr int HF = NF / 2;
+        bf16x8 rr[HF][2];
         auto request = [&](int h) {
 #pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < HF; q++)
 #pragma unroll
-                for (int it = 0; it < 2; it++) rr[q][it] = *(const bf16x8*)(rows_at(4 * h + q, it) + lane_off);
+                for (int it = 0; it < 2; it++) rr[q][it] = *(const bf16x8*)(rows_at(HF * h + q, it) + lane_off);
         };
         auto send = [&](int h) {
 #pragma unroll
-            for (int q = 0; q < 4; q++)
+            for (int q = 0; q < HF; q++)
 #pragma unroll
                 for (int it = 0; it < 2; it++) {
-                    const int gm = row_of(4 * h + q, it);
+                    const int gm = row_of(HF * h + q, it);
                     int64_t orow = gm;
                     if (EPI == EPI_PATCH) { const int t = gm / p.group; orow = (int64_t)t * (p.group + 1) + 1 + (gm - t * p.group); }
                     __builtin_nontemporal_store(rr[q][it], (bf16x8*)((bf16*)p.C + orow * p.ldc + gn));
@@ -347,8 +352,8 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
 #pragma unroll
         for (int h = 0; h < 2; h++) {
 #pragma unroll
-            for (int q = 0; q < 4; q++) {
-                const int mf = 4 * h + q;
+            for (int q = 0; q < HF; q++) {
+                const int mf = HF * h + q;
                 char* buf = stg + (mf & 1) * 2048;
                 stage_slice<EPI, F8>(acc[mf], bias_f, scale_f, has_bias, buf, lane, dq_f, dq_row(mf), lut);
                 __builtin_amdgcn_wave_barrier();
@@ -381,11 +386,11 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
             for (int q = 0; q < RPF; q++) load_rows(q, rring[q]);
         }
 #pragma unroll
-        for (int mf = 0; mf < 8; mf++) {
+        for (int mf = 0; mf < NF; mf++) {
             char* buf = stg + (EPI == EPI_GELU ? 0 : (mf & 1) * 2048);      // the GELU instance's tables leave room for one slice per wave
             stage_slice<EPI, F8>(acc[mf], bias_f, scale_f, has_bias, buf, lane, dq_f, dq_row(mf), lut);
             __builtin_amdgcn_wave_barrier();
-            if (PRE && mf + RPF < 8) load_rows(mf + RPF, rring[(mf + RPF) % (RPF + 1)]);
+            if (PRE && mf + RPF < NF) load_rows(mf + RPF, rring[(mf + RPF) % (RPF + 1)]);
 #pragma unroll
             for (int it = 0; it < 2; it++) {
                 const int gm = row_of(mf, it);
@@ -413,7 +418,7 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
     }
     // ragged N or unaligned rows: element by element
 #pragma unroll
-    for (int mf = 0; mf < 8; mf++) {
+    for (int mf = 0; mf < NF; mf++) {
         char* buf = stg + (EPI == EPI_GELU ? 0 : (mf & 1) * 2048);
         stage_slice<EPI, F8>(acc[mf], bias_f, scale_f, has_bias, buf, lane, dq_f, dq_row(mf), lut);
         __builtin_amdgcn_wave_barrier();
@@ -436,8 +441,8 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
 }
 
 // Grouped experts: rows r0 .. of tile t (expert, first position, rows), stored to position or perm[position]; N % 64 == 0.
-template <int EPI>
-__device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x4 (&acc)[8][4], char* stg, const int4 t, int r0, int col0, int lane) {
+template <int EPI, int NF>
+__device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x4 (&acc)[NF][4], char* stg, const int4 t, int r0, int col0, int lane) {
     if (col0 + 64 > p.N) return;                              // (wave-uniform)
     const int r = lane & 15, g = lane >> 4;
     typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
@@ -446,7 +451,7 @@ __device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x
         // row r at s ^ (r & 7)
         const int rr = lane >> 2, cc = lane & 3;
 #pragma unroll
-        for (int mf = 0; mf < 8; mf++) {
+        for (int mf = 0; mf < NF; mf++) {
             char* buf = stg + (mf & 1) * 1024;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
@@ -471,7 +476,7 @@ __device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x
     }
     const int rin = lane >> 3, c = lane & 7;
 #pragma unroll
-    for (int mf = 0; mf < 8; mf++) {
+    for (int mf = 0; mf < NF; mf++) {
         char* buf = stg + (mf & 1) * 2048;
 #pragma unroll
         for (int j = 0; j < 4; j++)
@@ -551,8 +556,9 @@ __device__ __forceinline__ i32x8 f8_put(const i32x8& v, int ks, const bf16x8& fr
 // of 128 bytes per row is 128 k instead of 64, and a matrix slot issues 8 v_mfma_scale_f32_16x16x128_f8f6f4 (unit block
 // scales, 32 cycles each) where the bf16 kernel issues 16 v_mfma_f32_16x16x32_bf16 (16 cycles each): the same slot length at
 // twice the k.  The per-row / per-column fp32 scales are applied to the finished sum in the epilogue.
-template <int EPI, bool F8 = false, bool BIG = false>
+template <int EPI, bool F8 = false, bool BIG = false, int F1 = 4>
 __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
+    constexpr int RW = 64 + F1 * 16, TM = 2 * RW;     // a wave's rows: 4 fragments of quadrant row mh = 0 and F1 of mh = 1; the tile's rows
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -560,7 +566,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     const int wm = wave >> 2, wn = wave & 3;
 
     constexpr bool GRP = EPI == EPI_X_GLU || EPI == EPI_X_ROWS;         // grouped experts: m0 is an index into p.tiles
-    const int ntm = GRP ? *p.n_tiles : (p.M + BM2 - 1) / BM2, ntn = (p.N + BN2 - 1) / BN2;
+    const int ntm = GRP ? *p.n_tiles : (p.M + TM - 1) / TM, ntn = (p.N + BN2 - 1) / BN2;
     const int ntiles = ntm * ntn;
     const int nk = p.K / BK2;
 
@@ -574,7 +580,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
         const int first_m = grp * GM;
         const int gsz = min(ntm - first_m, GM);
         const int in_g = pid - grp * per_group;
-        m0 = (first_m + in_g % gsz) * (GRP ? 1 : BM2);
+        m0 = (first_m + in_g % gsz) * (GRP ? 1 : TM);
         n0 = (in_g / gsz) * BN2;
     };
 
@@ -587,6 +593,8 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     const int schunk = (lane & 3) ^ ((srow >> 3) << 1);
     uint32_t qA[2];           // [mh]   offsets used by phases 2..8 (may already be the NEXT tile's); piece e = 1 is 64 B on
     uint32_t qB[2];           // [nh]
+    // first row of the fragment that this wave stages of A's quadrant row h; F1 = 2: U3 is 8 sub-tiles, one a wave: (wave row wave>>2, fragment (wave>>1)&1, ksub wave&1)
+    auto a_row = [&](int h) { return (wave >> 2) * RW + h * 64 + (h && F1 == 2 ? (wave >> 1) & 1 : wave & 3) * 16; };
     auto make_ptrs = [&](int m0, int n0) {
         // sub-tiles 2*wave and 2*wave + 1 are the two k-halves (ksub 0 / 1) of the same 16 rows
         int srow = lane >> 2, schunk = (lane & 3) ^ ((srow >> 3) << 1);
@@ -600,7 +608,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
             const int4 t = p.tiles[m0];
 #pragma unroll
             for (int h = 0; h < 2; h++) {
-                const int pos = t.y + min((wave >> 2) * 128 + h * 64 + (wave & 3) * 16 + srow, t.z - 1);
+                const int pos = t.y + min(a_row(h) + srow, t.z - 1);
                 const int arow = p.gather_div ? p.perm[pos] / p.gather_div : pos;
                 const int bblk = min((n0 + (wave >> 1) * 64 + h * 32 + (wave & 1) * 16) >> 4, (p.N >> 4) - 1);
                 qA[h] = (uint32_t)(((int64_t)arow * p.lda + schunk * 8) * 2);
@@ -610,7 +618,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
         }
 #pragma unroll
         for (int h = 0; h < 2; h++) {
-            const int arow = m0 + (wave >> 2) * 128 + h * 64 + (wave & 3) * 16 + srow;
+            const int arow = m0 + a_row(h) + srow;
             const int brow = n0 + (wave >> 1) * 64 + h * 32 + (wave & 1) * 16 + srow;
             qA[h] = (uint32_t)(((int64_t)min(arow, p.M - 1) * p.lda + schunk * 8) * 2);
             qB[h] = (uint32_t)(((int64_t)min(brow, p.N - 1) * p.ldw + schunk * 8) * 2);
@@ -618,6 +626,12 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
         }
     };
     auto dma = [&](const bf16* base, uint32_t o, int kt, int buf, int u) {
+        if (F1 == 2 && u == 3) {
+            char* dst = smem + buf * KBUF + 3 * UNIT + wave * 1024;
+            GM256_DIAG_POISON(dst)
+            __builtin_amdgcn_global_load_lds(CR_GLB((const char*)base + (int64_t)kt * (BK2 * 2) + (wave & 1) * 64 + o), CR_LDS(dst), 16, 0, 0);
+            return;
+        }
         char* dst = smem + buf * KBUF + u * UNIT + (2 * wave) * 1024;
         if (GRP && (u == 1 || u == 2)) {                      // fragment blocks: consecutive k-steps of 32 are consecutive KiB
             const char* src = (const char*)base + (int64_t)kt * 2048;
@@ -626,6 +640,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
             return;
         }
         GM256_DIAG_POISON(dst)
+        GM256_DIAG_POISON(dst + 1024)
         const char* src = (const char*)base + (int64_t)kt * (BK2 * 2);
         GM256_DIAG_ALT_DMA(base, src, o, dst, kt)
         __builtin_amdgcn_global_load_lds(CR_GLB(src + o), CR_LDS(dst), 16, 0, 0);
@@ -635,7 +650,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
 
     const int lrow = lane & 15;
     const int lane_off = lrow * 64 + (((lane >> 4) ^ ((lrow >> 3) << 1)) * 16);
-    int a_sub = wm * 8 * 1024 + lane_off;                // + (i*2 + ksub) * 1024
+    int a_sub = wm * 8 * 1024 + lane_off;                // + (i*2 + ksub) * 1024; U3: (wm * F1 + i) * 2 + ksub
     int b_sub = wn * 4 * 1024 + lane_off;                // + (j*2 + ksub) * 1024
     char* stg = smem + LDS_MAIN2 + wave * 4096;       // epilogue: two 2 KiB bf16 slices per wave
     const char* lut = nullptr;
@@ -644,15 +659,15 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
         stg = smem + LDS_MAIN2 + (wave == 0 ? 2 * LUT_N : 8192 + 2 * LUT_N + (wave - 1) * 2048);
     }
 
-    f32x4 acc[8][4];
+    f32x4 acc[4 + F1][4];
     bf16x8 ra[4][2];          // A fragments of the current quadrant row: [i][ksub]
     bf16x8 rb[2][2][2];       // B fragments: [nh][j][ksub]
     i32x8 ra8[4] = {};        // F8: the same fragments as 32-byte operands [i], [nh][j]
     i32x8 rb8[2][2] = {};
 
 #define READ_A(buf, unit)                                                                       \
-    _Pragma("unroll") for (int i = 0; i < 4; i++) _Pragma("unroll") for (int ks = 0; ks < 2; ks++) \
-        { const bf16x8 f_ = *(const bf16x8*)(smem + (buf) * KBUF + (unit) * UNIT + a_sub + (i * 2 + ks) * 1024); \
+    _Pragma("unroll") for (int i = 0; i < ((unit) == 3 ? F1 : 4); i++) _Pragma("unroll") for (int ks = 0; ks < 2; ks++) \
+        { const bf16x8 f_ = *(const bf16x8*)(smem + (buf) * KBUF + (unit) * UNIT + a_sub - ((unit) == 3 ? wm * (4 - F1) * 2048 : 0) + (i * 2 + ks) * 1024); \
           if (F8) ra8[i] = f8_put(ra8[i], ks, f_); else ra[i][ks] = f_; }
 #define READ_B(buf, unit, nh)                                                                   \
     _Pragma("unroll") for (int j = 0; j < 2; j++) _Pragma("unroll") for (int ks = 0; ks < 2; ks++) \
@@ -666,7 +681,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     DMA;                                                                                        \
     KI_VALU();                                                                                  \
     __builtin_amdgcn_sched_barrier(0);                                                          \
-    if (WAIT) WAIT_VM8();                                                                       \
+    if (WAIT) { if (F1 == 4) WAIT_VM8(); else WAIT_VM7(); }                                       \
     WAIT_LGKM0();                                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                          \
     __builtin_amdgcn_s_barrier();
@@ -675,18 +690,18 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     DMA;                                                                                        \
     KI_VALU();                                                                                  \
     __builtin_amdgcn_sched_barrier(0);                                                          \
-    if (WAIT) WAIT_VM8();                                                                       \
+    if (WAIT) { if (F1 == 4) WAIT_VM8(); else WAIT_VM7(); }                                       \
     __builtin_amdgcn_s_barrier();
 #define MFMA_SLOT(mh, nh)                                                                       \
     WAIT_LGKM0();                                                                               \
     __builtin_amdgcn_sched_barrier(0);                                                          \
     __builtin_amdgcn_s_setprio(1);                                                              \
     if (F8) {                                                                                   \
-        _Pragma("unroll") for (int i = 0; i < 4; i++) _Pragma("unroll") for (int j = 0; j < 2; j++) \
+        _Pragma("unroll") for (int i = 0; i < ((mh) ? F1 : 4); i++) _Pragma("unroll") for (int j = 0; j < 2; j++) \
             acc[(mh) * 4 + i][(nh) * 2 + j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(  \
                 rb8[nh][j], ra8[i], acc[(mh) * 4 + i][(nh) * 2 + j], 0, 0, 0, 0, 0, 0); \
     } else {                                                                                    \
-        _Pragma("unroll") for (int ks = 0; ks < 2; ks++) _Pragma("unroll") for (int i = 0; i < 4; i++) \
+        _Pragma("unroll") for (int ks = 0; ks < 2; ks++) _Pragma("unroll") for (int i = 0; i < ((mh) ? F1 : 4); i++) \
             _Pragma("unroll") for (int j = 0; j < 2; j++)                                       \
                 acc[(mh) * 4 + i][(nh) * 2 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rb[nh][j][ks], ra[i][ks], acc[(mh) * 4 + i][(nh) * 2 + j], 0, 0, 0); \
     }                                                                                           \
@@ -695,11 +710,11 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     __builtin_amdgcn_s_barrier();
 #define MFMA_QUAD(mh, nh)                                                                       \
     if (F8) {                                                                                   \
-        _Pragma("unroll") for (int i = 0; i < 4; i++) _Pragma("unroll") for (int j = 0; j < 2; j++) \
+        _Pragma("unroll") for (int i = 0; i < ((mh) ? F1 : 4); i++) _Pragma("unroll") for (int j = 0; j < 2; j++) \
             acc[(mh) * 4 + i][(nh) * 2 + j] = __builtin_amdgcn_mfma_scale_f32_16x16x128_f8f6f4(  \
                 rb8[nh][j], ra8[i], acc[(mh) * 4 + i][(nh) * 2 + j], 0, 0, 0, 0, 0, 0); \
     } else {                                                                                    \
-        _Pragma("unroll") for (int ks = 0; ks < 2; ks++) _Pragma("unroll") for (int i = 0; i < 4; i++) \
+        _Pragma("unroll") for (int ks = 0; ks < 2; ks++) _Pragma("unroll") for (int i = 0; i < ((mh) ? F1 : 4); i++) \
             _Pragma("unroll") for (int j = 0; j < 2; j++)                                       \
                 acc[(mh) * 4 + i][(nh) * 2 + j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(rb[nh][j][ks], ra[i][ks], acc[(mh) * 4 + i][(nh) * 2 + j], 0, 0, 0); \
     }
@@ -736,7 +751,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
             b_sub = wn * 4 * 1024 + off;
         }
 #pragma unroll
-        for (int i = 0; i < 8; i++)
+        for (int i = 0; i < 4 + F1; i++)
 #pragma unroll
             for (int j = 0; j < 4; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
         const int t_next = t_cur + gridDim.x;
@@ -820,9 +835,9 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
         GM256_STAMP(2)       // the look-ahead (K-tile 0 and U0, U1 of K-tile 1 of the next tile) has landed: slots 1..4 rely on it
 
         // ---- epilogue: eight 16-row slices per wave through its private 4 KiB (the K buffers stay untouched) ----
-        GM256_EPILOGUE(if constexpr (GRP) epilogue_grouped<EPI>(p, acc, stg, p.tiles[m0], wm * 128, n0 + wn * 64, lane);
-                       else if (EPI == EPI_GELU_Q8) epilogue_gelu_q8(p, acc, stg, m0 + wm * 128, n0 + wn * 64, lane);
-                       else epilogue_tile<EPI, F8>(p, acc, stg, m0 + wm * 128, n0 + wn * 64, lane, lut, pre_ok ? stg : nullptr);)
+        GM256_EPILOGUE(if constexpr (GRP) epilogue_grouped<EPI>(p, acc, stg, p.tiles[m0], wm * RW, n0 + wn * 64, lane);
+                       else if constexpr (EPI == EPI_GELU_Q8) epilogue_gelu_q8(p, acc, stg, m0 + wm * 128, n0 + wn * 64, lane);
+                       else epilogue_tile<EPI, F8>(p, acc, stg, m0 + wm * RW, n0 + wn * 64, lane, lut, pre_ok ? stg : nullptr);)
         GM256_STAMP_END
         if (!has_next) break;
         t_cur = t_next;
@@ -831,14 +846,25 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     WAIT_VM0();       // dead re-loads of the final pair must land before the workgroup releases its LDS
 }
 
-template <int EPI, bool F8, bool BIG>
+template <int EPI, bool F8, bool BIG, int F1 = 4>
 int launch_s(const GemmParams& p, hipStream_t stream) {
-    const int ntiles = ((p.M + BM2 - 1) / BM2) * ((p.N + BN2 - 1) / BN2);
+    constexpr int TM = 128 + 32 * F1;
+    const int ntiles = ((p.M + TM - 1) / TM) * ((p.N + BN2 - 1) / BN2);
     static std::atomic<uint64_t> attr_done{0};
-    if (!cr_dyn_lds_once(attr_done, (const void*)gemm256_kernel<EPI, F8, BIG>, LDS_BYTES2)) return CR_ERR_HIP;
+    if (!cr_dyn_lds_once(attr_done, (const void*)gemm256_kernel<EPI, F8, BIG, F1>, LDS_BYTES2)) return CR_ERR_HIP;
     const int n_cu = cr_device_cus();
-    hipLaunchKernelGGL((gemm256_kernel<EPI, F8, BIG>), dim3(ntiles < n_cu ? ntiles : n_cu), dim3(512), LDS_BYTES2, stream, p);
+    hipLaunchKernelGGL((gemm256_kernel<EPI, F8, BIG, F1>), dim3(ntiles < n_cu ? ntiles : n_cu), dim3(512), LDS_BYTES2, stream, p);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
+}
+
+// us of a launch of tiles of 256 (f1 = 4) or 192 rows (2), on the scale of gemm_mid_cost: rounds of one tile per CU, a K-tile of 256 rows 1.12 us (1000 x 4096 x 14336 takes
+// 251 us), of 192 rows 0.93 (203 us).  The shorter tile wins where it takes no more rounds (x 256 rows / 192 rows, us): 11275 x 3072 x 1024 (540 / 708 tiles) 73.7 / 62.8,
+// 11275 x 1024 x 4096 (180 / 236) 82.5 / 74.8, 8200 x 4096 x 1024 (528 / 688) 83.3 / 71.0, 6000 x 4096 x 14336 (384 / 512) 587 / 495; it loses where it takes one more:
+// 13325 x 1024 x 4096 (212 / 280) 91 / 130, 11275 x 4096 x 1024 (720 / 944) 89 / 94, 4700 x 28672 x 4096 (2128 / 2800) 799 / 811.
+double tile_us(const GemmParams& p, int f1) {
+    const int tm = 128 + 32 * f1;
+    const long tiles = (long)((p.M + tm - 1) / tm) * ((p.N + BN2 - 1) / BN2), cus = cr_device_cus();
+    return 3.5 + (double)((tiles + cus - 1) / cus) * (f1 == 4 ? p.K / BK2 * 1.12 + 3.0 : p.K / BK2 * 0.93 + 2.6);
 }
 
 // Two schedules of the same sums (bit-identical results): 32-MFMA matrix slots measured 2-5 % faster on the wide outputs at K <= 4096 (ViT QKV
@@ -849,7 +875,10 @@ int launch_t(const GemmParams& p, hipStream_t stream) {
     static const int pin = [] { const char* e = getenv("CR_GEMM_SLOTS"); return e ? atoi(e) : 0; }();
     const int want = p.slots ? p.slots : pin;
     const bool big = !F8 && (want == 32 || (want != 16 && p.N >= 2048 && p.K <= 8192));
-    if constexpr (!F8) { if (big) return launch_s<EPI, false, true>(p, stream); }
+    if constexpr (!F8) {
+        if (p.tile ? p.tile == 192 : tile_us(p, 2) < tile_us(p, 4)) return big ? launch_s<EPI, false, true, 2>(p, stream) : launch_s<EPI, false, false, 2>(p, stream);
+        if (big) return launch_s<EPI, false, true>(p, stream);
+    }
     return launch_s<EPI, F8, false>(p, stream);
 }
 
@@ -857,11 +886,7 @@ int launch_t(const GemmParams& p, hipStream_t stream) {
 
 bool gemm256_supported(int epi, const GemmParams& p) { return epi != EPI_PARTIAL && p.N >= 64 && p.K % 128 == 0 && !p.raw32; }
 
-// us of a launch, on the scale of gemm_mid_cost: rounds of one tile per CU, a K-tile 1.15 us of operand bytes (512 rows; 700 x 4096 x 14336 takes 244 us, 8200 x 1024 x 4096 75)
-double gemm256_cost(int epi, const GemmParams& p) {
-    const long tiles = (long)((p.M + BM2 - 1) / BM2) * ((p.N + BN2 - 1) / BN2), cus = cr_device_cus();
-    return 3.5 + (double)((tiles + cus - 1) / cus) * (p.K / BK2 * 1.12 + 3.0);
-}
+double gemm256_cost(const GemmParams& p) { const double a = tile_us(p, 4), b = tile_us(p, 2); return a < b ? a : b; }
 
 int launch_gemm256_grouped(int epi, const GemmParams& p, hipStream_t stream) {
     if (p.K <= 0 || p.K % 128 || p.N < 64 || p.N % 64 || (p.lda & 7) || (p.ldc & 7) || !p.tiles || !p.n_tiles || p.max_tiles <= 0 || ((p.gather_div || p.scatter) && !p.perm) ||

@@ -352,7 +352,7 @@ class KVCache:
 # ---- single operators (tests / profiling) ----
 def op_gemm(epi, A, Wt, bias=None, scale=None, res=None, group=0, out_dtype=torch.bfloat16, n_out=None, kernel=0, out=None, decode_layout=None):
     """kernel: 0 dispatcher's choice, 1 gemm_mid (16 + i: its tile shape i), 2 256x256 persistent (schedule per shape), 3 weight-streaming, 5 / 6 the 256x256 kernel with
-    its 16- / 32-MFMA-slot schedule pinned (tests pin one).  decode_layout = (kind, op_decode_swizzle(which, Wt)): the weight-streaming kernels
+    its 16- / 32-MFMA-slot schedule pinned, 7 / 8 the same with its 192-row tiles (tests pin one).  decode_layout = (kind, op_decode_swizzle(which, Wt)): the weight-streaming kernels
     (M <= 64) read that copy of the weight (kind 1: plain tiles, 2: wqkv's RoPE tile order with epi 7); Wt still gives N."""
     M, K = A.shape
     N = Wt.shape[0]

@@ -274,7 +274,7 @@ int cr_orderformer(cr_ctx* ctx, const void* boxes, int B, int L, float* scores, 
  * 8 row arg-max partials (cosine VQ: C = uint64 [M][ldc], one per row and 64-column block: bits of the bf16-rounded maximum in the
  *   high word, its first column in the low word; M > 64 tile kernels only).
  * Bits 8..15 of epi pin a kernel for the unit tests: 0 dispatcher's choice, 1 the kernel of many tile shapes (gemm_mid.hip; from 16 on one of its shapes), 2 256x256 persistent,
- * 3 weight-streaming (M <= 64), 5 / 6 the 256x256 kernel with its 16- / 32-MFMA-slot schedule (the same sums: the same bits);
+ * 3 weight-streaming (M <= 64), 5 / 6 the 256x256 kernel with its 16- / 32-MFMA-slot schedule, 7 / 8 the same with 192 rows a tile (the same sums: the same bits);
  * a pinned kernel that cannot take the shape returns CR_ERR_ARG.
  * Bits 18-19 (M <= 64, bf16 weights, the weight-streaming kernels): W is cr_op_decode_swizzle's copy of the weight (ldw ignored) -- 1: plain 16-row
  * tiles (its which = 1..4), 2: wqkv's RoPE tile order (which = 0; epi 7 only: the K-slices still land in their nn.Linear columns).  The same bits as
