@@ -444,6 +444,7 @@ __device__ __forceinline__ void epilogue_tile(const GemmParams& p, const f32x4 (
 template <int EPI, int NF>
 __device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x4 (&acc)[NF][4], char* stg, const int4 t, int r0, int col0, int lane) {
     if (col0 + 64 > p.N) return;                              // (wave-uniform)
+    asm volatile("" : "+v"(lane));                            // nothing of what follows is worked out ahead of the main loop: its registers are full (18 to 30 spills otherwise, 7 to 15 % of the launch)
     const int r = lane & 15, g = lane >> 4;
     typedef __attribute__((ext_vector_type(4))) unsigned u32x4;
     if (EPI == EPI_X_GLU) {
@@ -455,10 +456,14 @@ __device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x
             char* buf = stg + (mf & 1) * 1024;
 #pragma unroll
             for (int j = 0; j < 4; j++) {
-                bf16x4 o;
+                // halves of the wave trade: lanes 0..31 then hold gates and ups of their columns 0, 1 and lanes 32..63 those of columns 2, 3 of the lane 32 below
+                bf16x2 o;
 #pragma unroll
-                for (int e = 0; e < 4; e++) o[e] = f2bf(clamped_glu(acc[mf][j][e], __shfl_xor(acc[mf][j][e], 32, 64), p.limit));
-                if (g < 2) *(bf16x4*)(buf + r * 64 + (((j * 2 + g) ^ (r & 7)) << 3)) = o;
+                for (int e = 0; e < 2; e++) {
+                    const auto s = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[mf][j][e]), __float_as_uint(acc[mf][j][e + 2]), false, false);
+                    o[e] = f2bf(clamped_glu(__uint_as_float(s[0]), __uint_as_float(s[1]), p.limit));
+                }
+                *(bf16x2*)(buf + r * 64 + (((j * 2 + (g & 1)) ^ (r & 7)) << 3) + (g >> 1) * 4) = o;
             }
             __builtin_amdgcn_wave_barrier();
             const u32x4 v = *(const u32x4*)(buf + rr * 64 + ((cc ^ ((rr & 7) >> 1)) << 4));
@@ -466,15 +471,20 @@ __device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x
             const u32x4 w = {odd ? v[2] : v[0], odd ? v[3] : v[1], odd ? v[0] : v[2], odd ? v[1] : v[3]};
             const int row = r0 + mf * 16 + rr;
             if (row < t.z) {
-                const int pos = t.y + row;
-                const int64_t orow = p.scatter ? p.perm[pos] : pos;
-                __builtin_nontemporal_store(w, (u32x4*)((bf16*)p.C + orow * p.ldc + col0 / 2 + cc * 8));
+                __builtin_nontemporal_store(w, (u32x4*)((bf16*)p.C + (int64_t)(t.y + row) * p.ldc + col0 / 2 + cc * 8));
             }
             __builtin_amdgcn_wave_barrier();
         }
         return;
     }
     const int rin = lane >> 3, c = lane & 7;
+    // every output row's place up front (lane i: rows i and 64 + i), dealt out by shuffles: a load per slice would wait for all the slices' stores before it, as vmcnt is in order
+    int place[2];
+#pragma unroll
+    for (int h = 0; h < 2; h++) {
+        const int pos = t.y + min(r0 + h * 64 + lane, t.z - 1);
+        place[h] = p.scatter ? p.perm[pos] : pos;
+    }
 #pragma unroll
     for (int mf = 0; mf < NF; mf++) {
         char* buf = stg + (mf & 1) * 2048;
@@ -486,11 +496,8 @@ __device__ __forceinline__ void epilogue_grouped(const GemmParams& p, const f32x
         for (int it = 0; it < 2; it++) {
             const int row = r0 + mf * 16 + it * 8 + rin;
             const bf16x8 v = read_chunk(buf, it * 8 + rin, c);
-            if (row < t.z) {
-                const int pos = t.y + row;
-                const int64_t orow = p.scatter ? p.perm[pos] : pos;
-                __builtin_nontemporal_store(v, (bf16x8*)((bf16*)p.C + orow * p.ldc + col0 + c * 8));
-            }
+            const int64_t orow = __shfl(place[mf >> 2], (mf & 3) * 16 + it * 8 + rin, 64);
+            if (row < t.z) __builtin_nontemporal_store(v, (bf16x8*)((bf16*)p.C + orow * p.ldc + col0 + c * 8));
         }
         __builtin_amdgcn_wave_barrier();
     }
@@ -575,6 +582,12 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
         const int xcd = orig & 7, q = ntiles >> 3, r = ntiles & 7;
         const int pid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
         constexpr int GM = GM256_TILE_GM;                     // 8 (gemm256_diag.inc: CR_TILE_GM for scripts/traffic_clock.py)
+        if constexpr (GRP) {                                  // row tiles of ONE expert together (at most 8; the plan says which): 32 tiles that run on an XCD then share weight panels
+            const int r = pid / ntn, w = p.tiles[r].w, first = r - (w & 15), in_g = pid - first * ntn;
+            m0 = first + in_g % (w >> 4);
+            n0 = (in_g / (w >> 4)) * BN2;
+            return;
+        }
         const int per_group = GM * ntn;
         const int grp = pid / per_group;
         const int first_m = grp * GM;
@@ -598,21 +611,27 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     auto make_ptrs = [&](int m0, int n0) {
         // sub-tiles 2*wave and 2*wave + 1 are the two k-halves (ksub 0 / 1) of the same 16 rows
         int srow = lane >> 2, schunk = (lane & 3) ^ ((srow >> 3) << 1);
-        if (F8) {                                             // the e4m3 instance has no register to keep these across a tile: derive them again
+        if (F8 || GRP) {                                      // the e4m3 and grouped instances have no register to keep these across a tile: derive them again
             int l = tid;
             asm volatile("" : "+v"(l));
             l &= 63;
             srow = l >> 2; schunk = (l & 3) ^ ((srow >> 3) << 1);
         }
         if constexpr (GRP) {
+            // weight blocks are MFMA operands as a lane reads them (lane -> row lane & 15, chunk lane >> 4): they come in lane order, so that four lanes share a 64-byte piece of a
+            // line, and lie so in LDS.  Brought into the A units' row order instead, every lane of a quad fetched from another line and the loads
+            // bound the kernel: 24 496 rows over 32 experts, N = K = 2048 258 -> 222 us, N = 2048 and K = 1024 138 -> 123.
             const int4 t = p.tiles[m0];
+            int blane = tid;
+            asm volatile("" : "+v"(blane));
+            blane &= 63;
 #pragma unroll
             for (int h = 0; h < 2; h++) {
                 const int pos = t.y + min(a_row(h) + srow, t.z - 1);
                 const int arow = p.gather_div ? p.perm[pos] / p.gather_div : pos;
                 const int bblk = min((n0 + (wave >> 1) * 64 + h * 32 + (wave & 1) * 16) >> 4, (p.N >> 4) - 1);
                 qA[h] = (uint32_t)(((int64_t)arow * p.lda + schunk * 8) * 2);
-                qB[h] = (uint32_t)(((int64_t)t.x * p.expert_stride + ((int64_t)bblk * (p.K >> 5) * 64 + schunk * 16 + srow) * 8) * 2);
+                qB[h] = (uint32_t)(((int64_t)t.x * p.expert_stride + ((int64_t)bblk * (p.K >> 5) * 64 + blane) * 8) * 2);
             }
             return;
         }
@@ -743,12 +762,12 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     __builtin_amdgcn_s_barrier();
 
     while (true) {
-        if (F8) {           // not kept across the epilogue (no register to spare there: a spilled copy would drain vmcnt at the tile's start)
+        if (F8 || GRP) {    // not kept across the epilogue (no register to spare there: a spilled copy would drain vmcnt at the tile's start)
             int l = tid;
             asm volatile("" : "+v"(l));
             const int r16 = l & 15, off = r16 * 64 + ((((l & 63) >> 4) ^ ((r16 >> 3) << 1)) * 16);
             a_sub = wm * 8 * 1024 + off;
-            b_sub = wn * 4 * 1024 + off;
+            b_sub = wn * 4 * 1024 + (GRP ? (l & 63) * 16 : off);
         }
 #pragma unroll
         for (int i = 0; i < 4 + F1; i++)
@@ -893,7 +912,7 @@ int launch_gemm256_grouped(int epi, const GemmParams& p, hipStream_t stream) {
         (((uintptr_t)p.A | (uintptr_t)p.W | (uintptr_t)p.C) & 15))
         return CR_ERR_ARG;
     switch (epi) {
-        case EPI_X_GLU: return launch_s<EPI_X_GLU, false, true>(p, stream);
+        case EPI_X_GLU: return p.scatter ? CR_ERR_ARG : launch_s<EPI_X_GLU, false, true>(p, stream);
         case EPI_X_ROWS: return launch_s<EPI_X_ROWS, false, true>(p, stream);
     }
     return CR_ERR_ARG;

@@ -230,7 +230,7 @@ __global__ __launch_bounds__(1024) void lm_plan_kernel(const int32_t* __restrict
     __syncthreads();
     cur[tid] = off;
     for (int k = 0; k < t; k++)
-        if (t0 + k < max_tiles) tiles[t0 + k] = make_int4(tid, off + k * tile_m, min(tile_m, c - k * tile_m), 0);
+        if (t0 + k < max_tiles) tiles[t0 + k] = make_int4(tid, off + k * tile_m, min(tile_m, c - k * tile_m), (k & 7) | min(8, t - (k & ~7)) << 4);
     __syncthreads();
     for (int i0 = tid; i0 < n; i0 += 8192) {
         int e[8], at[8];
