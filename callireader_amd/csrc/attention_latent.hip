@@ -23,7 +23,7 @@ __global__ __launch_bounds__(TPB) void latent_attn_plain_kernel(const LatentAttn
 }
 template <typename T>
 void launch_plain_t(const LatentAttnParams& p, hipStream_t st) {
-    if ((int64_t)p.M * p.H <= 1024) hipLaunchKernelGGL((latent_attn_plain_kernel<T, 1024>), dim3(p.M, p.H), dim3(1024), plain_lds_floats(p.Rp, 1024) * 4, st, p);
+    if (!p.ix.row_pos) hipLaunchKernelGGL((latent_attn_plain_kernel<T, 1024>), dim3(p.M, p.H), dim3(1024), plain_lds_floats(p.Rp, 1024) * 4, st, p);
     else hipLaunchKernelGGL((latent_attn_plain_kernel<T, 256>), dim3(p.M, p.H), dim3(256), plain_lds_floats(p.Rp, 256) * 4, st, p);
 }
 

@@ -2,7 +2,7 @@
 //
 // Bound by the latency of its loads when rows are few (16 workgroups for two rows of eight heads), so the loads are wide, many and coalesced: sixteen lanes share a key in q . k (64
 // elements a load round), a column quad per thread in P . V with the keys dealt over the thread groups that are left, four keys' loads in flight in both.  With one key per thread and
-// one column per thread instead, a row of 213 keys of 128 columns took 29 us; now 9.2 (1024 threads), and 402 prompt
+// one column per thread instead, a row of 213 keys of 128 columns took 29 us; now 9.2 (1024 threads, decode), and 402 prompt
 // rows 27 us for 37 (256 threads: the chip is full of workgroups).
 #pragma once
 #include "common.hpp"

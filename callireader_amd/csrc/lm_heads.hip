@@ -182,8 +182,9 @@ __global__ __launch_bounds__(TPB) void heads_attn_plain_kernel(const HeadsAttnPa
 
 template <typename T>
 void launch_plain_t(const HeadsAttnParams& p, hipStream_t st) {
-    // few workgroups: sixteen waves each (a row's chain of loads is what counts); many: four, and the chip is full
-    if ((int64_t)p.M * p.H <= 1024) hipLaunchKernelGGL((heads_attn_plain_kernel<T, 1024>), dim3(p.M, p.H), dim3(1024), plain_lds_floats(p.Ap, 1024) * 4, st, p);
+    // decode: few workgroups, sixteen waves each (a row's chain of loads is what counts); prompts: four, the chip is full.  (Not by the number of rows: the waves share a row's sums
+    // out, and a row's bits must not depend on what it is computed with.)
+    if (!p.ix.row_pos) hipLaunchKernelGGL((heads_attn_plain_kernel<T, 1024>), dim3(p.M, p.H), dim3(1024), plain_lds_floats(p.Ap, 1024) * 4, st, p);
     else hipLaunchKernelGGL((heads_attn_plain_kernel<T, 256>), dim3(p.M, p.H), dim3(256), plain_lds_floats(p.Ap, 256) * 4, st, p);
 }
 

@@ -39,3 +39,40 @@ def test_fp32_long_context_decode():
         z = torch.cat([m.step([('r', [x], [0])]) for x in t[-3:]]).cpu()
         m.close()
         assert cases.rel(z, oracle.forward(w, cfg, t)[-3:]) < 1e-4      # (angles of a thousand radians: 6e-5 radians of fp32 rounding)
+
+
+@pytest.mark.parametrize('rows', [1, 16, 17, 49, 127, 129, 290, 1030])
+@pytest.mark.parametrize('name', ['lugasun', 'linasun'])
+def test_fp32_prompt_rows(name, rows):
+    """Prompts in float32: row counts around the row tiles' fragments (16) and heights, widths that leave columns over in every tile shape, a K of one K-tile, of odd and even numbers of
+    them; the last rows and some inside against the oracle, and the same bits whatever else is prefilled with them."""
+    from callireader_amd import modeling_decoder as MD
+    if name == 'lugasun':
+        cases, oracle, cls = LUG, OLUG, MD.LugasunForCausalLM
+        cfg = LUG.config(192, 300, [LUG.layer(LUG.heads(3, 1, 64, 40, 4096), LUG.ret(64, 72, (0.9,)), 328)], side=20)
+    else:
+        cases, oracle, cls, cfg = LIN, OLIN, MD.LinasunForCausalLM, LIN.config(320, 300, [(LIN.mixer(3, 64, 72, 96, 64, 0.15), LIN.moe(3, 2, 200, 1.5))])
+    w = cases.weights(cfg, 43)
+    m = cls.from_state_dict(w, cfg, dtype=torch.float32, max_tokens=rows, max_seqs=2)
+    t, want = cases.tokens(cfg, rows, seed=5), sorted({0, rows // 3, max(rows - 17, 0), rows - 1})
+    z = m.step([('a', t, want)]).cpu()
+    m.end('a')
+    both = m.step([('a', t, want), ('b', t[:min(rows, 70)], [0])]).cpu()
+    m.close()
+    assert cases.rel(z, oracle.forward(w, cfg, t)[want]) < 2e-5
+    assert torch.equal(both[:len(want)], z)
+
+
+@pytest.mark.parametrize('name', ['lugasun_huge', 'linasun_many_heads'])
+def test_fp32_decode_row_alone_and_among_others(name):
+    from callireader_amd import modeling_decoder as MD
+    cases, _, cfg = CASES[name]
+    cls = MD.LugasunForCausalLM if cases is LUG else MD.LinasunForCausalLM
+    m = cls.from_state_dict(cases.weights(cfg, 44), cfg, dtype=torch.float32, max_tokens=48, max_seqs=61)
+    toks = [cases.tokens(cfg, 3 + 7 * i % 40, seed=i) for i in range(60)]
+    m.step([(i, t[:-1], []) for i, t in enumerate(toks)])
+    z = m.step([(i, t[-1:], [0]) for i, t in enumerate(toks)]).cpu()
+    m.step([('a', toks[7][:-1], [])])
+    alone = m.step([('a', toks[7][-1:], [0])]).cpu()
+    m.close()
+    assert torch.equal(alone[0], z[7])
