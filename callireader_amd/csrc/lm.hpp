@@ -87,13 +87,14 @@ struct LmGemmParams {
     float softcap, limit;
     const void* gate; int64_t ldg;
     const int32_t* tok;
-    int stream;                                     // fp32, M <= LM_ROWS_MAX (grouped: M = the tokens, an expert sees at most that many): lm_gemm_rows.hip
+    int stream;                                     // fp32, M <= LM_ROWS_MAX (grouped: M = the tokens, an expert sees at most that many): lm_gemm_rows.hip's few-row form
     int slices;                                     // stream, LM_RAW32: K-slices C [slices][M][ldc] for a consumer that adds them
 };
 int launch_lm_gemm(bool f32, int epi, const LmGemmParams& p, hipStream_t st);
 constexpr int LM_TILE_M = 64;
 constexpr int LM_ROWS_MAX = 64, LM_ROWS_MAX_SLICES = 8;
 int launch_lm_gemm_rows(int epi, const LmGemmParams& p, hipStream_t st);
+int launch_lm_gemm_tiles(int epi, const LmGemmParams& p, hipStream_t st);
 int lm_rows_slices(int N, int K);
 
 // ---- rows (lm_rows.hip): one workgroup per token ----

@@ -1,5 +1,5 @@
-// Matrix products of described decoders that the dense bf16 kernels do not take: everything in true fp32 (v_mfma_f32_16x16x4_f32), products batched over heads, and products
-// grouped over experts with gathered rows and scattered results.  C = epi(A[M,K] . W[N,K]^T), K % 64 == 0.
+// Matrix products of described decoders that the dense bf16 kernels do not take: products batched over heads, and products grouped over experts with gathered rows and scattered
+// results.  C = epi(A[M,K] . W[N,K]^T), K % 64 == 0.  (Everything in fp32: lm_gemm_rows.hip.)
 //
 // 64 x 64 tile, 4 waves of 32 x 32 (2 x 2 accumulators of 16 x 16), K in steps of 32 through LDS.  The weights are the MFMA's A operand, so a lane's accumulator holds four
 // consecutive output columns of one row (the same roles as gemm256 / gemm_skinny).  A row's sum runs over K in ascending steps whatever tile it sits in.
@@ -9,8 +9,7 @@ namespace {
 
 constexpr int BM = LM_TILE_M, BN = 64, BK = 32;
 
-template <typename T> struct Frag;
-template <> struct Frag<bf16> {
+struct F {
     static constexpr int LD = BK + 8;              // elements per LDS row: 80 bytes, 16-byte aligned, rows spread over the banks
     static constexpr int VEC = 8;
     typedef bf16x8 vec;
@@ -19,20 +18,10 @@ template <> struct Frag<bf16> {
         return __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf, af, acc, 0, 0, 0);
     }
 };
-template <> struct Frag<float> {
-    static constexpr int LD = BK + 4;
-    static constexpr int VEC = 4;
-    typedef f32x4 vec;
-    static __device__ __forceinline__ f32x4 mma(const float* w, const float* a, int lane, f32x4 acc) {
-#pragma unroll
-        for (int k = 0; k < BK / 4; k++) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(w[4 * k + (lane >> 4)], a[4 * k + (lane >> 4)], acc, 0, 0, 0);
-        return acc;
-    }
-};
+typedef bf16 T;
 
-template <typename T, int EPI>
+template <int EPI>
 __global__ __launch_bounds__(256) void lm_gemm_kernel(const LmGemmParams p) {
-    typedef Frag<T> F;
     __shared__ __attribute__((aligned(16))) T sA[BM][F::LD];
     __shared__ __attribute__((aligned(16))) T sW[BN][F::LD];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -66,21 +55,21 @@ __global__ __launch_bounds__(256) void lm_gemm_kernel(const LmGemmParams p) {
 #pragma unroll
         for (int j = 0; j < 2; j++) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
     const int wn = (wave & 1) * 32, wm = (wave >> 1) * 32;
-    typename F::vec ra[NL], rw[NL];
+    F::vec ra[NL], rw[NL];
 #pragma unroll
-    for (int i = 0; i < NL; i++) { ra[i] = *(const typename F::vec*)ga[i]; rw[i] = *(const typename F::vec*)gw[i]; }
+    for (int i = 0; i < NL; i++) { ra[i] = *(const F::vec*)ga[i]; rw[i] = *(const F::vec*)gw[i]; }
     for (int k0 = 0; k0 < p.K; k0 += BK) {
         __syncthreads();
 #pragma unroll
         for (int i = 0; i < NL; i++) {
             const int v = tid + i * 256, r = v / CPR, c = (v % CPR) * F::VEC;
-            *(typename F::vec*)&sA[r][c] = ra[i];
-            *(typename F::vec*)&sW[r][c] = rw[i];
+            *(F::vec*)&sA[r][c] = ra[i];
+            *(F::vec*)&sW[r][c] = rw[i];
         }
         __syncthreads();
         if (k0 + BK < p.K) {
 #pragma unroll
-            for (int i = 0; i < NL; i++) { ra[i] = *(const typename F::vec*)(ga[i] + k0 + BK); rw[i] = *(const typename F::vec*)(gw[i] + k0 + BK); }
+            for (int i = 0; i < NL; i++) { ra[i] = *(const F::vec*)(ga[i] + k0 + BK); rw[i] = *(const F::vec*)(gw[i] + k0 + BK); }
         }
 #pragma unroll
         for (int i = 0; i < 2; i++)
@@ -145,16 +134,15 @@ __global__ __launch_bounds__(256) void lm_gemm_kernel(const LmGemmParams p) {
     }
 }
 
-template <typename T>
 int launch_t(int epi, const LmGemmParams& p, hipStream_t st) {
     const dim3 grid((p.N + BN - 1) / BN, p.tiles ? p.max_tiles : (p.M + BM - 1) / BM, p.batch > 0 ? p.batch : 1), block(256);
     switch (epi) {
-        case LM_STORE: hipLaunchKernelGGL((lm_gemm_kernel<T, LM_STORE>), grid, block, 0, st, p); break;
-        case LM_RAW32: hipLaunchKernelGGL((lm_gemm_kernel<T, LM_RAW32>), grid, block, 0, st, p); break;
-        case LM_GLU: hipLaunchKernelGGL((lm_gemm_kernel<T, LM_GLU>), grid, block, 0, st, p); break;
-        case LM_GATE: hipLaunchKernelGGL((lm_gemm_kernel<T, LM_GATE>), grid, block, 0, st, p); break;
-        case LM_RELU2: hipLaunchKernelGGL((lm_gemm_kernel<T, LM_RELU2>), grid, block, 0, st, p); break;
-        case LM_SIDE: hipLaunchKernelGGL((lm_gemm_kernel<T, LM_SIDE>), grid, block, 0, st, p); break;
+        case LM_STORE: hipLaunchKernelGGL((lm_gemm_kernel<LM_STORE>), grid, block, 0, st, p); break;
+        case LM_RAW32: hipLaunchKernelGGL((lm_gemm_kernel<LM_RAW32>), grid, block, 0, st, p); break;
+        case LM_GLU: hipLaunchKernelGGL((lm_gemm_kernel<LM_GLU>), grid, block, 0, st, p); break;
+        case LM_GATE: hipLaunchKernelGGL((lm_gemm_kernel<LM_GATE>), grid, block, 0, st, p); break;
+        case LM_RELU2: hipLaunchKernelGGL((lm_gemm_kernel<LM_RELU2>), grid, block, 0, st, p); break;
+        case LM_SIDE: hipLaunchKernelGGL((lm_gemm_kernel<LM_SIDE>), grid, block, 0, st, p); break;
         default: return cr_fail(CR_ERR_ARG, "lm_gemm: epilogue %d", epi);
     }
     CR_HIP(hipGetLastError());
@@ -169,5 +157,5 @@ int launch_lm_gemm(bool f32, int epi, const LmGemmParams& p, hipStream_t st) {
         (p.gather_div && !p.perm) || (epi == LM_GLU && (p.N % 16 || p.batch > 1)) || ((epi == LM_GATE || epi == LM_SIDE) && !p.gate) || (epi == LM_SIDE && !p.tok) || (((uintptr_t)p.A | (uintptr_t)p.W) & 15))
         return cr_fail(CR_ERR_ARG, "lm_gemm(epi=%d M=%d N=%d K=%d): bad argument", epi, p.M, p.N, p.K);
     if (p.stream) return f32 ? launch_lm_gemm_rows(epi, p, st) : cr_fail(CR_ERR_ARG, "lm_gemm: the few-row form is fp32");
-    return f32 ? launch_t<float>(epi, p, st) : launch_t<bf16>(epi, p, st);
+    return f32 ? launch_lm_gemm_tiles(epi, p, st) : launch_t(epi, p, st);
 }
