@@ -13,6 +13,8 @@
 #include <algorithm>
 
 #include "attention_merge.hpp"
+#include <type_traits>
+
 #include "lm.hpp"
 
 namespace {
@@ -29,10 +31,17 @@ template <> __device__ __forceinline__ f32x4 ld4f<bf16>(const bf16* p) {
 }
 // the sixteen dk groups of a wave sit four lanes apart
 __device__ __forceinline__ f32x4 sum_groups(f32x4 o) {
+    // lane ^ 4, ^ 8, ^ 16, ^ 32 on the vector pipe (LDS shuffles made a chain of four round trips of every token): the bank masks of two row shifts make the first
 #pragma unroll
-    for (int s = 4; s < 64; s <<= 1)
-#pragma unroll
-        for (int e = 0; e < 4; e++) o[e] += __shfl_xor(o[e], s, 64);
+    for (int e = 0; e < 4; e++) {
+        const int x = __float_as_int(o[e]);
+        o[e] += __int_as_float(__builtin_amdgcn_update_dpp(__builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, false), x, 0x114, 0xf, 0xa, false));
+        o[e] += dpp<0x128>(o[e]);
+        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(o[e]), __float_as_uint(o[e]), false, false);
+        o[e] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
+        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[e]), __float_as_uint(o[e]), false, false);
+        o[e] = __uint_as_float(h[0]) + __uint_as_float(h[1]);
+    }
     return o;
 }
 __device__ __forceinline__ float silu32(float x) { return x / (1.0f + expf(-x)); }
@@ -92,7 +101,9 @@ __global__ __launch_bounds__(dec_waves(NR) * 64) void ret_decode_kernel(const Re
         ((T*)p.ao)[(int64_t)row * p.ldo + (int64_t)h * p.vdim + c] = (T)(so[c] * rs * silu32((float)((const T*)p.g)[(int64_t)row * p.lda + h * p.Vp + c]));
 }
 
-// one wave = 16 value columns, the tokens of a segment in turn
+// one wave = 16 value columns, the tokens of a segment in turn, U at a time.  Bound by the chain of loads: the rows of the next U tokens are fetched under the current ones' arithmetic
+// (201 tokens of 64 x 64 heads: one token ahead, sums over LDS shuffles 94 us; eight ahead 78; and sums on the vector pipe 62, whose
+// issue of some 110 instructions a token is what is left).
 template <typename T, int NR>
 __global__ __launch_bounds__(256) void ret_recurrent_kernel(const RetParams p) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -105,28 +116,46 @@ __global__ __launch_bounds__(256) void ret_recurrent_kernel(const RetParams p) {
     f32x4 s[NR];
 #pragma unroll
     for (int r = 0; r < NR; r++) s[r] = sg[2] == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : *(const f32x4*)(sb + r * 256);
-    f32x4 q[NR / 4], k[NR / 4], v;
-    auto load = [&](int t) {
-        const int64_t o = ((int64_t)(row0 + t) * p.H + h) * p.Kp + g * NR;
+    constexpr int U = NR <= 4 ? 8 : NR <= 8 ? 4 : NR <= 16 ? 2 : 1;       // (two groups of U tokens: at most 100 registers beside the state's 4 NR)
+    struct Rows { f32x4 q[U][NR / 4], k[U][NR / 4], v[U]; };
+    auto load = [&](Rows& f, int t0) {
 #pragma unroll
-        for (int r = 0; r < NR / 4; r++) { q[r] = *(const f32x4*)(p.rq + o + 4 * r); k[r] = *(const f32x4*)(p.rk + o + 4 * r); }
-        v = ld4f((const T*)p.v + (int64_t)(row0 + t) * p.lda + h * p.Vp + b * 16 + c4);
-    };
-    load(0);
-    for (int t = 0; t < S; t++) {
-        f32x4 qc[NR / 4], kc[NR / 4];
-        const f32x4 vc = v;
+        for (int u = 0; u < U; u++) {
+            const int64_t row = row0 + min(t0 + u, S - 1), o = (row * p.H + h) * p.Kp + g * NR;
 #pragma unroll
-        for (int r = 0; r < NR / 4; r++) { qc[r] = q[r]; kc[r] = k[r]; }
-        load(min(t + 1, S - 1));
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            s[r] = s[r] * decay + kc[r / 4][r % 4] * vc;
-            o += s[r] * qc[r / 4][r % 4];
+            for (int r = 0; r < NR / 4; r++) { f.q[u][r] = *(const f32x4*)(p.rq + o + 4 * r); f.k[u][r] = *(const f32x4*)(p.rk + o + 4 * r); }
+            f.v[u] = ld4f((const T*)p.v + row * p.lda + h * p.Vp + b * 16 + c4);
         }
-        o = sum_groups(o);
-        if (lane < 4) *(f32x4*)(p.raw + ((int64_t)(row0 + t) * p.H + h) * p.Vp + b * 16 + c4) = o;
+    };
+    auto work = [&](const Rows& f, int t0, auto all) {
+#pragma unroll
+        for (int u = 0; u < U; u++) {
+            if (!decltype(all)::value && t0 + u >= S) break;  // (uniform)
+            f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int r = 0; r < NR; r++) {
+                s[r] = s[r] * decay + f.k[u][r / 4][r % 4] * f.v[u];
+                o += s[r] * f.q[u][r / 4][r % 4];
+            }
+            o = sum_groups(o);
+            if (lane < 4) *(f32x4*)(p.raw + ((int64_t)(row0 + t0 + u) * p.H + h) * p.Vp + b * 16 + c4) = o;
+        }
+    };
+    Rows f0, f1;
+    load(f0, 0);
+    int t = 0;
+    for (; t + 2 * U <= S; t += 2 * U) {
+        load(f1, t + U);
+        __builtin_amdgcn_sched_barrier(0);
+        work(f0, t, std::true_type{});
+        load(f0, t + 2 * U);
+        __builtin_amdgcn_sched_barrier(0);
+        work(f1, t + U, std::true_type{});
+    }
+    if (t < S) {
+        load(f1, t + U);
+        work(f0, t, std::false_type{});
+        work(f1, t + U, std::false_type{});
     }
 #pragma unroll
     for (int r = 0; r < NR; r++) *(f32x4*)(sb + r * 256) = s[r];
