@@ -308,18 +308,22 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
         read(f0, 0, count);
         int buf = 0;                                          // buffer of tile kt
         auto step = [&](int kt, Frags& now, Frags& next) {
-            if (kt + 1 < nk) {
-                arrive(kt + 1);
-                if (kt + NBUF < nk) ask(kt + NBUF, buf);      // the buffer that tile kt was read from
-                buf = buf + 1 == NBUF ? 0 : buf + 1;
-                read(next, buf, count);
-            }
+            arrive(kt + 1);
+            if (kt + NBUF < nk) ask(kt + NBUF, buf);          // the buffer that tile kt was read from
+            buf = buf + 1 == NBUF ? 0 : buf + 1;
+            read(next, buf, count);
+            __builtin_amdgcn_sched_barrier(0);
             multiply(now, count);
         };
-        for (int kt = 0; kt < nk; kt += 2) {
+        int kt = 0;
+        for (; kt + 2 < nk; kt += 2) {                        // (no read of the loop is conditional: the compiler waited for it ahead of the multiplications then)
             step(kt, f0, f1);
-            if (kt + 1 < nk) step(kt + 1, f1, f0);
+            step(kt + 1, f1, f0);
         }
+        if (kt + 1 < nk) {
+            step(kt, f0, f1);
+            multiply(f1, count);
+        } else multiply(f0, count);
     };
     if (live == FM) loop(std::integral_constant<int, FM>{});
     else if (FM > 1 && live == FM - 1) loop(std::integral_constant<int, FM - 1>{});
