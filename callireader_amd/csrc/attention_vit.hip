@@ -8,11 +8,11 @@
 //   * the CLS KEY enters each query's softmax as the INITIAL state instead of a tile: s0 = q . k_cls by 32 FMAs per lane, the
 //     reference point of the exponentials m = bf16(s0), row sum 1, O = v_cls -- so every tile of the sweep takes the lean softmax
 //     path (attention.hip) from the first one on; a row sum that is not finite or >= 2^100 at the END of the sweep (a score ~88 above
-//     that point) flags the block, and vit_attn_exact_kernel redoes flagged blocks in the exact rescaling form;
+//     that point) flags the block, and vit_attn_finish_kernel redoes flagged blocks in the exact rescaling form;
 //   * the CLS QUERY is spread over all workgroups of its (tile, head): block b sweeps its key tiles in the rotated order
 //     2b+2, ..., 2b+1 (a softmax does not care; it also spreads the eight blocks' K/V fetches over the tiles), so its LAST two tiles
 //     are 2b and 2b+1 and are both still in LDS when the sweep ends; each of the four waves then takes one 32-key half of them for the
-//     CLS query (4 + 4 MFMAs, exact softmax) and writes an un-normalised partial (m, l, O[64]); vit_cls_combine_kernel merges the
+//     CLS query (4 + 4 MFMAs, exact softmax) and writes an un-normalised partial (m, l, O[64]); vit_attn_finish_kernel merges the
 //     4n + 1 partials (the +1: the CLS key itself, by block 0) in index order, like the decode path's split combine.
 // Work per (tile, head): 8 x 16.6 tile-times instead of 9 x 17.
 // The sweep is bound by the vector pipe (77 % busy against 42 % for the matrix pipe: the reference's own per-score arithmetic), so: 124
@@ -47,7 +47,7 @@ __device__ __forceinline__ int kswz(int r) { return (r >> 1) & 7; }
 __device__ __forceinline__ int vswz(int r) { return ((r >> 1) & 1) << 2; }
 
 // One 128-query block of one (tile, head).  EXACT = false: the lean sweep, the block's verdict on it (flag), the output, the block's
-// share of the CLS query.  EXACT = true: the same block again in the exact rescaling form (vit_attn_exact_kernel, flagged blocks only).
+// share of the CLS query.  EXACT = true: the same block again in the exact rescaling form (vit_attn_finish_kernel, flagged blocks only).
 // NW = waves per workgroup (of 128 queries): 4 waves of 32 queries (round 2..4), or -- round 5, CR_VIT_ATTN_NW=2 -- 2 waves of 64: a wave then holds TWO 32-query
 // sub-blocks and every K / V fragment it reads from LDS feeds two MFMAs instead of one (the knock-outs of profiles/round5/06_* put the matrix side of this
 // kernel -- MFMAs + fragment reads + fills, no softmax -- at 0.281 ms of the launch's 0.346 and the vector side alone at 0.246: the matrix side is the longer
@@ -380,7 +380,7 @@ __device__ __forceinline__ void vit_attn_body(const AttnParams& p, const int qb,
         }
     };
     // The lean sweep's verdict (NaN compares false: a non-finite row sum is flagged as well) goes to the block's flag word; flagged
-    // blocks are redone by vit_attn_exact_kernel.  (With the exact sweep inside this kernel -- a workgroup-uniform branch behind the
+    // blocks are redone by vit_attn_finish_kernel.  (With the exact sweep inside this kernel -- a workgroup-uniform branch behind the
     // vote -- the kernel took 168 registers for code that all but never runs: 3 waves per SIMD; alone the lean form fits 128 and
     // four: 1.478 -> 1.412 ms per 255-tile launch in one process.)
     int* const flags = (int*)(p.part_o + (size_t)p.B * p.H * (4 * gx + 1) * D);
@@ -498,11 +498,11 @@ __global__ __launch_bounds__(256, 4) void vit_attn_kernel(const AttnParams p) {
     const int pid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (lin >> 3);
     vit_attn_body<false>(p, pid % gx, (pid / gx) % gy, pid / (gx * gy), gx);
 }
-// One workgroup per tile: redo the (head, query block)s the lean sweep flagged (a score ~88 above the CLS key's: none on real pages).
+// A tile's workgroup: redo the (head, query block)s the lean sweep flagged (a score ~88 above the CLS key's: none on real pages).
 // The tile's H * nb flag words are fetched in ONE round trip (a loop of dependent one-word loads per (tile, head) cost 47 us per
 // 255-tile launch with nothing flagged).
-__global__ __launch_bounds__(256) void vit_attn_exact_kernel(const AttnParams p, const int nb) {
-    const int batch = blockIdx.x, n = p.H * nb;
+__device__ __forceinline__ void vit_attn_exact(const AttnParams& p, int batch, int nb) {
+    const int n = p.H * nb;
     const int* flags = (const int*)(p.part_o + (size_t)p.B * p.H * (4 * nb + 1) * D) + (int64_t)batch * n;
     for (int j0 = 0; j0 < n; j0 += 256) {
         const int j = j0 + (int)threadIdx.x;
@@ -517,9 +517,8 @@ __global__ __launch_bounds__(256) void vit_attn_exact_kernel(const AttnParams p,
 // shuffles -- then lane d sums the weighted O rows with every load of the loop independent (a plain loop over a run-time count
 // waited for each partial's load in turn: 33 dependent L2 round trips, 15.8 us per launch at 32 tiles).
 template <int NS>
-__global__ __launch_bounds__(64) void vit_cls_combine_kernel(const AttnParams p) {
+__device__ __forceinline__ void vit_cls_combine(const AttnParams& p, int head, int batch, int lane) {
     static_assert(NS <= 64, "one lane per partial");
-    const int head = blockIdx.x, batch = blockIdx.y, lane = threadIdx.x;
     const int64_t base = ((int64_t)batch * p.H + head) * NS;
     const float m = lane < NS ? p.part_ml[(base + lane) * 2] : -INFINITY;
     const float l = lane < NS ? p.part_ml[(base + lane) * 2 + 1] : 0.f;
@@ -539,8 +538,7 @@ __global__ __launch_bounds__(64) void vit_cls_combine_kernel(const AttnParams p)
 }
 
 // any other partial count (S = 1 + 128 n with n != 8)
-__global__ __launch_bounds__(64) void vit_cls_combine_any_kernel(const AttnParams p, int nsplit) {
-    const int head = blockIdx.x, batch = blockIdx.y, d = threadIdx.x;
+__device__ __forceinline__ void vit_cls_combine_any(const AttnParams& p, int nsplit, int head, int batch, int d) {
     const int64_t base = ((int64_t)batch * p.H + head) * nsplit;
     float M = -INFINITY;
     for (int s = 0; s < nsplit; s++) M = fmaxf(M, p.part_ml[(base + s) * 2]);
@@ -551,6 +549,16 @@ __global__ __launch_bounds__(64) void vit_cls_combine_any_kernel(const AttnParam
         acc += w * p.part_o[(base + s) * D + d];
     }
     p.O[(int64_t)batch * p.o_bs + (int64_t)head * p.o_hs + d] = f2bf(acc / L);
+}
+
+// Both in one launch: block 0 of a tile redoes what was flagged (patch rows), the others merge the class rows of four heads, a wave each.  (A launch of 4.8 us each, and a layer of one
+// tile has seven launches in all.)
+__global__ __launch_bounds__(256) void vit_attn_finish_kernel(const AttnParams p, const int nb) {
+    const int batch = blockIdx.y, head = 4 * ((int)blockIdx.x - 1) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+    if (blockIdx.x == 0) vit_attn_exact(p, batch, nb);
+    else if (head >= p.H) return;
+    else if (nb == 8) vit_cls_combine<33>(p, head, batch, lane);
+    else vit_cls_combine_any(p, 4 * nb + 1, head, batch, lane);
 }
 
 }  // namespace
@@ -569,7 +577,7 @@ size_t vit_attn_ws_floats(int B, int H, int S) { const int nb = (S - 1) / 128; r
 int launch_vit_attn(const AttnParams& p, hipStream_t stream) {
     constexpr int LDS = 2 * 2 * TILE;
     static std::atomic<uint64_t> attr_done{0}, attr_done_x{0}, attr_done_2{0};
-    if (!cr_dyn_lds_once(attr_done, (const void*)vit_attn_kernel, LDS) || !cr_dyn_lds_once(attr_done_x, (const void*)vit_attn_exact_kernel, LDS) ||
+    if (!cr_dyn_lds_once(attr_done, (const void*)vit_attn_kernel, LDS) || !cr_dyn_lds_once(attr_done_x, (const void*)vit_attn_finish_kernel, LDS) ||
         !cr_dyn_lds_once(attr_done_2, (const void*)vit_attn2_kernel, LDS)) return CR_ERR_HIP;
     const char* e_nw = getenv("CR_VIT_ATTN_NW");                 // read per call (a bench flips it in one process)
     const bool two_waves = e_nw && e_nw[0] == '2';
@@ -578,8 +586,6 @@ int launch_vit_attn(const AttnParams& p, hipStream_t stream) {
     q.part_o = p.part_ml + (size_t)p.B * p.H * (4 * nb + 1) * 2;       // one allocation: [m, l] pairs, then the O partials
     if (two_waves) hipLaunchKernelGGL(vit_attn2_kernel, dim3(nb, p.H, p.B), dim3(128), LDS, stream, q);
     else hipLaunchKernelGGL(vit_attn_kernel, dim3(nb, p.H, p.B), dim3(256), LDS, stream, q);
-    hipLaunchKernelGGL(vit_attn_exact_kernel, dim3(p.B), dim3(256), LDS, stream, q, nb);
-    if (nb == 8) hipLaunchKernelGGL(vit_cls_combine_kernel<33>, dim3(p.H, p.B), dim3(64), 0, stream, q);
-    else hipLaunchKernelGGL(vit_cls_combine_any_kernel, dim3(p.H, p.B), dim3(64), 0, stream, q, 4 * nb + 1);
+    hipLaunchKernelGGL(vit_attn_finish_kernel, dim3(1 + (p.H + 3) / 4, p.B), dim3(256), LDS, stream, q, nb);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
