@@ -201,6 +201,8 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(const LatentDecod
 }
 
 // RW tokens of one head: 8 / RW waves per token merge its splits (each in index order) and the attended latent is rounded once; then the row block is carried back by W_uv, gated and stored
+// Bound, at few splits, by the loads of W_uv: a fragment's four neighbouring lanes hold four rows, so a KiB takes 64 clocks, 128 columns of a 512-wide latent 4 us of one CU.  gridDim.z
+// workgroups share a row block's columns then (each merges for itself, see the launch): 24 rows of 16 heads 9.2 us alone, 6.6 with four.
 template <int R, int RW>
 __global__ __launch_bounds__(512) void latent_combine_kernel(const LatentDecodeParams p) {
     __shared__ __attribute__((aligned(16))) bf16 sA[RW][R + 8];
@@ -212,9 +214,11 @@ __global__ __launch_bounds__(512) void latent_combine_kernel(const LatentDecodeP
     typedef typename std::conditional<CPL == 1, one, vecf_>::type vecf;
     // the projection's weights of this wave's first column block travel under the merge
     const bf16* W = p.wuv + (int64_t)head * p.uv_hs;
+    const int cw = 8 / (int)gridDim.z, col0 = wave < cw ? ((int)blockIdx.z * cw + wave) * 16 : p.vdim;      // waves that take columns: col0, col0 + 128, ..
     bf16x8 wf[R / 32];
+    if (col0 < p.vdim)
 #pragma unroll
-    for (int k = 0; k < R / 32; k++) wf[k] = *(const bf16x8*)(W + (int64_t)min(wave * 16 + (lane & 15), p.vdim - 1) * R + (lane >> 4) * 8 + k * 32);
+        for (int k = 0; k < R / 32; k++) wf[k] = *(const bf16x8*)(W + (int64_t)min(col0 + (lane & 15), p.vdim - 1) * R + (lane >> 4) * 8 + k * 32);
     {
         const int row = min(m0 + wave / SW, p.a.M - 1), sw = wave % SW;
         const int64_t base = ((int64_t)row * H + head) * p.nsplit;
@@ -268,7 +272,7 @@ __global__ __launch_bounds__(512) void latent_combine_kernel(const LatentDecodeP
         __syncthreads();
     }
     const int g = lane >> 4, li = lane & 15, row = m0 + (li & (RW - 1));       // (the product's other token columns repeat the first RW)
-    for (int n16 = wave * 16; n16 < p.vdim; n16 += 128) {
+    for (int n16 = col0; n16 < p.vdim; n16 += 128) {
         f32x4 acc = {0.f, 0.f, 0.f, 0.f};
         if (n16 >= 128)                                        // heads wider than a block per wave
 #pragma unroll
@@ -291,6 +295,15 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const float* __restr
     bf16* sq = (bf16*)smem;                            // [16 MT][Ap + 8]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15, head = blockIdx.y, ld = Ap + 8;
     const int per = Ap / 4;                            // vectors of four per row
+    bf16x8 w0[2][2], w1[2][2];                         // the weights' first 128 columns travel under the sums below (5.7 us -> 5.0 at 24 rows of 16 heads)
+#pragma unroll
+    for (int t = 0; t < 2; t++)
+#pragma unroll
+        for (int k = 0; k < 2; k++) {
+            const bf16* w = ukT + ((int64_t)head * Rp + min((int)blockIdx.x * 128 + (wave * 2 + t) * 16, Rp - 16) + li) * Ap + min(k * 64, Ap - 64) + g * 8;
+            w0[t][k] = *(const bf16x8*)w;
+            w1[t][k] = *(const bf16x8*)(w + 32);
+        }
     for (int v = tid; v < 16 * MT * per; v += 256) {
         const int m = v / per, c = (v % per) * 4;
         f32x4 s = {0.f, 0.f, 0.f, 0.f};
@@ -310,15 +323,17 @@ __global__ __launch_bounds__(256) void latent_absorb_kernel(const float* __restr
 #pragma unroll
         for (int m = 0; m < MT; m++) acc[m] = f32x4{0.f, 0.f, 0.f, 0.f};
         const bf16* w = ukT + ((int64_t)head * Rp + n16 + li) * Ap + g * 8;
-        for (int k = 0; k < Ap; k += 64) {
-            const bf16x8 w0 = *(const bf16x8*)(w + k), w1 = *(const bf16x8*)(w + k + 32);
+        auto step = [&](int k, const bf16x8& a, const bf16x8& b) {
 #pragma unroll
             for (int m = 0; m < MT; m++) {
                 const bf16* q = sq + (m * 16 + li) * ld + k + g * 8;
-                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w0, *(const bf16x8*)q, acc[m], 0, 0, 0);
-                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w1, *(const bf16x8*)(q + 32), acc[m], 0, 0, 0);
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, *(const bf16x8*)q, acc[m], 0, 0, 0);
+                acc[m] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b, *(const bf16x8*)(q + 32), acc[m], 0, 0, 0);
             }
-        }
+        };
+        step(0, w0[t][0], w1[t][0]);
+        if (Ap > 64) step(64, w0[t][1], w1[t][1]);
+        for (int k = 128; k < Ap; k += 64) step(k, *(const bf16x8*)(w + k), *(const bf16x8*)(w + k + 32));
 #pragma unroll
         for (int m = 0; m < MT; m++) {
             const int row = m * 16 + li;
@@ -334,8 +349,11 @@ int launch_decode_t(const LatentDecodeParams& p, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
     if (!cr_dyn_lds_once(done, (const void*)latent_decode_kernel<R, HT>, LDS)) return CR_ERR_HIP;
     hipLaunchKernelGGL((latent_decode_kernel<R, HT>), dim3(p.nsplit, p.a.M * ((p.a.H + 16 * HT - 1) / (16 * HT))), dim3(256), LDS, st, p);
-    if (p.a.M * p.a.H <= cr_device_cus()) hipLaunchKernelGGL((latent_combine_kernel<R, 1>), dim3(p.a.H, p.a.M), dim3(512), 0, st, p);      // few rows: eight waves share one row's splits
-    else hipLaunchKernelGGL((latent_combine_kernel<R, 8>), dim3(p.a.H, (p.a.M + 7) / 8), dim3(512), 0, st, p);
+    const bool few = p.a.M * p.a.H <= cr_device_cus();        // few rows: eight waves share one row's splits
+    const int wgs = p.a.H * (few ? p.a.M : (p.a.M + 7) / 8);
+    const int z = p.nsplit > 4 ? 1 : 4 * wgs <= cr_device_cus() ? 4 : 2 * wgs <= cr_device_cus() ? 2 : 1;      // (past four splits merging them again costs more than the columns save)
+    if (few) hipLaunchKernelGGL((latent_combine_kernel<R, 1>), dim3(p.a.H, p.a.M, z), dim3(512), 0, st, p);
+    else hipLaunchKernelGGL((latent_combine_kernel<R, 8>), dim3(p.a.H, (p.a.M + 7) / 8, z), dim3(512), 0, st, p);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }

@@ -1,0 +1,24 @@
+"""Latent decode in bf16 with one, two and four workgroups sharing a row block's value columns (by rows x heads), value widths that leave some of them without columns or with a part of
+sixteen, and a context of more key splits than the sharing takes: against the oracle, 0.03 of the logits' spread (test_gpu_linasun.py's bar for bfloat16)."""
+import pytest
+import torch
+
+import linasun_cases as LC
+from oracle import linasun as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('rows', [1, 4, 9, 33])
+@pytest.mark.parametrize('heads,dim,vdim,kv_rank', [(3, 64, 24, 64), (16, 128, 128, 512), (33, 64, 72, 128), (5, 192, 160, 256)])
+def test_columns_shared_out(rows, heads, dim, vdim, kv_rank):
+    from callireader_amd.modeling_decoder import LinasunForCausalLM
+    cfg = LC.config(192, 150, [(LC.mixer(heads, dim, vdim, 64, kv_rank, dim ** -0.5), LC.moe(3, 2, 64, 1.5))])
+    w = LC.weights(cfg, 51)
+    m = LinasunForCausalLM.from_state_dict(w, cfg, dtype=torch.bfloat16, max_tokens=1400 if rows == 1 else 80, max_seqs=rows)
+    toks = [LC.tokens(cfg, 1390 if rows == 1 else 3 + 11 * i % 70, seed=i) for i in range(rows)]
+    m.step([(i, t[:-1], []) for i, t in enumerate(toks)])
+    z = m.step([(i, t[-1:], [0]) for i, t in enumerate(toks)]).cpu()
+    m.close()
+    for i in sorted({0, rows // 2, rows - 1}):
+        assert LC.rel(z[i:i + 1], O.forward(w, cfg, toks[i])[-1:]) < 0.03, i
