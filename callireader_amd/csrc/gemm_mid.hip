@@ -373,7 +373,7 @@ int launch_t(int epi, const GemmParams& p, int rt, hipStream_t stream) {
 namespace {
 
 // Tile shapes (launch_gemm_mid's `tile` = index + 1).  Eight waves where the tile is large enough to feed them: two waves a SIMD cover each other's LDS reads and barriers (64 x 64 at
-// M = 1025, N = 1024, K = 4096: four waves 27.5 us, eight 26.6; 128 x 128 at N = 3072, K = 1024: 20 and 13.4).
+// M = 1025, N = 1024, K = 4096: four waves 27.5 us, eight 26.6, now 26.2; 128 x 128 at N = 3072, K = 1024: 20 and 13.4).
 struct MidShape { int bm, bn; };
 constexpr MidShape SHAPES[] = {{16, 32}, {16, 64}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {64, 128}, {96, 128}, {128, 128}, {96, 256}, {128, 256}};
 constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
@@ -383,7 +383,8 @@ constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 // The time a launch takes, in us, and the tile shape (and number of row tiles) that takes least.  Every shape measured here (M 1 .. 4100, N 512 .. 28672, K 512 .. 16384) follows one law:
 // a CU brings in its workgroups' operand bytes at 61 GB/s and does the rest under that, so a K-tile (64) of a workgroup costs 0.05 us + 2.1 ns per row of A or W in it; a workgroup
 // more on a CU costs its time again; launch, first fill and drain 3.5 us, the epilogue 0.1 ns an element.  (32 x 64, K 14336: 52.3 us measured, 57 by the law; 64 x 64, K 4096: 21.7 and
-// 24.1; 96 x 64, K 14336: 79.5 and 90; 128 x 128, K 4096: 43.5 and 42.5; 128 x 256, K 4096: 55.1 and 56.8.)
+// 24.1; 96 x 64, K 14336: 79.5 and 90; 128 x 128, K 4096: 43.5 and 42.5; 128 x 256, K 4096: 55.1 and 56.8.  With the operand reads under the
+// multiplications the same shapes take 2 to 12 % less, evenly enough that the choice stands.)
 double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
     const int nf = (p.M + 15) / 16, slices = epi == EPI_PARTIAL && p.group > 0 ? p.group : 1, nk = p.K / 64 / slices, cus = cr_device_cus();
     double best = 1e30;

@@ -2,8 +2,10 @@
 //
 // Bound by the weights' bytes.  A workgroup owns 16 rows of W (one v_mfma_f32_16x16x4_f32 operand tile) and the K range of its slice; its eight waves divide that range, so a product
 // of 1024 rows keeps 64 x slices x 8 waves of loads in flight where the 64 x 64 tiles of lm_gemm.hip give 16 workgroups that walk all of K alone (two rows, products of 1024 x 1536 .. 4096: 46 us there,
-// 6.8 here; 3584 x 1024: 27 and 10; 4096 x 1024 with the squared relu: 27 and 8.8; token side's 64 x 1024: 28 and 6.2).
-// A lane loads 16 bytes of its weight row, k = 4 (lane >> 4) .. + 3 of a 16-deep step, and the same four k of its activation row: the four multiplications of a step take one element
+// 5.5 here; 3584 x 1024: 27 and 7.2; 4096 x 1024 with the squared relu: 27 and 7.1; token side's 64 x 1024: 28 and 4.6).
+// W comes by LDS-DMA, a KiB of 16 rows x 16 k an instruction, four neighbouring lanes a row's 64 bytes; loaded straight as operands, four neighbouring lanes hold four rows and a KiB takes
+// 64 clocks of the CU's load path instead of 16 (two rows: 1024 x 1536 .. 4096 6.9 us -> 5.5, 3584 x 1024 10.3 -> 7.2, 4096 x 1024 8.8 -> 7.1, 64 x 1024 6.0 -> 4.6).
+// A lane multiplies with k = 4 (lane >> 4) .. + 3 of a 16-deep step of its weight row and of its activation row: the four multiplications of a step take one element
 // of each, which permutes k inside the step for both operands alike.  Partial tiles of the waves meet in LDS and are added in wave order; slices go to the consumer, which adds them
 // in slice order.  A row's sum depends on N and K (slices), never on the other rows.
 #include "lm.hpp"
@@ -15,8 +17,10 @@ constexpr int NW = 8;                        // waves of a workgroup
 template <int MT, int EPI>
 __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) {
     constexpr int U = MT == 4 ? 4 : 8;       // 16-deep steps whose loads are issued together
-    __shared__ float red[NW][MT * 16][17];
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    constexpr int RED = NW * MT * 16 * 17 * 4, RING = NW * U * 1024;
+    __shared__ __attribute__((aligned(16))) char sm[RED > RING ? RED : RING];      // the waves' U steps of W; after the products their partial tiles
+    auto red = (float (*)[MT * 16][17])sm;
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = blockIdx.x * 16;
     const float* A = (const float*)p.A + (int64_t)blockIdx.z * p.a_bs;
     const float* W = (const float*)p.W;
@@ -30,7 +34,11 @@ __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) 
     const int slice = p.tiles ? 0 : blockIdx.y, steps = p.K / 16 / max(p.slices, 1);      // 16-deep steps of this slice
     const int per = (steps + NW - 1) / NW, s0 = slice * steps + min(wave * per, steps), s1 = slice * steps + min(wave * per + per, steps);
 
-    const float* w = W + (int64_t)min(n0 + (lane & 15), p.N - 1) * p.ldw + 4 * (lane >> 4);
+    // a load instruction brings 16 rows x 16 k, four neighbouring lanes a row's 64 bytes, into the wave's own KiB of LDS; the 16-byte chunks of rows 8..15 are exchanged in pairs on both
+    // sides (reads without bank conflicts)
+    const float* w = W + (int64_t)min(n0 + (lane >> 2), p.N - 1) * p.ldw + 4 * ((lane & 3) ^ (((lane >> 2) >> 3) << 1));
+    char* ring = sm + wave * U * 1024;
+    const char* frag = ring + (lane & 15) * 64 + ((lane >> 4) ^ (((lane & 15) >> 3) << 1)) * 16;
     const float* a[MT];
 #pragma unroll
     for (int j = 0; j < MT; j++) {
@@ -46,10 +54,16 @@ __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) 
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int k = min(s + u, s1 - 1) * 16;
-            wf[u] = __builtin_nontemporal_load((const f32x4*)(w + k));
+            __builtin_amdgcn_global_load_lds(CR_GLB(w + k), CR_LDS(ring + u * 1024), 16, 0, 0);
 #pragma unroll
             for (int j = 0; j < MT; j++) af[u][j] = *(const f32x4*)(a[j] + k);
         }
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int u = 0; u < U; u++) wf[u] = *(const f32x4*)(frag + u * 1024);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");     // (the next round's loads overwrite what was read here)
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int u = 0; u < U; u++)
             if (s + u < s1) {
@@ -59,6 +73,7 @@ __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) 
                     for (int j = 0; j < MT; j++) acc[j] = __builtin_amdgcn_mfma_f32_16x16x4f32(wf[u][e], af[u][j][e], acc[j], 0, 0, 0);
             }
     }
+    __syncthreads();                                          // every wave has read its last steps
     // lane: columns 4 (lane >> 4) + e of row lane & 15
 #pragma unroll
     for (int j = 0; j < MT; j++)

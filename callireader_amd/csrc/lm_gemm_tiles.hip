@@ -4,8 +4,8 @@
 // Bound by the matrix cores (v_mfma_f32_16x16x4_f32: 256 operations a clock and CU) where the grid fills the card, by what lies between K-tiles where it does not.  The form of
 // gemm_mid.hip: NBUF K-tiles in LDS, NBUF - 1 of them under way, one barrier a K-tile, eight rows of 128 bytes a load instruction; the tile shape is picked by the rounds it gives.
 // 402 rows, us: products of 1024 columns over K = 64, 1536 and 4096 49 on average -> 5, 21 and 46 (32 x 64 tiles, K-tiles of 64: 52 with K-tiles of 32), 3584 x 1024 50 -> 43 and
-// 4096 x 1024 with the squared relu 51 -> 43 (112 x 64; 22 us of multiplications; 41 with one chain a sum, whose error
-// against 64 bits is 1.4 to 1.7 times that of two).  Before: 64 x 64 tiles, one K-tile of 32 in LDS, two barriers each.
+// 4096 x 1024 with the squared relu 51 -> 43 (112 x 64; 22 us of multiplications; 41 with one chain a sum, whose error against 64 bits is 1.4 to 1.7 times that of two).  Before:
+// 64 x 64 tiles, one K-tile of 32 in LDS, two barriers each.
 // A lane reads 16 bytes of its row, k = 16 h + 4 (lane >> 4) .. + 3; the four multiplications take one element of each, which permutes k inside 16 for both operands alike.  A row's
 // sum runs over K in two chains, the even and the odd 16-steps, whatever the tile.
 #include <algorithm>
