@@ -20,6 +20,7 @@
 #include "decode.hpp"
 #include "kv.hpp"
 #include "lm.hpp"
+#include "lm_upload.hpp"
 
 bool gemm_stream_supported(int epi, const GemmParams& p, int splits);      // gemm_stream.hip
 
@@ -225,8 +226,7 @@ int derive_layer(Deriver& dv, int i, LmLayer& L) {
     return CR_OK;
 }
 
-// Where a prompt's keys sit for layers of one chunk size: per sequence its cached rows of the chunk the portion goes on in, then the portion; pieces are the chunks (causal segments
-// {first row, rows, place of the first row in its chunk, key row of the chunk's start}).  Device pointers into the step's one upload.
+// a prompt's key plan (lm_upload.hpp) on the device
 struct KeyPlan {
     int ring, n_pieces, longest, n_pre; size_t Mk;
     const int32_t *row_key, *row_slot, *pieces, *pre_key, *pre_slot;
@@ -238,8 +238,7 @@ struct Step {
     int M; bool decode;
     const int64_t* tokens;          // device; null: the sequences' last generated ids
     LmRowIndex ix;
-    struct Seg { int row0, S, pos0, seq, key0; };
-    std::vector<Seg> segs;          // prefill
+    std::vector<PromptSeg> segs;    // prefill
     const int32_t* d_seg;           // prefill: {first row, rows, first position, first key row} per segment
     bool fresh;                     // prefill: every sequence starts empty (key rows = token rows)
     int Mk;                         // key rows
@@ -393,14 +392,14 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
         const int64_t ldk = (int64_t)2 * H * L.Ap;
         if (sp.fresh) CR_TRY(dense(c, lm, b.c, L.Rp, L.wkv, b.kv, ldk, M, 2 * H * L.Ap, L.Rp, st, true));
         else
-            for (const Step::Seg& sg : sp.segs)
+            for (const PromptSeg& sg : sp.segs)
                 CR_TRY(dense(c, lm, cache + (size_t)sg.seq * kv->max_tokens * L.Rp * es, L.Rp, L.wkv, (bf16*)b.kv + (size_t)sg.key0 * ldk, ldk, sg.pos0 + sg.S, 2 * H * L.Ap, L.Rp, st, true));
         AttnParams ap{};
         ap.Q = (const bf16*)b.q; ap.K = (const bf16*)b.kv; ap.V = (const bf16*)b.kv + (size_t)H * L.Ap; ap.O = (bf16*)b.ao;
         ap.q_rs = (int64_t)H * L.Ap; ap.q_hs = L.Ap; ap.k_bs = ap.v_bs = ap.k_rs = ap.v_rs = ldk; ap.k_hs = ap.v_hs = L.Ap; ap.o_rs = L.Gp; ap.o_hs = s.vdim;
         ap.B = (int)sp.segs.size(); ap.H = H; ap.kv_group = 1; ap.seg = sp.d_seg; ap.q_prescale = 1.f; ap.s_div = 1.f;
         ap.wide = 1; ap.s_mul = s.scale; ap.vdim = s.vdim; ap.gate = (const bf16*)gate; ap.g_rs = L.Na;
-        for (const Step::Seg& sg : sp.segs) ap.Sq = std::max(ap.Sq, sg.S);
+        for (const PromptSeg& sg : sp.segs) ap.Sq = std::max(ap.Sq, sg.S);
         if (launch_flash_attn(ap, L.Ap, true, st) != CR_OK) return cr_fail(CR_ERR_HIP, "latent attention (expanded): launch failed");
     } else {
         LmGemmParams g{};
@@ -758,35 +757,6 @@ int size_heads(int i, Lm& lm, LmLayer& L) {
     return CR_OK;
 }
 
-// the key plan of one chunk size, appended to the upload `hv` (offsets until the upload has an address)
-struct KeyPlanAt { KeyPlan k; size_t row_key, row_slot, pieces, pre_key, pre_slot; };
-KeyPlanAt plan_keys(const Step& sp, int chunk, int max_tokens, std::vector<int32_t>& hv) {
-    KeyPlanAt o{};
-    o.k.ring = std::min(chunk, max_tokens);
-    std::vector<int32_t> key, slot, pieces, pk, ps;
-    int base = 0;
-    for (const Step::Seg& g : sp.segs) {
-        const int pre = g.pos0 % chunk, last_chunk = (g.pos0 + g.S - 1) / chunk;
-        for (int i = 0; i < pre; i++) { pk.push_back(base + i); ps.push_back(g.seq * o.k.ring + i); }
-        for (int t = 0; t < g.S; t++) {
-            const int pos = g.pos0 + t;
-            key.push_back(base + pre + t);
-            slot.push_back(pos / chunk == last_chunk ? g.seq * o.k.ring + pos % chunk : -1);
-        }
-        for (int t = 0; t < g.S;) {
-            const int at = (g.pos0 + t) % chunk, n = std::min(g.S - t, chunk - at);
-            for (int32_t v : {g.row0 + t, n, at, base + pre + t - at}) pieces.push_back(v);
-            o.k.longest = std::max(o.k.longest, n);
-            t += n;
-        }
-        base += pre + g.S;
-    }
-    o.k.Mk = base; o.k.n_pieces = (int)pieces.size() / 4; o.k.n_pre = (int)pk.size();
-    auto put = [&](const std::vector<int32_t>& v) { const size_t at = hv.size(); hv.insert(hv.end(), v.begin(), v.end()); return at; };
-    o.row_key = put(key); o.row_slot = put(slot); o.pieces = put(pieces); o.pre_key = put(pk); o.pre_slot = put(ps);
-    return o;
-}
-
 }  // namespace
 
 extern "C" {
@@ -858,56 +828,36 @@ int cr_llm_prefill_tokens(cr_ctx* c, cr_kv* kv, const int32_t* seqs, int n, cons
     CR_HIP(hipSetDevice(c->device));
     hipStream_t st = (hipStream_t)stream;
     const int V = lm.d.vocab, piece = std::max(n, std::min(std::max(n_want, 1), 4096));
-    // one host-to-device copy: tokens, then per row sequence and position, per segment its bounds (two orders), the last rows, first retention chunks, the rows asked for, the chunks, key plans
-    const size_t fixed = (size_t)M * 4 + (size_t)n * 10 + n_want;
-    std::vector<int32_t> hv(fixed);
-    memcpy(hv.data(), tokens, (size_t)M * 8);
-    int32_t *h_seq = hv.data() + 2 * (size_t)M, *h_pos = h_seq + M, *h_seg = h_pos + M, *h_rseg = h_seg + 4 * n, *h_last = h_rseg + 4 * n, *h_snap = h_last + n, *h_want = h_snap + n;
-    for (int i = 0; i < n; i++) {
-        const Step::Seg& sg = sp.segs[i];
-        for (int r = 0; r < sg.S; r++) { h_seq[sg.row0 + r] = sg.seq; h_pos[sg.row0 + r] = sg.pos0 + r; }
-        const int32_t b0[4] = {sg.row0, sg.S, sg.pos0, sg.key0}, b1[4] = {sg.row0, sg.S, sg.pos0, sg.seq};
-        memcpy(h_seg + 4 * i, b0, 16);
-        memcpy(h_rseg + 4 * i, b1, 16);
-        h_last[i] = sg.row0 + sg.S - 1;
-        h_snap[i] = sp.snaps;
-        sp.snaps += ret_chunks(sg.S);
-        sp.longest = std::max(sp.longest, sg.S);
-    }
-    if (n_want) memcpy(h_want, want, (size_t)n_want * 4);
-    const size_t at_chunks = hv.size();
-    for (const Step::Seg& sg : sp.segs)
-        for (int t = 0; t < sg.S; t += RET_CHUNK) { hv.push_back(sg.row0 + t); hv.push_back(std::min(RET_CHUNK, sg.S - t)); }
-    std::vector<KeyPlanAt> at;
-    for (int chunk : lm.chunks) { at.push_back(plan_keys(sp, chunk, kv->max_tokens, hv)); sp.plans.push_back(at.back().k); }
-    CR_TRY(ws_ensure(c, carve_bytes(lm, sp) + (size_t)piece * lm.Wp * lm.esz() + (size_t)n * V * 4 + hv.size() * 4 + 8192));
+    const PromptUpload up = prompt_upload(sp.segs, M, tokens, want, n_want, lm.chunks, kv->max_tokens, RET_CHUNK);
+    sp.snaps = up.snaps; sp.longest = up.longest;
+    for (const PromptKeys& k : up.keys) sp.plans.push_back({k.ring, k.n_pieces, k.longest, k.n_pre, k.Mk, nullptr, nullptr, nullptr, nullptr, nullptr});
+    CR_TRY(ws_ensure(c, carve_bytes(lm, sp) + (size_t)piece * lm.Wp * lm.esz() + (size_t)n * V * 4 + up.words.size() * 4 + 8192));
     Arena ar(c->ws);
     Buffers b = carve(lm, ar, sp);
     void* hl = ar.take<char>((size_t)piece * lm.Wp * lm.esz());
     float* lg = ar.take<float>((size_t)n * V);
-    int32_t* dv = ar.take<int32_t>(hv.size());
-    CR_HIP(hipMemcpyAsync(dv, hv.data(), hv.size() * 4, hipMemcpyHostToDevice, st));       // pageable source: staged before return
+    int32_t* dv = ar.take<int32_t>(up.words.size());
+    CR_HIP(hipMemcpyAsync(dv, up.words.data(), up.words.size() * 4, hipMemcpyHostToDevice, st));       // pageable source: staged before return
     CR_HIP(hipMemcpyAsync(kv->d_seqs, seqs, (size_t)n * 4, hipMemcpyHostToDevice, st));
     kv->seqs_on_device.assign(seqs, seqs + n);
     sp.tokens = (const int64_t*)dv;
-    sp.ix.row_seq = dv + 2 * (size_t)M; sp.ix.row_pos = sp.ix.row_seq + M; sp.d_seg = sp.ix.row_pos + M; sp.d_rseg = sp.d_seg + 4 * n;
-    const int32_t *d_last = sp.d_rseg + 4 * n, *d_want = d_last + 2 * n;
-    sp.d_snap0 = d_last + n; sp.d_chunks = dv + at_chunks;
-    for (size_t i = 0; i < at.size(); i++) {
+    sp.ix.row_seq = dv + up.row_seq; sp.ix.row_pos = dv + up.row_pos; sp.d_seg = dv + up.seg; sp.d_rseg = dv + up.rseg; sp.d_snap0 = dv + up.snap0; sp.d_chunks = dv + up.chunks;
+    for (size_t i = 0; i < up.keys.size(); i++) {
         KeyPlan& k = sp.plans[i];
-        k.row_key = dv + at[i].row_key; k.row_slot = dv + at[i].row_slot; k.pieces = dv + at[i].pieces; k.pre_key = dv + at[i].pre_key; k.pre_slot = dv + at[i].pre_slot;
+        const PromptKeys& at = up.keys[i];
+        k.row_key = dv + at.row_key; k.row_slot = dv + at.row_slot; k.pieces = dv + at.pieces; k.pre_key = dv + at.pre_key; k.pre_slot = dv + at.pre_slot;
     }
     CR_TRY(run_passes(c, kv, sp, b, nullptr, st));
-    if (n_want) CR_TRY(lm_head(c, lm, b.x, d_want, n_want, hl, piece, want_logits, st));
+    if (n_want) CR_TRY(lm_head(c, lm, b.x, dv + up.want, n_want, hl, piece, want_logits, st));
     // the rows asked for are often the last rows: their logits serve the pick too
-    const bool same = n_want == n && memcmp(h_want, h_last, (size_t)n * 4) == 0;
+    const bool same = up.want_is_last;
     const bool own = logits_in_place(same ? want_logits : last_logits, penalty);
     if (own) lg = same ? want_logits : last_logits;
-    if (!same) CR_TRY(lm_head(c, lm, b.x, d_last, n, hl, piece, lg, st));
+    if (!same) CR_TRY(lm_head(c, lm, b.x, dv + up.last, n, hl, piece, lg, st));
     else if (!own) CR_HIP(hipMemcpyAsync(lg, want_logits, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
     if (last_logits && last_logits != lg) CR_HIP(hipMemcpyAsync(last_logits, lg, (size_t)n * V * 4, hipMemcpyDeviceToDevice, st));
     CR_TRY(launch_pick(lg, V, V, penalty, n, kv->d_seqs, kv, 0, st));
-    for (const Step::Seg& sg : sp.segs) {
+    for (const PromptSeg& sg : sp.segs) {
         kv->len[sg.seq] += sg.S;
         if (kv->ngen[sg.seq] < kv->gen_cap) kv->ngen[sg.seq] += 1;
     }

@@ -220,7 +220,6 @@ struct RetParams {
     const int32_t* chunks; int n_chunks;              // prompts, matrix form: {first row, rows} of every chunk of RET_CHUNK rows
 };
 bool ret_matrix_supported(int Kp, int Vp);
-inline int ret_chunks(int rows) { return (rows + RET_CHUNK - 1) / RET_CHUNK; }
 // merge: decode splits that the attention beside it left (AttnParams::no_merge), of heads of merge_dim columns
 int launch_ret_decode(bool f32, const RetParams& p, const AttnParams* merge, int merge_dim, hipStream_t st);
 int launch_ret_recurrent(bool f32, const RetParams& p, hipStream_t st);

@@ -81,3 +81,27 @@ def test_decode_attention_of_one_split(n):
     lens = torch.tensor([n - 1, 0, max(n - 2, 0), n // 2], dtype=torch.int32, device='cuda')
     one, two = (E.op_decode_attention(q, kc, vc, seqs, lens, max_keys=k) for k in (256, 257))
     assert torch.isfinite(one.float()).all() and torch.equal(one, two)
+
+
+def test_rows_asked_for_in_a_long_call():
+    """A call of more than 8190 prompt rows (its upload is past the heap's largest block), one row asked for of each prompt: the last ones, the ones ahead of them, the last ones in
+    another order.  The picked ids are those of the last rows each time."""
+    from callireader_amd.modeling_decoder import LinasunForCausalLM
+    cfg = dict(LC.TINY, vocab=211)
+    m = LinasunForCausalLM.from_state_dict(LC.weights(cfg, 6), cfg, dtype=torch.float32, max_tokens=2100, max_seqs=4)
+    toks = [LC.tokens(cfg, 2050 - i, seed=i) for i in range(4)]
+
+    def ids_and_logits(places):
+        z = m.step([(i, t, [p]) for i, (t, p) in enumerate(zip(toks, places))])
+        ids = [m.slots.kv.generated(m.slots.slot[i]) for i in range(4)]
+        m.slots.clear()
+        return ids, z
+
+    last = [len(t) - 1 for t in toks]
+    ids, z = ids_and_logits(last)
+    assert ids == [[int(i)] for i in z.argmax(-1)] and torch.isfinite(z).all()
+    other, z2 = ids_and_logits([p - 1 for p in last])
+    assert other == ids and not torch.equal(z2, z)
+    mixed, z3 = ids_and_logits(last[:2] + [0, 0])
+    assert mixed == ids and torch.equal(z3[:2], z[:2])
+    m.close()
