@@ -348,10 +348,10 @@ size_t carve_bytes(const Lm& lm, const Step& sp) {
 
 // C[M, N] = A . W^T in the model's element type: the engine's dense kernels for bf16, the fp32 tile kernel otherwise
 int dense(cr_ctx* c, const Lm& lm, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, hipStream_t st, bool prompt, const bf16* dl = nullptr,
-          bool relu2 = false) {
+          bool relu2 = false, bool parts = false) {
     if (lm.f32) {
         LmGemmParams p{};
-        p.A = A; p.lda = lda; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.stream = !prompt && M <= LM_ROWS_MAX;
+        p.A = A; p.lda = lda; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.stream = !prompt && M <= LM_ROWS_MAX; p.slices = parts ? lm_rows_slices(N, K) : 1;
         return launch_lm_gemm(true, relu2 ? LM_RELU2 : LM_STORE, p, st);
     }
     GemmParams p{};
@@ -361,7 +361,7 @@ int dense(cr_ctx* c, const Lm& lm, const void* A, int64_t lda, const void* W, vo
     return ctx_gemm(c, relu2 ? EPI_RELU2 : EPI_STORE, p, st);
 }
 // the same product left in fp32 (router scores, logits, the looped span's entry); few: rows that fp32 streams the weights for (decode steps, logits)
-int raw32(cr_ctx* c, const Lm& lm, const void* A, const void* W, float* C, int64_t ldc, int M, int N, int K, float softcap, hipStream_t st, bool few, const bf16* dl = nullptr) {
+int raw32(cr_ctx* c, const Lm& lm, const void* A, const void* W, float* C, int64_t ldc, int M, int N, int K, float softcap, hipStream_t st, bool few, const bf16* dl = nullptr, bool parts = false) {
     if (!lm.f32) {
         GemmParams p{};
         p.A = (const bf16*)A; p.lda = K; p.W = (const bf16*)W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.raw32 = 1; p.softcap = softcap;
@@ -369,7 +369,7 @@ int raw32(cr_ctx* c, const Lm& lm, const void* A, const void* W, float* C, int64
         return ctx_gemm(c, EPI_F32, p, st);
     }
     LmGemmParams p{};
-    p.A = A; p.lda = K; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.softcap = softcap; p.stream = few && M <= LM_ROWS_MAX;
+    p.A = A; p.lda = K; p.W = W; p.ldw = K; p.C = C; p.ldc = ldc; p.M = M; p.N = N; p.K = K; p.softcap = softcap; p.stream = few && M <= LM_ROWS_MAX; p.slices = parts ? lm_rows_slices(N, K) : 1;
     return launch_lm_gemm(lm.f32, LM_RAW32, p, st);
 }
 
@@ -382,7 +382,7 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
     char* cache = kv->lat + kv->lat_off[r];
     const int s_a = slices_of(lm, M, L.Na, Wp, sp.decode);
     if (s_a) CR_TRY(sliced(c, b.h, Wp, L.wa, L.wa_dl, b.sl, M, L.Na, Wp, st));
-    else CR_TRY(dense(c, lm, b.h, Wp, L.wa, b.a, L.Na, M, L.Na, Wp, st, !sp.decode, L.wa_dl));
+    else CR_TRY(dense(c, lm, b.h, Wp, L.wa, b.a, L.Na, M, L.Na, Wp, st, !sp.decode, L.wa_dl, false, true));
     CR_TRY(launch_lm_latents(lm.f32, lm, L, M, b.a, s_a ? b.sl : nullptr, s_a, b.cq, sp.decode ? nullptr : b.c, cache, kv->max_tokens, sp.ix, b.ao, st));
     const int s_q = !lm.f32 && L.Ap <= 512 ? slices_of(lm, M, H * L.Ap, L.Qp, sp.decode) : 0;
     if (s_q) CR_TRY(sliced(c, b.cq, L.Qp, L.wuq, L.wuq_dl, b.sl, M, H * L.Ap, L.Qp, st));
@@ -435,7 +435,7 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
     const size_t es = lm.esz();
     const int s_a = slices_of(lm, M, L.Na, Wp, sp.decode);
     if (s_a) CR_TRY(sliced(c, b.h, Wp, L.wa, L.wa_dl, b.sl, M, L.Na, Wp, st));
-    else CR_TRY(dense(c, lm, b.h, Wp, L.wa, b.a, L.Na, M, L.Na, Wp, st, !sp.decode, L.wa_dl));
+    else CR_TRY(dense(c, lm, b.h, Wp, L.wa, b.a, L.Na, M, L.Na, Wp, st, !sp.decode, L.wa_dl, false, true));
     const KeyPlan* kp = L.heads() && !sp.decode ? &sp.plans[L.chunk_ix] : nullptr;
     const int ring = L.heads() ? std::min(lm.chunks[L.chunk_ix], kv->max_tokens) : 1, chunk = L.heads() ? lm.chunks[L.chunk_ix] : 1;
     char *ck = kv->lat + kv->lat_off[r], *cv = ck + (size_t)kv->n_seqs * a.kv_heads * ring * L.Ap * es;
@@ -546,7 +546,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
     auto project = [&](const void* A, const void* W, const bf16* dl, int K, LmPostIn& out) -> int {
         const int n = slices_of(lm, M, Wp, K, sp.decode);
         out = LmPostIn{n ? (const void*)b.sl : b.y, Wp, n, nullptr, 0};
-        return n ? sliced(c, A, K, W, dl, b.sl, M, Wp, K, st) : dense(c, lm, A, K, W, b.y, Wp, M, Wp, K, st, !sp.decode, dl);
+        return n ? sliced(c, A, K, W, dl, b.sl, M, Wp, K, st) : dense(c, lm, A, K, W, b.y, Wp, M, Wp, K, st, !sp.decode, dl, false, true);
     };
     CR_TRY(launch_lm_embed(lm.f32, lm, M, sp.tokens, sp.ix, kv->d_gen, kv->d_ngen, kv->gen_cap, b.x, entry(0), b.tok, lm.d.loop_in ? (char*)b.cat + (size_t)Wp * es : nullptr, 2 * Wp, st));
     CR_TRY(probe(0));
@@ -560,7 +560,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
                 CR_TRY(sliced(c, b.cat, 2 * Wp, lm.loop_in, lm.loop_dl, b.sl, M, Wp, 2 * Wp, st));
                 CR_TRY(launch_lm_post(lm.f32, lm, M, LmPostIn{b.sl, Wp, n, nullptr, 0}, b.x, nullptr, true, to, st));
             } else {
-                CR_TRY(raw32(c, lm, b.cat, lm.loop_in, b.x, Wp, M, Wp, 2 * Wp, 0.f, st, sp.decode, sp.decode ? lm.loop_dl : nullptr));
+                CR_TRY(raw32(c, lm, b.cat, lm.loop_in, b.x, Wp, M, Wp, 2 * Wp, 0.f, st, sp.decode, sp.decode ? lm.loop_dl : nullptr, true));
                 CR_TRY(launch_lm_pick_rows(lm.f32, lm, M, b.x, nullptr, b.h, L.n1, st));
             }
         }

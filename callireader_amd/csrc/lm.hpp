@@ -88,10 +88,16 @@ struct LmGemmParams {
     const void* gate; int64_t ldg;
     const int32_t* tok;
     int stream;                                     // fp32, M <= LM_ROWS_MAX (grouped: M = the tokens, an expert sees at most that many): lm_gemm_rows.hip's few-row form
-    int slices;                                     // stream, LM_RAW32: K-slices C [slices][M][ldc] for a consumer that adds them
+    int slices;                                     // fp32: parts of K (see below), 0 = 1; stream with more than one: LM_RAW32, C [slices][M][ldc] for a consumer that adds them
 };
 int launch_lm_gemm(bool f32, int epi, const LmGemmParams& p, hipStream_t st);
 constexpr int LM_TILE_M = 64;
+// The order of a sum in an fp32 product, the same from the few-row and the tile kernel, so that its bits depend neither on the rows it comes with nor on decode or prompt: K in `slices`
+// equal parts, a part in LM_CHAINS chains of consecutive blocks of 32 (as many blocks as divide the part evenly, rounded up; the last chains may be shorter or empty), a chain in ascending
+// steps; chains are added in order, then parts in order.
+constexpr int LM_CHAINS = 8;
+__host__ __device__ inline int lm_part_blocks(int K, int slices) { return K / 32 / (slices > 1 ? slices : 1); }
+__host__ __device__ inline int lm_chain_blocks(int part) { return (part + LM_CHAINS - 1) / LM_CHAINS; }
 constexpr int LM_ROWS_MAX = 64, LM_ROWS_MAX_SLICES = 8;
 int launch_lm_gemm_rows(int epi, const LmGemmParams& p, hipStream_t st);
 int launch_lm_gemm_tiles(int epi, const LmGemmParams& p, hipStream_t st);

@@ -154,7 +154,7 @@ int launch_t(int epi, const LmGemmParams& p, hipStream_t st) {
 int launch_lm_gemm(bool f32, int epi, const LmGemmParams& p, hipStream_t st) {
     const int vec = f32 ? 4 : 8;
     if (p.N <= 0 || p.K <= 0 || p.K % 64 || p.lda % vec || p.ldw % vec || p.a_bs % vec || p.w_bs % vec || (p.tiles ? p.max_tiles <= 0 || p.batch > 1 || !p.n_tiles : p.M <= 0) ||
-        (p.gather_div && !p.perm) || (epi == LM_GLU && (p.N % 16 || p.batch > 1)) || ((epi == LM_GATE || epi == LM_SIDE) && !p.gate) || (epi == LM_SIDE && !p.tok) || (((uintptr_t)p.A | (uintptr_t)p.W) & 15))
+        (p.gather_div && !p.perm) || (epi == LM_GLU && (p.N % 16 || p.batch > 1)) || ((epi == LM_GATE || epi == LM_SIDE) && !p.gate) || (epi == LM_SIDE && !p.tok) || (p.slices > 1 && (!f32 || p.K % (32 * p.slices))) || (((uintptr_t)p.A | (uintptr_t)p.W) & 15))
         return cr_fail(CR_ERR_ARG, "lm_gemm(epi=%d M=%d N=%d K=%d): bad argument", epi, p.M, p.N, p.K);
     if (p.stream) return f32 ? launch_lm_gemm_rows(epi, p, st) : cr_fail(CR_ERR_ARG, "lm_gemm: the few-row form is fp32");
     return f32 ? launch_lm_gemm_tiles(epi, p, st) : launch_t(epi, p, st);

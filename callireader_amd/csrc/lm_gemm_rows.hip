@@ -7,12 +7,12 @@
 // 64 clocks of the CU's load path instead of 16 (two rows: 1024 x 1536 .. 4096 6.9 us -> 5.5, 3584 x 1024 10.3 -> 7.2, 4096 x 1024 8.8 -> 7.1, 64 x 1024 6.0 -> 4.6).
 // A lane multiplies with k = 4 (lane >> 4) .. + 3 of a 16-deep step of its weight row and of its activation row: the four multiplications of a step take one element
 // of each, which permutes k inside the step for both operands alike.  Partial tiles of the waves meet in LDS and are added in wave order; slices go to the consumer, which adds them
-// in slice order.  A row's sum depends on N and K (slices), never on the other rows.
+// in slice order: the order of lm.hpp, a wave a chain.
 #include "lm.hpp"
 
 namespace {
 
-constexpr int NW = 8;                        // waves of a workgroup
+constexpr int NW = LM_CHAINS;                // waves of a workgroup, one chain of the sum each
 
 template <int MT, int EPI>
 __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) {
@@ -31,8 +31,8 @@ __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) 
         W += (int64_t)t.x * p.w_bs;
         pos0 = t.y; rows = min(t.z, MT * 16);
     } else W += (int64_t)blockIdx.z * p.w_bs;
-    const int slice = p.tiles ? 0 : blockIdx.y, steps = p.K / 16 / max(p.slices, 1);      // 16-deep steps of this slice
-    const int per = (steps + NW - 1) / NW, s0 = slice * steps + min(wave * per, steps), s1 = slice * steps + min(wave * per + per, steps);
+    const int slice = p.tiles ? 0 : blockIdx.y, blocks = lm_part_blocks(p.K, p.slices), steps = 2 * blocks;      // 16-deep steps of this slice
+    const int per = 2 * lm_chain_blocks(blocks), s0 = slice * steps + min(wave * per, steps), s1 = slice * steps + min(wave * per + per, steps);
 
     // a load instruction brings 16 rows x 16 k, four neighbouring lanes a row's 64 bytes, into the wave's own KiB of LDS; the 16-byte chunks of rows 8..15 are exchanged in pairs on both
     // sides (reads without bank conflicts)
@@ -126,16 +126,16 @@ int launch_t(int epi, const LmGemmParams& p, hipStream_t st) {
 
 }  // namespace
 
-// Slices of a product whose consumer adds them: enough 16-row tiles for one workgroup per CU, at least 16 steps (two per wave) a slice.
+// Slices of a product whose consumer adds them: enough 16-row tiles for one workgroup per CU, at least 16 steps (two per wave) a slice, whole blocks of 32.
 int lm_rows_slices(int N, int K) {
     int s = 1;
-    while (s < LM_ROWS_MAX_SLICES && (N + 15) / 16 * s < 256 && K % (32 * s) == 0 && K / (2 * s) >= 256) s *= 2;
+    while (s < LM_ROWS_MAX_SLICES && (N + 15) / 16 * s < 256 && K % (64 * s) == 0 && K / (2 * s) >= 256) s *= 2;
     return s;
 }
 
 int launch_lm_gemm_rows(int epi, const LmGemmParams& p, hipStream_t st) {      // (checked by launch_lm_gemm)
     const int most = p.tiles ? std::min(p.M, LM_TILE_M) : p.M;
-    if (p.M <= 0 || most > LM_ROWS_MAX || (p.slices > 1 && (p.tiles || p.batch > 1 || epi != LM_RAW32 || p.softcap > 0.f || p.K % (16 * p.slices))))
+    if (p.M <= 0 || most > LM_ROWS_MAX || (p.slices > 1 && (p.tiles || p.batch > 1 || epi != LM_RAW32 || p.softcap > 0.f)))
         return cr_fail(CR_ERR_ARG, "lm_gemm_rows(epi=%d M=%d N=%d K=%d slices=%d): bad argument", epi, p.M, p.N, p.K, p.slices);
     return most <= 16 ? launch_t<1>(epi, p, st) : most <= 32 ? launch_t<2>(epi, p, st) : launch_t<4>(epi, p, st);
 }

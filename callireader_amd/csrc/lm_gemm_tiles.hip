@@ -3,11 +3,11 @@
 //
 // Bound by the matrix cores (v_mfma_f32_16x16x4_f32: 256 operations a clock and CU) where the grid fills the card, by what lies between K-tiles where it does not.  The form of
 // gemm_mid.hip: NBUF K-tiles in LDS, NBUF - 1 of them under way, one barrier a K-tile, eight rows of 128 bytes a load instruction; the tile shape is picked by the rounds it gives.
-// 402 rows, us: products of 1024 columns over K = 64, 1536 and 4096 49 on average -> 5, 21 and 46 (32 x 64 tiles, K-tiles of 64: 52 with K-tiles of 32), 3584 x 1024 50 -> 43 and
-// 4096 x 1024 with the squared relu 51 -> 43 (112 x 64; 22 us of multiplications; 41 with one chain a sum, whose error against 64 bits is 1.4 to 1.7 times that of two).  Before:
-// 64 x 64 tiles, one K-tile of 32 in LDS, two barriers each.
+// 402 rows, us: products of 1024 columns over K = 64, 1536 and 4096 49 on average -> 5, 22 and 49 (32 x 64 tiles, K-tiles of 64), 3584 x 1024 50 -> 42 and
+// 4096 x 1024 with the squared relu 51 -> 42 (112 x 64; 22 us of multiplications).  Before: 64 x 64 tiles, one K-tile of 32 in LDS, two barriers each.
 // A lane reads 16 bytes of its row, k = 16 h + 4 (lane >> 4) .. + 3; the four multiplications take one element of each, which permutes k inside 16 for both operands alike.  A row's
-// sum runs over K in two chains, the even and the odd 16-steps, whatever the tile.
+// sum has the order of lm.hpp whatever the tile: an accumulator is a chain, and goes to the part's sum and that to the total when it ends.  That costs 1.6 us of the 22 where a chain is one block of 32 (two chains over all of K: 20), nothing on
+// the larger tiles, whose waves multiply under each other's additions.
 #include <algorithm>
 #include <type_traits>
 
@@ -119,11 +119,13 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
         for (int i = 0; i < G::PER; i++)
             if (!dead[i] || lane == 0) __builtin_amdgcn_global_load_lds(CR_GLB(src[i] + (int64_t)kt * (32 * KB)), CR_LDS(smem + buf * G::STAGE + dst[i]), 16, 0, 0);
     };
-    f32x4 acc[FM][FN], odd[FM][FN];                           // the even and the odd 16-steps of K: two chains of half the length
+    f32x4 acc[FM][FN], part[FM][FN], total[FM][FN];           // of the chain, of the part, of the whole sum
 #pragma unroll
     for (int i = 0; i < FM; i++)
 #pragma unroll
-        for (int j = 0; j < FN; j++) acc[i][j] = odd[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < FN; j++) acc[i][j] = part[i][j] = total[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+    const int part_blocks = lm_part_blocks(p.K, p.slices), chain_blocks = lm_chain_blocks(part_blocks);
+    int in_part = part_blocks, in_chain = chain_blocks;       // blocks of 32 until they end
     const int swz = (lane >> 1) & 7;
     const int c_off[2] = {((lane >> 4) ^ swz) * 16, ((4 + (lane >> 4)) ^ swz) * 16};
     const int a_off = (wf0 * 16 + (lane & 15)) * 128, w_off = (G::BM + wn * FN * 16 + (lane & 15)) * 128;
@@ -140,20 +142,34 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
                 if (i < decltype(count)::value) f.a[h][i] = *(const f32x4*)(s + a_off + i * 2048 + at);
         }
     };
+    auto fold = [&](f32x4 (&to)[FM][FN], f32x4 (&from)[FM][FN], auto count) {
+#pragma unroll
+        for (int i = 0; i < FM; i++)
+            if (i < decltype(count)::value) {
+#pragma unroll
+                for (int j = 0; j < FN; j++) { to[i][j] += from[i][j]; from[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
+            }
+    };
     auto multiply = [&](const Frags& f, auto count) {
 #pragma unroll
-        for (int h = 0; h < 2 * KB; h++)
+        for (int kb = 0; kb < KB; kb++) {
 #pragma unroll
-            for (int e = 0; e < 4; e++)
+            for (int h = 2 * kb; h < 2 * kb + 2; h++)
 #pragma unroll
-                for (int i = 0; i < FM; i++)
-                    if (i < decltype(count)::value) {
+                for (int e = 0; e < 4; e++)
 #pragma unroll
-                        for (int j = 0; j < FN; j++) {
-                            f32x4& c = h & 1 ? odd[i][j] : acc[i][j];
-                            c = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[h][j][e], f.a[h][i][e], c, 0, 0, 0);
+                    for (int i = 0; i < FM; i++)
+                        if (i < decltype(count)::value) {
+#pragma unroll
+                            for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[h][j][e], f.a[h][i][e], acc[i][j], 0, 0, 0);
                         }
-                    }
+            in_chain--; in_part--;
+            if (in_chain == 0 || in_part == 0) {              // (uniform)
+                fold(part, acc, count);
+                in_chain = chain_blocks;
+                if (in_part == 0) { fold(total, part, count); in_part = part_blocks; }
+            }
+        }
     };
     auto arrive = [&](int t) {                                // K-tile t has landed in every wave's pieces, and every wave holds tile t - 1 in registers
         const int behind = nk - 1 - t;
@@ -192,18 +208,14 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
     if (live == FM) loop(std::integral_constant<int, FM>{});
     else if (FM > 1 && live == FM - 1) loop(std::integral_constant<int, FM - 1>{});
     else loop(std::integral_constant<int, 0>{});
-#pragma unroll
-    for (int i = 0; i < FM; i++)
-#pragma unroll
-        for (int j = 0; j < FN; j++) acc[i][j] += odd[i][j];
     const int row0 = m0 + wf0 * 16, col0 = n0 + wn * FN * 16;
     switch (epi) {                                            // (uniform)
-        case LM_STORE: epilogue<LM_STORE, FM, FN>(p, acc, row0, live, rows, pos0, col0, lane); break;
-        case LM_RAW32: epilogue<LM_RAW32, FM, FN>(p, acc, row0, live, rows, pos0, col0, lane); break;
-        case LM_GLU: epilogue<LM_GLU, FM, FN>(p, acc, row0, live, rows, pos0, col0, lane); break;
-        case LM_GATE: epilogue<LM_GATE, FM, FN>(p, acc, row0, live, rows, pos0, col0, lane); break;
-        case LM_RELU2: epilogue<LM_RELU2, FM, FN>(p, acc, row0, live, rows, pos0, col0, lane); break;
-        case LM_SIDE: epilogue<LM_SIDE, FM, FN>(p, acc, row0, live, rows, pos0, col0, lane); break;
+        case LM_STORE: epilogue<LM_STORE, FM, FN>(p, total, row0, live, rows, pos0, col0, lane); break;
+        case LM_RAW32: epilogue<LM_RAW32, FM, FN>(p, total, row0, live, rows, pos0, col0, lane); break;
+        case LM_GLU: epilogue<LM_GLU, FM, FN>(p, total, row0, live, rows, pos0, col0, lane); break;
+        case LM_GATE: epilogue<LM_GATE, FM, FN>(p, total, row0, live, rows, pos0, col0, lane); break;
+        case LM_RELU2: epilogue<LM_RELU2, FM, FN>(p, total, row0, live, rows, pos0, col0, lane); break;
+        case LM_SIDE: epilogue<LM_SIDE, FM, FN>(p, total, row0, live, rows, pos0, col0, lane); break;
     }
 }
 

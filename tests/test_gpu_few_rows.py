@@ -76,3 +76,38 @@ def test_fp32_decode_row_alone_and_among_others(name):
     alone = m.step([('a', toks[7][-1:], [0])]).cpu()
     m.close()
     assert torch.equal(alone[0], z[7])
+
+
+# sums cut into parts (K of 1024 and 2048 in four, the feed-forward's 1088 in two of 17 blocks, which chains of three do not divide)
+WIDE_SUMS = LUG.config(1024, 300, [LUG.layer(LUG.heads(4, 2, 64, 64, 4096), LUG.ret(64, 64, (0.9, 0.99)), 1088)], side=20, loop=(0, 1, 2))
+
+
+@pytest.mark.parametrize('name', [*CASES, 'lugasun_wide_sums'])
+def test_fp32_row_among_64_and_65(name):
+    """64 rows are the few-row kernel's, 65 the tile kernel's: a row's bits are the same alone, among 64 and among 65, decoded or asked for in a prompt."""
+    from callireader_amd import modeling_decoder as MD
+    cases, oracle, cfg = CASES.get(name, (LUG, OLUG, WIDE_SUMS))
+    cls = MD.LugasunForCausalLM if cases is LUG else MD.LinasunForCausalLM
+    w = cases.weights(cfg, 45)
+    m = cls.from_state_dict(w, cfg, dtype=torch.float32, max_tokens=100, max_seqs=65)
+    toks = [cases.tokens(cfg, 3 + 7 * i % 40, seed=i) for i in range(65)]
+
+    def decoded(n):
+        m.step([(i, t[:-1], []) for i, t in enumerate(toks[:n])])
+        z = m.step([(i, t[-1:], [0]) for i, t in enumerate(toks[:n])])
+        m.slots.clear()
+        return z
+
+    def asked(n):
+        z = m.step([('a', t, list(range(90 - n, 90)))])
+        m.slots.clear()
+        return z
+
+    one, few, many = decoded(1), decoded(64), decoded(65)
+    assert torch.equal(few, many[:64]) and torch.equal(one, few[:1])
+    assert cases.rel(many[64:].cpu(), oracle.forward(w, cfg, toks[64])[-1:]) < 2e-5
+    t = cases.tokens(cfg, 90, seed=3)
+    one, few, many = asked(1), asked(64), asked(65)
+    assert torch.equal(few, many[1:]) and torch.equal(one, few[-1:])
+    assert cases.rel(many.cpu(), oracle.forward(w, cfg, t)[25:]) < 2e-5
+    m.close()
