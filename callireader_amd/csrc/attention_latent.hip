@@ -12,7 +12,7 @@ namespace {
 template <typename T, int TPB>
 __global__ __launch_bounds__(TPB) void latent_attn_plain_kernel(const LatentAttnParams p) {
     extern __shared__ __attribute__((aligned(16))) float sm[];
-    __shared__ float red[2 * TPB / 64];
+    __shared__ float red[PLAIN_RED];
     const int row = blockIdx.x, head = blockIdx.y;
     const int seq = p.ix.row_seq ? p.ix.row_seq[row] : p.ix.seqs[row];
     const int n = (p.ix.row_pos ? p.ix.row_pos[row] : p.ix.lens[seq]) + 1;

@@ -169,7 +169,7 @@ __global__ __launch_bounds__(256) void lm_prefix_kernel(const int32_t* __restric
 template <typename T, int TPB>
 __global__ __launch_bounds__(TPB) void heads_attn_plain_kernel(const HeadsAttnParams p) {
     extern __shared__ __attribute__((aligned(16))) float sm[];
-    __shared__ float red[2 * TPB / 64];
+    __shared__ float red[PLAIN_RED];
     const int row = blockIdx.x, head = blockIdx.y;
     const int g = head / (p.H / p.G);
     const int seq = p.ix.row_seq ? p.ix.row_seq[row] : p.ix.seqs[row];
@@ -182,8 +182,7 @@ __global__ __launch_bounds__(TPB) void heads_attn_plain_kernel(const HeadsAttnPa
 
 template <typename T>
 void launch_plain_t(const HeadsAttnParams& p, hipStream_t st) {
-    // decode: few workgroups, sixteen waves each (a row's chain of loads is what counts); prompts: four, the chip is full.  (Not by the number of rows: the waves share a row's sums
-    // out, and a row's bits must not depend on what it is computed with.)
+    // decode: few workgroups, sixteen waves each (a row's chain of loads is what counts); prompts: four, the chip is full.  The same bits either way.
     if (!p.ix.row_pos) hipLaunchKernelGGL((heads_attn_plain_kernel<T, 1024>), dim3(p.M, p.H), dim3(1024), plain_lds_floats(p.Ap, 1024) * 4, st, p);
     else hipLaunchKernelGGL((heads_attn_plain_kernel<T, 256>), dim3(p.M, p.H), dim3(256), plain_lds_floats(p.Ap, 256) * 4, st, p);
 }

@@ -111,3 +111,27 @@ def test_fp32_row_among_64_and_65(name):
     assert torch.equal(few, many[1:]) and torch.equal(one, few[-1:])
     assert cases.rel(many.cpu(), oracle.forward(w, cfg, t)[25:]) < 2e-5
     m.close()
+
+
+# a latent of more column quads than a prompt's workgroup has threads
+WIDE_LATENT = LIN.config(128, 90, [(LIN.mixer(2, 90, 100, 40, 1100, 0.1), None)])
+
+
+@pytest.mark.parametrize('name,n', [('linasun_ragged', 60), ('linasun_many_heads', 90), ('deep_latent', 70), ('deep_latent', 1030), ('wide_latent', 40), ('wide_latent', 1100)])
+def test_fp32_row_decoded_and_in_a_prompt(name, n):
+    """The last tokens of a sequence as one prompt, as decode steps, and as a prompt of one token beside another request: the same bits.  (Cached rows of 64 to 1152 columns, one and two
+    blocks of keys.  Retention's two kernels add the squares of a row in orders of their own.)"""
+    from callireader_amd import modeling_decoder as MD
+    cfg = {'deep_latent': LIN.DEEP_LATENT, 'wide_latent': WIDE_LATENT}.get(name) or CASES[name][2]
+    w, t = LIN.weights(cfg, 46), LIN.tokens(cfg, n, seed=4)
+    m = MD.LinasunForCausalLM.from_state_dict(w, cfg, dtype=torch.float32, max_tokens=n, max_seqs=2)
+    whole = m.step([('a', t, [n - 2, n - 1])])
+    m.slots.clear()
+    m.step([('a', t[:-2], [])])
+    steps = torch.cat([m.step([('a', [x], [0])]) for x in t[-2:]])
+    m.slots.clear()
+    m.step([('a', t[:-1], [])])
+    beside = m.step([('a', t[-1:], [0]), ('b', t[:9], [])])
+    m.close()
+    assert torch.equal(whole, steps) and torch.equal(whole[1:], beside)
+    assert LIN.rel(whole.cpu(), OLIN.forward(w, cfg, t)[-2:]) < (2e-5 if n < 1000 else 1e-4)      # (angles of a thousand radians: 6e-5 radians of fp32 rounding)
