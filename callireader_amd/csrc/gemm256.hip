@@ -600,7 +600,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     // DMA sources: this wave fills sub-tiles s = 2*wave + e (e = 0,1) of every unit
     //   A units: s -> (wave row s>>3, fragment (s>>1)&3, ksub s&1);  B units: s -> (wave col s>>2, fragment (s>>1)&1, ksub s&1)
     //   lane -> row lane>>2 of the sub-tile, 16-B chunk (lane&3) ^ 2*(row>>3)
-    // kept as 32-bit byte offsets from the (uniform) operand base: operands are < 4 GiB, and the fragment double
+    // kept as 32-bit byte offsets from the (uniform) operand base: operands are < 4 GiB (rows_within_4g), and the fragment double
     // buffer below needs the registers
     const int srow = lane >> 2;
     const int schunk = (lane & 3) ^ ((srow >> 3) << 1);
@@ -903,7 +903,13 @@ int launch_t(const GemmParams& p, hipStream_t stream) {
 
 }  // namespace
 
-bool gemm256_supported(int epi, const GemmParams& p) { return epi != EPI_PARTIAL && p.N >= 64 && p.K % 128 == 0 && !p.raw32; }
+// rows reach their operand by a 32-bit byte offset from its base
+static bool rows_within_4g(const GemmParams& p) {
+    constexpr int64_t most = (1ll << 31) - 64;                // elements, a row's first K-tile included
+    return (int64_t)(p.M - 1) * p.lda < most && (int64_t)(p.N - 1) * p.ldw < most;
+}
+
+bool gemm256_supported(int epi, const GemmParams& p) { return epi != EPI_PARTIAL && p.N >= 64 && p.K % 128 == 0 && !p.raw32 && rows_within_4g(p); }
 
 double gemm256_cost(const GemmParams& p) { const double a = tile_us(p, 4), b = tile_us(p, 2); return a < b ? a : b; }
 
@@ -938,6 +944,7 @@ int launch_gemm256_f8(int epi, const GemmParams& p8, hipStream_t stream) {
 }
 
 int launch_gemm256(int epi, const GemmParams& p, hipStream_t stream) {
+    if (!rows_within_4g(p)) return CR_ERR_ARG;
     switch (epi) {
         case EPI_STORE: return launch_t<EPI_STORE>(p, stream);
         case EPI_GELU: return launch_t<EPI_GELU>(p, stream);

@@ -39,6 +39,27 @@ def test_every_shape_and_epilogue(M, N, K):
             assert torch.equal(out, first), (name, tile)
 
 
+@pytest.mark.parametrize('far', ['activations', 'weights'])
+def test_rows_more_than_4_gib_apart(far):
+    """The 256x256 kernel, which this shape would take, reaches its rows by 32-bit byte offsets; an operand that spans more goes to the tile shapes here, and a pin is an error."""
+    from callireader_amd import engine as E
+    g = torch.Generator().manual_seed(7)
+    dev = torch.device('cuda', 0)
+    M, N, K = 1536, 8192, 512
+    A, W = torch.randn(M, K, generator=g).bfloat16().to(dev), (torch.randn(N, K, generator=g) * K ** -0.5).bfloat16().to(dev)
+    want = E.op_gemm(0, A, W)
+    rows = M if far == 'activations' else N
+    ld = (2 ** 31 // (rows - 1) + 15) // 8 * 8
+    wide = torch.zeros(rows * ld, device=dev, dtype=torch.bfloat16).view(rows, ld)[:, :K]
+    wide.copy_(A if far == 'activations' else W)
+    args = (wide, W) if far == 'activations' else (A, wide)
+    assert torch.equal(E.op_gemm(0, *args), want)
+    with pytest.raises(RuntimeError):
+        E.op_gemm(0, *args, kernel=2)
+    near = (args[0][:-2], W) if far == 'activations' else (A, args[1][:-2])      # the last offset below 4 GiB
+    torch.testing.assert_close(E.op_gemm(0, *near, kernel=2), want[:-2] if far == 'activations' else want[:, :-2], rtol=0, atol=0)
+
+
 def test_rows_of_patches_keys_of_the_table_and_slices():
     """Position rows behind a class row (epi 5), first maxima of 64-column blocks (epi 8), K-slices (epi 7), an output in place of its residual."""
     from callireader_amd import engine as E
