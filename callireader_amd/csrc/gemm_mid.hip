@@ -407,6 +407,7 @@ double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
 int launch_gemm_mid(int epi, const GemmParams& p, hipStream_t stream) {
     int tile = p.tile, rt = 0;
     if (!tile) gemm_mid_cost(epi, p, &tile, &rt);
+    if (tile < 1 || tile > N_SHAPES || (epi == EPI_ARGMAX && SHAPES[tile - 1].bn != 256)) return CR_ERR_ARG;      // (a pin; a wave's columns have to be a partial's 64)
     switch (tile) {
         case 1: return launch_t<1, 2, 1, 1, 12>(epi, p, rt, stream);
         case 2: return launch_t<1, 4, 1, 1, 8>(epi, p, rt, stream);

@@ -39,6 +39,15 @@ def test_every_shape_and_epilogue(M, N, K):
             assert torch.equal(out, first), (name, tile)
 
 
+@pytest.mark.parametrize('tile', [*range(16, 26), 28, 255])
+def test_a_shape_that_cannot_take_the_epilogue_is_an_error(tile):
+    """First maxima of 64-column blocks need a wave of 64 columns; pins past the last shape name none."""
+    from callireader_amd import engine as E
+    A, W = torch.zeros(70, 128, device='cuda', dtype=torch.bfloat16), torch.zeros(192, 128, device='cuda', dtype=torch.bfloat16)
+    with pytest.raises(RuntimeError):
+        E.op_gemm(8, A, W, kernel=tile)
+
+
 @pytest.mark.parametrize('far', ['activations', 'weights'])
 def test_rows_more_than_4_gib_apart(far):
     """The 256x256 kernel, which this shape would take, reaches its rows by 32-bit byte offsets; an operand that spans more goes to the tile shapes here, and a pin is an error."""
