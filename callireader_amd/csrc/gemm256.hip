@@ -876,8 +876,9 @@ int launch_s(const GemmParams& p, hipStream_t stream) {
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
 
-// us of a launch of tiles of 256 (f1 = 4) or 192 rows (2), on the scale of gemm_mid_cost: rounds of one tile per CU, a K-tile of 256 rows 1.12 us (1000 x 4096 x 14336 takes
-// 251 us), of 192 rows 0.93 (203 us).  The shorter tile wins where it takes no more rounds (x 256 rows / 192 rows, us): 11275 x 3072 x 1024 (540 / 708 tiles) 73.7 / 62.8,
+// us of a launch of tiles of 256 (f1 = 4) or 192 rows (2), on the scale of gemm_mid_cost and like it a law to choose by: rounds of one tile per CU, a K-tile of 256 rows 1.12 us
+// (1000 x 4096 x 14336 takes 251 us), of 192 rows 0.93 (203 us).  One round is up to 14 % faster than that (1025 x 3072 x 1024 21.2 measured / 24.4, 77 x 4096 x 14336 238 / 257), rounds
+// that fill the card 5 to 16 % slower, as its clock falls (11275 x 4096 x 1024 76.7 / 66.3, 3164 x 28672 x 4096 527 / 452, 6000 x 4096 x 14336 559 / 511).  The shorter tile wins where it takes no more rounds (x 256 rows / 192 rows, us): 11275 x 3072 x 1024 (540 / 708 tiles) 73.7 / 62.8,
 // 11275 x 1024 x 4096 (180 / 236) 82.5 / 74.8, 8200 x 4096 x 1024 (528 / 688) 83.3 / 71.0, 6000 x 4096 x 14336 (384 / 512) 587 / 495; it loses where it takes one more:
 // 13325 x 1024 x 4096 (212 / 280) 91 / 130, 11275 x 4096 x 1024 (720 / 944) 89 / 94, 4700 x 28672 x 4096 (2128 / 2800) 799 / 811.
 double tile_us(const GemmParams& p, int f1) {

@@ -1,13 +1,14 @@
 // bf16 MFMA GEMM for the row counts between decode (gemm_skinny.hip) and the persistent 256x256 kernel (gemm256.hip):  C = epi(A[M,K] . W[N,K]^T),  K % 64 == 0.
 //
 // What bounds these shapes is not arithmetic but how many bytes are under way: a 128x128 grid over M = 1025, N = 1024 is 72 workgroups, and a K loop that waits for each K-tile's
-// loads before it asks for the next-but-one pays a memory round trip per 64 of K.  So (a) the tile shape is a template and picked by the grid it gives (mid_pick below), down to
-// 16 x 16 for a single wave, and (b) NBUF K-tiles live in LDS and NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles.
+// loads before it asks for the next-but-one pays a memory round trip per 64 of K.  So (a) the tile shape is a template and picked by the grid it gives (gemm_mid_cost below), down to
+// 16 x 32 for two waves, and (b) NBUF K-tiles live in LDS and NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles.
 //   * one global_load_lds_dwordx4 brings eight rows x 64 k, whole 128-byte lines (pieces of 16 rows x 32 k reach 56 of the 69 GB/s per CU that these do on cold weights);
 //     LDS rows of 128 bytes, the 16-byte chunk XORed with (row >> 1) & 7 on both sides: a fragment's ds_read_b128 is free of bank conflicts;
 //   * step t: wait until K-tile t + 1 has landed (this wave's pieces), barrier (everybody's have, and everybody holds tile t in registers), ask for tile t + NBUF into the buffer
 //     tile t leaves, read the fragments of t + 1, multiply t: the LDS reads' latency runs under the MFMAs;
-//   * the weights are the MFMA's A operand: a lane's accumulator holds four consecutive columns of one row, and the epilogue works there, without a stage in LDS;
+//   * the weights are the MFMA's A operand: a lane's accumulator holds four consecutive columns of one row; what a column can do by itself happens there, and bf16 rows leave in whole
+//     16-byte chunks through a stage in the K-tile buffers (epilogue_staged; ragged edges and fp32 straight from the accumulators);
 //   * a row tile's fragments past M are neither read nor multiplied (M = 1025: the last row costs a sixteenth of a tile, not a tile);
 //   * a row's sum runs over K in ascending 32-steps of the same MFMA as in gemm256, whatever the tile: the same bits from every kernel and every shape here.
 #include <algorithm>
@@ -380,11 +381,12 @@ constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 }  // namespace
 
-// The time a launch takes, in us, and the tile shape (and number of row tiles) that takes least.  Every shape measured here (M 1 .. 4100, N 512 .. 28672, K 512 .. 16384) follows one law:
-// a CU brings in its workgroups' operand bytes at 61 GB/s and does the rest under that, so a K-tile (64) of a workgroup costs 0.05 us + 2.1 ns per row of A or W in it; a workgroup
-// more on a CU costs its time again; launch, first fill and drain 3.5 us, the epilogue 0.1 ns an element.  (32 x 64, K 14336: 52.3 us measured, 57 by the law; 64 x 64, K 4096: 21.7 and
-// 24.1; 96 x 64, K 14336: 79.5 and 90; 128 x 128, K 4096: 43.5 and 42.5; 128 x 256, K 4096: 55.1 and 56.8.  With the operand reads under the
-// multiplications the same shapes take 2 to 12 % less, evenly enough that the choice stands.)
+// A law to choose by, in us, and the tile shape (and number of row tiles) that takes least by it: a CU brings in its workgroups' operand bytes at 61 GB/s and does the rest under that, so
+// a K-tile (64) of a workgroup costs 0.05 us + 2.1 ns per row of A or W in it; a workgroup more on a CU costs its time again; launch, first fill and drain 3.5 us, the epilogue 0.1 ns
+// an element.  It is no prediction.  Measured / law on cold weights: one round of short tiles is up to a fifth faster (1025 x 3072 x 1024 12.4 / 13.8, 1025 x 1024 x 4096 21.1 / 26.6,
+// 77 x 4096 x 14336 44 / 53, 333 x 4096 x 14336 78 / 91), many rounds of large ones up to 8 % slower (8192 x 7168 x 2048 236 / 218, 6000 x 4096 x 14336 637 / 589), and no term stands for the
+// rate of HBM itself, which bounds wide weights at few rows (77 x 28672 x 4096 54 / 36).  At 22 products of M 77 .. 13325, N 1024 .. 28672, K 1024 .. 14336 the kernel that the two
+// laws (here and tile_us in gemm256.hip) choose was the fastest of gemm_mid, 256-row and 192-row tiles, or within 3 % of it.
 double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
     const int nf = (p.M + 15) / 16, slices = epi == EPI_PARTIAL && p.group > 0 ? p.group : 1, nk = p.K / 64 / slices, cus = cr_device_cus();
     double best = 1e30;

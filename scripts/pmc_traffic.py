@@ -1,6 +1,6 @@
 #!/usr/bin/env python3
 """Aggregate rocprofv3 --pmc passes (FETCH_SIZE in one run, WRITE_SIZE in another) of the bench into per-launch
-memory-side traffic of the dominant kernel class, as MI355X_MICROARCH.md "HBM" prescribes:
+memory-side traffic of the dominant kernels (`gemm_tiled_big`: every launch of gemm256_kernel), as MI355X_MICROARCH.md "HBM" prescribes:
   bytes = (2 * FETCH_SIZE + WRITE_SIZE) * 1024      (gfx950 reports half the bytes of wide coalesced reads; units KB)
 Note: these counters sit on the L2's fabric side, so Infinity-Cache hits are included.
 usage: pmc_traffic.py <fetch_dir> <write_dir> <out.json> ["bench arguments of the two runs"]"""

@@ -52,8 +52,8 @@ def test_gemm_exact_integers(E, M, N, K):
 @pytest.mark.parametrize('M,N,K', [(2049, 520, 128), (2304, 768, 256), (4100, 1024, 640), (2048, 512, 1024), (5000, 300 * 3, 384),
                                    (8300, 2304, 1024), (2100, 520, 4096), (16500, 1280, 256)])
 def test_gemm256_exact_integers(E, M, N, K):
-    """The 256x256 8-phase kernel, pinned (the dispatcher's cost model would hand several of these shapes to the
-    128x128 kernel): exact integer data checks the unit/sub-tile/swizzle maps, the K-tile pairing (K = 128 is a single
+    """The 256x256 8-phase kernel, pinned (the dispatcher's cost model would hand several of these shapes to
+    gemm_mid's tile shapes): exact integer data checks the unit/sub-tile/swizzle maps, the K-tile pairing (K = 128 is a single
     pair), ragged M/N edges, long K loops on data that misses L2, and workgroups that walk several tiles (> 256 tiles:
     the look-ahead across the tile boundary, fragments prefetched over the epilogue)."""
     g = torch.Generator().manual_seed(M + N + K)
@@ -157,7 +157,7 @@ def _bit_exact_epilogues(E, g, M, N, K, kern):
 
 
 def test_gelu_packed_pairs_equal_the_scalar_form(E):
-    """The 256x256 kernel evaluates GELU on pairs with packed fp32 instructions (common.hpp: gelu_erf2), the 128x128 kernel one
+    """The 256x256 kernel evaluates GELU on pairs (common.hpp: gelu_erf2), gemm_mid's tile shapes one
     element at a time (gelu_erf): the same bits on every bf16 input, in both positions of a pair and beside any neighbour."""
     bits = torch.arange(0, 65536, dtype=torch.int32)
     x = (bits << 16).view(torch.float32)
@@ -425,7 +425,7 @@ def test_gemm_row_argmax_partials(E, M, N, K, kern):
 @pytest.mark.parametrize('M,N,K', [(32800, 1024, 1024), (32800, 1024, 4096), (32800, 3072, 1024), (2100, 512, 256)])
 def test_gemm_tail_rows_take_the_small_kernel(E, M, N, K):
     """BASELINE config 2 (32 tiles) is 128 x 256 + 32 rows: the dispatcher cuts the 32 rows off the 256x256 launch (they would cost a
-    whole round of tiles) and sends them through the 128x128 kernel.  A row's result must not depend on which kernel made it:
+    whole round of tiles) and sends them through one of gemm_mid's tile shapes.  A row's result must not depend on which kernel made it:
     random data, every epilogue of the ViT layer, dispatcher's choice against the pinned un-split 256x256 launch, bit for bit."""
     g = torch.Generator().manual_seed(M + K)
     A = bf(_rand((M, K), g)).to(dev())
@@ -439,7 +439,7 @@ def test_gemm_tail_rows_take_the_small_kernel(E, M, N, K):
         small = E.op_gemm(epi, A[-300:], W, kernel=1, **{k: (v[-300:] if k == 'res' else v) for k, v in kw.items()})
         torch.cuda.synchronize()
         assert torch.equal(auto, pinned), epi
-        assert torch.equal(small, pinned[-300:]), epi          # and the 128x128 kernel agrees on rows well inside a 256-row tile too
+        assert torch.equal(small, pinned[-300:]), epi          # and the small kernel agrees on rows well inside a 256-row tile too
 
 
 def test_gemm_rejects_bad_k(E):
