@@ -593,7 +593,7 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
         const int first_m = grp * GM;
         const int gsz = min(ntm - first_m, GM);
         const int in_g = pid - grp * per_group;
-        m0 = (first_m + in_g % gsz) * (GRP ? 1 : TM);
+        m0 = (first_m + in_g % gsz) * TM;
         n0 = (in_g / gsz) * BN2;
     };
 

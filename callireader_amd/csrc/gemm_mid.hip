@@ -298,7 +298,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
         else if constexpr (NBUF > 2) wait_tail<NBUF - 3, G::PER>(behind);
         __builtin_amdgcn_s_waitcnt(0xC07F);                   // lgkmcnt(0)
         __builtin_amdgcn_sched_barrier(0);
-        if constexpr (G::WAVES > 1) __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_s_barrier();
         __builtin_amdgcn_sched_barrier(0);
     };
     auto loop = [&](auto count) {
@@ -332,10 +332,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
     else if (FM > 3 && live == FM - 3) loop(std::integral_constant<int, (FM > 3 ? FM - 3 : 0)>{});
     else loop(std::integral_constant<int, 0>{});
 
-    if constexpr (G::WAVES > 1) {
-        __builtin_amdgcn_s_waitcnt(0xC07F);
-        __builtin_amdgcn_s_barrier();                         // everybody has read the last K-tile: the buffers become the epilogue's stage
-    }
+    __builtin_amdgcn_s_waitcnt(0xC07F);
+    __builtin_amdgcn_s_barrier();                             // everybody has read the last K-tile: the buffers become the epilogue's stage
     char* stg = smem + wave * (2 * 16 * (FN * 32 + 16));
     const int row0 = m0 + wf0 * 16, col0 = n0 + wn * FN * 16;
     switch (epi) {                                            // (uniform)

@@ -1,7 +1,7 @@
 // Few-row products of described decoders in true fp32: C = epi(A[M,K] . W[N,K]^T), M <= 64 (per expert where grouped), every weight read once.
 //
 // Bound by the weights' bytes.  A workgroup owns 16 rows of W (one v_mfma_f32_16x16x4_f32 operand tile) and the K range of its slice; its eight waves divide that range, so a product
-// of 1024 rows keeps 64 x slices x 8 waves of loads in flight where the 64 x 64 tiles of lm_gemm.hip give 16 workgroups that walk all of K alone (two rows, products of 1024 x 1536 .. 4096: 46 us there,
+// of 1024 rows keeps 64 x slices x 8 waves of loads in flight where 64 x 64 tiles give 16 workgroups that walk all of K alone (two rows, products of 1024 x 1536 .. 4096: 46 us there,
 // 5.5 here; 3584 x 1024: 27 and 7.2; 4096 x 1024 with the squared relu: 27 and 7.1; token side's 64 x 1024: 28 and 4.6).
 // W comes by LDS-DMA, a KiB of 16 rows x 16 k an instruction, four neighbouring lanes a row's 64 bytes; loaded straight as operands, four neighbouring lanes hold four rows and a KiB takes
 // 64 clocks of the CU's load path instead of 16 (two rows: 1024 x 1536 .. 4096 6.9 us -> 5.5, 3584 x 1024 10.3 -> 7.2, 4096 x 1024 8.8 -> 7.1, 64 x 1024 6.0 -> 4.6).
