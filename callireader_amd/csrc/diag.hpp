@@ -1,6 +1,6 @@
 // Diagnostic builds, quarantined.
 //
-// The knock-out / knock-in / poison / stamp blocks inside the product kernels (gemm256.hip, gemm_skinny.hip, attention_vit.hip) are cost-structure
+// The knock-out / knock-in / poison / stamp blocks inside the product kernels (gemm256.hip, gemm_mid.hip, gemm_skinny.hip, lm_gemm_rows.hip, lm_gemm_tiles.hip, attention_vit.hip) are cost-structure
 // and hazard-screen tools: several of them give WRONG RESULTS by design.  Every translation unit that has such blocks includes this header, and this header is
 // the only door to them:
 //   * a diagnostic macro without -DCR_DIAG_BUILD is a compile error -- callireader_amd/build.py (the product build, __graft_entry__.build()) never defines
@@ -81,4 +81,19 @@ struct CrDiagRegistration {
 };
 static CrDiagRegistration cr_diag_registration_;
 }  // namespace
+#endif
+
+// ---- hazard screen (CR_POISON): the KiB of LDS that a wave is about to refill by LDS-DMA is overwritten with NaNs first (bf16 pairs and fp32 alike; `lane` in scope).  By a schedule's WAR
+//      rule nobody may still read it, by its RAW rule nobody reads it again before the new bytes have landed: a read that breaks either rule returns NaNs, and the exact tests fail
+//      instead of passing by luck (tests/test_gpu_hazards.py) ----
+#ifdef CR_POISON
+#define CR_DIAG_POISON(dst)                                                                                  \
+    {                                                                                                        \
+        typedef __attribute__((ext_vector_type(4))) unsigned u32x4_p;                                        \
+        const u32x4_p nan4 = {0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u, 0x7fc07fc0u};                           \
+        *(u32x4_p*)((dst) + lane * 16) = nan4;                                                               \
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");                                                   \
+    }
+#else
+#define CR_DIAG_POISON(dst)
 #endif

@@ -647,19 +647,21 @@ __global__ __launch_bounds__(512, 2) void gemm256_kernel(const GemmParams p) {
     auto dma = [&](const bf16* base, uint32_t o, int kt, int buf, int u) {
         if (F1 == 2 && u == 3) {
             char* dst = smem + buf * KBUF + 3 * UNIT + wave * 1024;
-            GM256_DIAG_POISON(dst)
+            CR_DIAG_POISON(dst)
             __builtin_amdgcn_global_load_lds(CR_GLB((const char*)base + (int64_t)kt * (BK2 * 2) + (wave & 1) * 64 + o), CR_LDS(dst), 16, 0, 0);
             return;
         }
         char* dst = smem + buf * KBUF + u * UNIT + (2 * wave) * 1024;
         if (GRP && (u == 1 || u == 2)) {                      // fragment blocks: consecutive k-steps of 32 are consecutive KiB
+            CR_DIAG_POISON(dst)
+            CR_DIAG_POISON(dst + 1024)
             const char* src = (const char*)base + (int64_t)kt * 2048;
             __builtin_amdgcn_global_load_lds(CR_GLB(src + o), CR_LDS(dst), 16, 0, 0);
             __builtin_amdgcn_global_load_lds(CR_GLB(src + o), CR_LDS(dst), 16, 1024, 0);
             return;
         }
-        GM256_DIAG_POISON(dst)
-        GM256_DIAG_POISON(dst + 1024)
+        CR_DIAG_POISON(dst)
+        CR_DIAG_POISON(dst + 1024)
         const char* src = (const char*)base + (int64_t)kt * (BK2 * 2);
         GM256_DIAG_ALT_DMA(base, src, o, dst, kt)
         __builtin_amdgcn_global_load_lds(CR_GLB(src + o), CR_LDS(dst), 16, 0, 0);

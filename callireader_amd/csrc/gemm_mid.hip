@@ -15,6 +15,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "diag.hpp"
 
 namespace {
 
@@ -256,8 +257,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
     }
     auto ask = [&](int kt, int buf) {
 #pragma unroll
-        for (int i = 0; i < G::PER; i++)
+        for (int i = 0; i < G::PER; i++) {
+            CR_DIAG_POISON(smem + buf * G::STAGE + dst[i])
             if (!dead[i] || lane == 0) __builtin_amdgcn_global_load_lds(CR_GLB(src[i] + (int64_t)kt * 64), CR_LDS(smem + buf * G::STAGE + dst[i]), 16, 0, 0);
+        }
     };
 
     f32x4 acc[FM][FN];

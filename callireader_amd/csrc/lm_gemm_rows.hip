@@ -8,6 +8,7 @@
 // A lane multiplies with k = 4 (lane >> 4) .. + 3 of a 16-deep step of its weight row and of its activation row: the four multiplications of a step take one element
 // of each, which permutes k inside the step for both operands alike.  Partial tiles of the waves meet in LDS and are added in wave order; slices go to the consumer, which adds them
 // in slice order: the order of lm.hpp, a wave a chain.
+#include "diag.hpp"
 #include "lm.hpp"
 
 namespace {
@@ -54,6 +55,7 @@ __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) 
 #pragma unroll
         for (int u = 0; u < U; u++) {
             const int k = min(s + u, s1 - 1) * 16;
+            CR_DIAG_POISON(ring + u * 1024)
             __builtin_amdgcn_global_load_lds(CR_GLB(w + k), CR_LDS(ring + u * 1024), 16, 0, 0);
 #pragma unroll
             for (int j = 0; j < MT; j++) af[u][j] = *(const f32x4*)(a[j] + k);

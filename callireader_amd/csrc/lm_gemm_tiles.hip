@@ -11,6 +11,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "diag.hpp"
 #include "lm.hpp"
 
 namespace {
@@ -116,8 +117,10 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
     const int nk = p.K / (32 * KB);
     auto ask = [&](int kt, int buf) {
 #pragma unroll
-        for (int i = 0; i < G::PER; i++)
+        for (int i = 0; i < G::PER; i++) {
+            CR_DIAG_POISON(smem + buf * G::STAGE + dst[i])
             if (!dead[i] || lane == 0) __builtin_amdgcn_global_load_lds(CR_GLB(src[i] + (int64_t)kt * (32 * KB)), CR_LDS(smem + buf * G::STAGE + dst[i]), 16, 0, 0);
+        }
     };
     f32x4 acc[FM][FN], part[FM][FN], total[FM][FN];           // of the chain, of the part, of the whole sum
 #pragma unroll

@@ -22,14 +22,16 @@ if 'api.hip' not in srcs:
     srcs_id = srcs + ['api.hip']
 else:
     srcs_id = srcs
-new_objs = []
+new_objs, jobs = [], []
 for one in srcs_id:
     obj = os.path.join(ROOT, 'ab', f'{name}_{one[:-4]}.o')
     own = flags if one in srcs else []
     cmd = ['hipcc', '--offload-arch=gfx950', '-O3', '-std=c++17', '-fPIC', '-Wno-unused-value', *B.DEVICE_FLAGS, '-DCR_DIAG_BUILD=1', f'-DCR_BUILD_ID="CR_BUILD_ID={vid}"'] \
         + B.EXTRA_FLAGS.get(one, []) + own + ['-c', os.path.join(B.CSRC, one), '-o', obj]
-    subprocess.check_call(cmd)
+    jobs.append(subprocess.Popen(cmd))
     new_objs.append(obj)
+if any([j.wait() for j in jobs]):
+    sys.exit('a compile failed')
 srcs = srcs_id
 objs = [os.path.join(B.CSRC, 'build', os.path.basename(s)[:-4] + '.o') for s in B.sources() if os.path.basename(s) not in srcs] + new_objs
 out = os.path.join(ROOT, 'ab', f'lib{name}.so')
