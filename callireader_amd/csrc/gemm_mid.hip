@@ -5,8 +5,7 @@
 // 16 x 32 for two waves, and (b) NBUF K-tiles live in LDS and NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles.
 //   * one global_load_lds_dwordx4 brings eight rows x 64 k, whole 128-byte lines (pieces of 16 rows x 32 k reach 56 of the 69 GB/s per CU that these do on cold weights);
 //     LDS rows of 128 bytes, the 16-byte chunk XORed with (row >> 1) & 7 on both sides: a fragment's ds_read_b128 is free of bank conflicts;
-//   * step t: wait until K-tile t + 1 has landed (this wave's pieces), barrier (everybody's have, and everybody holds tile t in registers), ask for tile t + NBUF into the buffer
-//     tile t leaves, read the fragments of t + 1, multiply t: the LDS reads' latency runs under the MFMAs;
+//   * the steps and their waits are k_ring.hpp's;
 //   * the weights are the MFMA's A operand: a lane's accumulator holds four consecutive columns of one row; what a column can do by itself happens there, and bf16 rows leave in whole
 //     16-byte chunks through a stage in the K-tile buffers (epilogue_staged; ragged edges and fp32 straight from the accumulators);
 //   * a row tile's fragments past M are neither read nor multiplied (M = 1025: the last row costs a sixteenth of a tile, not a tile);
@@ -16,15 +15,9 @@
 
 #include "common.hpp"
 #include "diag.hpp"
+#include "k_ring.hpp"
 
 namespace {
-
-template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-// ... with `behind` <= R K-tiles of PER instructions left under way
-template <int R, int PER> __device__ __forceinline__ void wait_tail(int behind) {
-    if (behind >= R) wait_vm<R * PER>();
-    else if constexpr (R > 0) wait_tail<R - 1, PER>(behind);
-}
 
 // ---- epilogue of four consecutive columns gn .. gn + 3 (gn % 4 == 0) of row gm: the reference's bf16 rounding sequence ----
 template <int EPI>
@@ -294,16 +287,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
                     for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[h][j], f.a[h][i], acc[i][j], 0, 0, 0);
                 }
     };
-    // K-tile t has landed in every wave's pieces, and every wave holds tile t - 1 in registers
-    auto arrive = [&](int t) {
-        const int behind = nk - 1 - t;                        // tiles after t: at most NBUF - 2 of them are under way
-        if (behind >= NBUF - 2) wait_vm<(NBUF - 2) * G::PER>();
-        else if constexpr (NBUF > 2) wait_tail<NBUF - 3, G::PER>(behind);
-        __builtin_amdgcn_s_waitcnt(0xC07F);                   // lgkmcnt(0)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-    };
+    auto arrive = [&](int t) { ring_arrive<NBUF, G::PER>(nk, t); };
     auto loop = [&](auto count) {
         for (int t = 0; t < min(NBUF - 1, nk); t++) ask(t, t);
         Frags f0, f1;

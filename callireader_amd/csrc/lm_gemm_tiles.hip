@@ -12,15 +12,10 @@
 #include <type_traits>
 
 #include "diag.hpp"
+#include "k_ring.hpp"
 #include "lm.hpp"
 
 namespace {
-
-template <int N> __device__ __forceinline__ void wait_vm() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
-template <int R, int PER> __device__ __forceinline__ void wait_tail(int behind) {
-    if (behind >= R) wait_vm<R * PER>();
-    else if constexpr (R > 0) wait_tail<R - 1, PER>(behind);
-}
 
 // four consecutive columns gn .. gn + 3 of row cr (`whole`: all inside N, 16-byte places)
 template <int EPI>
@@ -174,15 +169,7 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
             }
         }
     };
-    auto arrive = [&](int t) {                                // K-tile t has landed in every wave's pieces, and every wave holds tile t - 1 in registers
-        const int behind = nk - 1 - t;
-        if (behind >= NBUF - 2) wait_vm<(NBUF - 2) * G::PER>();
-        else if constexpr (NBUF > 2) wait_tail<NBUF - 3, G::PER>(behind);
-        __builtin_amdgcn_s_waitcnt(0xC07F);                   // lgkmcnt(0)
-        __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_barrier();
-        __builtin_amdgcn_sched_barrier(0);
-    };
+    auto arrive = [&](int t) { ring_arrive<NBUF, G::PER>(nk, t); };
     auto loop = [&](auto count) {
         for (int t = 0; t < min(NBUF - 1, nk); t++) ask(t, t);
         Frags f0, f1;
