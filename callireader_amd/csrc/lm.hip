@@ -346,7 +346,8 @@ size_t carve_bytes(const Lm& lm, const Step& sp) {
     return ar.off + 512;
 }
 
-// C[M, N] = A . W^T in the model's element type: the engine's dense kernels for bf16, the fp32 tile kernel otherwise
+// C[M, N] = A . W^T in the model's element type: the engine's dense kernels for bf16, the fp32 kernels otherwise.  parts: a product that few decode rows leave in K-slices to its consumer;
+// in fp32 its sum has that order here too
 int dense(cr_ctx* c, const Lm& lm, const void* A, int64_t lda, const void* W, void* C, int64_t ldc, int M, int N, int K, hipStream_t st, bool prompt, const bf16* dl = nullptr,
           bool relu2 = false, bool parts = false) {
     if (lm.f32) {
