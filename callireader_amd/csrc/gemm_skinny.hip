@@ -8,7 +8,7 @@
 //   * RT = 16-row weight tiles per wave (4 where N >= 16384 and M > 16): the X fragments are loaded once per RT
 //     tiles; X comes from L2 but through the same per-CU load path as W, and at M = 32 it is 2 x the W bytes at RT = 1;
 //   * per k-step a lane loads 16 B of W (row n = lane&15, k = 8*(lane>>4) .. +7) and 16 B of each X tile,
-//     UNROLL k-steps of loads are issued before the first MFMA; with p.wsw the weights come from their DECODE-LAYOUT copy (gemm_decode.hip:
+//     a batch of k-steps is loaded before its first MFMA, and up to 32 rows the next batch too; with p.wsw the weights come from their DECODE-LAYOUT copy (gemm_decode.hip:
 //     decode_swizzle_kernel -- the 64 lanes' fragments of a tile and k-step side by side), so a load instruction is one contiguous KiB instead of
 //     16 rows x 64 bytes: wqkv / wo / w2 at 64 rows 19.6 / 14.6 / 37.7 -> 17.2 / 13.6 / 29.7 us, the same bits;
 //   * accumulator = C^T tile [16 n][16 m] per X tile, so the lane holds 4 consecutive n of one m;
@@ -41,12 +41,14 @@ __device__ __forceinline__ bf16x8 fp8x8_to_bf16(unsigned lo, unsigned hi) {
     return bf16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
 }
 
+// shapes whose grids put more than one workgroup on a CU: few row tiles each
+constexpr bool skinny_two(int RT, int MT) { return RT == 1 || (RT == 2 && MT <= 2); }
+
 template <int EPI, int WAVES, int MT, int RT = 1, bool W8 = false>
-__global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const GemmParams p) {
+__global__ __launch_bounds__(WAVES * 64, !W8 && skinny_two(RT, MT) ? 4 : 1) void gemm_skinny_kernel(const GemmParams p) {
     // RT = 16-row weight tiles per wave: X fragments are loaded once per RT tiles (X re-reads through L2 are the
     // bottleneck once M > 16), used where N is large enough to still fill the chip
     __shared__ float red[WAVES][RT * MT][16][17];
-    constexpr int UNROLL = 8;
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int n0 = blockIdx.x * 16 * RT;
@@ -72,7 +74,8 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const GemmParam
     constexpr int XSTEP = 32;
 #endif
 
-    constexpr int UR = UNROLL / RT;
+    // k-steps a batch: two batches of RT + MT fragments of 4 registers each, 96 registers where two workgroups are to share a CU and 160 beyond; one batch of 80 registers past 32 rows
+    constexpr int UR = MT > 2 ? (RT == 1 ? 20 / (1 + MT) : 8 / RT) : skinny_two(RT, MT) ? 12 / (RT + MT) : RT + MT <= 5 ? 4 : 3;
     f32x4 acc[RT][MT];
 #pragma unroll
     for (int r = 0; r < RT; r++)
@@ -97,7 +100,7 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const GemmParam
         const bf16* x8p[MT];
 #pragma unroll
         for (int t = 0; t < MT; t++) x8p[t] = p.A + (int64_t)min(t * 16 + (lane & 15), p.M - 1) * p.lda + kbase + kq16;
-        constexpr int U8 = UR > 1 ? UR / 2 : 1;               // 64-deep steps in flight per batch
+        constexpr int U8 = RT < 4 ? 4 / RT : 1;               // 64-deep steps in flight per batch
         int s8 = 0;
         for (; s8 + U8 <= steps; s8 += U8) {
             u32x4_t w[RT][U8];
@@ -138,34 +141,46 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const GemmParam
             }
         }
     }
-    int ks = W8 ? ksteps : 0;
-    for (; ks + UR <= ksteps; ks += UR) {
-        bf16x8 w[RT][UR], x[MT][UR];
+    if (!W8) {
+        // Batches of UR k-steps, the last one partial.  Described decoders give a wave 1..8 k-steps (K = 1024 .. 4096 over eight waves and the slices): fewer than a batch, they used to be
+        // loaded one by one, a round trip to memory each (one row, us before -> after: 4096 x 1024 5.4 -> 4.5, 3584 x 1024 5.5 -> 4.2, 1024 x 4096 4.9 -> 3.9, 1024 x 1536 4.2 -> 3.5;
+        // 24 rows: 3328 x 2048 6.7 -> 6.0, 2048 x 2048 6.4 -> 5.4).  Up to 32 rows the next batch's loads are issued ahead of this one's MFMAs; beyond that the volume of X through the
+        // CU's load path is what counts and a second batch changes nothing (64 rows, 6144 x 4096: 17.9 without, 18.5 with).
+        struct Batch { bf16x8 w[RT][UR], x[MT][UR]; };
+        auto load = [&](Batch& f, int ks) {
 #pragma unroll
-        for (int r = 0; r < RT; r++)
+            for (int u = 0; u < UR; u++) {
+                if (ks + u >= ksteps) break;                      // (uniform)
 #pragma unroll
-            for (int u = 0; u < UR; u++) w[r][u] = __builtin_nontemporal_load((const bf16x8*)(wp[r] + (ks + u) * wstep));
+                for (int r = 0; r < RT; r++) f.w[r][u] = __builtin_nontemporal_load((const bf16x8*)(wp[r] + (ks + u) * wstep));
 #pragma unroll
-        for (int t = 0; t < MT; t++)
+                for (int t = 0; t < MT; t++) f.x[t][u] = *(const bf16x8*)(xp[t] + (ks + u) * XSTEP);
+            }
+        };
+        auto mul = [&](const Batch& f, int ks) {
 #pragma unroll
-            for (int u = 0; u < UR; u++) x[t][u] = *(const bf16x8*)(xp[t] + (ks + u) * XSTEP);
+            for (int u = 0; u < UR; u++) {
+                if (ks + u >= ksteps) break;
 #pragma unroll
-        for (int u = 0; u < UR; u++)
+                for (int r = 0; r < RT; r++)
 #pragma unroll
-            for (int r = 0; r < RT; r++)
-#pragma unroll
-                for (int t = 0; t < MT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r][u], x[t][u], acc[r][t], 0, 0, 0);
-    }
-    for (; ks < ksteps; ks++) {
-        bf16x8 x[MT];
-#pragma unroll
-        for (int t = 0; t < MT; t++) x[t] = *(const bf16x8*)(xp[t] + ks * 32);
-#pragma unroll
-        for (int r = 0; r < RT; r++) {
-            const bf16x8 w = __builtin_nontemporal_load((const bf16x8*)(wp[r] + ks * wstep));
-#pragma unroll
-            for (int t = 0; t < MT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, x[t], acc[r][t], 0, 0, 0);
-        }
+                    for (int t = 0; t < MT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[r][u], f.x[t][u], acc[r][t], 0, 0, 0);
+            }
+        };
+        Batch f0, f1;
+        if (MT <= 2) {
+            load(f0, 0);
+            for (int ks = 0; ks < ksteps; ks += 2 * UR) {
+                load(f1, ks + UR);
+                mul(f0, ks);
+                load(f0, ks + 2 * UR);
+                mul(f1, ks + UR);
+            }
+        } else
+            for (int ks = 0; ks < ksteps; ks += UR) {
+                load(f0, ks);
+                mul(f0, ks);
+            }
     }
     // C^T tile: row (n) = (lane>>4)*4 + e, col (m) = lane&15; staged tile index = r * MT + t
 #pragma unroll
@@ -176,44 +191,35 @@ __global__ __launch_bounds__(WAVES * 64) void gemm_skinny_kernel(const GemmParam
             for (int e = 0; e < 4; e++) red[wave][r * MT + t][(lane >> 4) * 4 + e][lane & 15] = acc[r][t][e];
     __syncthreads();
 
-    // thread -> (m tile, n, m); sum the waves' partials in wave order
-    for (int idx = tid; idx < RT * MT * 256; idx += WAVES * 64) {
-        const int t = idx >> 8, n = idx & 15, m = (idx >> 4) & 15;
+    // thread -> (tile, n, m); the waves' partials are added in wave order
+    auto total = [&](int t, int n, int m) -> float {
         float s = 0.f;
 #pragma unroll
         for (int w = 0; w < WAVES; w++) s += red[w][t][n][m];
         if (W8) s *= p.wscale[min(n0 + (t / MT) * 16 + n, p.N - 1)];      // fp8 weights: the row's scale, once, on the fp32 sum
-        red[0][t][n][m] = s;       // own element only: no hazard with other threads' reads
-    }
-    __syncthreads();
-    if (EPI == EPI_PARTIAL) {
-        float* out = (float*)p.C + (int64_t)blockIdx.y * p.M * p.ldc;
-        for (int idx = tid; idx < RT * MT * 256; idx += WAVES * 64) {
-            const int t = idx >> 8, n = idx & 15, m = (idx >> 4) & 15;
-            const int gm = (t % MT) * 16 + m, gn = p.wsw == 2 ? rope_tile_row(n0 / 16 + t / MT, n) : n0 + (t / MT) * 16 + n;
-            if (gm < p.M && gn < p.N) out[(int64_t)gm * p.ldc + gn] = red[0][t][n][m];
-        }
-        return;
-    }
+        return s;
+    };
     if (EPI == EPI_SWIGLU) {
         for (int idx = tid; idx < RT * MT * 128; idx += WAVES * 64) {
-            const int q = idx >> 7, j = idx & 7, m = (idx >> 3) & 15;
-            const int t = q;
-            const int gm = (q % MT) * 16 + m, gno = (n0 + (q / MT) * 16) / 2 + j;
+            const int t = idx >> 7, j = idx & 7, m = (idx >> 3) & 15;
+            const int gm = (t % MT) * 16 + m, gno = (n0 + (t / MT) * 16) / 2 + j;
             if (gm < p.M && gno < p.N / 2) {
-                const float g = rbf(red[0][t][j][m]), u = rbf(red[0][t][8 + j][m]);
+                const float g = rbf(total(t, j, m)), u = rbf(total(t, 8 + j, m));
                 ((bf16*)p.C)[(int64_t)gm * p.ldc + gno] = f2bf(rbf(silu(g)) * u);
             }
         }
         return;
     }
+    float* part = (float*)p.C + (int64_t)blockIdx.y * p.M * p.ldc;       // EPI_PARTIAL: this K-slice
     for (int idx = tid; idx < RT * MT * 256; idx += WAVES * 64) {
         const int t = idx >> 8, n = idx & 15, m = (idx >> 4) & 15;
-        const int gm = (t % MT) * 16 + m, gn = n0 + (t / MT) * 16 + n;
+        const int gm = (t % MT) * 16 + m, gn = EPI == EPI_PARTIAL && p.wsw == 2 ? rope_tile_row(n0 / 16 + t / MT, n) : n0 + (t / MT) * 16 + n;
         if (gm >= p.M || gn >= p.N) continue;
-        const float sum = red[0][t][n][m] + (p.bias ? bf2f(p.bias[gn]) : 0.f);
-        if (EPI == EPI_F32) { ((float*)p.C)[(int64_t)gm * p.ldc + gn] = f32_out(p, sum); continue; }
-        float x = EPI == EPI_RELU2 ? relu2(sum) : rbf(sum);
+        const float sum = total(t, n, m);
+        if (EPI == EPI_PARTIAL) { part[(int64_t)gm * p.ldc + gn] = sum; continue; }
+        const float biased = sum + (p.bias ? bf2f(p.bias[gn]) : 0.f);
+        if (EPI == EPI_F32) { ((float*)p.C)[(int64_t)gm * p.ldc + gn] = f32_out(p, biased); continue; }
+        float x = EPI == EPI_RELU2 ? relu2(biased) : rbf(biased);
         if (EPI == EPI_RES) x = bf2f(p.res[(int64_t)gm * p.ldr + gn]) + x;
         ((bf16*)p.C)[(int64_t)gm * p.ldc + gn] = f2bf(x);
     }
