@@ -49,7 +49,6 @@ __device__ __forceinline__ float rbf1(float x) {
 #endif
 
 template <int D> __device__ __forceinline__ int kswz(int r) { return D == 64 ? ((r >> 1) & 7) : (r & 15); }
-template <int D> __device__ __forceinline__ int vswz(int r) { return D == 64 ? (((r >> 1) & 1) << 2) : ((r & 3) << 2); }
 
 // Measured nulls at the ViT shape (0.55 ms either way; PMC: waves issue 27 % of their cycles, sit in issue stalls 40 %,
 // parked 33 %): three K/V stages with a counted wait instead of two drained ones (-5 %: one workgroup fewer per CU),
@@ -149,7 +148,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void flash_attn_kernel(const
         const int r = (wave * IPW + ii) * RPI + lane / CPR;
         const int cp = lane % CPR;
         kbase[ii] = Kb + (int64_t)r * p.k_rs + ((cp ^ kswz<D>(r)) * 8);
-        vbase[ii] = Vb + (int64_t)r * p.v_rs + ((cp ^ vswz<D>(r)) * 8);
+        vbase[ii] = Vb + (int64_t)r * p.v_rs + ((cp ^ attn_vswz<D>(r)) * 8);
     }
     auto stage = [&](int buf, int kt) {
         const bool full = kt * 64 + 64 <= Sk;
@@ -165,7 +164,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void flash_attn_kernel(const
                 const int cp = lane % CPR;
                 const int key = min(kt * 64 + r, Sk - 1);
                 ks = Kb + (int64_t)key * p.k_rs + ((cp ^ kswz<D>(r)) * 8);
-                vs = Vb + (int64_t)key * p.v_rs + ((cp ^ vswz<D>(r)) * 8);
+                vs = Vb + (int64_t)key * p.v_rs + ((cp ^ attn_vswz<D>(r)) * 8);
             }
             char* dst = smem + buf * (2 * TILE) + (wave * IPW + ii) * 1024;
             __builtin_amdgcn_global_load_lds(CR_GLB(ks), CR_LDS(dst), 16, 0, 0);
@@ -201,7 +200,7 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void flash_attn_kernel(const
     const int k_sw = kswz<D>(l31);
     const int g = lane >> 4, li = lane & 15, tq = li >> 2, tp = li & 3;
     const int v_lane_row = 4 * hh + tq;
-    const int v_sw = vswz<D>(v_lane_row);
+    const int v_sw = attn_vswz<D>(v_lane_row);
     const int v_clow = (g & 1) * 2 + (tp >> 1);
     const int v_lane_off = v_lane_row * ROWB + (tp & 1) * 8;
 

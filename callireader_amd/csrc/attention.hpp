@@ -1,6 +1,9 @@
 #pragma once
 #include "common.hpp"
 
+// value tiles in LDS, [key][D]: the 16-byte chunk c of row r sits at c ^ attn_vswz(r) (the transposing reads of P . V then meet no bank twice)
+template <int D> __device__ __forceinline__ int attn_vswz(int r) { return D == 64 ? (((r >> 1) & 1) << 2) : ((r & 3) << 2); }
+
 // Strides are in elements.  Q/K/V/O are addressed as base + b*bs + row*rs + head*hs + d.
 struct AttnParams {
     const bf16* Q; const bf16* K; const bf16* V; bf16* O;

@@ -139,6 +139,17 @@ int derive_heads(Deriver& dv, const std::string& p, const std::string& o, LmLaye
         for (int i = 0; i < dims / 2; i++) f[i] = (float)pow(base, -2.0 * i / dims);
         return dv.table(n, f);
     };
+    // its place among a decoded row's angles: the same rotation of another layer, or a new one
+    auto place_rot = [&](double base, int dims) {
+        const int half = dims / 2, pad = (half + 7) / 8 * 8;
+        std::vector<float> f(2 * pad, 0.f);
+        for (int i = 0; i < half; i++) f[pad + i] = -(f[i] = (float)pow(base, -2.0 * i / dims));
+        std::vector<float>& all = dv.lm.rot;
+        for (size_t at = 0; at + f.size() <= all.size(); at += 16)
+            if (std::equal(f.begin(), f.end(), all.begin() + at)) return (int)at;
+        all.insert(all.end(), f.begin(), f.end());
+        return (int)(all.size() - f.size());
+    };
     auto rows = [&](int kind, const std::string& name, int size) -> int {
         const LmRegion* g = L.region(kind);
         const DevTensor* t = dv.src(name, (int64_t)g->heads * size, W);
@@ -156,6 +167,7 @@ int derive_heads(Deriver& dv, const std::string& p, const std::string& o, LmLaye
         CR_TRY(dv.place(wo, 0, W, L.wo, 0, L.Gp));
         if (a.qk_norm && (!(L.nq = dv.gain(o + "nq", q + "q.norm", a.dim, L.Ap, 0.f)) || !(L.nc = dv.gain(o + "nk", q + "k.norm", a.dim, L.Ap, 0.f)))) return CR_ERR_STATE;
         if (a.rot_dims && !(L.fq_a = rotations(o + "fa", a.rot_base, a.rot_dims))) return CR_ERR_NOMEM;
+        if (a.rot_dims) L.rot_a = place_rot(a.rot_base, a.rot_dims);
     }
     if (L.retention()) {
         const std::string q = p + "mix." + std::string(r.name, strnlen(r.name, sizeof r.name));
@@ -167,6 +179,7 @@ int derive_heads(Deriver& dv, const std::string& p, const std::string& o, LmLaye
         if (!wo) return CR_ERR_STATE;
         CR_TRY(dv.place(wo, 0, W, L.wo, L.off_r, L.Gp));
         if (r.rot_dims && !(L.fq_r = rotations(o + "fr", r.rot_base, r.rot_dims))) return CR_ERR_NOMEM;
+        if (r.rot_dims) L.rot_r = place_rot(r.rot_base, r.rot_dims);
         std::vector<float> pw((size_t)r.heads * (RET_CHUNK + 1));
         for (int h = 0; h < r.heads; h++)
             for (int i = 0; i <= RET_CHUNK; i++) pw[(size_t)h * (RET_CHUNK + 1) + i] = i ? (float)pow(L.decay[h], (double)i) : 1.f;
@@ -253,6 +266,7 @@ struct Step {
 struct Buffers {
     float* x; void *h, *a, *cq, *q, *c, *kv, *qp, *ol, *ao, *y, *act, *ye, *cat, *z2; float *z, *wt, *part, *sl, *rq, *rk, *raw; bf16 *rq2, *rk2, *snap;
     int32_t *idx, *perm, *n_tiles, *tok; int4* tiles;
+    int2* where; float* ang;
 };
 bool expanded(const Lm& lm, const LmLayer& L, bool decode) { return !lm.f32 && !decode && L.s.scale > 0.f && (L.Ap == 64 || L.Ap == 128 || L.Ap == 256); }
 bool split_decode(const Lm& lm, const LmLayer& L, bool decode) { return !lm.f32 && decode && latent_decode_supported(L.Rp); }
@@ -337,6 +351,7 @@ Buffers carve(const Lm& lm, Arena& ar, const Step& sp) {
     b.z = ar.take<float>((size_t)M * Ep * (M <= 128 ? LM_ROUTER_SLICES : 1)); b.wt = ar.take<float>((size_t)M * top);
     b.idx = ar.take<int32_t>((size_t)M * top); b.perm = ar.take<int32_t>((size_t)M * top); b.n_tiles = ar.take<int32_t>(1); b.tiles = ar.take<int4>(tiles);
     b.rq = ar.take<float>(r32); b.rk = ar.take<float>(r32); b.rq2 = ar.take<bf16>(r16); b.rk2 = ar.take<bf16>(r16); b.raw = ar.take<float>(raw); b.snap = ar.take<bf16>(snap);
+    b.where = ar.take<int2>(decode ? M : 0); b.ang = ar.take<float>(decode ? M * std::max<size_t>(lm.rot.size(), 1) : 0);
     b.tok = ar.take<int32_t>(M); b.z2 = T((size_t)M * lm.Sp); b.cat = T(lm.d.loop_in ? (size_t)M * 2 * Wp : 0);
     return b;
 }
@@ -440,6 +455,18 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
     const KeyPlan* kp = L.heads() && !sp.decode ? &sp.plans[L.chunk_ix] : nullptr;
     const int ring = L.heads() ? std::min(lm.chunks[L.chunk_ix], kv->max_tokens) : 1, chunk = L.heads() ? lm.chunks[L.chunk_ix] : 1;
     char *ck = kv->lat + kv->lat_off[r], *cv = ck + (size_t)kv->n_seqs * a.kv_heads * ring * L.Ap * es;
+    float* state = (float*)(kv->lat + kv->state_off[r]);
+    // by the layer's sizes alone (and 64 rows, where slices end): a row's bits do not depend on the rows it is decoded with
+    if (s_a && lm_mix_supported(lm.f32, L)) {
+        LmMixIn in{};
+        in.M = M; in.part = b.sl; in.slices = s_a; in.where = b.where; in.ang = b.ang; in.ao = b.ao; in.cache_k = ck; in.cache_v = cv; in.ring = ring; in.chunk = chunk; in.rows = in.nsplit = 1;
+        in.state = state;
+        if (L.heads() && !lm.f32) {
+            in.rows = heads_per_split(a); in.nsplit = sp.hsplit[L.chunk_ix];
+            in.part_o = b.part; in.part_ml = b.part + (size_t)M * a.heads * in.nsplit * L.Ap;
+        }
+        return launch_lm_mix(lm.f32, lm, L, in, st);
+    }
     if (kp) CR_TRY(launch_lm_prefix(lm.f32, L, kp->n_pre, kp->pre_key, kp->pre_slot, b.kv, ck, cv, ring, st));
     const bool matrix = L.retention() && matrix_retention(lm, L, sp.decode);
     LmHeadsIn in{};
@@ -482,7 +509,7 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
     if (!L.retention()) return CR_OK;
     RetParams rp{};
     rp.rq = b.rq; rp.rk = b.rk; rp.rq2 = b.rq2; rp.rk2 = b.rk2; rp.lda = L.Na; rp.v = (char*)b.a + (size_t)L.region(LM_RV)->off * es; rp.g = (char*)b.a + (size_t)L.region(LM_RG)->off * es;
-    rp.ao = (char*)b.ao + (size_t)L.off_r * es; rp.ldo = L.Gp; rp.state = (float*)(kv->lat + kv->state_off[r]); rp.raw = b.raw; rp.snap = b.snap; rp.pw = L.pw;
+    rp.ao = (char*)b.ao + (size_t)L.off_r * es; rp.ldo = L.Gp; rp.state = state; rp.raw = b.raw; rp.snap = b.snap; rp.pw = L.pw;
     rp.M = M; rp.H = rt.heads; rp.Kp = L.Kp; rp.Vp = L.Vp; rp.vdim = rt.vdim; rp.eps = lm.d.eps; rp.out_scale = rt.out_scale; rp.ix = sp.ix;
     rp.seg = sp.d_rseg; rp.snap0 = sp.d_snap0; rp.n_segs = (int)sp.segs.size(); rp.longest = sp.longest; rp.chunks = sp.d_chunks; rp.n_chunks = sp.snaps;
     return sp.decode ? launch_ret_decode(lm.f32, rp, merge ? &ap : nullptr, L.Ap, st) : matrix ? launch_ret_matrix(rp, st) : launch_ret_recurrent(lm.f32, rp, st);
@@ -549,7 +576,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
         out = LmPostIn{n ? (const void*)b.sl : b.y, Wp, n, nullptr, 0};
         return n ? sliced(c, A, K, W, dl, b.sl, M, Wp, K, st) : dense(c, lm, A, K, W, b.y, Wp, M, Wp, K, st, !sp.decode, dl, false, true);
     };
-    CR_TRY(launch_lm_embed(lm.f32, lm, M, sp.tokens, sp.ix, kv->d_gen, kv->d_ngen, kv->gen_cap, b.x, entry(0), b.tok, lm.d.loop_in ? (char*)b.cat + (size_t)Wp * es : nullptr, 2 * Wp, st));
+    CR_TRY(launch_lm_embed(lm.f32, lm, M, sp.tokens, sp.ix, kv->d_gen, kv->d_ngen, kv->gen_cap, b.x, entry(0), b.tok, lm.d.loop_in ? (char*)b.cat + (size_t)Wp * es : nullptr, 2 * Wp, LmEmbedOut{sp.decode ? b.where : nullptr, b.ang}, st));
     CR_TRY(probe(0));
     for (size_t r = 0; r < lm.passes.size(); r++) {
         const LmLayer& L = lm.layers[lm.passes[r]];
@@ -655,7 +682,9 @@ int lm_finalize(cr_ctx* c, hipStream_t st) {
         CR_HIP(hipMemcpyAsync(lm->freq, f.data(), (size_t)n * 4, hipMemcpyHostToDevice, st));
         CR_HIP(hipStreamSynchronize(st));
     }
+    lm->rot.clear();
     for (size_t i = 0; i < lm->layers.size(); i++) CR_TRY(derive_layer(dv, (int)i, lm->layers[i]));
+    if (!lm->rot.empty() && !(lm->rot_freq = dv.table("derived.lm.rot", lm->rot))) return CR_ERR_NOMEM;
     CR_HIP(hipStreamSynchronize(st));
     for (const std::string& n : dv.used) {
         auto it = c->w.find(n);

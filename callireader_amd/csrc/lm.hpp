@@ -41,6 +41,7 @@ struct LmLayer {
     // fp32: gains (one plus the stored weight for the norms about zero), router correction
     float *n1, *n1b, *n2, *n2b, *nq, *nc, *corr, *ns;
     float *fq_a, *fq_r;        // rotation frequencies of attention and of retention
+    int rot_a, rot_r;          // and where their cos start in a row's angles (Lm::rot)
     float *pw;                 // retention: decay^0 .. decay^RET_CHUNK of every head
 
     const LmRegion* region(int kind) const {
@@ -63,6 +64,9 @@ struct Lm {
     void *embed = nullptr, *head = nullptr, *side = nullptr, *loop_in = nullptr;
     bf16 *head_dl = nullptr, *loop_dl = nullptr;
     float *fin = nullptr, *freq = nullptr;
+    // the angles a decoded row needs, once for all layers: per distinct rotation cos of its pairs, then sin, each padded to eight; frequencies, negative where the sine is meant
+    std::vector<float> rot;
+    float* rot_freq = nullptr;
     float gain_base() const { return d.norm_plain ? 0.f : 1.f; }
     size_t esz() const { return f32 ? 4 : 2; }
 };
@@ -110,10 +114,12 @@ struct LmRowIndex {            // where a row's token sits: prefill gives arrays
 };
 // where a row of the residual goes for its next reader, in the element type: rms(x) * gain, or with a null gain x itself
 struct LmSink { void* h; int64_t ldh; const float* gain; };
+// (decode) where: {sequence, position} of every row, ang: cos and sin of its angles (Lm::rot)
+struct LmEmbedOut { int2* where; float* ang; };
 // x = embed[token] + sinusoid(pos), then the sink.  token = tokens[row], or the last generated id of the row's sequence; also written to tok[row], and the row as it is to
 // x0 (rows ldx0 apart) when given
 int launch_lm_embed(bool f32, const Lm& lm, int M, const int64_t* tokens, const LmRowIndex& ix, const int64_t* gen, const int32_t* ngen, int gen_cap,
-                    float* x, const LmSink& to, int32_t* tok, void* x0, int64_t ldx0, hipStream_t st);
+                    float* x, const LmSink& to, int32_t* tok, void* x0, int64_t ldx0, const LmEmbedOut& out, hipStream_t st);
 // what a sublayer left for a row: one row of Y in the element type (fp32 rows: slices = 1); with `slices` the sum of fp32 K-slices Y [slices][M][ldy]; with `top` the weighted
 // sum of the row's expert rows
 struct LmPostIn { const void* Y; int64_t ldy; int slices; const float* wt; int top; };
@@ -230,6 +236,18 @@ bool ret_matrix_supported(int Kp, int Vp);
 int launch_ret_decode(bool f32, const RetParams& p, const AttnParams* merge, int merge_dim, hipStream_t st);
 int launch_ret_recurrent(bool f32, const RetParams& p, hipStream_t st);
 int launch_ret_matrix(const RetParams& p, hipStream_t st);
+// ---- one decode step's mixers in one launch (lm_mix.hip): rows, attention and retention from the fused projection's K-slices ----
+struct LmMixIn {
+    int M;
+    const float* part; int slices;                    // [slices][M][Na]
+    const int2* where; const float* ang; void* ao;    // launch_lm_embed's; out
+    void *cache_k, *cache_v; int ring, chunk;         // attention (LmHeadsIn)
+    int rows, nsplit;                                 //   query heads of one key head a workgroup takes (fp32: 1), splits of 256 keys of the longest row (fp32: 1)
+    float *part_o, *part_ml;                          //   more than one split: partials (AttnParams)
+    float* state;                                     // retention (RetParams)
+};
+bool lm_mix_supported(bool f32, const LmLayer& L);
+int launch_lm_mix(bool f32, const Lm& lm, const LmLayer& L, const LmMixIn& in, hipStream_t st);
 // decode of <= 64 rows: z[m][n] = gelu_tanh(sum of K-slices) * side[tok[m]][n]
 int launch_lm_side_act(const Lm& lm, int M, const float* part, int slices, const void* side, int64_t lds, const int32_t* tok, void* z, hipStream_t st);
 // ... and y [M][Wp] = z . W^T in the same launch (few rows)

@@ -5,31 +5,9 @@
 // one wave: its norm is a lane reduction, its rotation partner (half a rotation away, at any distance) comes through 2 KiB of the wave's own LDS.  Angles are fp32 and are
 // computed once per row.
 #include "attention_plain.hpp"
-#include "lm.hpp"
+#include "lm_heads.hpp"
 
 namespace {
-
-template <typename T> __device__ __forceinline__ void ld8(const T* p, float (&v)[8]);
-template <> __device__ __forceinline__ void ld8<bf16>(const bf16* p, float (&v)[8]) {
-    const bf16x8 x = *(const bf16x8*)p;
-#pragma unroll
-    for (int e = 0; e < 8; e++) v[e] = (float)x[e];
-}
-template <> __device__ __forceinline__ void ld8<float>(const float* p, float (&v)[8]) {
-    const f32x4 a = *(const f32x4*)p, b = *(const f32x4*)(p + 4);
-#pragma unroll
-    for (int e = 0; e < 4; e++) { v[e] = a[e]; v[4 + e] = b[e]; }
-}
-__device__ __forceinline__ void st8(bf16* p, const float (&v)[8]) {
-    bf16x8 x;
-#pragma unroll
-    for (int e = 0; e < 8; e++) x[e] = (bf16)v[e];
-    *(bf16x8*)p = x;
-}
-__device__ __forceinline__ void st8(float* p, const float (&v)[8]) {
-    *(f32x4*)p = f32x4{v[0], v[1], v[2], v[3]};
-    *(f32x4*)(p + 4) = f32x4{v[4], v[5], v[6], v[7]};
-}
 
 struct HeadsArgs {
     LmHeadsIn in;
@@ -84,51 +62,10 @@ __global__ __launch_bounds__(256) void lm_heads_kernel(const HeadsArgs p) {
                 }
             } else if (!raw) ld8<T>((const T*)p.in.a + row * p.in.lda + col, v);
         }
-        // the norm of a query or key head
-        const float* gain = rg.kind == LM_Q ? p.nq : rg.kind == LM_K ? p.nk : nullptr;
-        float ss = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; e++) ss += v[e] * v[e];
-#pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const float other = __shfl_xor(ss, o, 64);
-            ss += o < rg.P / 8 ? other : 0.f;
-        }
-        if (gain) {
-            const float rs = 1.0f / sqrtf(ss / (float)p.dim + p.eps);
-            float g[8];
-            ld8<float>(gain + e0, g);
-#pragma unroll
-            for (int e = 0; e < 8; e++) v[e] *= rs * g[e];
-        }
-        // the rotation: partners through LDS
-        st8(&sx[wave][lane * 8], v);
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();
         const bool rq = rg.kind == LM_RQ || rg.kind == LM_RK;
-        const int half = rg.kind == LM_Q || rg.kind == LM_K ? p.half_a : rq ? p.half_r : 0;
-        if (e0 < 2 * half) {
-            const float *c = cs[rq][0], *s = cs[rq][1];
-            if (half % 8 == 0) {
-                const bool first = e0 < half;
-                const int i = first ? e0 : e0 - half;
-                float u[8], cc[8], sn[8];
-                ld8<float>(&sx[wave][lane * 8 + (first ? half : -half)], u);
-                ld8<float>(c + i, cc);
-                ld8<float>(s + i, sn);
-#pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = first ? v[e] * cc[e] - u[e] * sn[e] : v[e] * cc[e] + u[e] * sn[e];
-            } else {
-#pragma unroll
-                for (int e = 0; e < 8; e++) {
-                    const int q = e0 + e;
-                    if (q < half) v[e] = v[e] * c[q] - sx[wave][lane * 8 + e + half] * s[q];
-                    else if (q < 2 * half) v[e] = v[e] * c[q - half] + sx[wave][lane * 8 + e - half] * s[q - half];
-                }
-            }
-        }
-        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
-        __builtin_amdgcn_wave_barrier();                        // (the next round overwrites sx)
+        HeadLane hl;
+        hl.ask(e0, rg.kind == LM_Q ? p.nq : rg.kind == LM_K ? p.nk : nullptr, rg.kind == LM_Q || rg.kind == LM_K ? p.half_a : rq ? p.half_r : 0, cs[rq][0], cs[rq][1]);
+        hl.apply(rg.P, p.dim, p.eps, &sx[wave][lane * 8], v);
         if (rg.kind == LM_Q) st8((T*)p.in.q + row * ((int64_t)rg.heads * rg.P) + at, v);
         else if (rg.kind == LM_K || rg.kind == LM_V) {
             if (p.in.kv) st8((T*)p.in.kv + ((int64_t)p.in.row_key[row] * 2 + (rg.kind == LM_V)) * p.G * p.Ap + at, v);

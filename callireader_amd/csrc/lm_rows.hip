@@ -64,11 +64,19 @@ __device__ __forceinline__ int row_pos(const LmRowIndex& ix, int row) { return i
 template <typename T, int TPB, int NV>
 __global__ __launch_bounds__(TPB) void lm_embed_kernel(const T* __restrict__ table, const float* __restrict__ freq, int Wp, int W, int vocab, float eps, const int64_t* __restrict__ tokens,
                                                        const LmRowIndex ix, const int64_t* __restrict__ gen, const int32_t* __restrict__ ngen, int gen_cap,
-                                                       float* __restrict__ xo, const LmSink to, int32_t* __restrict__ tok, T* __restrict__ x0, int64_t ldx0) {
+                                                       float* __restrict__ xo, const LmSink to, int32_t* __restrict__ tok, T* __restrict__ x0, int64_t ldx0, const LmEmbedOut out,
+                                                       const float* __restrict__ rot, int n_rot) {
     __shared__ float red[TPB / 64];
     const int row = blockIdx.x, tid = threadIdx.x;
     const int seq = row_seq(ix, row);
     const float pos = (float)row_pos(ix, row);
+    if (out.where) {
+        if (tid == 0) out.where[row] = int2{seq, (int)row_pos(ix, row)};
+        for (int i = tid; i < n_rot; i += TPB) {
+            const float f = rot[i], a = pos * fabsf(f);
+            out.ang[(int64_t)row * n_rot + i] = signbit(f) ? sinf(a) : cosf(a);
+        }
+    }
     const int64_t t = tokens ? tokens[row] : gen[(int64_t)seq * gen_cap + ngen[seq] - 1];
     const int64_t id = t < 0 ? 0 : (t >= vocab ? vocab - 1 : t);      // (the host checks ids; a clamped read stays in bounds whatever arrives)
     if (tok && tid == 0) tok[row] = (int32_t)id;
@@ -239,9 +247,9 @@ __global__ __launch_bounds__(256) void lm_latents_kernel(T* __restrict__ a, cons
     } while (0)
 
 int launch_lm_embed(bool f32, const Lm& lm, int M, const int64_t* tokens, const LmRowIndex& ix, const int64_t* gen, const int32_t* ngen, int gen_cap, float* x, const LmSink& to, int32_t* tok,
-                    void* x0, int64_t ldx0, hipStream_t st) {
-    if (f32) LM_NV_DISPATCH(lm_embed_kernel, float, M, (const float*)lm.embed, lm.freq, lm.Wp, lm.d.width, lm.d.vocab, lm.d.eps, tokens, ix, gen, ngen, gen_cap, x, to, tok, (float*)x0, ldx0);
-    LM_NV_DISPATCH(lm_embed_kernel, bf16, M, (const bf16*)lm.embed, lm.freq, lm.Wp, lm.d.width, lm.d.vocab, lm.d.eps, tokens, ix, gen, ngen, gen_cap, x, to, tok, (bf16*)x0, ldx0);
+                    void* x0, int64_t ldx0, const LmEmbedOut& out, hipStream_t st) {
+    if (f32) LM_NV_DISPATCH(lm_embed_kernel, float, M, (const float*)lm.embed, lm.freq, lm.Wp, lm.d.width, lm.d.vocab, lm.d.eps, tokens, ix, gen, ngen, gen_cap, x, to, tok, (float*)x0, ldx0, out, lm.rot_freq, (int)lm.rot.size());
+    LM_NV_DISPATCH(lm_embed_kernel, bf16, M, (const bf16*)lm.embed, lm.freq, lm.Wp, lm.d.width, lm.d.vocab, lm.d.eps, tokens, ix, gen, ngen, gen_cap, x, to, tok, (bf16*)x0, ldx0, out, lm.rot_freq, (int)lm.rot.size());
 }
 
 int launch_lm_post(bool f32, const Lm& lm, int M, const LmPostIn& in, float* x, const float* gain_b, bool replace, const LmSink& to, hipStream_t st) {

@@ -15,7 +15,7 @@
 #include "attention_merge.hpp"
 #include <type_traits>
 
-#include "lm.hpp"
+#include "retention.hpp"
 
 namespace {
 
@@ -29,23 +29,6 @@ template <> __device__ __forceinline__ f32x4 ld4f<bf16>(const bf16* p) {
     const bf16x4 v = *(const bf16x4*)p;
     return f32x4{(float)v[0], (float)v[1], (float)v[2], (float)v[3]};
 }
-// the sixteen dk groups of a wave sit four lanes apart
-__device__ __forceinline__ f32x4 sum_groups(f32x4 o) {
-    // lane ^ 4, ^ 8, ^ 16, ^ 32 on the vector pipe (LDS shuffles made a chain of four round trips of every token): the bank masks of two row shifts make the first
-#pragma unroll
-    for (int e = 0; e < 4; e++) {
-        const int x = __float_as_int(o[e]);
-        o[e] += __int_as_float(__builtin_amdgcn_update_dpp(__builtin_amdgcn_update_dpp(0, x, 0x104, 0xf, 0x5, false), x, 0x114, 0xf, 0xa, false));
-        o[e] += dpp<0x128>(o[e]);
-        const auto r = __builtin_amdgcn_permlane16_swap(__float_as_uint(o[e]), __float_as_uint(o[e]), false, false);
-        o[e] = __uint_as_float(r[0]) + __uint_as_float(r[1]);
-        const auto h = __builtin_amdgcn_permlane32_swap(__float_as_uint(o[e]), __float_as_uint(o[e]), false, false);
-        o[e] = __uint_as_float(h[0]) + __uint_as_float(h[1]);
-    }
-    return o;
-}
-__device__ __forceinline__ float silu32(float x) { return x / (1.0f + expf(-x)); }
-
 constexpr int dec_waves(int NR) { return NR > 16 ? 8 : 16; }
 
 // workgroups past the heads merge the attention's key splits of the same row (the mixer beside this one), a wave per 64 columns: two short launches in one
@@ -60,45 +43,13 @@ __global__ __launch_bounds__(dec_waves(NR) * 64) void ret_decode_kernel(const Re
         return;
     }
     const int seq = p.ix.seqs[row];
-    const bool fresh = p.ix.lens[seq] == 0;                   // a state starts at zero, whatever the slot held before
-    const int g = lane >> 2, c4 = (lane & 3) * 4, blocks = p.Vp >> 4;
-    float* st = p.state + ((int64_t)seq * p.H + h) * p.Vp * p.Kp;
-    const float decay = p.pw[h * (RET_CHUNK + 1) + 1];
-    const float* qr = p.rq + ((int64_t)row * p.H + h) * p.Kp + g * NR;
-    const float* kr = p.rk + ((int64_t)row * p.H + h) * p.Kp + g * NR;
-    for (int b = wave; b < blocks; b += nw) {
-        f32x4 s[NR];
-        float* sb = st + (int64_t)b * NR * 256 + lane * 4;
-#pragma unroll
-        for (int r = 0; r < NR; r++) s[r] = fresh ? f32x4{0.f, 0.f, 0.f, 0.f} : __builtin_nontemporal_load((const f32x4*)(sb + r * 256));
-        float q[NR], k[NR];
-#pragma unroll
-        for (int r = 0; r < NR; r += 4) {
-            const f32x4 a = *(const f32x4*)(qr + r), c = *(const f32x4*)(kr + r);
-#pragma unroll
-            for (int e = 0; e < 4; e++) { q[r + e] = a[e]; k[r + e] = c[e]; }
-        }
-        const f32x4 v = ld4f((const T*)p.v + (int64_t)row * p.lda + h * p.Vp + b * 16 + c4);
-        f32x4 o = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int r = 0; r < NR; r++) {
-            s[r] = s[r] * decay + k[r] * v;
-            o += s[r] * q[r];
-            __builtin_nontemporal_store(s[r], (f32x4*)(sb + r * 256));
-        }
-        o = sum_groups(o);
-        if (lane < 4) *(f32x4*)&so[b * 16 + c4] = o;
-        float ss = o[0] * o[0] + o[1] * o[1] + o[2] * o[2] + o[3] * o[3];
-        ss += __shfl_xor(ss, 1, 64);
-        ss += __shfl_xor(ss, 2, 64);
-        if (lane == 0) red[b] = ss;
-    }
+    const RetHead head{p.state, p.pw, p.H, p.Kp, p.Vp, p.vdim, p.eps, p.out_scale};
+    RetStep<NR> step(head, seq, h);
+    step.ask();
+    const int64_t at = ((int64_t)row * p.H + h) * p.Kp;
+    step.run(p.ix.lens[seq] == 0, p.rq + at, p.rk + at, [&](int c) { return ld4f((const T*)p.v + (int64_t)row * p.lda + h * p.Vp + c); }, so, red);
     __syncthreads();
-    float ss = 0.f;
-    for (int b = 0; b < blocks; b++) ss += red[b];
-    const float rs = p.out_scale / sqrtf(ss / (float)p.vdim + p.eps);
-    for (int c = tid; c < p.vdim; c += blockDim.x)
-        ((T*)p.ao)[(int64_t)row * p.ldo + (int64_t)h * p.vdim + c] = (T)(so[c] * rs * silu32((float)((const T*)p.g)[(int64_t)row * p.lda + h * p.Vp + c]));
+    step.finish(so, red, [&](int c, float o) { ((T*)p.ao)[(int64_t)row * p.ldo + (int64_t)h * p.vdim + c] = (T)(o * silu32((float)((const T*)p.g)[(int64_t)row * p.lda + h * p.Vp + c])); });
 }
 
 // one wave = 16 value columns, the tokens of a segment in turn, U at a time.  Bound by the chain of loads: the rows of the next U tokens are fetched under the current ones' arithmetic

@@ -1,0 +1,42 @@
+"""One launch for a decode step's attention and retention (lm_mix.hip): key counts around its 32-key blocks, 64-key tiles and 256-key splits, groups of query heads from one to the most a
+workgroup takes, heads of 64 and 128, rotations whose halves are no multiple of eight, value sizes that no vector divides."""
+import pytest
+import torch
+
+import lugasun_cases as LC
+from oracle import lugasun as O
+
+pytestmark = pytest.mark.gpu
+F32, BF16 = torch.float32, torch.bfloat16
+LENS = [1, 2, 31, 32, 33, 63, 64, 65, 96, 254, 255, 256, 257, 511, 513]
+LAYERS = {
+    'group4_128': LC.layer(LC.heads(8, 2, 128, 128, 4096, softcap=20.0), LC.ret(64, 64, (0.97, 0.9)), 64),
+    'group1_64': LC.layer(LC.heads(3, 3, 50, 50, 4096, rot=(100.0, 36)), LC.ret(100, 300, (0.95,), rot=(100.0, 12)), None),
+    'group32_128': LC.layer(LC.heads(32, 1, 72, 70, 4096), LC.ret(40, 33, (0.9, 0.99, 0.5)), None),
+    'chunks': LC.layer(LC.heads(4, 1, 64, 64, 256), LC.ret(128, 64, (0.99,)), 64),
+}
+
+
+@pytest.mark.parametrize('dtype', [F32, BF16])
+@pytest.mark.parametrize('name', LAYERS)
+def test_rows_of_every_length_together_and_alone(name, dtype):
+    """Against the oracle, and a row's bits are the same whatever longer or shorter rows it is decoded with."""
+    from callireader_amd.modeling_decoder import LugasunForCausalLM
+    cfg = LC.config(128, 60, [LAYERS[name]], side=8)
+    w = LC.weights(cfg, 31, qk_gain=1.5 if dtype == F32 else 1.0)
+    m = LugasunForCausalLM.from_state_dict(w, cfg, dtype=dtype, max_tokens=640, max_seqs=len(LENS))
+    toks = [LC.tokens(cfg, n + 3, seed=n) for n in LENS]
+
+    def run(which):
+        for i in which:                                       # (a prompt alone, so that its bits are given)
+            m.step([(i, toks[i][:LENS[i]], [])])
+        z = torch.stack([m.step([(i, [toks[i][LENS[i] + k]], [0]) for i in which]) for k in range(3)], 1).cpu()
+        for i in which:
+            m.end(i)
+        return z
+    together = run(range(len(LENS)))
+    for i, n in enumerate(LENS):
+        assert LC.close(together[i], O.forward(w, cfg, toks[i])[n:], dtype), n
+    for i in (0, 3, 6, 9, 12):
+        assert torch.equal(run([i])[0], together[i]), LENS[i]
+    m.close()
