@@ -240,10 +240,18 @@ class Engine:
         B.check(B.lib.cr_llm_hidden_probe(self._h, _p(self._probe), row0, rows), 'cr_llm_hidden_probe')
         return self._probe
 
+    def upload(self, t):
+        """A small host tensor on the device, through a pinned copy of its own: a copy from pageable memory waits for all that the stream has still to do, and a step that fed it one ran
+        with nothing enqueued behind it."""
+        return torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t).to(self.device, non_blocking=True)
+
     def decode(self, kv, seqs, penalty=1.0, force_tokens=None, want_logits=False):
         n = len(seqs)
         seq_arr = (C.c_int32 * n)(*seqs)
-        ft = force_tokens.reshape(-1).to(self.device, torch.int64).contiguous() if force_tokens is not None else None
+        ft = None
+        if force_tokens is not None:
+            ft = force_tokens.reshape(-1).to(torch.int64)
+            ft = self.upload(ft) if ft.device.type == 'cpu' else ft.to(self.device).contiguous()
         logits = torch.empty(n, self.dims.vocab, device=self.device, dtype=torch.float32) if want_logits else None
         B.check(B.lib.cr_llm_decode(self._h, kv._h, seq_arr, n, _p(ft), float(penalty), _p(logits), _stream()), 'cr_llm_decode')
         return logits

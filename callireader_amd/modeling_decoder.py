@@ -73,7 +73,9 @@ class DecoderLM:
         if not new and all(len(t) == 1 for _, t, _ in entries):
             logits = self.engine.decode(kv, seqs, penalty=penalty, force_tokens=torch.tensor([t[0] for _, t, _ in entries], dtype=torch.int64), want_logits=True)
             rows = [i for i, (_, _, w) in enumerate(entries) for _ in w]
-            return logits[rows] if rows else None
+            if rows == list(range(len(entries))):
+                return logits
+            return logits.index_select(0, self.engine.upload(torch.tensor(rows))) if rows else None
         want, base = [], 0
         for _, t, w in entries:
             want += [base + p for p in w]
