@@ -233,3 +233,4 @@ __device__ __forceinline__ unsigned long long argmax_pack(float v, int c) {
 int launch_gemm(int epi, const GemmParams& p, hipStream_t stream);
 // K-slices of the EPI_PARTIAL decode GEMM for an [N, K] weight (depends on N and K only, never on M); 0 = unsupported
 int gemm_partial_splits(int N, int K);
+int gemm_partial_tiles(int N, int K);      // 16-row weight tiles of a workgroup of the same

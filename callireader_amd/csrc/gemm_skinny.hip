@@ -293,6 +293,7 @@ PartialGeom partial_geom(int N, int K) {
 }  // namespace
 
 int gemm_partial_splits(int N, int K) { return partial_geom(N, K).splits; }
+int gemm_partial_tiles(int N, int K) { return partial_geom(N, K).rt; }
 
 bool gemm_skinny_supported(int epi, const GemmParams& p) {
     if (p.M > 64 || p.K % 128 != 0) return false;

@@ -267,6 +267,8 @@ struct Buffers {
     float* x; void *h, *a, *cq, *q, *c, *kv, *qp, *ol, *ao, *y, *act, *ye, *cat, *z2; float *z, *wt, *part, *sl, *rq, *rk, *raw; bf16 *rq2, *rk2, *snap;
     int32_t *idx, *perm, *n_tiles, *tok; int4* tiles;
     int2* where; float* ang;
+    float *x2, *sl2;             // few decode rows: the residual's and the slices' other place (lm_ahead.hip reads one and writes the other)
+    LmAhead ahead;               // a residual update that the next product makes (Y null: none)
 };
 bool expanded(const Lm& lm, const LmLayer& L, bool decode) { return !lm.f32 && !decode && L.s.scale > 0.f && (L.Ap == 64 || L.Ap == 128 || L.Ap == 256); }
 bool split_decode(const Lm& lm, const LmLayer& L, bool decode) { return !lm.f32 && decode && latent_decode_supported(L.Rp); }
@@ -298,6 +300,15 @@ int sliced(cr_ctx* c, const void* A, int64_t lda, const void* W, const bf16* dl,
     if (!one_slice(M, N, K)) return ctx_gemm(c, EPI_PARTIAL, p, st);
     p.raw32 = 1;
     return ctx_gemm(c, EPI_F32, p, st);
+}
+
+// the product that reads the residual next, with the update ahead of it; K-slices (LM_RAW32) to b.sl, of which the update reads the other half
+int behind(const Lm& lm, Buffers& b, int epi, const void* W, const bf16* dl, void* C, int N, const void* gate, int64_t ldg, hipStream_t st) {
+    CR_TRY(launch_lm_ahead(lm.f32, b.ahead, epi, lm.f32 ? W : dl, epi == LM_RAW32 ? b.sl2 : C, N, gate, ldg, b.tok, st));
+    std::swap(b.x, b.x2);
+    if (epi == LM_RAW32) std::swap(b.sl, b.sl2);
+    b.ahead.Y = nullptr;
+    return CR_OK;
 }
 
 // K-slices of the token side's gate in the 128-row kernel: four where K allows (depends on K alone)
@@ -344,10 +355,10 @@ Buffers carve(const Lm& lm, Arena& ar, const Step& sp) {
     if (lm.d.loop_in) slices(Wp, 2 * Wp);
     auto T = [&](size_t n) { return (void*)ar.take<char>(n * es); };
     Buffers b{};
-    b.x = ar.take<float>((size_t)M * Wp); b.h = T((size_t)M * Wp); b.a = T((size_t)M * Na); b.cq = T((size_t)M * Qp); b.q = T((size_t)M * qn);
+    b.x = ar.take<float>((size_t)M * Wp); b.x2 = ar.take<float>(decode && M <= 8 ? (size_t)M * Wp : 0); b.h = T((size_t)M * Wp); b.a = T((size_t)M * Na); b.cq = T((size_t)M * Qp); b.q = T((size_t)M * qn);
     b.c = T((size_t)M * Rp); b.kv = T(std::max((size_t)sp.Mk * kvn, kvh)); b.qp = T((size_t)M * hr); b.ol = T((size_t)M * hr); b.ao = T((size_t)M * Gp); b.y = T((size_t)M * Wp);
     b.act = T((size_t)M * act); b.ye = T((size_t)M * top * Wp);
-    b.part = ar.take<float>(part); b.sl = ar.take<float>(sl);
+    b.part = ar.take<float>(part); b.sl = ar.take<float>(sl); b.sl2 = ar.take<float>(decode && M <= 8 ? sl : 0);
     b.z = ar.take<float>((size_t)M * Ep * (M <= 128 ? LM_ROUTER_SLICES : 1)); b.wt = ar.take<float>((size_t)M * top);
     b.idx = ar.take<int32_t>((size_t)M * top); b.perm = ar.take<int32_t>((size_t)M * top); b.n_tiles = ar.take<int32_t>(1); b.tiles = ar.take<int4>(tiles);
     b.rq = ar.take<float>(r32); b.rk = ar.take<float>(r32); b.rq2 = ar.take<bf16>(r16); b.rk2 = ar.take<bf16>(r16); b.raw = ar.take<float>(raw); b.snap = ar.take<bf16>(snap);
@@ -397,7 +408,8 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
     const size_t es = lm.esz();
     char* cache = kv->lat + kv->lat_off[r];
     const int s_a = slices_of(lm, M, L.Na, Wp, sp.decode);
-    if (s_a) CR_TRY(sliced(c, b.h, Wp, L.wa, L.wa_dl, b.sl, M, L.Na, Wp, st));
+    if (b.ahead.Y) CR_TRY(behind(lm, b, LM_RAW32, L.wa, L.wa_dl, nullptr, L.Na, nullptr, 0, st));
+    else if (s_a) CR_TRY(sliced(c, b.h, Wp, L.wa, L.wa_dl, b.sl, M, L.Na, Wp, st));
     else CR_TRY(dense(c, lm, b.h, Wp, L.wa, b.a, L.Na, M, L.Na, Wp, st, !sp.decode, L.wa_dl, false, true));
     CR_TRY(launch_lm_latents(lm.f32, lm, L, M, b.a, s_a ? b.sl : nullptr, s_a, b.cq, sp.decode ? nullptr : b.c, cache, kv->max_tokens, sp.ix, b.ao, st));
     const int s_q = !lm.f32 && L.Ap <= 512 ? slices_of(lm, M, H * L.Ap, L.Qp, sp.decode) : 0;
@@ -450,7 +462,8 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
     const int M = sp.M, Wp = lm.Wp;
     const size_t es = lm.esz();
     const int s_a = slices_of(lm, M, L.Na, Wp, sp.decode);
-    if (s_a) CR_TRY(sliced(c, b.h, Wp, L.wa, L.wa_dl, b.sl, M, L.Na, Wp, st));
+    if (b.ahead.Y) CR_TRY(behind(lm, b, LM_RAW32, L.wa, L.wa_dl, nullptr, L.Na, nullptr, 0, st));
+    else if (s_a) CR_TRY(sliced(c, b.h, Wp, L.wa, L.wa_dl, b.sl, M, L.Na, Wp, st));
     else CR_TRY(dense(c, lm, b.h, Wp, L.wa, b.a, L.Na, M, L.Na, Wp, st, !sp.decode, L.wa_dl, false, true));
     const KeyPlan* kp = L.heads() && !sp.decode ? &sp.plans[L.chunk_ix] : nullptr;
     const int ring = L.heads() ? std::min(lm.chunks[L.chunk_ix], kv->max_tokens) : 1, chunk = L.heads() ? lm.chunks[L.chunk_ix] : 1;
@@ -576,6 +589,15 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
         out = LmPostIn{n ? (const void*)b.sl : b.y, Wp, n, nullptr, 0};
         return n ? sliced(c, A, K, W, dl, b.sl, M, Wp, K, st) : dense(c, lm, A, K, W, b.y, Wp, M, Wp, K, st, !sp.decode, dl, false, true);
     };
+    // x += ..., then the sink: left to the product behind it where few rows allow it (N columns; 0: no product reads this sink next)
+    auto update = [&](const LmPostIn& y, const float* gain_b, bool replace, const LmSink& to, int epi, int N, const bf16* dl) -> int {
+        if (!N || !sp.decode || y.top || !lm_ahead_supported(lm.f32, M, Wp, N, epi, dl != nullptr)) return launch_lm_post(lm.f32, lm, M, y, b.x, gain_b, replace, to, st);
+        b.ahead = LmAhead{y.Y, y.slices, replace, b.x, b.x2, gain_b, to.gain, M, Wp, lm.d.width, lm.d.eps};
+        return CR_OK;
+    };
+    // what the update ahead of pass r's first product is left to: that product, unless the embedding is mixed in first or there is no such pass
+    auto first_n = [&](size_t r) { return r < lm.passes.size() && !lm.starts[r] && slices_of(lm, M, lm.layers[lm.passes[r]].Na, Wp, sp.decode) ? lm.layers[lm.passes[r]].Na : 0; };
+    auto first_dl = [&](size_t r) -> const bf16* { return r < lm.passes.size() ? lm.layers[lm.passes[r]].wa_dl : nullptr; };
     CR_TRY(launch_lm_embed(lm.f32, lm, M, sp.tokens, sp.ix, kv->d_gen, kv->d_ngen, kv->gen_cap, b.x, entry(0), b.tok, lm.d.loop_in ? (char*)b.cat + (size_t)Wp * es : nullptr, 2 * Wp, LmEmbedOut{sp.decode ? b.where : nullptr, b.ang}, st));
     CR_TRY(probe(0));
     for (size_t r = 0; r < lm.passes.size(); r++) {
@@ -586,7 +608,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
             const int n = slices_of(lm, M, Wp, 2 * Wp, sp.decode);
             if (n) {
                 CR_TRY(sliced(c, b.cat, 2 * Wp, lm.loop_in, lm.loop_dl, b.sl, M, Wp, 2 * Wp, st));
-                CR_TRY(launch_lm_post(lm.f32, lm, M, LmPostIn{b.sl, Wp, n, nullptr, 0}, b.x, nullptr, true, to, st));
+                CR_TRY(update(LmPostIn{b.sl, Wp, n, nullptr, 0}, nullptr, true, to, LM_RAW32, slices_of(lm, M, L.Na, Wp, sp.decode) ? L.Na : 0, L.wa_dl));
             } else {
                 CR_TRY(raw32(c, lm, b.cat, lm.loop_in, b.x, Wp, M, Wp, 2 * Wp, 0.f, st, sp.decode, sp.decode ? lm.loop_dl : nullptr, true));
                 CR_TRY(launch_lm_pick_rows(lm.f32, lm, M, b.x, nullptr, b.h, L.n1, st));
@@ -595,11 +617,16 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
         CR_TRY(L.latent() ? latent_mixer(c, kv, sp, b, L, r, st) : heads_mixer(c, kv, sp, b, L, r, st));
         CR_TRY(project(b.ao, L.wo, L.wo_dl, L.Gp, y));
         const LmSink next = entry(r + 1), end = lm.Sp ? LmSink{b.h, Wp, nullptr} : next;
-        CR_TRY(launch_lm_post(lm.f32, lm, M, y, b.x, L.n1b, false, L.s.ff == CR_FF_NONE ? end : LmSink{b.h, Wp, L.n2}, st));
+        // the last update of a pass ahead of the token side
+        const int end_epi = lm.Sp && lm.f32 ? LM_SIDE : LM_RAW32, end_n = !lm.Sp ? first_n(r + 1) : lm.f32 ? (M <= LM_ROWS_MAX ? lm.Sp : 0) : slices_of(lm, M, lm.Sp, Wp, sp.decode) ? lm.Sp : 0;
+        const bf16* end_dl = lm.Sp ? L.sgate_dl : first_dl(r + 1);
+        if (L.s.ff == CR_FF_NONE) CR_TRY(update(y, L.n1b, false, end, end_epi, end_n, end_dl));
+        else CR_TRY(update(y, L.n1b, false, LmSink{b.h, Wp, L.n2}, LM_RELU2, L.s.ff == CR_FF_DENSE && M <= LM_ROWS_MAX ? L.ffp : 0, L.wgu_dl));
         if (L.s.ff == CR_FF_DENSE) {
-            CR_TRY(dense(c, lm, b.h, Wp, L.wgu, b.act, L.ffp, M, L.ffp, Wp, st, !sp.decode, L.wgu_dl, true));
+            if (b.ahead.Y) CR_TRY(behind(lm, b, LM_RELU2, L.wgu, L.wgu_dl, b.act, L.ffp, nullptr, 0, st));
+            else CR_TRY(dense(c, lm, b.h, Wp, L.wgu, b.act, L.ffp, M, L.ffp, Wp, st, !sp.decode, L.wgu_dl, true));
             CR_TRY(project(b.act, L.wdn, L.wdn_dl, L.ffp, y));
-            CR_TRY(launch_lm_post(lm.f32, lm, M, y, b.x, L.n2b, false, end, st));
+            CR_TRY(update(y, L.n2b, false, end, end_epi, end_n, end_dl));
         } else if (L.s.ff == CR_FF_MOE) {
             CR_TRY(expert_mixture(c, sp, b, L, st));
             CR_TRY(launch_lm_post(lm.f32, lm, M, LmPostIn{b.ye, Wp, 0, b.wt, L.s.top}, b.x, L.n2b, false, end, st));
@@ -611,11 +638,13 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
             if (lm.f32) {
                 LmGemmParams g{};
                 g.A = b.h; g.lda = Wp; g.W = L.sgate; g.ldw = Wp; g.C = b.z2; g.ldc = lm.Sp; g.M = M; g.N = lm.Sp; g.K = Wp; g.gate = side; g.ldg = lds; g.tok = b.tok; g.stream = sp.decode && M <= LM_ROWS_MAX;
-                CR_TRY(launch_lm_gemm(true, LM_SIDE, g, st));
+                if (b.ahead.Y) CR_TRY(behind(lm, b, LM_SIDE, L.sgate, nullptr, b.z2, lm.Sp, side, lds, st));
+                else CR_TRY(launch_lm_gemm(true, LM_SIDE, g, st));
             } else {
                 // few columns: K-slices keep the chip busy, and the kernel that adds them applies the activation and the token's row
                 int n = slices_of(lm, M, lm.Sp, Wp, sp.decode);
-                if (n) CR_TRY(sliced(c, b.h, Wp, L.sgate, L.sgate_dl, b.sl, M, lm.Sp, Wp, st));
+                if (b.ahead.Y) CR_TRY(behind(lm, b, LM_RAW32, L.sgate, L.sgate_dl, nullptr, lm.Sp, nullptr, 0, st));
+                else if (n) CR_TRY(sliced(c, b.h, Wp, L.sgate, L.sgate_dl, b.sl, M, lm.Sp, Wp, st));
                 else {
                     GemmParams g = slice_params(b.h, Wp, L.sgate, nullptr, b.sl, M, lm.Sp, Wp);
                     g.kernel = 128; g.group = n = side_slices(Wp);
@@ -627,7 +656,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
             }
             if (projected) y = LmPostIn{b.y, Wp, 0, nullptr, 0};
             else CR_TRY(project(b.z2, L.sproj, L.sproj_dl, lm.Sp, y));
-            CR_TRY(launch_lm_post(lm.f32, lm, M, y, b.x, L.ns, false, next, st));
+            CR_TRY(update(y, L.ns, false, next, LM_RAW32, first_n(r + 1), first_dl(r + 1)));
         }
         CR_TRY(probe((int)r + 1));
     }

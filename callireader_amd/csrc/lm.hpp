@@ -125,6 +125,11 @@ int launch_lm_embed(bool f32, const Lm& lm, int M, const int64_t* tokens, const 
 struct LmPostIn { const void* Y; int64_t ldy; int slices; const float* wt; int top; };
 // x += gain_b ? rms(y) * gain_b : y (x = y with `replace`), then the sink (h may be null)
 int launch_lm_post(bool f32, const Lm& lm, int M, const LmPostIn& in, float* x, const float* gain_b, bool replace, const LmSink& to, hipStream_t st);
+// The same update at the start of the few-row product that reads its result (lm_ahead.hip): C = epi(h . W^T), epi LM_RAW32 (K-slices [slices][M][N] for a consumer that adds them), LM_RELU2
+// (element type) or, in fp32, LM_SIDE.  bf16: W is the decode-layout copy.  x and x_out are not the same rows: other workgroups still read x.
+struct LmAhead { const void* Y; int slices, replace; const float* x; float* x_out; const float *gain_b, *gain; int M, Wp, W; float eps; };      // Y: slices of [M][Wp], or (0) rows in the element type
+bool lm_ahead_supported(bool f32, int M, int Wp, int N, int epi, bool decode_layout);
+int launch_lm_ahead(bool f32, const LmAhead& a, int epi, const void* W, void* C, int N, const void* gate, int64_t ldg, const int32_t* tok, hipStream_t st);
 // h[i] = rms(x[rows[i]]) * gain
 int launch_lm_pick_rows(bool f32, const Lm& lm, int n, const float* x, const int32_t* rows, void* h, const float* gain, hipStream_t st);
 // the down projection (rows `a`, or fp32 K-slices `part` [slices][M][Na]: then the gate's columns are also written to `a`) -> its two latents: cq = rms(a[0 .. q_rank)) * nq; c = rms(a[off_c .. + kv_rank)) * nc -> the cache row and (prefill) a dense copy

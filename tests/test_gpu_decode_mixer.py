@@ -40,3 +40,28 @@ def test_rows_of_every_length_together_and_alone(name, dtype):
     for i in (0, 3, 6, 9, 12):
         assert torch.equal(run([i])[0], together[i]), LENS[i]
     m.close()
+
+
+@pytest.mark.parametrize('dtype', [F32, BF16])
+@pytest.mark.parametrize('width', [200, 1024, 2048])
+def test_residual_updates_inside_the_next_product(width, dtype):
+    """One to a few rows leave each residual update to the product behind it (lm_ahead.hip), more rows take a launch for it: the same bits, with and without norms on the way, at the entry of
+    a looped span and ahead of the token side."""
+    from callireader_amd.modeling_decoder import LugasunForCausalLM
+    cfg = LC.config(width, 90, [LC.layer(LC.heads(2, 1, 64, 64, 64), LC.ret(64, 64, (0.9, 0.99)), 640), LC.layer(LC.heads(1, 1, 64, 40, 64), LC.ret(16, 16, (0.9,)), None)], side=24, loop=(1, 2, 2))
+    w = LC.weights(cfg, 32)
+    m = LugasunForCausalLM.from_state_dict(w, cfg, dtype=dtype, max_tokens=64, max_seqs=20)
+    toks = [LC.tokens(cfg, 12, seed=i) for i in range(20)]
+
+    def run(which):
+        for i in which:
+            m.step([(i, toks[i][:9], [])])
+        z = torch.stack([m.step([(i, [toks[i][9 + k]], [0]) for i in which]) for k in range(3)], 1).cpu()
+        for i in which:
+            m.end(i)
+        return z
+    together = run(range(20))
+    assert LC.close(together[5], O.forward(w, cfg, toks[5])[9:], dtype)
+    for which in ([0], [3], [0, 1], [4, 5, 6, 7], range(8)):
+        assert torch.equal(run(which), together[list(which)]), which
+    m.close()
