@@ -228,6 +228,7 @@ int derive_layer(Deriver& dv, int i, LmLayer& L) {
     L.router = dv.mat(o + "router", (size_t)L.Ep * Wp); L.wgu = dv.mat(o + "gu", (size_t)s.experts * 2 * L.ffp * Wp); L.wdn = dv.mat(o + "dn", (size_t)s.experts * Wp * L.ffp);
     if (!L.router || !L.wgu || !L.wdn) return CR_ERR_NOMEM;
     CR_TRY(dv.place(rt, 0, s.experts, L.router, 0, Wp));
+    L.router_dl = dv.swizzled(o + "router.dl", L.router, s.experts, Wp);
     for (int e = 0; e < s.experts; e++) {
         const std::string q = p + "mlp.e" + std::to_string(e) + ".";
         const DevTensor *ga = dv.src(q + "gate", s.expert_ff, W), *up = dv.src(q + "up", s.expert_ff, W), *dn = dv.src(q + "down", W, s.expert_ff);
@@ -265,7 +266,7 @@ struct Step {
 // one activations carve-up for a step; the same function sizes the workspace and lays it out
 struct Buffers {
     float* x; void *h, *a, *cq, *q, *c, *kv, *qp, *ol, *ao, *y, *act, *ye, *cat, *z2; float *z, *wt, *part, *sl, *rq, *rk, *raw; bf16 *rq2, *rk2, *snap;
-    int32_t *idx, *perm, *n_tiles, *tok; int4* tiles;
+    int32_t *idx, *perm, *n_tiles, *hist, *tok; int4* tiles;
     int2* where; float* ang;
     float *x2, *sl2;             // few decode rows: the residual's and the slices' other place (lm_ahead.hip reads one and writes the other)
     LmAhead ahead;               // a residual update that the next product makes (Y null: none)
@@ -318,7 +319,7 @@ Buffers carve(const Lm& lm, Arena& ar, const Step& sp) {
     const size_t es = lm.esz();
     const int M = sp.M, Wp = lm.Wp;
     const bool decode = sp.decode, sliced = decode && M <= 64;
-    size_t Na = 0, Qp = 0, Rp = 0, Gp = 0, qn = 0, kvn = 0, hr = 0, Ep = 0, top = 0, act = 0, tiles = 0, part = 0, sl = 0, kvh = 0, r32 = 0, r16 = 0, raw = 0, snap = 0;
+    size_t Na = 0, Qp = 0, Rp = 0, Gp = 0, qn = 0, kvn = 0, hr = 0, Ep = 0, top = 0, act = 0, tiles = 0, part = 0, sl = 0, kvh = 0, r32 = 0, r16 = 0, raw = 0, snap = 0, hist = 0;
     auto slices = [&](int N, int K) { if (sliced) sl = std::max(sl, (size_t)M * std::max(1, lm.f32 ? lm_rows_slices(N, K) : gemm_partial_splits(N, K)) * N); };
     for (const LmLayer& L : lm.layers) {
         Na = std::max<size_t>(Na, L.Na); Gp = std::max<size_t>(Gp, L.Gp);
@@ -347,6 +348,7 @@ Buffers carve(const Lm& lm, Arena& ar, const Step& sp) {
         if (L.s.ff != CR_FF_MOE) continue;
         Ep = std::max<size_t>(Ep, L.Ep); top = std::max<size_t>(top, L.s.top); act = std::max<size_t>(act, (size_t)L.s.top * L.ffp);
         tiles = std::max<size_t>(tiles, lm_max_tiles(M * L.s.top, L.s.experts, LM_TILE_M));
+        hist = std::max(hist, lm_plan_ints(M, L.s.top, L.s.experts));
     }
     if (lm.Sp) {
         slices(lm.Sp, Wp); slices(Wp, lm.Sp);
@@ -360,7 +362,7 @@ Buffers carve(const Lm& lm, Arena& ar, const Step& sp) {
     b.act = T((size_t)M * act); b.ye = T((size_t)M * top * Wp);
     b.part = ar.take<float>(part); b.sl = ar.take<float>(sl); b.sl2 = ar.take<float>(decode && M <= 8 ? sl : 0);
     b.z = ar.take<float>((size_t)M * Ep * (M <= 128 ? LM_ROUTER_SLICES : 1)); b.wt = ar.take<float>((size_t)M * top);
-    b.idx = ar.take<int32_t>((size_t)M * top); b.perm = ar.take<int32_t>((size_t)M * top); b.n_tiles = ar.take<int32_t>(1); b.tiles = ar.take<int4>(tiles);
+    b.idx = ar.take<int32_t>((size_t)M * top); b.perm = ar.take<int32_t>((size_t)M * top); b.n_tiles = ar.take<int32_t>(1); b.hist = ar.take<int32_t>(hist); b.tiles = ar.take<int4>(tiles);
     b.rq = ar.take<float>(r32); b.rk = ar.take<float>(r32); b.rq2 = ar.take<bf16>(r16); b.rk2 = ar.take<bf16>(r16); b.raw = ar.take<float>(raw); b.snap = ar.take<bf16>(snap);
     b.where = ar.take<int2>(decode ? M : 0); b.ang = ar.take<float>(decode ? M * std::max<size_t>(lm.rot.size(), 1) : 0);
     b.tok = ar.take<int32_t>(M); b.z2 = T((size_t)M * lm.Sp); b.cat = T(lm.d.loop_in ? (size_t)M * 2 * Wp : 0);
@@ -546,7 +548,7 @@ int expert_mixture(cr_ctx* c, const Step& sp, Buffers& b, const LmLayer& L, hipS
         if (!stream) {
             mp.grouped256 = moe_grouped256(M, s.top, s.experts, 2 * L.ffp, Wp) && moe_grouped256(M, s.top, s.experts, Wp, L.ffp);
             const int tile_m = mp.grouped256 ? 256 : MOE_TILE_M;
-            CR_TRY(launch_lm_plan(L, M, tile_m, b.idx, b.perm, b.tiles, b.n_tiles, st));
+            CR_TRY(launch_lm_plan(L, M, tile_m, b.idx, b.perm, b.tiles, b.n_tiles, b.hist, st));
             mp.tiles = b.tiles; mp.n_tiles = b.n_tiles; mp.max_tiles = lm_max_tiles(M * s.top, s.experts, tile_m); mp.perm = b.perm;
         }
         CR_TRY(stream ? launch_moe_stream(true, mp, st) : launch_moe_tiled(true, mp, st));
@@ -555,7 +557,7 @@ int expert_mixture(cr_ctx* c, const Step& sp, Buffers& b, const LmLayer& L, hipS
         CR_TRY(stream ? launch_moe_stream(false, mp, st) : launch_moe_tiled(false, mp, st));
         return CR_OK;
     }
-    CR_TRY(launch_lm_plan(L, M, LM_TILE_M, b.idx, b.perm, b.tiles, b.n_tiles, st));
+    CR_TRY(launch_lm_plan(L, M, LM_TILE_M, b.idx, b.perm, b.tiles, b.n_tiles, b.hist, st));
     LmGemmParams g{};
     g.A = b.h; g.lda = Wp; g.W = L.wgu; g.ldw = Wp; g.w_bs = (int64_t)2 * L.ffp * Wp; g.C = b.act; g.ldc = L.ffp; g.N = 2 * L.ffp; g.K = Wp;
     g.tiles = b.tiles; g.n_tiles = b.n_tiles; g.max_tiles = lm_max_tiles(M * s.top, s.experts, LM_TILE_M); g.perm = b.perm; g.gather_div = s.top; g.limit = s.limit;

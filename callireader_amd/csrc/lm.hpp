@@ -37,7 +37,7 @@ struct LmLayer {
     // element type of the model (bf16 or float)
     void *wa, *wuq, *wkv, *wukT, *wo, *router, *wgu, *wdn;      // (wgu, wdn: fragment-ordered blocks for bf16, rows for float; dense feed-forward: up and down in rows)
     void *sgate, *sproj;
-    bf16 *wa_dl, *wuq_dl, *wo_dl, *wgu_dl, *wdn_dl, *sgate_dl, *sproj_dl;      // bf16: decode-layout copies for the weight-streaming kernels (gemm_skinny.hip), may be null
+    bf16 *wa_dl, *wuq_dl, *wo_dl, *wgu_dl, *wdn_dl, *sgate_dl, *sproj_dl, *router_dl;      // bf16: decode-layout copies for the weight-streaming kernels (gemm_skinny.hip), may be null
     // fp32: gains (one plus the stored weight for the norms about zero), router correction
     float *n1, *n1b, *n2, *n2b, *nq, *nc, *corr, *ns;
     float *fq_a, *fq_r;        // rotation frequencies of attention and of retention
@@ -139,7 +139,9 @@ int launch_lm_latents(bool f32, const Lm& lm, const LmLayer& L, int M, void* a, 
 // z [slices][M][ldz] fp32 (summed in slice order) -> idx [M][top], wt [M][top]
 int launch_lm_route(const LmLayer& L, int M, const float* z, int64_t ldz, int slices, int32_t* idx, float* wt, hipStream_t st);
 // assignments sorted by expert: perm[pos] = row * top + slot, tiles of at most tile_m positions
-int launch_lm_plan(const LmLayer& L, int M, int tile_m, const int32_t* idx, int32_t* perm, int4* tiles, int32_t* n_tiles, hipStream_t st);
+// hist: lm_plan_ints of scratch
+int launch_lm_plan(const LmLayer& L, int M, int tile_m, const int32_t* idx, int32_t* perm, int4* tiles, int32_t* n_tiles, int32_t* hist, hipStream_t st);
+size_t lm_plan_ints(int M, int top, int experts);
 inline int lm_max_tiles(int rows, int experts, int tile_m) { return rows / tile_m + (experts < rows ? experts : rows); }
 
 // router product + routing in one kernel (bf16): z = h . router^T accumulated in fp32 and kept on the chip

@@ -4,6 +4,7 @@
 namespace {
 
 constexpr int MAX_E = 1024;
+constexpr int LM_PLAN_ONE = 4096;      // assignments one workgroup places by itself
 
 // order of a wave's own LDS accesses (each wave below works in LDS of its own: no workgroup barrier)
 #define WAVE_LDS_FENCE()                                      \
@@ -112,43 +113,66 @@ __global__ __launch_bounds__(256) void lm_route_kernel(const float* __restrict__
 }
 
 // bf16 models: the router product and the routing of 16 tokens in one workgroup of 16 waves.  Wave = a quarter of K x a quarter of the experts (EB blocks of 16); the four K-slices
-// meet in LDS in slice order, then wave w routes token w.
+// meet in LDS in slice order, then wave w routes token w.  Bound by the CU's load path: loaded straight as operands, a fragment is 16 rows x 64 bytes and takes four times its bytes' time,
+// and four waves fetched the same tokens.  So the tokens come once, by LDS-DMA, a contiguous KiB an instruction (16 k-steps of a row and slice; the 16-byte chunks of rows in fours XORed for
+// the reads), the weights from their fragment-ordered copy (wsw; without it row by row as before), and waves past the experts stay idle.  6124 tokens, 2048 x 32: 28 -> 15.8 us.
 template <int EB>
-__global__ __launch_bounds__(1024) void lm_router_kernel(const bf16* __restrict__ h, int64_t ldh, const bf16* __restrict__ Wr, int K, const float* __restrict__ corr, int M, int E, int top,
+__global__ __launch_bounds__(1024) void lm_router_kernel(const bf16* __restrict__ h, int64_t ldh, const bf16* __restrict__ Wr, int wsw, int K, const float* __restrict__ corr, int M, int E, int top,
                                                          int groups, int keep, int32_t* __restrict__ idx, float* __restrict__ wt) {
-    extern __shared__ float sm[];
-    constexpr int ELD = EB * 64 + 4;
+    extern __shared__ __attribute__((aligned(16))) float sm[];
+    constexpr int ELD = EB * 64 + 4, STEPS = 16;
     float* part = sm;                                  // [4][16][ELD]
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15;
+    char* xs = (char*)sm;                              // [slice][token][KiB], until the products are done: two workgroups a CU
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, li = lane & 15;
     const int kq = wave >> 2, eq = wave & 3, m0 = blockIdx.x * 16;
     const int steps = K / 32, per = (steps + 3) / 4, k_lo = min(kq * per, steps), k_hi = min(k_lo + per, steps);
-    const bf16* x = h + (int64_t)min(m0 + li, M - 1) * ldh + g * 8;
+    const bf16* row = h + (int64_t)min(m0 + wave, M - 1) * ldh;
+    const int own = (lane ^ ((wave & 3) << 2)) * 8;    // the lane's column of a KiB of row `wave`
+    const char* x = xs + (kq * 16 + li) * 1024;
     const bf16* w[EB];
+    const int wstep = wsw ? 512 : 32;
 #pragma unroll
-    for (int b = 0; b < EB; b++) w[b] = Wr + (int64_t)min((eq * EB + b) * 16 + li, E - 1) * K + g * 8;
+    for (int b = 0; b < EB; b++) {
+        const int blk = min(eq * EB + b, (E + 15) / 16 - 1);
+        w[b] = wsw ? Wr + (int64_t)blk * (K / 32) * 512 + lane * 8 : Wr + (int64_t)min(blk * 16 + li, E - 1) * K + g * 8;
+    }
     f32x4 acc[EB];
 #pragma unroll
     for (int b = 0; b < EB; b++) acc[b] = f32x4{0.f, 0.f, 0.f, 0.f};
     constexpr int U = EB > 2 ? 2 : 8 / EB;
-    int ks = k_lo;
-    for (; ks + U <= k_hi; ks += U) {
-        bf16x8 xf[U], wf[EB][U];
+    const bool mine = eq * EB * 16 < E;
+    for (int c = 0; c < per; c += STEPS) {
+        if (c) __syncthreads();
 #pragma unroll
-        for (int u = 0; u < U; u++) {
-            xf[u] = *(const bf16x8*)(x + (ks + u) * 32);
+        for (int s = 0; s < 4; s++)
+            __builtin_amdgcn_global_load_lds(CR_GLB(row + min((min(s * per, steps) + c) * 32 + own, K - 8)), CR_LDS(xs + (s * 16 + wave) * 1024), 16, 0, 0);
+        const int n = min(STEPS, k_hi - k_lo - c), k0 = k_lo + c;
+        bf16x8 wf[EB][U];
+        auto load = [&](int ks) {
 #pragma unroll
-            for (int b = 0; b < EB; b++) wf[b][u] = *(const bf16x8*)(w[b] + (ks + u) * 32);
+            for (int u = 0; u < U; u++)
+#pragma unroll
+                for (int b = 0; b < EB; b++)
+                    if (ks + u < n) wf[b][u] = *(const bf16x8*)(w[b] + (int64_t)(k0 + ks + u) * wstep);
+        };
+        if (mine) load(0);
+        __syncthreads();
+        if (!mine) continue;
+        for (int ks = 0; ks < n; ks += U) {
+            if (ks) load(ks);
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                if (ks + u >= n) break;                // (uniform)
+                const bf16x8 xf = *(const bf16x8*)(x + ((((ks + u) * 4 + g) ^ ((li & 3) << 2)) << 4));
+#pragma unroll
+                for (int b = 0; b < EB; b++) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][u], xf, acc[b], 0, 0, 0);
+            }
         }
-#pragma unroll
-        for (int u = 0; u < U; u++)
-#pragma unroll
-            for (int b = 0; b < EB; b++) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[b][u], xf[u], acc[b], 0, 0, 0);
     }
-    for (; ks < k_hi; ks++)
+    __syncthreads();
+    if (mine)
 #pragma unroll
-        for (int b = 0; b < EB; b++) acc[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(*(const bf16x8*)(w[b] + ks * 32), *(const bf16x8*)(x + ks * 32), acc[b], 0, 0, 0);
-#pragma unroll
-    for (int b = 0; b < EB; b++) *(f32x4*)(part + (kq * 16 + li) * ELD + (eq * EB + b) * 16 + 4 * g) = acc[b];      // experts 4 g + 0..3 of the block, token li
+        for (int b = 0; b < EB; b++) *(f32x4*)(part + (kq * 16 + li) * ELD + (eq * EB + b) * 16 + 4 * g) = acc[b];      // experts 4 g + 0..3 of the block, token li
     __syncthreads();
     float* z = part + wave * ELD;                      // slice 0 of token `wave` becomes its sum
     for (int e = lane; e < E; e += 64) z[e] = ((z[e] + part[(16 + wave) * ELD + e]) + part[(32 + wave) * ELD + e]) + part[(48 + wave) * ELD + e];
@@ -189,59 +213,93 @@ __global__ __launch_bounds__(256) void lm_router_slice_kernel(const bf16* __rest
 
 template <int EB>
 int launch_router_t(const Lm& lm, const LmLayer& L, int M, const void* h, int32_t* idx, float* wt, hipStream_t st) {
-    constexpr int LDS = 4 * 16 * (EB * 64 + 4) * 4;
+    constexpr int PART = 4 * 16 * (EB * 64 + 4) * 4, LDS = PART > 64 * 1024 ? PART : 64 * 1024;
     static std::atomic<uint64_t> done{0};
     if (!cr_dyn_lds_once(done, (const void*)lm_router_kernel<EB>, LDS)) return CR_ERR_HIP;
-    hipLaunchKernelGGL(lm_router_kernel<EB>, dim3((M + 15) / 16), dim3(1024), LDS, st, (const bf16*)h, (int64_t)lm.Wp, (const bf16*)L.router, lm.Wp, L.corr, M, L.s.experts, L.s.top, L.s.groups,
-                       L.s.keep, idx, wt);
+    hipLaunchKernelGGL(lm_router_kernel<EB>, dim3((M + 15) / 16), dim3(1024), LDS, st, (const bf16*)h, (int64_t)lm.Wp, L.router_dl ? L.router_dl : (const bf16*)L.router, L.router_dl != nullptr,
+                       lm.Wp, L.corr, M, L.s.experts, L.s.top, L.s.groups, L.s.keep, idx, wt);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }
 
-// One workgroup: counts per expert, their prefix sums, the tile table, then every assignment's place.  The order of an expert's rows is the order its wave-sized chunks of
-// assignments reach the cursor; a row's result does not depend on its place in a tile.
-__global__ __launch_bounds__(1024) void lm_plan_kernel(const int32_t* __restrict__ idx, int n, int E, int tile_m, int32_t* __restrict__ perm, int4* __restrict__ tiles,
-                                                       int32_t* __restrict__ n_tiles, int max_tiles) {
-    __shared__ int cnt[MAX_E], cur[MAX_E], tl[MAX_E];
-    const int tid = threadIdx.x;
-    for (int e = tid; e < MAX_E; e += 1024) cnt[e] = 0;
+// Assignments sorted by expert.  The order of an expert's rows is the order its wave-sized chunks of assignments reach the cursor; a row's result does not depend on its place in a tile.
+// offsets of the experts (exclusive scans of counts and tiles over MAX_E slots) for thread e's expert of c rows; the tile table by the workgroup that `writes`
+__device__ __forceinline__ int plan_offsets(int c, int tile_m, int* cur, int* tl, int4* tiles, int32_t* n_tiles, int max_tiles, bool writes) {
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, t = (c + tile_m - 1) / tile_m;
+    int sc = c, st = t;
+#pragma unroll
+    for (int o = 1; o < 64; o <<= 1) {
+        const int a = __shfl_up(sc, o, 64), b = __shfl_up(st, o, 64);
+        if (lane >= o) { sc += a; st += b; }
+    }
+    if (lane == 63) { cur[wave] = sc; tl[wave] = st; }
     __syncthreads();
-    for (int i0 = tid; i0 < n; i0 += 8192) {
-        int e[8];
-#pragma unroll
-        for (int q = 0; q < 8; q++) e[q] = i0 + 1024 * q < n ? idx[i0 + 1024 * q] : -1;
-#pragma unroll
-        for (int q = 0; q < 8; q++)
-            if (e[q] >= 0) atomicAdd(&cnt[e[q]], 1);
+    int off = sc - c, t0 = st - t;
+    for (int w = 0; w < wave; w++) { off += cur[w]; t0 += tl[w]; }
+    if (writes) {
+        if (tid == MAX_E - 1) *n_tiles = min(t0 + t, max_tiles);
+        for (int k = 0; k < t; k++)
+            if (t0 + k < max_tiles) tiles[t0 + k] = make_int4(tid, off + k * tile_m, min(tile_m, c - k * tile_m), (k & 7) | min(8, t - (k & ~7)) << 4);
     }
     __syncthreads();
-    // inclusive scans over MAX_E slots (positions and tiles)
-    const int c = cnt[tid], t = (c + tile_m - 1) / tile_m;
-    cur[tid] = c; tl[tid] = t;
-    __syncthreads();
-    for (int o = 1; o < MAX_E; o <<= 1) {
-        const int a = tid >= o ? cur[tid - o] : 0, b = tid >= o ? tl[tid - o] : 0;
-        __syncthreads();
-        cur[tid] += a; tl[tid] += b;
-        __syncthreads();
-    }
-    const int off = cur[tid] - c, t0 = tl[tid] - t;
-    if (tid == MAX_E - 1) *n_tiles = min(tl[tid], max_tiles);
-    __syncthreads();
-    cur[tid] = off;
-    for (int k = 0; k < t; k++)
-        if (t0 + k < max_tiles) tiles[t0 + k] = make_int4(tid, off + k * tile_m, min(tile_m, c - k * tile_m), (k & 7) | min(8, t - (k & ~7)) << 4);
-    __syncthreads();
-    for (int i0 = tid; i0 < n; i0 += 8192) {
+    return off;
+}
+// LDS counters of an expert each, over assignments [lo, hi): f(assignment, what the counter held)
+template <typename F> __device__ __forceinline__ void plan_count(const int32_t* idx, int lo, int hi, int* cnt, F f) {
+    for (int i0 = lo + threadIdx.x; i0 < hi; i0 += 8192) {
         int e[8], at[8];
 #pragma unroll
-        for (int q = 0; q < 8; q++) e[q] = i0 + 1024 * q < n ? idx[i0 + 1024 * q] : -1;
+        for (int q = 0; q < 8; q++) e[q] = i0 + 1024 * q < hi ? idx[i0 + 1024 * q] : -1;
 #pragma unroll
-        for (int q = 0; q < 8; q++) at[q] = e[q] >= 0 ? atomicAdd(&cur[e[q]], 1) : 0;
+        for (int q = 0; q < 8; q++) at[q] = e[q] >= 0 ? atomicAdd(&cnt[e[q]], 1) : 0;
 #pragma unroll
         for (int q = 0; q < 8; q++)
-            if (e[q] >= 0) perm[at[q]] = i0 + 1024 * q;
+            if (e[q] >= 0) f(i0 + 1024 * q, at[q]);
     }
+}
+
+// One workgroup for all assignments, as long as they are few
+__global__ __launch_bounds__(1024) void lm_plan_kernel(const int32_t* __restrict__ idx, int n, int E, int tile_m, int32_t* __restrict__ perm, int4* __restrict__ tiles,
+                                                       int32_t* __restrict__ n_tiles, int max_tiles) {
+    __shared__ int cnt[MAX_E], cur[16], tl[16];
+    const int tid = threadIdx.x;
+    cnt[tid] = 0;
+    __syncthreads();
+    plan_count(idx, 0, n, cnt, [](int, int) {});
+    __syncthreads();
+    const int off = plan_offsets(cnt[tid], tile_m, cur, tl, tiles, n_tiles, max_tiles, true);
+    cnt[tid] = off;
+    __syncthreads();
+    plan_count(idx, 0, n, cnt, [&](int i, int at) { perm[at] = i; });
+}
+
+// Many assignments: counting and placing them is bound by one CU's LDS atomics (24 496 of 32 experts: 18.5 us), so PLAN_PARTS workgroups count a part each, and as many place it behind what
+// the parts ahead of it hold.
+constexpr int PLAN_PARTS = 32;
+__global__ __launch_bounds__(1024) void lm_plan_count_kernel(const int32_t* __restrict__ idx, int n, int E, int32_t* __restrict__ hist) {
+    __shared__ int cnt[MAX_E];
+    const int tid = threadIdx.x, per = (n + PLAN_PARTS - 1) / PLAN_PARTS, lo = min((int)blockIdx.x * per, n);
+    cnt[tid] = 0;
+    __syncthreads();
+    plan_count(idx, lo, min(lo + per, n), cnt, [](int, int) {});
+    __syncthreads();
+    if (tid < E) hist[blockIdx.x * E + tid] = cnt[tid];
+}
+__global__ __launch_bounds__(1024) void lm_plan_place_kernel(const int32_t* __restrict__ idx, int n, int E, int tile_m, const int32_t* __restrict__ hist, int32_t* __restrict__ perm,
+                                                             int4* __restrict__ tiles, int32_t* __restrict__ n_tiles, int max_tiles) {
+    __shared__ int cnt[MAX_E], cur[16], tl[16];
+    const int tid = threadIdx.x, per = (n + PLAN_PARTS - 1) / PLAN_PARTS, lo = min((int)blockIdx.x * per, n);
+    int c = 0, ahead = 0;
+    if (tid < E)
+#pragma unroll 8
+        for (int p = 0; p < PLAN_PARTS; p++) {
+            const int v = hist[p * E + tid];
+            c += v;
+            ahead += p < (int)blockIdx.x ? v : 0;
+        }
+    cnt[tid] = plan_offsets(c, tile_m, cur, tl, tiles, n_tiles, max_tiles, blockIdx.x == 0) + ahead;
+    __syncthreads();
+    plan_count(idx, lo, min(lo + per, n), cnt, [&](int i, int at) { perm[at] = i; });
 }
 
 }  // namespace
@@ -275,10 +333,18 @@ int launch_lm_route(const LmLayer& L, int M, const float* z, int64_t ldz, int sl
     return CR_OK;
 }
 
-int launch_lm_plan(const LmLayer& L, int M, int tile_m, const int32_t* idx, int32_t* perm, int4* tiles, int32_t* n_tiles, hipStream_t st) {
+int launch_lm_plan(const LmLayer& L, int M, int tile_m, const int32_t* idx, int32_t* perm, int4* tiles, int32_t* n_tiles, int32_t* hist, hipStream_t st) {
     if (L.s.experts > MAX_E) return cr_fail(CR_ERR_ARG, "routing: %d experts (at most %d)", L.s.experts, MAX_E);
-    const int n = M * L.s.top;
-    hipLaunchKernelGGL(lm_plan_kernel, dim3(1), dim3(1024), 0, st, idx, n, L.s.experts, tile_m, perm, tiles, n_tiles, lm_max_tiles(n, L.s.experts, tile_m));
+    const int n = M * L.s.top, E = L.s.experts, most = lm_max_tiles(n, E, tile_m);
+    if (n <= LM_PLAN_ONE) {
+        hipLaunchKernelGGL(lm_plan_kernel, dim3(1), dim3(1024), 0, st, idx, n, E, tile_m, perm, tiles, n_tiles, most);
+    } else {
+        if (!hist) return cr_fail(CR_ERR_ARG, "routing: %d assignments without a place for their counts", n);
+        hipLaunchKernelGGL(lm_plan_count_kernel, dim3(PLAN_PARTS), dim3(1024), 0, st, idx, n, E, hist);
+        hipLaunchKernelGGL(lm_plan_place_kernel, dim3(PLAN_PARTS), dim3(1024), 0, st, idx, n, E, tile_m, hist, perm, tiles, n_tiles, most);
+    }
     CR_HIP(hipGetLastError());
     return CR_OK;
 }
+
+size_t lm_plan_ints(int M, int top, int experts) { return M * top <= LM_PLAN_ONE ? 0 : (size_t)PLAN_PARTS * experts; }

@@ -1,0 +1,24 @@
+"""Routing of many tokens: the router product through LDS and the fragment-ordered weights, at widths and expert counts that its chunks of 512 columns and blocks of 16 do not divide, and the
+assignments' plan in one workgroup (up to 4096) and in parts (above): against the oracle."""
+import pytest
+import torch
+
+import linasun_cases as LC
+from oracle import linasun as O
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize('width,experts,top,groups,keep,n', [(320, 3, 1, 1, 1, 333), (2304, 40, 2, 5, 3, 700), (1024, 96, 6, 8, 4, 683), (4224, 33, 4, 3, 2, 1025), (512, 200, 5, 10, 4, 1400)])
+def test_many_tokens(width, experts, top, groups, keep, n):
+    from callireader_amd.modeling_decoder import LinasunForCausalLM
+    cfg = LC.config(width, 120, [(LC.mixer(2, 64, 64, 64, 64, 0.15), LC.moe(experts, top, 64, 2.0, (groups, keep)))])
+    w = {k: (6 * v.float()).to(v.dtype) if k.endswith('router') else v for k, v in LC.weights(cfg, 51).items()}      # (choices that rounding does not turn)
+    t = LC.tokens(cfg, n, seed=3)
+    m = LinasunForCausalLM.from_state_dict(w, cfg, dtype=torch.bfloat16, max_tokens=n)
+    z = m.step([('r', t, list(range(n)))]).cpu()
+    m.close()
+    ref = O.forward(w, cfg, t)
+    d = z - ref
+    err = (d - d.mean(-1, keepdim=True)).pow(2).mean(-1).sqrt() / ref.std()
+    assert float(err.median()) < 2e-2 and float((err > 0.1).float().mean()) < 0.02, (float(err.median()), float(err.max()))
