@@ -531,11 +531,12 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
 }
 
 // h -> ye, wt: the rows of every chosen expert and their weights
-int expert_mixture(cr_ctx* c, const Step& sp, Buffers& b, const LmLayer& L, hipStream_t st) {
+int expert_mixture(cr_ctx* c, const Step& sp, Buffers& b, const LmLayer& L, bool routed, hipStream_t st) {
     const Lm& lm = *c->lm;
     const cr_lm_layer& s = L.s;
     const int M = sp.M, Wp = lm.Wp;
-    if (!lm.f32 && lm_router_supported(L)) CR_TRY(launch_lm_router(lm, L, M, b.h, b.idx, b.wt, b.z, st));
+    if (routed) ;
+    else if (!lm.f32 && lm_router_supported(L)) CR_TRY(launch_lm_router(lm, L, M, b.h, b.idx, b.wt, b.z, st));
     else {
         CR_TRY(raw32(c, lm, b.h, L.router, b.z, L.Ep, M, s.experts, Wp, 0.f, st, sp.decode));
         CR_TRY(launch_lm_route(L, M, b.z, L.Ep, 1, b.idx, b.wt, st));
@@ -622,7 +623,9 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
         // the last update of a pass ahead of the token side
         const int end_epi = lm.Sp && lm.f32 ? LM_SIDE : LM_RAW32, end_n = !lm.Sp ? first_n(r + 1) : lm.f32 ? (M <= LM_ROWS_MAX ? lm.Sp : 0) : slices_of(lm, M, lm.Sp, Wp, sp.decode) ? lm.Sp : 0;
         const bf16* end_dl = lm.Sp ? L.sgate_dl : first_dl(r + 1);
-        if (L.s.ff == CR_FF_NONE) CR_TRY(update(y, L.n1b, false, end, end_epi, end_n, end_dl));
+        const bool routed = L.s.ff == CR_FF_MOE && sp.decode && M <= 64 && lm_post_route_supported(lm, L);      // (by the layer and 64 rows, as the slices)
+        if (routed) CR_TRY(launch_lm_post_route(lm, L, LmAhead{y.Y, y.slices, 0, b.x, b.x, L.n1b, L.n2, M, Wp, lm.d.width, lm.d.eps}, b.h, b.idx, b.wt, st));
+        else if (L.s.ff == CR_FF_NONE) CR_TRY(update(y, L.n1b, false, end, end_epi, end_n, end_dl));
         else CR_TRY(update(y, L.n1b, false, LmSink{b.h, Wp, L.n2}, LM_RELU2, L.s.ff == CR_FF_DENSE && M <= LM_ROWS_MAX ? L.ffp : 0, L.wgu_dl));
         if (L.s.ff == CR_FF_DENSE) {
             if (b.ahead.Y) CR_TRY(behind(lm, b, LM_RELU2, L.wgu, L.wgu_dl, b.act, L.ffp, nullptr, 0, st));
@@ -630,7 +633,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
             CR_TRY(project(b.act, L.wdn, L.wdn_dl, L.ffp, y));
             CR_TRY(update(y, L.n2b, false, end, end_epi, end_n, end_dl));
         } else if (L.s.ff == CR_FF_MOE) {
-            CR_TRY(expert_mixture(c, sp, b, L, st));
+            CR_TRY(expert_mixture(c, sp, b, L, routed, st));
             CR_TRY(launch_lm_post(lm.f32, lm, M, LmPostIn{b.ye, Wp, 0, b.wt, L.s.top}, b.x, L.n2b, false, end, st));
         }
         if (lm.Sp) {

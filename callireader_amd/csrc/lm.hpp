@@ -147,6 +147,9 @@ inline int lm_max_tiles(int rows, int experts, int tile_m) { return rows / tile_
 // router product + routing in one kernel (bf16): z = h . router^T accumulated in fp32 and kept on the chip
 bool lm_router_supported(const LmLayer& L);
 int launch_lm_router(const Lm& lm, const LmLayer& L, int M, const void* h, int32_t* idx, float* wt, float* part, hipStream_t st);
+// decode rows: the residual update, h = rms(x) * gain and the routing in one launch (x_out may be x)
+bool lm_post_route_supported(const Lm& lm, const LmLayer& L);
+int launch_lm_post_route(const Lm& lm, const LmLayer& L, const LmAhead& a, void* h, int32_t* idx, float* wt, hipStream_t st);
 constexpr int LM_ROUTER_SLICES = 16;          // few rows: K-slices of the router product in `part` [slices][M][Ep], summed by the routing kernel
 
 // ---- expert products in bf16 (moe_gemm.hip) ----

@@ -1,5 +1,5 @@
 // Expert routing: scores, grouped choice, and the assignments sorted by expert for the grouped products.
-#include "lm.hpp"
+#include "lm_ahead.hpp"
 
 namespace {
 
@@ -211,6 +211,48 @@ __global__ __launch_bounds__(256) void lm_router_slice_kernel(const bf16* __rest
     }
 }
 
+// Decode: a row's residual update, its router scores and its choice in one workgroup of eight waves, where those were three launches (24 rows, 2048 x 32: 4.6 + 3.4 + 4.8 us).  A wave scores
+// its share of the experts, 512 columns a load instruction, the first POST_EXPERTS of them asked for ahead of the update.
+constexpr int POST_EXPERTS = 4, POST_COLS = 2048;
+__global__ __launch_bounds__(512) void lm_post_route_kernel(const LmAhead a, bf16* __restrict__ h, const bf16* __restrict__ Wr, const float* __restrict__ corr, int E, int top, int groups, int keep,
+                                                            int32_t* __restrict__ idx, float* __restrict__ wt) {
+    constexpr int NC = POST_COLS / 512;
+    __shared__ __attribute__((aligned(16))) bf16 hs[POST_COLS];
+    __shared__ float sums[AHEAD_SEGS], z[64], ch[64], gs[64];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = blockIdx.x, K = a.Wp, per = (E + 7) / 8, e_hi = min(wave * per + per, E);
+    bf16x8 w[POST_EXPERTS][NC];
+    auto load = [&](int e0) {
+#pragma unroll
+        for (int j = 0; j < POST_EXPERTS; j++)
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+                if (e0 + j < e_hi) w[j][c] = *(const bf16x8*)(Wr + (int64_t)(e0 + j) * K + min(c * 512 + lane * 8, K - 8));
+    };
+    load(wave * per);
+    __builtin_amdgcn_sched_barrier(0);
+    update_rows<bf16>(a, row, 1, hs, K, sums, true);
+    bf16x8 x[NC];
+#pragma unroll
+    for (int c = 0; c < NC; c++) x[c] = c * 512 + lane * 8 < K ? *(const bf16x8*)(hs + c * 512 + lane * 8) : bf16x8{};
+    if (wave < NC && wave * 512 + lane * 8 < K) *(bf16x8*)(h + (int64_t)row * K + wave * 512 + lane * 8) = *(const bf16x8*)(hs + wave * 512 + lane * 8);
+    for (int e0 = wave * per; e0 < e_hi; e0 += POST_EXPERTS) {
+        if (e0 != wave * per) load(e0);
+#pragma unroll
+        for (int j = 0; j < POST_EXPERTS; j++) {
+            if (e0 + j >= e_hi) break;                         // (uniform)
+            float s = 0.f;
+#pragma unroll
+            for (int c = 0; c < NC; c++)
+#pragma unroll
+                for (int q = 0; q < 8; q++) s = fmaf((float)w[j][c][q], (float)x[c][q], s);
+            s = wave_sum_s(s);
+            if (lane == 0) z[e0 + j] = s;
+        }
+    }
+    __syncthreads();
+    if (wave == 0) route_row<1>(z, ch, gs, corr, E, top, groups, keep, lane, true, idx + (int64_t)row * top, wt + (int64_t)row * top);
+}
+
 template <int EB>
 int launch_router_t(const Lm& lm, const LmLayer& L, int M, const void* h, int32_t* idx, float* wt, hipStream_t st) {
     constexpr int PART = 4 * 16 * (EB * 64 + 4) * 4, LDS = PART > 64 * 1024 ? PART : 64 * 1024;
@@ -303,6 +345,16 @@ __global__ __launch_bounds__(1024) void lm_plan_place_kernel(const int32_t* __re
 }
 
 }  // namespace
+
+// a row's workgroup reads the whole router from L2: 256 KiB of it are about the time of the launches it saves
+bool lm_post_route_supported(const Lm& lm, const LmLayer& L) { return !lm.f32 && lm.Wp <= POST_COLS && lm.Wp % 64 == 0 && L.s.experts <= 64; }
+
+int launch_lm_post_route(const Lm& lm, const LmLayer& L, const LmAhead& a, void* h, int32_t* idx, float* wt, hipStream_t st) {
+    if (a.M <= 0 || !a.Y || !a.x || !a.x_out || !h || !idx || !wt || a.Wp != lm.Wp || !lm_post_route_supported(lm, L)) return cr_fail(CR_ERR_ARG, "update and routing: %d rows, %d experts", a.M, L.s.experts);
+    hipLaunchKernelGGL(lm_post_route_kernel, dim3(a.M), dim3(512), 0, st, a, (bf16*)h, (const bf16*)L.router, L.corr, L.s.experts, L.s.top, L.s.groups, L.s.keep, idx, wt);
+    CR_HIP(hipGetLastError());
+    return CR_OK;
+}
 
 bool lm_router_supported(const LmLayer& L) { return L.s.experts <= 256; }
 
