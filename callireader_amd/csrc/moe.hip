@@ -211,46 +211,61 @@ __global__ __launch_bounds__(256) void lm_router_slice_kernel(const bf16* __rest
     }
 }
 
-// Decode: a row's residual update, its router scores and its choice in one workgroup of eight waves, where those were three launches (24 rows, 2048 x 32: 4.6 + 3.4 + 4.8 us).  A wave scores
-// its share of the experts, 512 columns a load instruction, the first POST_EXPERTS of them asked for ahead of the update.
-constexpr int POST_EXPERTS = 4, POST_COLS = 2048;
-__global__ __launch_bounds__(512) void lm_post_route_kernel(const LmAhead a, bf16* __restrict__ h, const bf16* __restrict__ Wr, const float* __restrict__ corr, int E, int top, int groups, int keep,
-                                                            int32_t* __restrict__ idx, float* __restrict__ wt) {
-    constexpr int NC = POST_COLS / 512;
+// Decode: a row's residual update, its router scores and its choice in one workgroup of eight waves, where those were three launches (24 rows, 2048 x 32: 4.6 + 3.4 + 4.8 us and two gaps -> 8.9).  Scores are
+// the ones lm_router_slice_kernel and lm_route_kernel form, bit for bit -- the same K-slices on the matrix cores, added in slice order: a choice between close experts must not hang on the
+// path.  A wave takes every eighth slice of all experts; the weights of its first 32 experts (fragment-ordered with wsw) are asked for ahead of the update.
+constexpr int POST_COLS = 2048, POST_E = 64;
+__global__ __launch_bounds__(512) void lm_post_route_kernel(const LmAhead a, bf16* __restrict__ h, const bf16* __restrict__ Wr, int wsw, const float* __restrict__ corr, int E, int top, int groups,
+                                                            int keep, int32_t* __restrict__ idx, float* __restrict__ wt) {
+    constexpr int SL = LM_ROUTER_SLICES / 8, MAX_PER = POST_COLS / 32 / LM_ROUTER_SLICES, PAIR = 2;      // slices a wave, k-steps a slice, blocks of 16 experts a batch
     __shared__ __attribute__((aligned(16))) bf16 hs[POST_COLS];
-    __shared__ float sums[AHEAD_SEGS], z[64], ch[64], gs[64];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = blockIdx.x, K = a.Wp, per = (E + 7) / 8, e_hi = min(wave * per + per, E);
-    bf16x8 w[POST_EXPERTS][NC];
-    auto load = [&](int e0) {
+    __shared__ __attribute__((aligned(16))) float part[LM_ROUTER_SLICES][POST_E];
+    __shared__ float sums[AHEAD_SEGS], z[POST_E], ch[POST_E], gs[POST_E];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), row = blockIdx.x, K = a.Wp, g = lane >> 4, li = lane & 15;
+    const int steps = K / 32, per = (steps + LM_ROUTER_SLICES - 1) / LM_ROUTER_SLICES, blocks = (E + 15) / 16;
+    bf16x8 w[PAIR][SL][MAX_PER];
+    auto load = [&](int b0) {
 #pragma unroll
-        for (int j = 0; j < POST_EXPERTS; j++)
+        for (int j = 0; j < PAIR; j++) {
+            const int b = min(b0 + j, blocks - 1);
+            const bf16* p = wsw ? Wr + (int64_t)b * steps * 512 + lane * 8 : Wr + (int64_t)min(b * 16 + li, E - 1) * K + g * 8;
 #pragma unroll
-            for (int c = 0; c < NC; c++)
-                if (e0 + j < e_hi) w[j][c] = *(const bf16x8*)(Wr + (int64_t)(e0 + j) * K + min(c * 512 + lane * 8, K - 8));
+            for (int s = 0; s < SL; s++)
+#pragma unroll
+                for (int u = 0; u < MAX_PER; u++)
+                    if (u < per) w[j][s][u] = *(const bf16x8*)(p + (int64_t)min((wave + 8 * s) * per + u, steps - 1) * (wsw ? 512 : 32));
+        }
     };
-    load(wave * per);
+    load(0);
     __builtin_amdgcn_sched_barrier(0);
     update_rows<bf16>(a, row, 1, hs, K, sums, true);
-    bf16x8 x[NC];
+    if (wave * 512 + lane * 8 < K) *(bf16x8*)(h + (int64_t)row * K + wave * 512 + lane * 8) = *(const bf16x8*)(hs + wave * 512 + lane * 8);
+    for (int b0 = 0; b0 < blocks; b0 += PAIR) {
+        if (b0) load(b0);
 #pragma unroll
-    for (int c = 0; c < NC; c++) x[c] = c * 512 + lane * 8 < K ? *(const bf16x8*)(hs + c * 512 + lane * 8) : bf16x8{};
-    if (wave < NC && wave * 512 + lane * 8 < K) *(bf16x8*)(h + (int64_t)row * K + wave * 512 + lane * 8) = *(const bf16x8*)(hs + wave * 512 + lane * 8);
-    for (int e0 = wave * per; e0 < e_hi; e0 += POST_EXPERTS) {
-        if (e0 != wave * per) load(e0);
+        for (int j = 0; j < PAIR; j++)
 #pragma unroll
-        for (int j = 0; j < POST_EXPERTS; j++) {
-            if (e0 + j >= e_hi) break;                         // (uniform)
-            float s = 0.f;
+            for (int s = 0; s < SL; s++) {
+                const int k_lo = min((wave + 8 * s) * per, steps), k_hi = min(k_lo + per, steps);
+                f32x4 acc = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-            for (int c = 0; c < NC; c++)
-#pragma unroll
-                for (int q = 0; q < 8; q++) s = fmaf((float)w[j][c][q], (float)x[c][q], s);
-            s = wave_sum_s(s);
-            if (lane == 0) z[e0 + j] = s;
-        }
+                for (int u = 0; u < MAX_PER; u++) {
+                    if (k_lo + u >= k_hi) break;               // (uniform)
+                    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j][s][u], *(const bf16x8*)(hs + (k_lo + u) * 32 + g * 8), acc, 0, 0, 0);
+                }
+                if (li == 0 && b0 + j < blocks) *(f32x4*)(&part[wave + 8 * s][(b0 + j) * 16 + 4 * g]) = acc;      // (every column is the row)
+            }
     }
     __syncthreads();
-    if (wave == 0) route_row<1>(z, ch, gs, corr, E, top, groups, keep, lane, true, idx + (int64_t)row * top, wt + (int64_t)row * top);
+    if (wave) return;
+    if (lane < E) {
+        float v = 0.f;
+#pragma unroll
+        for (int s = 0; s < LM_ROUTER_SLICES; s++) v += part[s][lane];
+        z[lane] = v;
+    }
+    WAVE_LDS_FENCE();
+    route_row<1>(z, ch, gs, corr, E, top, groups, keep, lane, true, idx + (int64_t)row * top, wt + (int64_t)row * top);
 }
 
 template <int EB>
@@ -347,11 +362,12 @@ __global__ __launch_bounds__(1024) void lm_plan_place_kernel(const int32_t* __re
 }  // namespace
 
 // a row's workgroup reads the whole router from L2: 256 KiB of it are about the time of the launches it saves
-bool lm_post_route_supported(const Lm& lm, const LmLayer& L) { return !lm.f32 && lm.Wp <= POST_COLS && lm.Wp % 64 == 0 && L.s.experts <= 64; }
+bool lm_post_route_supported(const Lm& lm, const LmLayer& L) { return !lm.f32 && lm.Wp <= POST_COLS && lm.Wp % 64 == 0 && L.s.experts <= POST_E; }
 
 int launch_lm_post_route(const Lm& lm, const LmLayer& L, const LmAhead& a, void* h, int32_t* idx, float* wt, hipStream_t st) {
     if (a.M <= 0 || !a.Y || !a.x || !a.x_out || !h || !idx || !wt || a.Wp != lm.Wp || !lm_post_route_supported(lm, L)) return cr_fail(CR_ERR_ARG, "update and routing: %d rows, %d experts", a.M, L.s.experts);
-    hipLaunchKernelGGL(lm_post_route_kernel, dim3(a.M), dim3(512), 0, st, a, (bf16*)h, (const bf16*)L.router, L.corr, L.s.experts, L.s.top, L.s.groups, L.s.keep, idx, wt);
+    hipLaunchKernelGGL(lm_post_route_kernel, dim3(a.M), dim3(512), 0, st, a, (bf16*)h, L.router_dl ? L.router_dl : (const bf16*)L.router, L.router_dl != nullptr,
+                       L.corr, L.s.experts, L.s.top, L.s.groups, L.s.keep, idx, wt);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }

@@ -22,3 +22,21 @@ def test_many_tokens(width, experts, top, groups, keep, n):
     d = z - ref
     err = (d - d.mean(-1, keepdim=True)).pow(2).mean(-1).sqrt() / ref.std()
     assert float(err.median()) < 2e-2 and float((err > 0.1).float().mean()) < 0.02, (float(err.median()), float(err.max()))
+
+
+@pytest.mark.parametrize('width,experts,top,groups,keep', [(64, 3, 1, 1, 1), (320, 17, 2, 1, 1), (1088, 33, 3, 3, 2), (2048, 64, 4, 8, 4)])
+def test_decoded_rows(width, experts, top, groups, keep):
+    """Decoded rows: update, scores and choice in one launch, at widths that the sixteen K-slices and expert counts that the blocks of 16 do not divide."""
+    from callireader_amd.modeling_decoder import LinasunForCausalLM
+    cfg = LC.config(width, 120, [(LC.mixer(2, 64, 64, 64, 64, 0.15), LC.moe(experts, top, 64, 2.0, (groups, keep)))])
+    w = {k: (6 * v.float()).to(v.dtype) if k.endswith('router') else v for k, v in LC.weights(cfg, 53).items()}
+    rows, n, new = 7, 12, 6
+    t = [LC.tokens(cfg, n + new, seed=20 + r) for r in range(rows)]
+    m = LinasunForCausalLM.from_state_dict(w, cfg, dtype=torch.bfloat16, max_tokens=64)
+    m.step([(r, t[r][:n], []) for r in range(rows)])
+    z = torch.stack([m.step([(r, [t[r][n + i]], [0]) for r in range(rows)]).cpu() for i in range(new)], 1)
+    m.close()
+    ref = torch.stack([O.forward(w, cfg, t[r])[n:] for r in range(rows)])
+    d = z - ref
+    err = (d - d.mean(-1, keepdim=True)).pow(2).mean(-1).sqrt() / ref.std()
+    assert float(err.median()) < 2e-2 and float((err > 0.1).float().mean()) < 0.05, (float(err.median()), float(err.max()))      # (at most two of 42 rows: a turned choice)
