@@ -47,18 +47,21 @@ struct HeadLane {
     }
     // sx: the lane's eight places in the wave's own 512 floats of LDS, through which partners are read.  Every lane of the wave calls it.
     __device__ __forceinline__ void apply(int P, int dim, float eps, float* sx, float (&v)[8]) const {
-        float ss = 0.f;
+        if (__builtin_amdgcn_ballot_w64(normed)) {              // (a head's lanes agree)
+            float ss = 0.f;
 #pragma unroll
-        for (int e = 0; e < 8; e++) ss += v[e] * v[e];
-        ss += dpp<0xB1>(ss); ss += dpp<0x4E>(ss); ss += dpp<0x141>(ss);      // lanes of eight; sixteen; half the wave; the wave
-        if (P > 64) { const float o = dpp<0x128>(ss); ss += o; }
-        if (P > 128) { const float o = __shfl_xor(ss, 16, 64); ss += o; }
-        if (P > 256) { const float o = __shfl_xor(ss, 32, 64); ss += o; }
-        if (normed) {
-            const float rs = 1.0f / sqrtf(ss / (float)dim + eps);
+            for (int e = 0; e < 8; e++) ss += v[e] * v[e];
+            ss += dpp<0xB1>(ss); ss += dpp<0x4E>(ss); ss += dpp<0x141>(ss);      // lanes of eight; sixteen; half the wave; the wave
+            if (P > 64) { const float o = dpp<0x128>(ss); ss += o; }
+            if (P > 128) { const float o = __shfl_xor(ss, 16, 64); ss += o; }
+            if (P > 256) { const float o = __shfl_xor(ss, 32, 64); ss += o; }
+            if (normed) {
+                const float rs = 1.0f / sqrtf(ss / (float)dim + eps);
 #pragma unroll
-            for (int e = 0; e < 8; e++) v[e] *= rs * g[e];
+                for (int e = 0; e < 8; e++) v[e] *= rs * g[e];
+            }
         }
+        if (!__builtin_amdgcn_ballot_w64(e0 < 2 * half)) return;
         st8(sx, v);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
