@@ -80,7 +80,8 @@ __global__ __launch_bounds__(512) void ahead_rows_kernel(const LmAhead a, const 
     const char* frag = ring + (lane & 15) * 64 + ((lane >> 4) ^ (((lane & 15) >> 3) << 1)) * 16;
     auto load = [&](int s) {
 #pragma unroll
-        for (int u = 0; u < U; u++) __builtin_amdgcn_global_load_lds(CR_GLB(w + min(s + u, s1 - 1) * 16), CR_LDS(ring + u * 1024), 16, 0, 0);
+        for (int u = 0; u < U; u++)
+            if (s + u < s1) __builtin_amdgcn_global_load_lds(CR_GLB(w + (s + u) * 16), CR_LDS(ring + u * 1024), 16, 0, 0);
     };
     if (s0 < s1) load(s0);
     update_rows<float>(a, 0, a.M, hf, K + 4, sums, blockIdx.x == 0 && blockIdx.y == 0);
