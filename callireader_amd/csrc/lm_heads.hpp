@@ -65,19 +65,20 @@ struct HeadLane {
         st8(sx, v);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
+        // (which product is rounded alone is spelled out: left to the compiler, entry 0 of every eight had the other one where half % 8 != 0)
         if (e0 < 2 * half) {
             if (half % 8 == 0) {
                 const bool first = e0 < half;
                 float u[8];
                 ld8<float>(sx + (first ? half : -half), u);
 #pragma unroll
-                for (int e = 0; e < 8; e++) v[e] = first ? v[e] * c[e] - u[e] * s[e] : v[e] * c[e] + u[e] * s[e];
+                for (int e = 0; e < 8; e++) v[e] = fmaf(v[e], c[e], first ? -(u[e] * s[e]) : u[e] * s[e]);
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
                     const int q = e0 + e;
-                    if (q < half) v[e] = v[e] * c[e] - sx[e + half] * s[e];
-                    else if (q < 2 * half) v[e] = v[e] * c[e] + sx[e - half] * s[e];
+                    if (q < half) v[e] = fmaf(v[e], c[e], -(sx[e + half] * s[e]));
+                    else if (q < 2 * half) v[e] = fmaf(v[e], c[e], sx[e - half] * s[e]);
                 }
             }
         }
