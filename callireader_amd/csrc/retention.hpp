@@ -49,7 +49,10 @@ template <int NR> struct RetStep {
 #pragma unroll
                 for (int e = 0; e < 4; e++) {
                     if (fresh) s[r + e] = f32x4{0.f, 0.f, 0.f, 0.f};              // a state starts at zero, whatever the slot held before
-                    s[r + e] = s[r + e] * decay + kv[e] * v;
+                    // the fused product is spelled out: states of 64 keys as a prompt's recurrence has it (ret_recurrent_kernel), larger ones the other way round, so that neither moves with
+                    // what the compiler finds around it
+                    if (NR == 4) s[r + e] = __builtin_elementwise_fma(f32x4{kv[e], kv[e], kv[e], kv[e]}, v, s[r + e] * decay);
+                    else s[r + e] = __builtin_elementwise_fma(s[r + e], f32x4{decay, decay, decay, decay}, kv[e] * v);
                     o += s[r + e] * qv[e];
                     __builtin_nontemporal_store(s[r + e], (f32x4*)(st + ((int64_t)b * NR + r + e) * 256));
                 }

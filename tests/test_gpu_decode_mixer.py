@@ -65,3 +65,22 @@ def test_residual_updates_inside_the_next_product(width, dtype):
     for which in ([0], [3], [0, 1], [4, 5, 6, 7], range(8)):
         assert torch.equal(run(which), together[list(which)]), which
     m.close()
+
+
+@pytest.mark.parametrize('dim', [16, 64])
+def test_decoded_state_steps_as_prompts_do(dim):
+    """float32, states of up to 64 keys: a decoded token moves its state as a prompt's token does, decay times state rounded ahead of the fused k v.  With one live value column the outputs' norms are
+    the same sums too, so decoded logits have the bits of the prompt that holds their tokens."""
+    from callireader_amd.modeling_decoder import LugasunForCausalLM
+    cfg = LC.config(128, 90, [LC.layer(LC.heads(1, 1, 64, 64, 64), LC.ret(dim, 16, (0.9, 0.97, 0.999)), None, (0.0, 0.8))], side=8)
+    w = LC.weights(cfg, 43)
+    v = w['l0.mix.right.v'].view(3, 16, 128)
+    v[:, 1:] = 0
+    m = LugasunForCausalLM.from_state_dict(w, cfg, dtype=torch.float32, max_tokens=64, max_seqs=2)
+    t = LC.tokens(cfg, 60, seed=9)
+    whole = m.step([('prompt', t, list(range(40, 60)))])
+    m.step([('row', t[:40], [])])
+    rows = torch.cat([m.step([('row', [x], [0])]) for x in t[40:]])
+    torch.cuda.synchronize()
+    assert torch.equal(rows, whole), float((rows - whole).abs().max())
+    m.close()
