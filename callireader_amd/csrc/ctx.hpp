@@ -40,6 +40,7 @@ struct cr_ctx {
     bool no_sliced_decode = false;      // CR_NO_SLICED_DECODE=1: decode through the one-tile weight-streaming GEMMs (A/B aid)
     bool perceiver_v1 = false;          // CR_PERCEIVER_ATTN_V1=1 at cr_create: round 1's perceiver attention kernel (the bit-for-bit yardstick of the current one)
     bool fold_rope = true;              // 9..64-row decode: RoPE + split + the new token's cache row inside the attention kernel (attention_decode.hip FOLD; bit-identical); CR_DECODE_FOLD_ROPE=0 at cr_create: rope_split_kernel as its own launch
+    bool joined_decode = true;          // decode steps of described decoders: mixer, residual update + product, residual update + routing as one launch each where sizes allow (the same bits); CR_DECODE_JOINED=0 at cr_create: the separate kernels
     std::unordered_map<std::string, DevTensor> w;
     std::shared_ptr<Lm> lm;             // cr_lm_configure: the language model of this context is a described decoder
     // workspace

@@ -472,7 +472,7 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
     char *ck = kv->lat + kv->lat_off[r], *cv = ck + (size_t)kv->n_seqs * a.kv_heads * ring * L.Ap * es;
     float* state = (float*)(kv->lat + kv->state_off[r]);
     // by the layer's sizes alone (and 64 rows, where slices end): a row's bits do not depend on the rows it is decoded with
-    if (s_a && lm_mix_supported(lm.f32, L)) {
+    if (s_a && c->joined_decode && lm_mix_supported(lm.f32, L)) {
         LmMixIn in{};
         in.M = M; in.part = b.sl; in.slices = s_a; in.where = b.where; in.ang = b.ang; in.ao = b.ao; in.cache_k = ck; in.cache_v = cv; in.ring = ring; in.chunk = chunk; in.rows = in.nsplit = 1;
         in.state = state;
@@ -594,7 +594,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
     };
     // x += ..., then the sink: left to the product behind it where few rows allow it (N columns; 0: no product reads this sink next)
     auto update = [&](const LmPostIn& y, const float* gain_b, bool replace, const LmSink& to, int epi, int N, const bf16* dl) -> int {
-        if (!N || !sp.decode || y.top || !lm_ahead_supported(lm.f32, M, Wp, N, epi, dl != nullptr)) return launch_lm_post(lm.f32, lm, M, y, b.x, gain_b, replace, to, st);
+        if (!N || !sp.decode || !c->joined_decode || y.top || !lm_ahead_supported(lm.f32, M, Wp, N, epi, dl != nullptr)) return launch_lm_post(lm.f32, lm, M, y, b.x, gain_b, replace, to, st);
         b.ahead = LmAhead{y.Y, y.slices, replace, b.x, b.x2, gain_b, to.gain, M, Wp, lm.d.width, lm.d.eps};
         return CR_OK;
     };
@@ -623,7 +623,7 @@ int run_passes(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, void* last, hip
         // the last update of a pass ahead of the token side
         const int end_epi = lm.Sp && lm.f32 ? LM_SIDE : LM_RAW32, end_n = !lm.Sp ? first_n(r + 1) : lm.f32 ? (M <= LM_ROWS_MAX ? lm.Sp : 0) : slices_of(lm, M, lm.Sp, Wp, sp.decode) ? lm.Sp : 0;
         const bf16* end_dl = lm.Sp ? L.sgate_dl : first_dl(r + 1);
-        const bool routed = L.s.ff == CR_FF_MOE && sp.decode && M <= 64 && lm_post_route_supported(lm, L);      // (by the layer and 64 rows, as the slices)
+        const bool routed = L.s.ff == CR_FF_MOE && sp.decode && c->joined_decode && M <= 64 && lm_post_route_supported(lm, L);      // (by the layer and 64 rows, as the slices)
         if (routed) CR_TRY(launch_lm_post_route(lm, L, LmAhead{y.Y, y.slices, 0, b.x, b.x, L.n1b, L.n2, M, Wp, lm.d.width, lm.d.eps}, b.h, b.idx, b.wt, st));
         else if (L.s.ff == CR_FF_NONE) CR_TRY(update(y, L.n1b, false, end, end_epi, end_n, end_dl));
         else CR_TRY(update(y, L.n1b, false, LmSink{b.h, Wp, L.n2}, LM_RELU2, L.s.ff == CR_FF_DENSE && M <= LM_ROWS_MAX ? L.ffp : 0, L.wgu_dl));

@@ -5,9 +5,10 @@
 // Bound by latency: with few rows none of it fills the chip, so the chain from the slices to the result is what counts.
 //
 // Attention in bf16 (heads of 64 or 128, any number of keys): a wave forms the scores of 32 of the split's 256 keys, which go from the cache straight into its registers as the A operand;
-// the values come by LDS-DMA.  Raw scores of a query lie in LDS before its softmax starts, so a wave takes a whole query (four keys a lane, one reference point, no running maximum) instead of
-// an accumulator's 32 query places of which a group fills a few.  Weights go through LDS as the P.V product's fragments (two bf16 terms, as in attention.hip), a wave of the first D / 32 takes
-// 32 value columns.  The token's own key and value never come from memory: they replace the stale row in the registers and in LDS.  Attention in fp32: attention_plain.hpp on the token's
+// the values come by LDS-DMA.  Scores of a query lie in LDS before its softmax starts, so a wave takes a whole query (four keys a lane) instead of an accumulator's 32 query places of which a
+// group fills a few.  Weights go through LDS as the P.V product's fragments (two bf16 terms, as in attention.hip), a wave of the first D / 32 takes 32 value columns.
+// The arithmetic is flash_attn_kernel's over the split's tiles of 64 keys (attention.hip, SPLIT with WIDE), bit for bit: its running reference point, which a vote over the unit's queries moves, its
+// rescaling, its order of sums (one row of 8 heads of 128 on 2, 49 .. 80 keys: 7.2 us; with one reference point a split and sums across the wave 7.0, and other bits).  The token's own key and value never come from memory: they replace the stale row in the registers and in LDS.  Attention in fp32: attention_plain.hpp on the token's
 // freshly written cache row, which every workgroup of a group of query heads writes for itself -- the same bits.
 #include "attention_merge.hpp"
 #include "attention_plain.hpp"
@@ -23,6 +24,8 @@ __device__ __forceinline__ unsigned pack_bf16x2(float a, float b) {
 }
 
 constexpr int MIX_THREADS16 = 512, MIX_THREADS32 = 1024, MIX_SC = 260;      // floats between the queries of a split's scores: 256 keys, the rows four banks apart
+constexpr int MIX_TILES = 4;                     // tiles of 64 keys a split: eight waves of 32 keys
+static_assert(MIX_TILES == ATTN_SPLIT_TILES, "the caller counts splits of ATTN_SPLIT_TILES tiles (lm.hip: HEADS_SPLIT)");
 
 struct MixArgs {
     const float* part; const int2* where; const float* ang; void* ao;      // K-slices; {sequence, position} and angles of every row
@@ -84,8 +87,8 @@ struct Columns {
     }
 };
 
-// bytes: value tiles, weights, scores (before them, in the same place, the waves' columns), queries, own key and value, sums and maxima
-template <int D> constexpr int mix_lds16(int rows) { return 4 * 64 * D * 2 + 1024 * rows + MIX_SC * 4 * rows + (rows + 2) * D * 2 + 256; }
+// bytes: value tiles, weights, scores (before them, in the same place, the waves' columns), queries, own key and value, maxima of the tiles
+template <int D> constexpr int mix_lds16(int rows) { return MIX_TILES * 64 * D * 2 + 1024 * rows + MIX_SC * 4 * rows + (rows + 2) * D * 2 + MIX_TILES * 32 * 4; }
 
 template <int D>
 __device__ __forceinline__ void mix_attend16(const MixArgs& p, int u, int row, char* smem) {
@@ -93,10 +96,10 @@ __device__ __forceinline__ void mix_attend16(const MixArgs& p, int u, int row, c
     constexpr float LOG2E = 1.4426950408889634f;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l31 = lane & 31, hh = lane >> 5;
     const int unit = u / p.nsplit, split = u - unit * p.nsplit, g = unit / p.kv_group, R = p.R, heads = R + 2;
-    char *vt = smem, *pt = vt + 4 * TILE;                      // [4][64][D] bf16, chunks swizzled; [32-key block][16-key step][term][half wave][query] x 16 bytes
+    char *vt = smem, *pt = vt + MIX_TILES * TILE;              // [tile][64][D] bf16, chunks swizzled; [32-key block][16-key step][term][half wave][query] x 16 bytes
     float* sc = (float*)(pt + 1024 * R);                       // [R][MIX_SC]
     bf16 *q = (bf16*)(sc + MIX_SC * R), *nk = q + R * D, *nv = nk + D;
-    float *mx = (float*)(nv + D), *ls = mx + 32, *sx = (float*)pt;      // [R], [R]; [wave][512]: (R + 2) * D floats in whole waves, at most 4096
+    float *mx = (float*)(nv + D), *sx = (float*)pt;      // [tile][32 queries]; [wave][512]: (R + 2) * D floats in whole waves, at most 4096
 
     // the unit's query heads, its key and its value: D / 8 lanes each
     const int e0 = (lane % CPR) * 8;
@@ -161,28 +164,55 @@ __device__ __forceinline__ void mix_attend16(const MixArgs& p, int u, int row, c
 #pragma unroll
             for (int i = 0; i < 4; i++) *(f32x4*)(sc + l31 * MIX_SC + r0 + 8 * i + 4 * hh) = f32x4{s[4 * i], s[4 * i + 1], s[4 * i + 2], s[4 * i + 3]};
     }
-    if (r0 < 64 * tiles && key0 + r0 + 32 >= n) {
-        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-        // the token's own value, also over what lies behind it (its weights are zero, but the rows hold anything)
-        for (int r = max(r0, n - 1 - key0) + lane / CPR; r < r0 + 32; r += RPI)
-            *(bf16x8*)(vt + r * ROWB + (((lane % CPR) ^ attn_vswz<D>(r)) * 16)) = *(const bf16x8*)(nv + e0);
-    }
-    __syncthreads();
-    for (int i = wave; i < R; i += 8) {
-        const f32x4 x = *(const f32x4*)(sc + i * MIX_SC + 4 * lane);
-        f32x4 z;
+    lds_barrier();
+    // a wave's queries, every eighth: four scores a lane, sixteen lanes a tile
+    const bool capped = p.softcap > 0.f;
+    f32x4 z[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) {
-            // softcap * tanh(z / softcap) = softcap - 2 softcap / (1 + exp(2 z / softcap))
-            const float y = x[e] * p.s_mul;
-            z[e] = p.softcap > 0.f ? fmaf(-2.0f * p.softcap, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(2.0f * LOG2E * y / p.softcap)), p.softcap) : y;
-            z[e] = 4 * lane + e < here ? z[e] : -INFINITY;
+    for (int j = 0; j < 4; j++) {
+        const int i = wave + 8 * j;
+        if (i >= R) break;
+        z[j] = *(const f32x4*)(sc + i * MIX_SC + 4 * lane);
+        if (capped) {                                          // softcap * tanh(z / softcap) = softcap - 2 softcap / (1 + exp(2 z / softcap))
+            const float cap2 = -2.0f * p.softcap, capx = 2.0f * LOG2E * p.s_mul / p.softcap;
+#pragma unroll
+            for (int e = 0; e < 4; e++) z[j][e] = fmaf(cap2, __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(z[j][e] * capx)), p.softcap);
         }
-        const float m = wave_max_s(fmaxf(fmaxf(z[0], z[1]), fmaxf(z[2], z[3])));
-        float w[4];
 #pragma unroll
-        for (int e = 0; e < 4; e++) w[e] = here > 0 ? __builtin_amdgcn_exp2f((z[e] - m) * LOG2E) : 0.f;
-        const float l = wave_sum_s((w[0] + w[1]) + (w[2] + w[3]));
+        for (int e = 0; e < 4; e++) z[j][e] = 4 * lane + e < here ? z[j][e] : -INFINITY;
+        float m = fmaxf(fmaxf(z[j][0], z[j][1]), fmaxf(z[j][2], z[j][3]));
+        m = fmaxf(m, dpp<0xB1>(m)); m = fmaxf(m, dpp<0x4E>(m)); m = fmaxf(m, dpp<0x141>(m)); m = fmaxf(m, dpp<0x128>(m));      // over the tile's lanes
+        if ((lane & 15) == 0) mx[(lane >> 4) * 32 + i] = capped ? m : m * p.s_mul;
+    }
+    lds_barrier();
+
+    // the reference point of each tile's exponentials (it stays while no query's maximum grows by more than 8) and what the sums ahead of the tile are scaled by; lane: query
+    float m = -INFINITY, ref[MIX_TILES] = {}, alpha[MIX_TILES] = {};
+    const int qi = min(l31, R - 1);
+#pragma unroll
+    for (int t = 0; t < MIX_TILES; t++) {
+        if (t >= tiles) break;                                 // (uniform)
+        const float top = mx[32 * t + qi], was = m;
+        const bool move = !__all(top - m <= 8.0f);
+        if (move) m = fmaxf(m, top);
+        ref[t] = m;
+        alpha[t] = move ? __builtin_amdgcn_exp2f((was - m) * LOG2E) : 1.0f;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+        const int i = wave + 8 * j;
+        if (i >= R) break;
+        float at_tile = 0.f;                                   // query i's reference point in the lane's tile
+#pragma unroll
+        for (int t = 0; t < MIX_TILES; t++) {
+            const float r = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(ref[t]), i));
+            at_tile = lane >> 4 == t ? r : at_tile;
+        }
+        const float scale = capped ? LOG2E : p.s_mul * LOG2E, m2 = at_tile * LOG2E;
+        f32x4 w;
+#pragma unroll
+        for (int e = 0; e < 4; e++) w[e] = __builtin_amdgcn_exp2f(fmaf(z[j][e], scale, -m2));
+        *(f32x4*)(sc + i * MIX_SC + 4 * lane) = w;             // (for their sums)
         u32x2 hi, lo;
 #pragma unroll
         for (int e = 0; e < 2; e++) {
@@ -193,16 +223,28 @@ __device__ __forceinline__ void mix_attend16(const MixArgs& p, int u, int row, c
         char* d = pt + ((lane >> 2) * 4 + (lane & 1)) * R * 16 + i * 16 + (lane >> 1 & 1) * 8;
         *(u32x2*)d = hi;
         *(u32x2*)(d + 2 * R * 16) = lo;
-        if (lane == 0) { mx[i] = m; ls[i] = l; }
+    }
+    if (r0 < 64 * tiles) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");       // the wave's values are in LDS, for all waves behind the barrier
+        // the token's own value, also over what lies behind it (its weights are zero, but the rows hold anything)
+        for (int r = max(r0, n - 1 - key0) + lane / CPR; r < r0 + 32; r += RPI)
+            *(bf16x8*)(vt + r * ROWB + (((lane % CPR) ^ attn_vswz<D>(r)) * 16)) = *(const bf16x8*)(nv + e0);
     }
     __syncthreads();
     if (wave >= DB) return;
-    const int db = wave, tq = (lane & 15) >> 2, tp = lane & 3, v_row = 4 * hh + tq, qi = min(l31, R - 1);
+    const int db = wave, tq = (lane & 15) >> 2, tp = lane & 3, v_row = 4 * hh + tq;
     const int v_at = v_row * ROWB + (tp & 1) * 8 + ((((db * 4) ^ attn_vswz<D>(v_row)) | (((lane >> 4) & 1) * 2 + (tp >> 1))) * 16);
     f32x16 o;
 #pragma unroll
     for (int e = 0; e < 16; e++) o[e] = 0.f;
-    for (int t = 0; t < tiles; t++)
+    float l = 0.f;
+#pragma unroll
+    for (int t = 0; t < MIX_TILES; t++) {
+        if (t >= tiles) break;
+        if (t)
+#pragma unroll
+            for (int e = 0; e < 16; e++) o[e] *= alpha[t];
+        float even = 0.f, odd = 0.f;                           // the tile's weights, as the lanes of its keys add them
 #pragma unroll
         for (int st = 0; st < 4; st++) {
             const char* w = pt + (((t * 4 + st) * 4 + hh) * R + qi) * 16;
@@ -213,13 +255,21 @@ __device__ __forceinline__ void mix_attend16(const MixArgs& p, int u, int row, c
             const bf16x8 vf = {x[0], x[1], x[2], x[3], y[0], y[1], y[2], y[3]};
             o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, hi, o, 0, 0, 0);
             o = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, lo, o, 0, 0, 0);
+#pragma unroll
+            for (int i = 0; i < 2; i++) {
+                const f32x4 z = *(const f32x4*)(sc + qi * MIX_SC + 64 * t + 16 * st + 8 * i + 4 * hh);
+                even += z[0]; odd += z[1];
+                even += z[2]; odd += z[3];
+            }
         }
+        l = fmaf(l, alpha[t], even + odd);
+    }
+    l += __shfl_xor(l, 32, 64);
     if (l31 >= R) return;
-    const float l = ls[l31];
     // lane (query, half) owns columns 32 db + 8 g4 + 4 hh + 0..3
     if (p.nsplit > 1) {
         const int64_t pr = (((int64_t)row * p.units + unit) * p.nsplit + split) * R + l31;
-        if (db == 0 && hh == 0) { p.part_ml[pr * 2] = mx[l31]; p.part_ml[pr * 2 + 1] = l; }
+        if (db == 0 && hh == 0) { p.part_ml[pr * 2] = m; p.part_ml[pr * 2 + 1] = l; }
 #pragma unroll
         for (int g4 = 0; g4 < 4; g4++) *(f32x4*)(p.part_o + pr * D + 32 * db + 8 * g4 + 4 * hh) = f32x4{o[4 * g4], o[4 * g4 + 1], o[4 * g4 + 2], o[4 * g4 + 3]};
         return;

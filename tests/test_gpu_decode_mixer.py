@@ -8,6 +8,7 @@ from oracle import lugasun as O
 
 pytestmark = pytest.mark.gpu
 F32, BF16 = torch.float32, torch.bfloat16
+WIDTH = 512      # (a bf16 layer of fewer than 256 columns has no K-slices and keeps the separate kernels)
 LENS = [1, 2, 31, 32, 33, 63, 64, 65, 96, 254, 255, 256, 257, 511, 513]
 LAYERS = {
     'group4_128': LC.layer(LC.heads(8, 2, 128, 128, 4096, softcap=20.0), LC.ret(64, 64, (0.97, 0.9)), 64),
@@ -22,7 +23,7 @@ LAYERS = {
 def test_rows_of_every_length_together_and_alone(name, dtype):
     """Against the oracle, and a row's bits are the same whatever longer or shorter rows it is decoded with."""
     from callireader_amd.modeling_decoder import LugasunForCausalLM
-    cfg = LC.config(128, 60, [LAYERS[name]], side=8)
+    cfg = LC.config(WIDTH, 60, [LAYERS[name]], side=8)
     w = LC.weights(cfg, 31, qk_gain=1.5 if dtype == F32 else 1.0)
     m = LugasunForCausalLM.from_state_dict(w, cfg, dtype=dtype, max_tokens=640, max_seqs=len(LENS))
     toks = [LC.tokens(cfg, n + 3, seed=n) for n in LENS]
@@ -40,6 +41,26 @@ def test_rows_of_every_length_together_and_alone(name, dtype):
     for i in (0, 3, 6, 9, 12):
         assert torch.equal(run([i])[0], together[i]), LENS[i]
     m.close()
+
+
+@pytest.mark.parametrize('dtype', [F32, BF16])
+@pytest.mark.parametrize('name', LAYERS)
+def test_one_launch_has_the_bits_of_the_separate_ones(name, dtype, monkeypatch):
+    """Against the kernels it stands for (row kernel, split attention, retention with its merge), which other sizes take: logits, and what later steps read from caches and states.  Sharp scores move
+    the reference point of the softmax from tile to tile, in some of a unit's queries and not in others."""
+    from callireader_amd.modeling_decoder import LugasunForCausalLM
+    cfg = LC.config(WIDTH, 60, [LAYERS[name], LAYERS[name]], side=8)
+    w = LC.weights(cfg, 33, qk_gain=1.5)
+    toks = [LC.tokens(cfg, n + 4, seed=n) for n in LENS]
+    got = []
+    for joined in ('1', '0'):
+        monkeypatch.setenv('CR_DECODE_JOINED', joined)
+        m = LugasunForCausalLM.from_state_dict(w, cfg, dtype=dtype, max_tokens=640, max_seqs=len(LENS))
+        for i, n in enumerate(LENS):
+            m.step([(i, toks[i][:n], [])])
+        got.append(torch.stack([m.step([(i, [toks[i][n + k]], [0]) for i, n in enumerate(LENS)]) for k in range(4)]).cpu())
+        m.close()
+    assert torch.equal(*got), [(int(k), LENS[int(i)]) for k, i in (got[0] != got[1]).any(-1).nonzero()]
 
 
 @pytest.mark.parametrize('dtype', [F32, BF16])
