@@ -246,6 +246,7 @@ class Engine:
         return torch.empty(t.shape, dtype=t.dtype, pin_memory=True).copy_(t).to(self.device, non_blocking=True)
 
     def decode(self, kv, seqs, penalty=1.0, force_tokens=None, want_logits=False):
+        """One step for `seqs`, enqueued on the current stream: its logits are there for what follows on that stream.  Steps of one context on several streams are the caller's to order."""
         n = len(seqs)
         seq_arr = (C.c_int32 * n)(*seqs)
         ft = None

@@ -2,6 +2,7 @@
 
 A design is a reader of its config.json (config.DecoderSpec.from_*), listed in registry.py; everything below is shared by all of them.
 """
+import functools
 import json
 import os
 
@@ -12,9 +13,26 @@ from .config import DecoderSpec
 from .engine import DecoderEngine
 
 
+def _in_order(call):
+    """Workspace, cache and states belong to the model: what a call enqueues on another stream than the last one's comes behind all that stream holds.  (No event behind every call: one costs the
+    stream 5 us, and nearly every program stays on one stream.)"""
+    @functools.wraps(call)
+    def run(self, *args, **kw):
+        now = torch.cuda.current_stream()
+        if self._on is not None and now != self._on:
+            try:
+                now.wait_stream(self._on)
+            except RuntimeError:                          # a foreign stream that is no more
+                torch.cuda.synchronize()
+        self._on = now
+        return call(self, *args, **kw)
+    return run
+
+
 class DecoderLM:
     main_input_name = 'input_ids'
     read_config = None               # config.json (parsed) -> DecoderSpec
+    _on = None                       # the stream of the last call that enqueued work
 
     def __init__(self, spec, dtype=torch.bfloat16, device=0, max_tokens=8192, max_seqs=1):
         self.spec, self.max_tokens = spec, max_tokens
@@ -62,9 +80,12 @@ class DecoderLM:
         self.engine.close()
 
     # ---- one step ------------------------------------------------------------------------------
+    @_in_order
     def step(self, entries, penalty=1.0):
         """entries: (request id, next token ids, places among them whose logits are wanted).  Runs exactly these tokens on top of what the requests have cached; unknown ids are new
-        requests.  -> fp32 logits [wanted, vocab] in the order of the entries and places, or None.  One token each on top of a cache is a decode step, anything else a prefill."""
+        requests.  -> fp32 logits [wanted, vocab] in the order of the entries and places, or None.  One token each on top of a cache is a decode step, anything else a prefill.
+        A step is enqueued on the current stream and returns: logits are read on that stream, on one that waits for it, or after a synchronisation.  Steps of one model may come on different
+        streams; each is ordered behind the one before."""
         new = [rid for rid, _, _ in entries if rid not in self.slots.slot]
         if new:
             self.slots.admit(new)
@@ -82,10 +103,12 @@ class DecoderLM:
             base += len(t)
         return self.engine.prefill_tokens(kv, seqs, [t for _, t, _ in entries], penalty=penalty, want=want)
 
+    @_in_order
     def end(self, rid):
         self.slots.release(rid)
 
     # ---- generation ----------------------------------------------------------------------------
+    @_in_order
     @torch.no_grad()
     def generate(self, prompts, max_new_tokens=128, eos_token_id=None, repetition_penalty=1.0, check_every=16, prefill_tokens=16384):
         """prompts: lists of token ids, decoded greedily as one batch; -> the new ids of each, EOS included."""
