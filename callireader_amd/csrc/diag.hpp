@@ -1,6 +1,6 @@
 // Diagnostic builds, quarantined.
 //
-// The knock-out / knock-in / poison / stamp blocks inside the product kernels (gemm256.hip, gemm_mid.hip, gemm_skinny.hip, lm_gemm_rows.hip, lm_gemm_tiles.hip, attention_vit.hip) are cost-structure
+// The knock-out / knock-in / poison / stamp blocks inside the product kernels (gemm256.hip, gemm_mid.hip, gemm_skinny.hip, lm_gemm_rows.hip, lm_gemm_tiles.hip, lm_mix.hip, lm_ahead.hip, moe.hip, attention_vit.hip) are cost-structure
 // and hazard-screen tools: several of them give WRONG RESULTS by design.  Every translation unit that has such blocks includes this header, and this header is
 // the only door to them:
 //   * a diagnostic macro without -DCR_DIAG_BUILD is a compile error -- callireader_amd/build.py (the product build, __graft_entry__.build()) never defines

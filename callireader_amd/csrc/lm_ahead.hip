@@ -3,6 +3,7 @@
 // it waiting, and a workgroup reads the few KiB of slices from L2 in about the time its weights take to arrive.  With many rows every workgroup would read megabytes: see lm_ahead_supported.
 //
 // Sums, norms and products have the order of the kernels they stand for (lm_post_kernel; gemm_skinny.hip; lm_gemm_rows.hip), so a row's bits do not depend on which of them ran.
+#include "diag.hpp"
 #include "lm_ahead.hpp"
 
 bool gemm_stream_supported(int epi, const GemmParams& p, int splits);      // gemm_stream.hip
@@ -81,7 +82,10 @@ __global__ __launch_bounds__(512) void ahead_rows_kernel(const LmAhead a, const 
     auto load = [&](int s) {
 #pragma unroll
         for (int u = 0; u < U; u++)
-            if (s + u < s1) __builtin_amdgcn_global_load_lds(CR_GLB(w + (s + u) * 16), CR_LDS(ring + u * 1024), 16, 0, 0);
+            if (s + u < s1) {
+                CR_DIAG_POISON(ring + u * 1024)
+                __builtin_amdgcn_global_load_lds(CR_GLB(w + (s + u) * 16), CR_LDS(ring + u * 1024), 16, 0, 0);
+            }
     };
     if (s0 < s1) load(s0);
     update_rows<float>(a, 0, a.M, hf, K + 4, sums, blockIdx.x == 0 && blockIdx.y == 0);

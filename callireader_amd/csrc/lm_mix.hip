@@ -12,6 +12,7 @@
 // freshly written cache row, which every workgroup of a group of query heads writes for itself -- the same bits.
 #include "attention_merge.hpp"
 #include "attention_plain.hpp"
+#include "diag.hpp"
 #include "lm_heads.hpp"
 #include "retention.hpp"
 
@@ -125,6 +126,7 @@ __device__ __forceinline__ void mix_attend16(const MixArgs& p, int u, int row, c
 #pragma unroll
             for (int i = 0; i < 32 / RPI; i++) {
                 const int r = r0 + i * RPI + lane / CPR;
+                CR_DIAG_POISON(vt + (r0 + i * RPI) * ROWB)
                 __builtin_amdgcn_global_load_lds(CR_GLB(Vb + (int64_t)min(key0 + r, old) * D + (((lane % CPR) ^ attn_vswz<D>(r)) * 8)), CR_LDS(vt + (r0 + i * RPI) * ROWB), 16, 0, 0);
             }
         }

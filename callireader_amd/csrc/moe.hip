@@ -1,4 +1,5 @@
 // Expert routing: scores, grouped choice, and the assignments sorted by expert for the grouped products.
+#include "diag.hpp"
 #include "lm_ahead.hpp"
 
 namespace {
@@ -144,8 +145,10 @@ __global__ __launch_bounds__(1024) void lm_router_kernel(const bf16* __restrict_
     for (int c = 0; c < per; c += STEPS) {
         if (c) __syncthreads();
 #pragma unroll
-        for (int s = 0; s < 4; s++)
+        for (int s = 0; s < 4; s++) {
+            CR_DIAG_POISON(xs + (s * 16 + wave) * 1024)
             __builtin_amdgcn_global_load_lds(CR_GLB(row + min((min(s * per, steps) + c) * 32 + own, K - 8)), CR_LDS(xs + (s * 16 + wave) * 1024), 16, 0, 0);
+        }
         const int n = min(STEPS, k_hi - k_lo - c), k0 = k_lo + c;
         bf16x8 wf[EB][U];
         auto load = [&](int ks) {
