@@ -217,10 +217,10 @@ __global__ __launch_bounds__(256) void lm_router_slice_kernel(const bf16* __rest
 // Decode: a row's residual update, its router scores and its choice in one workgroup of eight waves, where those were three launches (24 rows, 2048 x 32: 4.6 + 3.4 + 4.8 us and two gaps -> 8.9).  Scores are
 // the ones lm_router_slice_kernel and lm_route_kernel form, bit for bit -- the same K-slices on the matrix cores, added in slice order: a choice between close experts must not hang on the
 // path.  A wave takes every eighth slice of all experts; the weights of its first 32 experts (fragment-ordered with wsw) are asked for ahead of the update.
-constexpr int POST_COLS = 2048, POST_E = 64;
+constexpr int POST_COLS = 2048, POST_E = 64, POST_BATCH = 32, POST_COLS_TWO = 1536;      // columns and experts at most; experts of a batch of weights, columns at most with two batches
 __global__ __launch_bounds__(512) void lm_post_route_kernel(const LmAhead a, bf16* __restrict__ h, const bf16* __restrict__ Wr, int wsw, const float* __restrict__ corr, int E, int top, int groups,
                                                             int keep, int32_t* __restrict__ idx, float* __restrict__ wt) {
-    constexpr int SL = LM_ROUTER_SLICES / 8, MAX_PER = POST_COLS / 32 / LM_ROUTER_SLICES, PAIR = 2;      // slices a wave, k-steps a slice, blocks of 16 experts a batch
+    constexpr int SL = LM_ROUTER_SLICES / 8, MAX_PER = POST_COLS / 32 / LM_ROUTER_SLICES, PAIR = POST_BATCH / 16;      // slices a wave, k-steps a slice, blocks of 16 experts a batch
     __shared__ __attribute__((aligned(16))) bf16 hs[POST_COLS];
     __shared__ __attribute__((aligned(16))) float part[LM_ROUTER_SLICES][POST_E];
     __shared__ float sums[AHEAD_SEGS], z[POST_E], ch[POST_E], gs[POST_E];
@@ -364,8 +364,12 @@ __global__ __launch_bounds__(1024) void lm_plan_place_kernel(const int32_t* __re
 
 }  // namespace
 
-// a row's workgroup reads the whole router from L2: 256 KiB of it are about the time of the launches it saves
-bool lm_post_route_supported(const Lm& lm, const LmLayer& L) { return !lm.f32 && lm.Wp <= POST_COLS && lm.Wp % 64 == 0 && L.s.experts <= POST_E; }
+// A row's workgroup reads the whole router from L2.  One batch of weights travels under the update; a second one is a round trip and its bytes behind it, which pays up to 1536 columns.  A layer's
+// step, us saved against the separate kernels at 9 / 24 / 64 rows: 2048 x 32 3.3 / 3.1 / 3.3, 1024 x 64 3.0 / 2.9 / 1.8, 1536 x 64 0.7 / 0.9 / 0.4; 2048 x 36 -0.4 / -0.7 / -0.8, 2048 x 64
+// -2.2 / -1.9 / -1.6.
+bool lm_post_route_supported(const Lm& lm, const LmLayer& L) {
+    return !lm.f32 && lm.Wp <= (L.s.experts <= POST_BATCH ? POST_COLS : POST_COLS_TWO) && lm.Wp % 64 == 0 && L.s.experts <= POST_E;
+}
 
 int launch_lm_post_route(const Lm& lm, const LmLayer& L, const LmAhead& a, void* h, int32_t* idx, float* wt, hipStream_t st) {
     if (a.M <= 0 || !a.Y || !a.x || !a.x_out || !h || !idx || !wt || a.Wp != lm.Wp || !lm_post_route_supported(lm, L)) return cr_fail(CR_ERR_ARG, "update and routing: %d rows, %d experts", a.M, L.s.experts);

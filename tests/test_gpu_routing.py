@@ -24,7 +24,7 @@ def test_many_tokens(width, experts, top, groups, keep, n):
     assert float(err.median()) < 2e-2 and float((err > 0.1).float().mean()) < 0.02, (float(err.median()), float(err.max()))
 
 
-@pytest.mark.parametrize('width,experts,top,groups,keep', [(64, 3, 1, 1, 1), (320, 17, 2, 1, 1), (1088, 33, 3, 3, 2), (2048, 64, 4, 8, 4)])
+@pytest.mark.parametrize('width,experts,top,groups,keep', [(64, 3, 1, 1, 1), (320, 17, 2, 1, 1), (1088, 33, 3, 3, 2), (2048, 64, 4, 8, 4), (1536, 64, 4, 8, 4), (2048, 32, 4, 4, 2)])
 def test_decoded_rows(width, experts, top, groups, keep):
     """Decoded rows: update, scores and choice in one launch, at widths that the sixteen K-slices and expert counts that the blocks of 16 do not divide."""
     from callireader_amd.modeling_decoder import LinasunForCausalLM
@@ -43,7 +43,7 @@ def test_decoded_rows(width, experts, top, groups, keep):
 
 
 @pytest.mark.parametrize('layout', ['1', '0'])
-@pytest.mark.parametrize('width,experts,top,groups,keep', [(64, 3, 1, 1, 1), (320, 17, 3, 1, 1), (1088, 33, 3, 3, 2), (2048, 64, 5, 8, 4)])
+@pytest.mark.parametrize('width,experts,top,groups,keep', [(64, 3, 1, 1, 1), (320, 17, 3, 1, 1), (1088, 33, 3, 3, 2), (1536, 64, 5, 8, 4), (2048, 32, 3, 4, 2)])
 def test_joined_choice_has_the_bits_of_the_separate_kernels(width, experts, top, groups, keep, layout, monkeypatch):
     """Update, scores and choice in one launch against the residual update, the sliced router and the routing kernel, bit for bit, with fragment-ordered weights and without.  Experts come in pairs that
     only the rounding of sums tells apart: the second has the first's weights with columns of equal activations exchanged across K-slices, so another order of a sum turns choices."""
