@@ -471,15 +471,13 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
     const int ring = L.heads() ? std::min(lm.chunks[L.chunk_ix], kv->max_tokens) : 1, chunk = L.heads() ? lm.chunks[L.chunk_ix] : 1;
     char *ck = kv->lat + kv->lat_off[r], *cv = ck + (size_t)kv->n_seqs * a.kv_heads * ring * L.Ap * es;
     float* state = (float*)(kv->lat + kv->state_off[r]);
-    // by the layer's sizes alone (and 64 rows, where slices end): a row's bits do not depend on the rows it is decoded with
-    if (s_a && c->joined_decode && lm_mix_supported(lm.f32, L)) {
+    const bool split = L.heads() && !lm.f32 && sp.decode;
+    const int unit = split ? heads_per_split(a) : 1, splits = L.heads() && sp.decode ? sp.hsplit[L.chunk_ix] : 1;
+    if (s_a && c->joined_decode && lm_mix_supported(lm.f32, L) && lm_mix_pays(lm.f32, L, M, unit, splits)) {
         LmMixIn in{};
-        in.M = M; in.part = b.sl; in.slices = s_a; in.where = b.where; in.ang = b.ang; in.ao = b.ao; in.cache_k = ck; in.cache_v = cv; in.ring = ring; in.chunk = chunk; in.rows = in.nsplit = 1;
+        in.M = M; in.part = b.sl; in.slices = s_a; in.where = b.where; in.ang = b.ang; in.ao = b.ao; in.cache_k = ck; in.cache_v = cv; in.ring = ring; in.chunk = chunk; in.rows = unit; in.nsplit = split ? splits : 1;
         in.state = state;
-        if (L.heads() && !lm.f32) {
-            in.rows = heads_per_split(a); in.nsplit = sp.hsplit[L.chunk_ix];
-            in.part_o = b.part; in.part_ml = b.part + (size_t)M * a.heads * in.nsplit * L.Ap;
-        }
+        if (split) { in.part_o = b.part; in.part_ml = b.part + (size_t)M * a.heads * splits * L.Ap; }
         return launch_lm_mix(lm.f32, lm, L, in, st);
     }
     if (kp) CR_TRY(launch_lm_prefix(lm.f32, L, kp->n_pre, kp->pre_key, kp->pre_slot, b.kv, ck, cv, ring, st));

@@ -257,6 +257,7 @@ struct LmMixIn {
     float* state;                                     // retention (RetParams)
 };
 bool lm_mix_supported(bool f32, const LmLayer& L);
+bool lm_mix_pays(bool f32, const LmLayer& L, int M, int rows, int splits);      // (splits of 256 keys of the longest row) against the separate kernels, which give the same bits
 int launch_lm_mix(bool f32, const Lm& lm, const LmLayer& L, const LmMixIn& in, hipStream_t st);
 // decode of <= 64 rows: z[m][n] = gelu_tanh(sum of K-slices) * side[tok[m]][n]
 int launch_lm_side_act(const Lm& lm, int M, const float* part, int slices, const void* side, int64_t lds, const int32_t* tok, void* z, hipStream_t st);

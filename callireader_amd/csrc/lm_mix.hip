@@ -406,6 +406,23 @@ bool lm_mix_supported(bool f32, const LmLayer& L) {
     return !L.heads() || f32 || (L.s.attn.scale > 0.f && L.Ap <= 128);
 }
 
+// One launch saves two others and their round trips, 6 to 15 us a layer while the chip is not full.  Beyond that the separate kernels' smaller workgroups count.  Us of a layer's step saved:
+//   fp32: a workgroup of 16 waves has its CU to itself, so a second round of them loses: heads of 8 on 2 x 128 + 8 of retention, 16 rows +6.5 / +2.8 / -1.1 at 60 / 900 / 2500 keys, 20 rows
+//   +1.4 / -11, 64 rows -5 / -37.  Wide heads over many keys are bound by reading them, which a group's heads share better in the separate kernel's order: 16 on 4 x 128, 12 rows (216 workgroups)
+//   +6.7 / -2 / -10 at 60 / 900 / 2500; 4 x 256, 32 rows (256) +6.7 at 60, -3.4 at 400; 24 rows (192) +7 / +2.3 / +0.6 / -9 at 60 / 400 / 900 / 2500, 16 rows (128) +6 at 2500.
+//   bf16, one workgroup a CU (their LDS: groups of 8 of 128 and more, of 32 of 64): 16 on 2 x 128, 24 x 900 (192) +6.5, 24 x 2500 (480) -0.6, 64 x 2500 -6.6; 32 on 1 x 64, 64 x 900 (256) +2,
+//   40 x 2500 (400) -5.  Two a CU: heads of 128 gain throughout (16 on 16, 64 x 2500 +20); of 64, whose cache rows of 128 bytes come in pieces of 32, up to four rounds: 32 on 32,
+//   9 x 900 (1152) +1.7, 64 x 200 (2048) +4.5, 9 x 2500 (2880) -1.4, 64 x 900 (8192) -15; 32 on 2 (groups of 16), 64 x 900 (512) +0.6, 64 x 2500 (1280) -2.
+bool lm_mix_pays(bool f32, const LmLayer& L, int M, int rows, int splits) {
+    constexpr int64_t CUS = 256;
+    const int64_t att = L.heads() ? (int64_t)M * (L.s.attn.heads / rows) * (f32 ? 1 : splits) : 0, ret = L.retention() ? (int64_t)M * L.s.ret.heads : 0;
+    if (f32) return att + ret <= (!L.heads() || L.Ap <= 64 || splits <= 1 ? CUS : CUS * ((L.Ap <= 128 ? 4 : 3) - (splits > 4)) / 4);
+    if (!L.heads()) return true;
+    const int lds = L.Ap == 64 ? mix_lds16<64>(rows) : mix_lds16<128>(rows);
+    if (2 * lds > 160 * 1024) return att <= CUS;
+    return L.Ap == 128 || att <= (rows > 8 ? 4 : 8) * CUS;
+}
+
 int launch_lm_mix(bool f32, const Lm& lm, const LmLayer& L, const LmMixIn& in, hipStream_t st) {
     const cr_lm_heads& s = L.s.attn;
     const cr_lm_retention& r = L.s.ret;
