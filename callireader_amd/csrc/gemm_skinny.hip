@@ -22,6 +22,7 @@
 //     multiplies the fp32 sum once, before the epilogue's rounding.
 #include <stdio.h>
 #include <stdlib.h>
+#include <type_traits>
 
 #include "common.hpp"
 #include "diag.hpp"
@@ -74,7 +75,8 @@ __global__ __launch_bounds__(WAVES * 64, !W8 && skinny_two(RT, MT) ? 4 : 1) void
     constexpr int XSTEP = 32;
 #endif
 
-    // k-steps a batch: two batches of RT + MT fragments of 4 registers each, 96 registers where two workgroups are to share a CU and 160 beyond; one batch of 80 registers past 32 rows
+    // k-steps a batch: two batches of RT + MT fragments of 4 registers each, 96 registers where two workgroups are to share a CU and 160 beyond; past 32 rows one batch, of 56 (3 + 4)
+    // to 96 (2 + 4) registers
     constexpr int UR = MT > 2 ? (RT == 1 ? 20 / (1 + MT) : 8 / RT) : skinny_two(RT, MT) ? 12 / (RT + MT) : RT + MT <= 5 ? 4 : 3;
     f32x4 acc[RT][MT];
 #pragma unroll
@@ -145,60 +147,60 @@ __global__ __launch_bounds__(WAVES * 64, !W8 && skinny_two(RT, MT) ? 4 : 1) void
         // Batches of UR k-steps, the last one partial.  Described decoders give a wave 1..8 k-steps (K = 1024 .. 4096 over eight waves and the slices): fewer than a batch, they used to be
         // loaded one by one, a round trip to memory each (one row, us before -> after: 4096 x 1024 5.4 -> 4.5, 3584 x 1024 5.5 -> 4.2, 1024 x 4096 4.9 -> 3.9, 1024 x 1536 4.2 -> 3.5;
         // 24 rows: 3328 x 2048 6.7 -> 6.0, 2048 x 2048 6.4 -> 5.4).  Up to 32 rows the next batch's loads are issued ahead of this one's MFMAs; beyond that the volume of X through the
-        // CU's load path is what counts and a second batch changes nothing (64 rows, 6144 x 4096: 17.9 without, 18.5 with).
+        // CU's load path is what counts and a second batch gains nothing.  There a whole batch asks for all its weights, then for X, as the far loads have to lead, and the scheduler may not
+        // sink them between the MFMAs (64 rows, cold weights, us with / without that barrier: 6144 x 4096 20.0 / 20.6, 4096 x 4096 15.8 / 16.9, 4096 x 14336 31.8 / 34.4; 33 rows 15.7 / 15.8, 13.2 /
+        // 14.0, 26.9 / 26.8).
         struct Batch { bf16x8 w[RT][UR], x[MT][UR]; };
-        auto load = [&](Batch& f, int ks) {
+        auto load = [&](Batch& f, int ks, auto whole) {            // whole: all UR steps are there
+            if constexpr (MT > 2 && decltype(whole)::value) {
 #pragma unroll
-            for (int u = 0; u < UR; u++) {
-                if (ks + u >= ksteps) break;                      // (uniform)
+                for (int r = 0; r < RT; r++)
 #pragma unroll
-                for (int r = 0; r < RT; r++) f.w[r][u] = __builtin_nontemporal_load((const bf16x8*)(wp[r] + (ks + u) * wstep));
+                    for (int u = 0; u < UR; u++) f.w[r][u] = __builtin_nontemporal_load((const bf16x8*)(wp[r] + (ks + u) * wstep));
 #pragma unroll
-                for (int t = 0; t < MT; t++) f.x[t][u] = *(const bf16x8*)(xp[t] + (ks + u) * XSTEP);
-            }
+                for (int t = 0; t < MT; t++)
+#pragma unroll
+                    for (int u = 0; u < UR; u++) f.x[t][u] = *(const bf16x8*)(xp[t] + (ks + u) * XSTEP);
+            } else
+#pragma unroll
+                for (int u = 0; u < UR; u++) {
+                    if (ks + u >= ksteps) break;                  // (uniform)
+#pragma unroll
+                    for (int r = 0; r < RT; r++) f.w[r][u] = __builtin_nontemporal_load((const bf16x8*)(wp[r] + (ks + u) * wstep));
+#pragma unroll
+                    for (int t = 0; t < MT; t++) f.x[t][u] = *(const bf16x8*)(xp[t] + (ks + u) * XSTEP);
+                }
         };
-        auto mul = [&](const Batch& f, int ks) {
+        auto mul = [&](const Batch& f, int ks, auto whole) {
 #pragma unroll
             for (int u = 0; u < UR; u++) {
-                if (ks + u >= ksteps) break;
+                if (!decltype(whole)::value && ks + u >= ksteps) break;
 #pragma unroll
                 for (int r = 0; r < RT; r++)
 #pragma unroll
                     for (int t = 0; t < MT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[r][u], f.x[t][u], acc[r][t], 0, 0, 0);
             }
         };
+        constexpr std::false_type some{};
         Batch f0, f1;
         if (MT <= 2) {
-            load(f0, 0);
+            load(f0, 0, some);
             for (int ks = 0; ks < ksteps; ks += 2 * UR) {
-                load(f1, ks + UR);
-                mul(f0, ks);
-                load(f0, ks + 2 * UR);
-                mul(f1, ks + UR);
+                load(f1, ks + UR, some);
+                mul(f0, ks, some);
+                load(f0, ks + 2 * UR, some);
+                mul(f1, ks + UR, some);
             }
         } else {
-            // whole batches: all weights, then X, as the far loads have to lead (64 rows: 14336 x 4096 and 4096 x 4096 23.4 us on average, 6144 x 4096 17.5; k-step by k-step 24.2 and 18.3)
             int ks = 0;
             for (; ks + UR <= ksteps; ks += UR) {
-                bf16x8 w[RT][UR], x[MT][UR];
-#pragma unroll
-                for (int r = 0; r < RT; r++)
-#pragma unroll
-                    for (int u = 0; u < UR; u++) w[r][u] = __builtin_nontemporal_load((const bf16x8*)(wp[r] + (ks + u) * wstep));
-#pragma unroll
-                for (int t = 0; t < MT; t++)
-#pragma unroll
-                    for (int u = 0; u < UR; u++) x[t][u] = *(const bf16x8*)(xp[t] + (ks + u) * XSTEP);
-#pragma unroll
-                for (int u = 0; u < UR; u++)
-#pragma unroll
-                    for (int r = 0; r < RT; r++)
-#pragma unroll
-                        for (int t = 0; t < MT; t++) acc[r][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[r][u], x[t][u], acc[r][t], 0, 0, 0);
+                load(f0, ks, std::true_type{});
+                __builtin_amdgcn_sched_barrier(0);
+                mul(f0, ks, std::true_type{});
             }
             if (ks < ksteps) {
-                load(f0, ks);
-                mul(f0, ks);
+                load(f0, ks, some);
+                mul(f0, ks, some);
             }
         }
     }
