@@ -379,6 +379,18 @@ int cr_op_attention(const void* q, const void* k, const void* v, void* o, const 
     return CR_OK;
 }
 
+int cr_op_prompt_attention(const void* q, const void* k, const void* v, void* o, const int32_t* segs, int n_seg, int longest, const int64_t* s, int H, int kv_group, int head_dim, int vdim,
+                           float s_mul, float softcap, float out_mul, void* stream) {
+    if (!q || !k || !v || !o || !segs || !s || n_seg <= 0 || n_seg > 65535 || longest <= 0 || H <= 0 || kv_group <= 0 || H % kv_group) return cr_fail(CR_ERR_ARG, "cr_op_prompt_attention: bad argument");
+    AttnParams p{};
+    p.Q = (const bf16*)q; p.K = (const bf16*)k; p.V = (const bf16*)v; p.O = (bf16*)o;
+    p.q_rs = s[0]; p.q_hs = s[1]; p.k_bs = p.v_bs = p.k_rs = p.v_rs = s[2]; p.k_hs = p.v_hs = s[3]; p.o_rs = s[4]; p.o_hs = s[5];
+    p.B = n_seg; p.H = H; p.kv_group = kv_group; p.Sq = longest; p.seg = segs; p.q_prescale = p.s_div = 1.f;
+    p.wide = 1; p.s_mul = s_mul; p.softcap = softcap; p.out_mul = out_mul; p.vdim = vdim;
+    if (launch_flash_attn(p, head_dim, true, (hipStream_t)stream) != CR_OK) return cr_fail(CR_ERR_ARG, "cr_op_prompt_attention(d=%d) rejected or failed", head_dim);
+    return CR_OK;
+}
+
 int64_t cr_op_decode_attention_scratch_floats(int B, int max_keys) {
     const int nsplit = ((max_keys + 63) / 64 + ATTN_SPLIT_TILES - 1) / ATTN_SPLIT_TILES;
     return (int64_t)attn_split_ws_floats(B, 8, 4, nsplit, 128);

@@ -104,8 +104,9 @@ __global__ __launch_bounds__(256, D == 256 ? 1 : 2) void flash_attn_kernel(const
         head = (pid / gx) % gy;
         batch = pid / (gx * gy);
         // causal: query blocks have 2 .. 2 gx key tiles.  Head by head, an XCD's last heads bring their longest blocks when its CUs run dry; so where XCDs get whole heads, eight of them are
-        // taken together, the longest blocks of all of them first (more than eight would read as many heads' keys at once through one L2).  128 columns, us: 3164 tokens x 32 heads
-        // 144 -> 119, 4 x 1531 x 16 in 32-bit scores 113 -> 90, 8 x 1024 x 16 capped 129 -> 94; 64 x 333 x 32 184 either way (three blocks a head)
+        // taken together, the longest blocks of all of them first.  128 columns, us: 3164 tokens x 32 heads 144 -> 119, 4 x 1531 x 16 in 32-bit scores 113 -> 90, 8 x 1024 x 16 capped 129 -> 94;
+        // 64 x 333 x 32 184 either way (three blocks a head).  Groups of 4 / 8 / 16 / 64 heads (more of them read as many heads' keys at once through one L2): 13 x 3164 x 32 1450 / 1485 / 1506 / 1836,
+        // 8 x 1024 x 16 80 / 70 / 77 / 76, 24 x 500 x 16 65 / 66 / 66 / 71
         const int heads = gy * (int)gridDim.z, hx = heads >> 3;
         if (CAUSAL && !SPLIT && (heads & 7) == 0) {
             const int i = lin >> 3, g0 = i / (8 * gx) * 8, n = min(8, hx - g0), j = i - g0 * gx, hb = xcd * hx + g0 + j % n;

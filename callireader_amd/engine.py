@@ -509,3 +509,19 @@ def op_decode_attention(q, kc, vc, seqs, lens, s_div=11.313708498984761, which=0
     B.check(B.lib.cr_op_decode_attention(which, _p(q), _p(kc), _p(vc), max_tokens, _p(seqs), _p(lens), Bn, max_keys, float(s_div), _p(scratch), _p(out), _stream()),
             'cr_op_decode_attention')
     return out
+
+
+def op_prompt_attention(q, k, v, segments, s_mul, softcap=0.0, out_mul=1.0, vdim=None):
+    """cr_op_prompt_attention: q (rows, H, D), k / v (keys, G, D) bf16; segments: (first row, rows, first position, first key row) each; -> (rows, H, vdim) bf16, zeros where no segment is."""
+    (rows, H, D), (keys, G, _) = q.shape, k.shape
+    if k.shape != v.shape or k.shape[2] != D or H % G or not (q.is_contiguous() and k.is_contiguous() and v.is_contiguous()):
+        raise ValueError(f'op_prompt_attention: {tuple(q.shape)} on {tuple(k.shape)} / {tuple(v.shape)}, contiguous')
+    if any(n <= 0 or r < 0 or r + n > rows or p < 0 or kr < 0 or kr + p + n > keys for r, n, p, kr in segments):
+        raise ValueError('op_prompt_attention: a segment outside the rows or keys')
+    vdim = vdim or D
+    o = torch.zeros(rows, (H * vdim + 3) // 4 * 4, device=q.device, dtype=torch.bfloat16)      # (rows of whole 8-byte pieces)
+    seg = torch.tensor([x for s in segments for x in s], dtype=torch.int32, device=q.device)
+    st = (C.c_int64 * 6)(q.stride(0), q.stride(1), k.stride(0), k.stride(1), o.stride(0), vdim)
+    B.check(B.lib.cr_op_prompt_attention(_p(q), _p(k), _p(v), _p(o), _p(seg), len(segments), max(s[1] for s in segments), st, H, H // G, D, vdim, float(s_mul), float(softcap), float(out_mul),
+                                         _stream()), 'cr_op_prompt_attention')
+    return o[:, :H * vdim].reshape(rows, H, vdim)

@@ -25,7 +25,7 @@
 extern "C" {
 #endif
 
-#define CR_ABI_VERSION 12  /* 12: cr_lm_layer / cr_lm_desc: attention over heads, retention, dense feed-forward, token side input; 11: cr_lm_configure, cr_lm_passes, cr_llm_prefill_tokens; 10: cr_op_decode_attention(+_scratch_floats); 9: cr_build_flags, cr_diag_register; 8: cr_op_decode_swizzle, cr_op_decode_gemm flags bit 8, cr_op_gemm bits 18-19; 7: cr_op_decode_gemm; 6: cr_build_id, cr_llm_hidden_probe; 5: cr_share_weights, cr_op_gemm_q8, cr_op_norm_fp8 takes the next linear's bound; 4: cr_enable_fp8_mfma, cr_op_norm_fp8, cr_op_gemm bit 17; 2: cr_orderformer; cr_op_gemm kernel pin and EPI_PARTIAL (epi 7); 3: cr_profile_stats, cr_kv_read, cr_kv_reset takes a stream, cr_enable_fp8_decode, cr_op_quantize_fp8, epi 8 */
+#define CR_ABI_VERSION 13  /* 13: cr_op_prompt_attention; 12: cr_lm_layer / cr_lm_desc: attention over heads, retention, dense feed-forward, token side input; 11: cr_lm_configure, cr_lm_passes, cr_llm_prefill_tokens; 10: cr_op_decode_attention(+_scratch_floats); 9: cr_build_flags, cr_diag_register; 8: cr_op_decode_swizzle, cr_op_decode_gemm flags bit 8, cr_op_gemm bits 18-19; 7: cr_op_decode_gemm; 6: cr_build_id, cr_llm_hidden_probe; 5: cr_share_weights, cr_op_gemm_q8, cr_op_norm_fp8 takes the next linear's bound; 4: cr_enable_fp8_mfma, cr_op_norm_fp8, cr_op_gemm bit 17; 2: cr_orderformer; cr_op_gemm kernel pin and EPI_PARTIAL (epi 7); 3: cr_profile_stats, cr_kv_read, cr_kv_reset takes a stream, cr_enable_fp8_decode, cr_op_quantize_fp8, epi 8 */
 
 enum { CR_OK = 0, CR_ERR_ARG = -1, CR_ERR_HIP = -2, CR_ERR_STATE = -3, CR_ERR_NOMEM = -4 };
 enum { CR_BF16 = 0, CR_F32 = 1, CR_I64 = 2, CR_I32 = 3, CR_U8 = 4 /* library-internal: e4m3 weight copies */ };
@@ -326,6 +326,12 @@ int cr_op_attention(const void* q, const void* k, const void* v, void* o, const 
 int64_t cr_op_decode_attention_scratch_floats(int B, int max_keys);
 int cr_op_decode_attention(int which, const void* q, const void* kc, const void* vc, int max_tokens, const int32_t* seqs, const int32_t* lens, int B, int max_keys,
                            float s_div, float* scratch, void* out, void* stream);
+/* A described decoder's prompt attention alone (test / tuning entry): n_seg segments {first row, rows, first position, first key row} of 4 int32 each (DEVICE array; `longest` = the most rows of one),
+ * a row at position p of its segment over the p + 1 keys from the segment's first key row on.  q rows q_rs, heads q_hs elements apart, k and v likewise (k_rs, k_hs; kv_group query heads a key
+ * head), o (o_rs, o_hs; vdim <= head_dim columns a head): strides6 = {q_rs, q_hs, k_rs, k_hs, o_rs, o_hs}.  head_dim 64, 128 or 256; scores q . k * s_mul in 32 bits, soft-capped when softcap > 0;
+ * the result times out_mul.  ABI v13. */
+int cr_op_prompt_attention(const void* q, const void* k, const void* v, void* o, const int32_t* segs, int n_seg, int longest, const int64_t* strides6, int H, int kv_group, int head_dim, int vdim,
+                           float s_mul, float softcap, float out_mul, void* stream);
 
 #ifdef __cplusplus
 }
