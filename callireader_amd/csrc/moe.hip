@@ -5,7 +5,7 @@
 namespace {
 
 constexpr int MAX_E = 1024;
-constexpr int LM_PLAN_ONE = 4096;      // assignments one workgroup places by itself
+constexpr int LM_PLAN_ONE = 8192;      // assignments one workgroup places by itself
 
 // order of a wave's own LDS accesses (each wave below works in LDS of its own: no workgroup barrier)
 #define WAVE_LDS_FENCE()                                      \
@@ -333,8 +333,8 @@ __global__ __launch_bounds__(1024) void lm_plan_kernel(const int32_t* __restrict
     plan_count(idx, 0, n, cnt, [&](int i, int at) { perm[at] = i; });
 }
 
-// Many assignments: counting and placing them is bound by one CU's LDS atomics (24 496 of 32 experts: 18.5 us), so PLAN_PARTS workgroups count a part each, and as many place it behind what
-// the parts ahead of it hold.
+// Many assignments: counting and placing them is bound by one CU's LDS atomics, so PLAN_PARTS workgroups count a part each, and as many place it behind what the parts ahead of it hold.
+// One workgroup / parts, us: 32 experts 4096 6.4 / 6.8, 8192 9.4 / 9.0, 12 288 12.5 / 10.4, 24 576 19.7 / 11.5; 256 experts 4096 5.9 / 8.8, 8192 8.1 / 9.6, 12 288 10.7 / 10.6, 24 576 17.0 / 10.6.
 constexpr int PLAN_PARTS = 32;
 __global__ __launch_bounds__(1024) void lm_plan_count_kernel(const int32_t* __restrict__ idx, int n, int E, int32_t* __restrict__ hist) {
     __shared__ int cnt[MAX_E];

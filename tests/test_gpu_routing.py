@@ -1,5 +1,5 @@
 """Routing of many tokens: the router product through LDS and the fragment-ordered weights, at widths and expert counts that its chunks of 512 columns and blocks of 16 do not divide, and the
-assignments' plan in one workgroup (up to 4096) and in parts (above): against the oracle."""
+assignments' plan in one workgroup (up to 8192) and in parts (above): against the oracle."""
 import pytest
 import torch
 
@@ -9,7 +9,8 @@ from oracle import linasun as O
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize('width,experts,top,groups,keep,n', [(320, 3, 1, 1, 1, 333), (2304, 40, 2, 5, 3, 700), (1024, 96, 6, 8, 4, 683), (4224, 33, 4, 3, 2, 1025), (512, 200, 5, 10, 4, 1400)])
+@pytest.mark.parametrize('width,experts,top,groups,keep,n', [(320, 3, 1, 1, 1, 333), (2304, 40, 2, 5, 3, 700), (1024, 96, 6, 8, 4, 683), (4224, 33, 4, 3, 2, 1025), (512, 200, 5, 10, 4, 1400), (320, 33, 8, 3, 3, 1024),
+                                                                  (320, 33, 8, 3, 3, 1025), (512, 200, 10, 10, 9, 1300)])
 def test_many_tokens(width, experts, top, groups, keep, n):
     from callireader_amd.modeling_decoder import LinasunForCausalLM
     cfg = LC.config(width, 120, [(LC.mixer(2, 64, 64, 64, 64, 0.15), LC.moe(experts, top, 64, 2.0, (groups, keep)))])
