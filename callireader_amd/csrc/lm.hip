@@ -528,14 +528,13 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
     return sp.decode ? launch_ret_decode(lm.f32, rp, merge ? &ap : nullptr, L.Ap, st) : matrix ? launch_ret_matrix(rp, st) : launch_ret_recurrent(lm.f32, rp, st);
 }
 
-// h -> ye, wt: the rows of every chosen expert and their weights
+// h -> ye, wt: the rows of every chosen expert and their weights (routed: the choice is made)
 int expert_mixture(cr_ctx* c, const Step& sp, Buffers& b, const LmLayer& L, bool routed, hipStream_t st) {
     const Lm& lm = *c->lm;
     const cr_lm_layer& s = L.s;
     const int M = sp.M, Wp = lm.Wp;
-    if (routed) ;
-    else if (!lm.f32 && lm_router_supported(L)) CR_TRY(launch_lm_router(lm, L, M, b.h, b.idx, b.wt, b.z, st));
-    else {
+    if (!routed && !lm.f32 && lm_router_supported(L)) CR_TRY(launch_lm_router(lm, L, M, b.h, b.idx, b.wt, b.z, st));
+    else if (!routed) {
         CR_TRY(raw32(c, lm, b.h, L.router, b.z, L.Ep, M, s.experts, Wp, 0.f, st, sp.decode));
         CR_TRY(launch_lm_route(L, M, b.z, L.Ep, 1, b.idx, b.wt, st));
     }

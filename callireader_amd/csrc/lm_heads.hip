@@ -46,7 +46,7 @@ template <> struct Row8<float> {
 
 template <typename T>
 __global__ __launch_bounds__(256) void lm_heads_kernel(const HeadsArgs p) {
-    __shared__ float cs[2][2][LM_MAX_HEAD / 2];              // [attention, retention][cos, sin][pair]
+    __shared__ __attribute__((aligned(16))) float cs[2][2][LM_MAX_HEAD / 2];      // [attention, retention][cos, sin][pair], read as 16-byte vectors
     __shared__ __attribute__((aligned(16))) float sx[4][512];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int64_t row = blockIdx.x;

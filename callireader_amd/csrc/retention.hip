@@ -34,7 +34,8 @@ constexpr int dec_waves(int NR) { return NR > 16 ? 8 : 16; }
 // workgroups past the heads merge the attention's key splits of the same row (the mixer beside this one), a wave per 64 columns: two short launches in one
 template <typename T, int NR>
 __global__ __launch_bounds__(dec_waves(NR) * 64) void ret_decode_kernel(const RetParams p, const AttnParams merge, int merge_dim) {
-    __shared__ float so[LM_MAX_HEAD], red[LM_MAX_HEAD / 16];
+    __shared__ __attribute__((aligned(16))) float so[LM_MAX_HEAD];
+    __shared__ float red[LM_MAX_HEAD / 16];
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, nw = blockDim.x >> 6;
     const int h = blockIdx.x, row = blockIdx.y;
     if (h >= p.H) {
