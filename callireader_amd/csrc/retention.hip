@@ -155,12 +155,13 @@ __device__ __forceinline__ int3 xcd_block() {
 }
 
 // U[64 dk][64 dv] of one (chunk, head): sum over the chunk's n rows of decay^(n-1-j) k_j v_j^T.  Two tiles of 64 rows are under way while one is multiplied.  Every key column block meets every
-// value column block: those workgroups go to one XCD.  32 chunks of 8 heads, 128 x 256: 37.6 -> 33.4 us
+// value column block: those workgroups go to one XCD.  32 chunks of 8 heads, 128 x 256: 37.6 -> 33.4 us; with
+// one block a head (64 x 64) there is nothing to share, and chunks dealt out in turn take 8.1 us for 8.9
 __global__ __launch_bounds__(256) void ret_chunk_kernel(const RetParams p) {
     __shared__ __attribute__((aligned(16))) char sm[2][3][8192];          // [buffer][v, k, k's remainder][64 rows][64 columns]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int3 blk = xcd_block();
+    const int3 blk = gridDim.x > 1 ? xcd_block() : int3{0, (int)blockIdx.y, (int)blockIdx.z};
     const int kt = blk.x % (p.Kp / 64), vt = blk.x / (p.Kp / 64), h = blk.y;
     const int row0 = p.chunks[2 * blk.z], S = p.chunks[2 * blk.z + 1];
     const float* pw = p.pw + h * (RET_CHUNK + 1);
