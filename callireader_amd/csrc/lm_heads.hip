@@ -45,10 +45,10 @@ template <> struct Row8<float> {
 };
 
 template <typename T>
-__global__ __launch_bounds__(256) void lm_heads_kernel(const HeadsArgs p) {
+__global__ __launch_bounds__(512) void lm_heads_kernel(const HeadsArgs p) {
     __shared__ __attribute__((aligned(16))) float cs[2][2][LM_MAX_HEAD / 2];      // [attention, retention][cos, sin][pair], read as 16-byte vectors
-    __shared__ __attribute__((aligned(16))) float sx[4][512];
-    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    extern __shared__ __attribute__((aligned(16))) float sx[];                    // 512 floats a wave
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), threads = blockDim.x, waves = threads >> 6;
     const int64_t row = blockIdx.x;
     // task t's region; at: the lane's first column of it (past its end: none)
     auto region = [&](int t, int& at) -> LmRegion {
@@ -65,11 +65,11 @@ __global__ __launch_bounds__(256) void lm_heads_kernel(const HeadsArgs p) {
         const LmRegion rg = region(t, at);
         if (at < rg.heads * rg.P) raw.load((const T*)p.in.a + row * p.in.lda + rg.off + at);
     };
-    int t = blockIdx.y * 4 + wave, next, at;
+    int t = blockIdx.y * waves + wave, next, at;
     if (!p.in.part) fetch(t);
     const int seq = p.in.ix.row_seq ? p.in.ix.row_seq[row] : p.in.ix.seqs[row];
     const int pos = p.in.ix.row_pos ? p.in.ix.row_pos[row] : p.in.ix.lens[seq];
-    for (int i = tid; i < p.half_a + p.half_r; i += 256) {
+    for (int i = tid; i < p.half_a + p.half_r; i += threads) {
         const bool r = i >= p.half_a;
         const int j = r ? i - p.half_a : i;
         float s, c;
@@ -78,8 +78,8 @@ __global__ __launch_bounds__(256) void lm_heads_kernel(const HeadsArgs p) {
     }
     if (blockIdx.y == 0) {
         T* ao = (T*)p.in.ao + row * p.ldo;
-        for (int i = p.pad0 + tid; i < p.pad1; i += 256) ao[i] = (T)0.f;
-        for (int i = p.pad2 + tid; i < p.pad3; i += 256) ao[i] = (T)0.f;
+        for (int i = p.pad0 + tid; i < p.pad1; i += threads) ao[i] = (T)0.f;
+        for (int i = p.pad2 + tid; i < p.pad3; i += threads) ao[i] = (T)0.f;
     }
     __syncthreads();
     // cache row of the token, < 0: not kept
@@ -89,7 +89,7 @@ __global__ __launch_bounds__(256) void lm_heads_kernel(const HeadsArgs p) {
         if (slot >= 0) crow = (int64_t)(slot / p.in.ring) * p.G * p.in.ring + slot % p.in.ring;
     } else crow = (int64_t)seq * p.G * p.in.ring + pos % p.in.chunk;
     for (; t < p.tasks; t = next) {
-        next = t + gridDim.y * 4;
+        next = t + gridDim.y * waves;
         const LmRegion rg = region(t, at);
         const bool in = at < rg.heads * rg.P, rq = rg.kind == LM_RQ || rg.kind == LM_RK;
         const int e0 = at & (rg.P - 1), here = at;
@@ -106,7 +106,7 @@ __global__ __launch_bounds__(256) void lm_heads_kernel(const HeadsArgs p) {
             }
         HeadLane hl;
         hl.ask(e0, rg.kind == LM_Q ? p.nq : rg.kind == LM_K ? p.nk : nullptr, rg.kind == LM_Q || rg.kind == LM_K ? p.half_a : rq ? p.half_r : 0, cs[rq][0], cs[rq][1]);
-        hl.apply(rg.P, p.dim, p.eps, &sx[wave][lane * 8], v);
+        hl.apply(rg.P, p.dim, p.eps, &sx[wave * 512 + lane * 8], v);
         if (!in) continue;
         if (rg.kind == LM_Q) st8((T*)p.in.q + row * ((int64_t)rg.heads * rg.P) + here, v);
         else if (rg.kind == LM_K || rg.kind == LM_V) {
@@ -188,9 +188,20 @@ int launch_lm_heads(bool f32, const Lm& lm, const LmLayer& L, int M, const LmHea
     p.pad0 = L.heads() ? a.heads * a.vdim : 0; p.pad1 = L.off_r; p.pad2 = L.off_r + (L.retention() ? r.heads * r.vdim : 0); p.pad3 = L.Gp; p.ldo = L.Gp;
     p.rplane = (int64_t)M * r.heads * L.Kp;
     if (!L.heads()) { p.in.ring = p.in.chunk = 1; }
+    // Waves of a workgroup.  Up to 512 rows: four, the tasks beside each other in workgroups.  Then a row is one workgroup, angles computed once: a wave for every task (or every second ...,
+    // eight at most) while such workgroups are resident at once, 22 waves a CU; then four while these are, and past that even shares of four waves' rounds, so that none stands by while
+    // the last task runs (five or six tasks: three waves).  Two layers, four waves -> these: 700 rows, five tasks 7.2 -> 6.3 us, six 7.1 -> 6.4; 2000 rows, five 11.3 -> 9.9, six 12.1 -> 10.4
+    // (a wave each: 13.0, 15.0); 1000 rows, six: 7.7 with four, 8.0 with three, 9.2 with six.
+    constexpr int RESIDENT = 22 * 256;
+    auto shared = [&](int most) { const int rounds = (p.tasks + most - 1) / most; return (p.tasks + rounds - 1) / rounds; };
+    int waves = 4;
+    if (M > 512) {
+        if ((int64_t)M * shared(8) <= RESIDENT) waves = shared(8);
+        else if ((int64_t)M * 4 > RESIDENT) waves = shared(4);
+    }
     const int y = M <= 512 ? (p.tasks + 3) / 4 : 1;
-    if (f32) hipLaunchKernelGGL(lm_heads_kernel<float>, dim3((unsigned)M, y), dim3(256), 0, st, p);
-    else hipLaunchKernelGGL(lm_heads_kernel<bf16>, dim3((unsigned)M, y), dim3(256), 0, st, p);
+    if (f32) hipLaunchKernelGGL(lm_heads_kernel<float>, dim3((unsigned)M, y), dim3(64 * waves), 2048 * waves, st, p);
+    else hipLaunchKernelGGL(lm_heads_kernel<bf16>, dim3((unsigned)M, y), dim3(64 * waves), 2048 * waves, st, p);
     CR_HIP(hipGetLastError());
     return CR_OK;
 }

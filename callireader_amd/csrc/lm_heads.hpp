@@ -38,6 +38,14 @@ struct HeadLane {
             const int i = e0 < half ? e0 : e0 - half;
             ld8<float>(cos + i, c);
             ld8<float>(sin + i, s);
+        } else if (half % 4 == 0) {
+#pragma unroll
+            for (int e = 0; e < 8; e += 4) {
+                const int q = e0 + e, i = q < half ? q : q < 2 * half ? q - half : 0;
+                const f32x4 cos4 = *(const f32x4*)(cos + i), sin4 = *(const f32x4*)(sin + i);
+#pragma unroll
+                for (int j = 0; j < 4; j++) { c[e + j] = cos4[j]; s[e + j] = sin4[j]; }
+            }
         } else
 #pragma unroll
             for (int e = 0; e < 8; e++) {
@@ -65,7 +73,7 @@ struct HeadLane {
         st8(sx, v);
         __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
         __builtin_amdgcn_wave_barrier();
-        // (which product is rounded alone is spelled out: left to the compiler, entry 0 of every eight had the other one where half % 8 != 0)
+        // (which product is rounded alone is spelled out: left to the compiler, entry 0 of every eight had the other one where entries went one by one)
         if (e0 < 2 * half) {
             if (half % 8 == 0) {
                 const bool first = e0 < half;
@@ -73,6 +81,16 @@ struct HeadLane {
                 ld8<float>(sx + (first ? half : -half), u);
 #pragma unroll
                 for (int e = 0; e < 8; e++) v[e] = fmaf(v[e], c[e], first ? -(u[e] * s[e]) : u[e] * s[e]);
+            } else if (half % 4 == 0) {                        // four entries side by side have their partners side by side
+#pragma unroll
+                for (int e = 0; e < 8; e += 4) {
+                    const int q = e0 + e;
+                    const bool first = q < half;
+                    if (q >= 2 * half) continue;
+                    const f32x4 u = *(const f32x4*)(sx + e + (first ? half : -half));
+#pragma unroll
+                    for (int j = 0; j < 4; j++) v[e + j] = fmaf(v[e + j], c[e + j], first ? -(u[j] * s[e + j]) : u[j] * s[e + j]);
+                }
             } else {
 #pragma unroll
                 for (int e = 0; e < 8; e++) {
