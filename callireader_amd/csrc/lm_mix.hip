@@ -1,6 +1,6 @@
 // One decode step's mixers in one launch: from the fused projection's K-slices to the output projection's input.  A workgroup takes a (row, key head, split of keys) of the attention or a
 // (row, head) of retention, forms its own queries, keys, values and gate from the slices (lm_heads.hpp), and goes on with them on the chip; the caches and states it needs travel meanwhile.
-// What all layers of a step share -- a row's sequence and position, the cos and sin of its angles -- is there already (lm_embed_kernel).
+// What all layers of a step share -- a row's sequence and position, the cos and sin of its angles -- is there already (lm_embed_step_kernel).
 //
 // Bound by latency: with few rows none of it fills the chip, so the chain from the slices to the result is what counts.
 //
