@@ -8,7 +8,22 @@
 
 // units of unit_bytes side by side, unit u read by workgroups whose numbers leave u % 8; fetched in pieces (of a multiple of 16 bytes), a workgroup each.  at null: nothing
 struct L2Ahead { const void* at; int units, unit_bytes, pieces; };
-constexpr int L2_AHEAD_GROUPS = 256;
+constexpr int L2_AHEAD_GROUPS = 256, L2_AHEAD_PIECES = 8;
+
+// `bytes` of weights in `units` equal parts, or nothing where they cannot be cut so.  A power of two of pieces, as long as every fetching workgroup gets at most one.  (The count that just goes round, six for
+// 40 units, cuts at odd addresses and leaves the rest of the division out.  Us a step without fetching / so / in powers of two: float32, 768 wide, 4 and 12 rows 289 / 301 / 282 and 326 / 347 / 328; 640 wide,
+// 4 rows 257 / 270 / 250; bf16, 768 wide, 48 rows 369 / 383 / 371.)
+inline L2Ahead l2_ahead_of(const void* at, int64_t bytes, int units) {
+    if (!at || bytes <= 0 || units <= 0 || bytes % units || bytes / units % 16 || bytes / units > INT32_MAX) return {};
+    L2Ahead a{at, units, (int)(bytes / units), 1};
+    while (a.pieces < L2_AHEAD_PIECES && 2 * a.pieces * units <= L2_AHEAD_GROUPS && a.unit_bytes % (32 * a.pieces) == 0) a.pieces *= 2;
+    return a;
+}
+// A fetching workgroup takes pieces j = nth >> 3, then every L2_AHEAD_GROUPS / 8 further, of the units of its remainder: the offset of piece j's first byte, negative past the last unit
+__host__ __device__ inline int64_t l2_ahead_piece(const L2Ahead& a, int linear, int j) {
+    const int u = (linear & 7) + 8 * (j / a.pieces);
+    return u < a.units ? (int64_t)u * a.unit_bytes + j % a.pieces * (a.unit_bytes / a.pieces) : -1;
+}
 
 // linear: the workgroup's number in its launch; nth: its number among those that do this (linear and nth alike modulo 8), < L2_AHEAD_GROUPS
 __device__ __forceinline__ void l2_ahead(const L2Ahead& a, int linear, int nth) {
@@ -16,11 +31,11 @@ __device__ __forceinline__ void l2_ahead(const L2Ahead& a, int linear, int nth) 
     u32x4_t s = {0u, 0u, 0u, 0u};
     const int bytes = a.unit_bytes / a.pieces, step = (int)blockDim.x * 16;
     for (int j = nth >> 3; j < (a.units + 7) / 8 * a.pieces; j += L2_AHEAD_GROUPS / 8) {
-        const int u = (linear & 7) + 8 * (j / a.pieces);
-        if (u >= a.units) break;
-        const char* p = (const char*)a.at + (int64_t)u * a.unit_bytes + j % a.pieces * bytes;
+        const int64_t off = l2_ahead_piece(a, linear, j);
+        if (off < 0) break;
+        const char* p = (const char*)a.at + off;
         for (int i = threadIdx.x * 16; i < bytes; i += 8 * step) {
-            u32x4_t v[8];
+            u32x4_t v[8];                                     // (past a short piece's end its last vector again; fewer loads there: 1024 wide, a row 440 us a step -> 451)
 #pragma unroll
             for (int q = 0; q < 8; q++) v[q] = *(const u32x4_t*)(p + min(i + q * step, bytes - 16));
 #pragma unroll
@@ -42,4 +57,4 @@ __device__ __forceinline__ void l2_ahead(const L2AheadList& l, int linear, int n
 // workgroups behind the `groups` of a launch's own that make L2_AHEAD_GROUPS fetching ones, which start at a multiple of eight
 inline int l2_ahead_extra(int groups) { return (groups + 7) / 8 * 8 - groups + L2_AHEAD_GROUPS; }
 // number of workgroup `linear` among them (negative, or L2_AHEAD_GROUPS and more: none of them)
-__device__ __forceinline__ int l2_ahead_nth(int linear, int groups) { return linear - (groups + 7) / 8 * 8; }
+__host__ __device__ inline int l2_ahead_nth(int linear, int groups) { return linear - (groups + 7) / 8 * 8; }

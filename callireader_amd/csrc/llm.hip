@@ -408,7 +408,7 @@ int run_layers(cr_ctx* c, cr_kv* kv, bf16* x, int M, bool decode, const std::vec
             ap.nsplit = nsplit; ap.part_ml = part; ap.part_o = part + (size_t)M * NKV * nsplit * (NH / NKV) * 2;
             // wo's 34 MB travel while the attention computes: a step of four layers and the head 458 -> 447 us (1 row, 77 keys), 494 -> 486 (1 x 3164), 538 -> 524 (8 x 100), 611 -> 601 (8 x 3000).  (The first
             // layer's wqkv beside the embedding's rows the same way: no gain)
-            if (w.d_o) ap.ahead = L2Ahead{w.d_o->ptr, D / 16, 16 * D * 2, 1};
+            if (w.d_o) ap.ahead = l2_ahead_of(w.d_o->ptr, (int64_t)D * D * 2, D / 16);
             if (launch_flash_attn_split(ap, HD, st) != CR_OK) return cr_fail(CR_ERR_HIP, "decode attention launch failed");
             DecodeGemmParams dq{};
             dq.M = M; dq.eps = c->d.rms_eps;
@@ -485,7 +485,7 @@ int run_layers(cr_ctx* c, cr_kv* kv, bf16* x, int M, bool decode, const std::vec
             // wo travels beside, by the tiles of its workgroups: a step of four layers and the head 521 -> 511 us (9 rows of 200 keys), 653 -> 634 (13 x 3164), 586 -> 571 (24 x 100), 661 -> 643 (32 x 500),
             // 774 -> 757 (64 x 333); beside the merge of the splits instead a third of that (and the next layer's wqkv beside the update ahead of it, 50 MB for 32 of L2, 1 .. 4 us slower)
             const int o_units = D / (16 * std::max(1, gemm_partial_tiles(D, D)));
-            if (sliced && !f8 && w.d_o && o_units % 8 == 0) ap.ahead = L2Ahead{w.d_o->ptr, o_units, D / o_units * D * 2, std::max(1, L2_AHEAD_GROUPS / o_units)};
+            if (sliced && !f8 && w.d_o && o_units % 8 == 0) ap.ahead = l2_ahead_of(w.d_o->ptr, (int64_t)D * D * 2, o_units);
             if (rope_folded) { ap.qkv_part = pbuf; ap.qkv_splits = s_qkv; ap.qkv_ld = QKV; ap.rope_cos = cosT; ap.rope_sin = sinT; }
             if (launch_flash_attn_split(ap, HD, st) != CR_OK) return cr_fail(CR_ERR_HIP, "decode attention launch failed");
         }

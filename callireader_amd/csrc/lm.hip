@@ -407,8 +407,7 @@ int raw32(cr_ctx* c, const Lm& lm, const void* A, const void* W, float* C, int64
 L2Ahead few_row_reads(const Lm& lm, int M, const void* W, const bf16* dl, int N, int K, bool parts) {
     const int rt = lm.f32 || !parts ? 1 : gemm_partial_tiles(N, K);
     if (!(lm.f32 ? W : dl) || M > 64 || rt <= 0 || N % (128 * rt) || (parts ? one_slice(M, N, K) : !lm.f32 && N > 8192)) return {};
-    const int units = N / (16 * rt);
-    return {lm.f32 ? W : dl, units, 16 * rt * K * (int)lm.esz(), std::max(1, std::min(8, L2_AHEAD_GROUPS / units))};
+    return l2_ahead_of(lm.f32 ? W : dl, (int64_t)N * K * lm.esz(), N / (16 * rt));
 }
 
 // h -> ao, latent attention

@@ -1,0 +1,75 @@
+"""Which bytes the workgroups of csrc/l2_ahead.hpp fetch: its host arithmetic, compiled for this machine and walked as the kernel walks it."""
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+HIPCC = shutil.which('hipcc') or '/opt/rocm/bin/hipcc'
+pytestmark = pytest.mark.skipif(not os.path.exists(HIPCC), reason='hipcc not found')
+
+WALK = r'''
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#include "l2_ahead.hpp"
+
+// units of a weight of N rows and K columns, `tiles` tiles of 16 rows a workgroup of its reader; own workgroups ahead of the fetching ones, `width` of them side by side
+int main(int, char** v) {
+    const long N = atol(v[1]), K = atol(v[2]), es = atol(v[3]), tiles = atol(v[4]), own = atol(v[5]), width = atol(v[6]);
+    static char base;
+    const L2Ahead a = l2_ahead_of(&base, N * K * es, (int)(N / (16 * tiles)));
+    if (!a.at) return puts("nothing"), 0;
+    const long bytes = N * K * es, piece = a.unit_bytes / a.pieces, groups = (own + l2_ahead_extra((int)own) + width - 1) / width * width;
+    std::vector<char> seen(bytes / 16);
+    long most = 0;
+    for (long linear = own; linear < groups; linear++) {
+        const int nth = l2_ahead_nth((int)linear, (int)own);
+        if (nth < 0 || nth >= L2_AHEAD_GROUPS) continue;
+        if ((nth & 7) != (linear & 7)) return puts("remainder"), 1;
+        long took = 0;
+        for (int j = nth >> 3; j < (a.units + 7) / 8 * a.pieces; j += L2_AHEAD_GROUPS / 8) {
+            const long off = l2_ahead_piece(a, (int)linear, j);
+            if (off < 0) break;
+            if (off % 16 || piece % 16 || off + piece > bytes) return printf("piece %ld at %ld\n", piece, off), 1;
+            if (off / a.unit_bytes % 8 != (linear & 7)) return puts("another XCD"), 1;
+            for (long i = off / 16; i < (off + piece) / 16; i++) seen[i]++;
+            took += piece;
+        }
+        most = most > took ? most : took;
+    }
+    for (long i = 0; i < bytes / 16; i++)
+        if (seen[i] != 1) return printf("vector %ld read %d times\n", i, seen[i]), 1;
+    printf("pieces %d most %ld\n", a.pieces, most);
+}
+'''
+
+
+@pytest.fixture(scope='module')
+def walk(tmp_path_factory):
+    d = tmp_path_factory.mktemp('l2_ahead')
+    (d / 'walk.cpp').write_text(WALK)
+    subprocess.run([HIPCC, '-x', 'hip', '--offload-arch=gfx950', '--offload-host-only', '-std=c++17', '-O1', '-I', os.path.join(ROOT, 'callireader_amd', 'csrc'), str(d / 'walk.cpp'), '-o',
+                    str(d / 'walk')], check=True, capture_output=True, timeout=300)
+    return lambda *n: subprocess.run([str(d / 'walk'), *map(str, n)], capture_output=True, text=True, timeout=60)
+
+
+# widths whose tiles eight pieces, or any power of two of them, do not divide evenly among the fetching workgroups; tiles a workgroup as few-row products have them; own workgroups that eight and the
+# grid's width do not divide
+@pytest.mark.parametrize('own,width', [(8, 8), (10, 10), (51, 17), (480, 12)])
+@pytest.mark.parametrize('N,K,es,tiles', [(640, 640, 2, 1), (640, 640, 4, 1), (768, 1152, 4, 1), (1152, 768, 2, 3), (1280, 2560, 2, 2), (2560, 640, 4, 1), (2560, 5120, 2, 4), (4096, 4096, 2, 1), (4096, 4096, 2, 4),
+                                          (4096, 1024, 4, 1), (128, 128, 2, 1), (16, 64, 2, 1), (208, 64, 2, 1)])
+def test_every_byte_once_in_16_byte_vectors_on_its_readers_xcd(walk, N, K, es, tiles, own, width):
+    r = walk(N, K, es, tiles, own, width)
+    assert r.returncode == 0 and r.stdout.startswith('pieces'), r.stdout + r.stderr
+    pieces, most = int(r.stdout.split()[1]), int(r.stdout.split()[3])
+    assert pieces in (1, 2, 4, 8)
+    units = N // (16 * tiles)
+    if -(-units // 8) * 8 * pieces <= 256:                              # a piece a workgroup at most
+        assert most == N * K * es // units // pieces
+
+
+def test_what_cannot_be_cut_is_left_alone(walk):
+    assert walk(100, 64, 2, 1, 8, 8).stdout == 'nothing\n'             # 6 units, which do not divide 12 800 bytes
+    assert walk(8, 64, 2, 1, 8, 8).stdout == 'nothing\n'               # none
