@@ -364,7 +364,8 @@ int launch_decode_t(const LatentDecodeParams& p, hipStream_t st) {
     static std::atomic<uint64_t> done{0};
     if (!cr_dyn_lds_once(done, (const void*)latent_decode_kernel<R, HT>, LDS)) return CR_ERR_HIP;
     const int rows = p.a.M * ((p.a.H + 16 * HT - 1) / (16 * HT));
-    hipLaunchKernelGGL((latent_decode_kernel<R, HT>), dim3(p.nsplit, rows + (p.ahead.at ? (l2_ahead_extra(p.nsplit * rows) + p.nsplit - 1) / p.nsplit : 0)), dim3(256), LDS, st, p);
+    const bool ahead = p.ahead.at && l2_ahead_bytes(p.ahead) <= l2_ahead_beside_latent((int64_t)p.nsplit * rows, cr_device_cus());
+    hipLaunchKernelGGL((latent_decode_kernel<R, HT>), dim3(p.nsplit, rows + (ahead ? (l2_ahead_extra(p.nsplit * rows) + p.nsplit - 1) / p.nsplit : 0)), dim3(256), LDS, st, p);
     const bool few = p.a.M * p.a.H <= cr_device_cus();        // few rows: eight waves share one row's splits
     const int wgs = p.a.H * (few ? p.a.M : (p.a.M + 7) / 8);
     const int z = p.nsplit > 4 ? 1 : 4 * wgs <= cr_device_cus() ? 4 : 2 * wgs <= cr_device_cus() ? 2 : 1;      // (past four splits merging them again costs more than the columns save: 8 rows of 16 heads, 1000 keys, a step 790 / 788 / 810 us with 1 / 2 / 4)

@@ -19,6 +19,11 @@ inline L2Ahead l2_ahead_of(const void* at, int64_t bytes, int units) {
     while (a.pieces < L2_AHEAD_PIECES && 2 * a.pieces * units <= L2_AHEAD_GROUPS && a.unit_bytes % (32 * a.pieces) == 0) a.pieces *= 2;
     return a;
 }
+inline int64_t l2_ahead_bytes(const L2Ahead& a) { return (int64_t)a.units * a.unit_bytes; }
+// Most bytes that go beside `own` workgroups of latent attention.  What the caches do not hold is read twice, and where every second CU has a workgroup of its own the two share its load path.  A step with
+// fetching over one without, few experts, wo of 8 / 32 / 40 / 80 MiB: 1 .. 64 own 1.01 / 1.02 .. 1.05 / 1.04 / 0.98, 96 .. 128 1.01 / 1.00 / 1.02 / 0.96, 192 .. 256 1.00 / 0.98 / 0.99 / 0.94, 448 1.00 /
+// 0.99 / 0.97 / 0.88 (235 MB of 128 heads 0.85 throughout).
+inline int64_t l2_ahead_beside_latent(int64_t own, int cus) { return (int64_t)(2 * own <= cus ? 40 : 8) << 20; }
 // A fetching workgroup takes pieces j = nth >> 3, then every L2_AHEAD_GROUPS / 8 further, of the units of its remainder: the offset of piece j's first byte, negative past the last unit
 __host__ __device__ inline int64_t l2_ahead_piece(const L2Ahead& a, int linear, int j) {
     const int u = (linear & 7) + 8 * (j / a.pieces);

@@ -189,7 +189,7 @@ struct LatentDecodeParams {
     int64_t uv_hs; int vdim;
     const bf16* gate; int64_t ldg;
     bf16* out; int64_t ldo;    // [M][heads * vdim]
-    L2Ahead ahead;             // weights of the output projection
+    L2Ahead ahead;             // weights of the output projection, fetched where that pays (l2_ahead_beside_latent)
 };
 bool latent_decode_supported(int Rp);
 inline size_t latent_part_floats(int M, int H, int nsplit, int Rp) { return (size_t)M * H * nsplit * (Rp + 2); }

@@ -16,7 +16,8 @@ WALK = r'''
 #include "l2_ahead.hpp"
 
 // units of a weight of N rows and K columns, `tiles` tiles of 16 rows a workgroup of its reader; own workgroups ahead of the fetching ones, `width` of them side by side
-int main(int, char** v) {
+int main(int n, char** v) {
+    if (n == 3) return printf("%ld\n", (long)l2_ahead_beside_latent(atol(v[1]), atol(v[2]))), 0;
     const long N = atol(v[1]), K = atol(v[2]), es = atol(v[3]), tiles = atol(v[4]), own = atol(v[5]), width = atol(v[6]);
     static char base;
     const L2Ahead a = l2_ahead_of(&base, N * K * es, (int)(N / (16 * tiles)));
@@ -73,3 +74,9 @@ def test_every_byte_once_in_16_byte_vectors_on_its_readers_xcd(walk, N, K, es, t
 def test_what_cannot_be_cut_is_left_alone(walk):
     assert walk(100, 64, 2, 1, 8, 8).stdout == 'nothing\n'             # 6 units, which do not divide 12 800 bytes
     assert walk(8, 64, 2, 1, 8, 8).stdout == 'nothing\n'               # none
+
+
+def test_beside_latent_attention_as_much_as_the_caches_hold(walk):
+    room = lambda own: int(walk(own, 256).stdout)                      # noqa: E731
+    assert 4096 * 4096 * 2 <= room(1) == room(128) < 5120 * 8192 * 2   # 64 heads of 128 on 5120 columns: more than all L2 caches together
+    assert 2048 * 2048 * 2 <= room(129) == room(512) < 3072 * 3072 * 2
