@@ -8,7 +8,7 @@
 
 // units of unit_bytes side by side, unit u read by workgroups whose numbers leave u % 8; fetched in pieces (of a multiple of 16 bytes), a workgroup each.  at null: nothing
 struct L2Ahead { const void* at; int units, unit_bytes, pieces; };
-constexpr int L2_AHEAD_GROUPS = 256, L2_AHEAD_PIECES = 8;
+constexpr int L2_AHEAD_GROUPS = 256, L2_AHEAD_PIECES = 8, L2_AHEAD_MOST = 5;      // fetching workgroups, pieces of a unit, products of a list
 
 // `bytes` of weights in `units` equal parts, or nothing where they cannot be cut so.  A power of two of pieces, as long as every fetching workgroup gets at most one.  (The count that just goes round, six for
 // 40 units, cuts at odd addresses and leaves the rest of the division out.  Us a step without fetching / so / in powers of two: float32, 768 wide, 4 and 12 rows 289 / 301 / 282 and 326 / 347 / 328; 640 wide,
@@ -24,6 +24,17 @@ inline int64_t l2_ahead_bytes(const L2Ahead& a) { return (int64_t)a.units * a.un
 // fetching over one without, few experts, wo of 8 / 32 / 40 / 80 MiB: 1 .. 64 own 1.01 / 1.02 .. 1.05 / 1.04 / 0.98, 96 .. 128 1.01 / 1.00 / 1.02 / 0.96, 192 .. 256 1.00 / 0.98 / 0.99 / 0.94, 448 1.00 /
 // 0.99 / 0.97 / 0.88 (235 MB of 128 heads 0.85 throughout).
 inline int64_t l2_ahead_beside_latent(int64_t own, int cus) { return (int64_t)(2 * own <= cus ? 40 : 8) << 20; }
+// The same beside `own` workgroups of a decode mixer (lm_mix.hip), with how little it must be to go at all and how many products it may be.  A step with all that fits over one without:
+//   bf16, one key split: up to 256 own 0.98 .. 1.07; 288 .. 960 0.95 .. 1.05 with 34 MiB, 0.97 .. 1.05 with 26; where all that there is are 7 MiB, 320 .. 512 0.97 .. 0.99.
+//   Several splits (retention then streams its states through the caches before the weights' reader starts): up to 256 0.97 .. 1.05, 320 0.98 .. 1.04, 384 .. 1024 0.93 .. 1.03, mostly below one.
+//   float32, whose workgroups have a CU each: up to 128 0.99 .. 1.04; 144 .. 192 0.95 .. 1.03, the first product alone 1.00 .. 1.03 (of 32 MiB 0.99 .. 1.02); 200 .. 256 0.95 .. 1.03 and 0.98 .. 1.03.
+struct L2AheadRoom { int64_t most, least; int products; };
+inline L2AheadRoom l2_ahead_beside_mixer(bool f32, int64_t own, int splits, int cus) {
+    constexpr int64_t MiB = 1 << 20;
+    if (f32) return 2 * own <= cus ? L2AheadRoom{34 * MiB, 0, L2_AHEAD_MOST} : 4 * own <= 3 * cus ? L2AheadRoom{16 * MiB, 0, 1} : L2AheadRoom{};
+    if (own <= cus) return {34 * MiB, 0, L2_AHEAD_MOST};
+    return splits > 1 && 4 * own > 5 * cus ? L2AheadRoom{} : L2AheadRoom{26 * MiB, 8 * MiB, L2_AHEAD_MOST};
+}
 // A fetching workgroup takes pieces j = nth >> 3, then every L2_AHEAD_GROUPS / 8 further, of the units of its remainder: the offset of piece j's first byte, negative past the last unit
 __host__ __device__ inline int64_t l2_ahead_piece(const L2Ahead& a, int linear, int j) {
     const int u = (linear & 7) + 8 * (j / a.pieces);
@@ -52,8 +63,7 @@ __device__ __forceinline__ void l2_ahead(const L2Ahead& a, int linear, int nth) 
 
 // several, one behind the other
 struct L2AheadList {
-    static constexpr int MOST = 6;
-    L2Ahead w[MOST];
+    L2Ahead w[L2_AHEAD_MOST];
     int n;
 };
 __device__ __forceinline__ void l2_ahead(const L2AheadList& l, int linear, int nth) {

@@ -468,25 +468,33 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
     return CR_OK;
 }
 
-// What the products between this mixer and the next read, in the order they read it, as far as it fits into the L2 caches (32 MiB; a little more still gains).  The mixer leaves most of the chip and all of memory idle.  Us a step with nothing / the output projection alone /
-// all that fits (delay in lm_mix.hip): 1024 wide, 14 passes, 1 row 469 / 471 / 443; float32 2 rows 725 / 726 / 708, 8 rows 820 / 817 / 795; 2048 wide, 8 layers, 1 row 453 / 453 / 447, 4 rows 487 / 488 / 482,
-// 32 rows 720 / 723 / 710.
-L2AheadList behind_mixer(const Lm& lm, int M, const LmLayer& L, size_t r) {
+// What the products between this mixer and the next read, in the order they read it, as far as it fits beside the mixer's own workgroups (l2_ahead_beside_mixer): a product that has no such form is left
+// out, the first that is too large ends the list.  The token side's small products (0.3 MB and two launches that wait for each other) are not fetched.  float32 leaves the next projection out as well: 512 wide,
+// 2 rows 204 us a step without any fetching, 205 without it, 214 with it; 1024 wide it does not fit anyway.  Us a step with nothing / the output projection alone / all that fits (delay in lm_mix.hip): 1024 wide, 14
+// passes, 1 row 469 / 471 / 443; float32 2 rows 725 / 726 / 708, 8 rows 820 / 817 / 795; 2048 wide, 8 layers, whose up projection no longer fits, 1 row 453 / 447, 4 rows 487 / 482, 32 rows 720 / 710.
+L2AheadList behind_mixer(const Lm& lm, int M, const LmLayer& L, size_t r, int unit, int splits) {
+    const int64_t own = (L.heads() ? (int64_t)M * (L.s.attn.heads / unit) * (lm.f32 ? 1 : splits) : 0) + (L.retention() && (lm.f32 || splits == 1) ? (int64_t)M * L.s.ret.heads : 0);
+    const L2AheadRoom room = l2_ahead_beside_mixer(lm.f32, own, splits, cr_device_cus());
     L2AheadList l{};
-    int64_t room = (int64_t)34 << 20;
+    int64_t bytes = 0;
+    bool full = false;
     auto add = [&](const void* W, const bf16* dl, int N, int K, bool parts) {      // parts: left in K-slices
         const L2Ahead w = few_row_reads(lm, M, W, dl, N, K, parts);
-        const int64_t bytes = (int64_t)N * K * lm.esz();
-        if (!w.at || bytes > room || l.n == L2AheadList::MOST) { room = 0; return; }
+        if (full || !w.at) return;
+        full = l.n == room.products || bytes + l2_ahead_bytes(w) > room.most;
+        if (full) return;
         l.w[l.n++] = w;
-        room -= bytes;
+        bytes += l2_ahead_bytes(w);
     };
     add(L.wo, L.wo_dl, lm.Wp, L.Gp, true);
-    if (L.s.ff != CR_FF_DENSE) return l;
-    add(L.wgu, L.wgu_dl, L.ffp, lm.Wp, false);
-    add(L.wdn, L.wdn_dl, lm.Wp, L.ffp, true);
+    if (L.s.ff == CR_FF_MOE) return l;
+    if (L.s.ff == CR_FF_DENSE) {
+        add(L.wgu, L.wgu_dl, L.ffp, lm.Wp, false);
+        add(L.wdn, L.wdn_dl, lm.Wp, L.ffp, true);
+    }
     if (r + 1 < lm.passes.size() && lm.starts[r + 1]) add(lm.loop_in, lm.loop_dl, lm.Wp, 2 * lm.Wp, true);
-    if (r + 1 < lm.passes.size()) { const LmLayer& n = lm.layers[lm.passes[r + 1]]; add(n.wa, n.wa_dl, n.Na, lm.Wp, true); }
+    if (r + 1 < lm.passes.size() && !lm.f32) { const LmLayer& n = lm.layers[lm.passes[r + 1]]; add(n.wa, n.wa_dl, n.Na, lm.Wp, true); }
+    if (bytes < room.least) l.n = 0;
     return l;
 }
 
@@ -512,7 +520,7 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
         in.M = M; in.part = b.sl; in.slices = s_a; in.where = b.where; in.ang = b.ang; in.ao = b.ao; in.cache_k = ck; in.cache_v = cv; in.ring = ring; in.chunk = chunk; in.rows = unit; in.nsplit = split ? splits : 1;
         in.state = state;
         if (split) { in.part_o = b.part; in.part_ml = b.part + (size_t)M * a.heads * splits * L.Ap; }
-        const L2AheadList ahead = behind_mixer(lm, M, L, r);
+        const L2AheadList ahead = behind_mixer(lm, M, L, r, unit, splits);
         in.ahead = &ahead;
         return launch_lm_mix(lm.f32, lm, L, in, st);
     }

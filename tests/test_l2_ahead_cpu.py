@@ -18,6 +18,10 @@ WALK = r'''
 // units of a weight of N rows and K columns, `tiles` tiles of 16 rows a workgroup of its reader; own workgroups ahead of the fetching ones, `width` of them side by side
 int main(int n, char** v) {
     if (n == 3) return printf("%ld\n", (long)l2_ahead_beside_latent(atol(v[1]), atol(v[2]))), 0;
+    if (n == 5) {
+        const L2AheadRoom r = l2_ahead_beside_mixer(atoi(v[1]), atol(v[2]), atoi(v[3]), atoi(v[4]));
+        return printf("%ld %ld %d\n", (long)(r.most >> 20), (long)(r.least >> 20), r.products), 0;
+    }
     const long N = atol(v[1]), K = atol(v[2]), es = atol(v[3]), tiles = atol(v[4]), own = atol(v[5]), width = atol(v[6]);
     static char base;
     const L2Ahead a = l2_ahead_of(&base, N * K * es, (int)(N / (16 * tiles)));
@@ -80,3 +84,10 @@ def test_beside_latent_attention_as_much_as_the_caches_hold(walk):
     room = lambda own: int(walk(own, 256).stdout)                      # noqa: E731
     assert 4096 * 4096 * 2 <= room(1) == room(128) < 5120 * 8192 * 2   # 64 heads of 128 on 5120 columns: more than all L2 caches together
     assert 2048 * 2048 * 2 <= room(129) == room(512) < 3072 * 3072 * 2
+
+
+def test_beside_a_mixer_less_where_the_chip_is_full(walk):
+    room = lambda *n: tuple(map(int, walk(*n, 256).stdout.split()))    # noqa: E731  (float32, own workgroups, key splits)
+    assert room(0, 10, 1) == room(0, 256, 4) == (34, 0, 5)
+    assert room(0, 257, 1) == room(0, 320, 2) == (26, 8, 5) and room(0, 321, 2) == (0, 0, 0)
+    assert room(1, 128, 1) == (34, 0, 5) and room(1, 129, 1) == room(1, 192, 1) == (16, 0, 1) and room(1, 193, 1) == (0, 0, 0)
