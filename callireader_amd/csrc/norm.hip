@@ -56,7 +56,8 @@ __device__ __forceinline__ void store_row_e4m3(const NormParams& p, int64_t orow
     }
 }
 
-template <int TPR, int MODE>   // MODE 0: plain rows, 1: pixel-shuffle gather (N = 4096 from [T,1025,1024])
+// MODE 0: plain rows, 1: pixel-shuffle gather (N = 4096 from [T,1025,1024]).  LATE: the gains are asked for behind both sums instead of with the row (launch_layernorm)
+template <int TPR, int MODE, bool LATE>
 __global__ __launch_bounds__(256) void layernorm_kernel(const NormParams p) {
     __shared__ float red[4];
     const int tid = threadIdx.x;
@@ -76,10 +77,9 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const NormParams p) {
         src = p.in + r * p.ld_in + t * 16;
     }
     float x[16], g[16], bb[16], y[16];
+    auto gains = [&]() { load16(p.gamma + t * 16, g); load16(p.beta + t * 16, bb); };
     load16(src, x);
-    load16(p.gamma + t * 16, g);
-    load16(p.beta + t * 16, bb);
-    __builtin_amdgcn_sched_barrier(0);                         // (all loads are on their way together)
+    if (!LATE) { gains(); __builtin_amdgcn_sched_barrier(0); }      // (all loads are on their way together)
     float s = 0.f;
 #pragma unroll
     for (int e = 0; e < 16; e++) s += x[e];
@@ -90,6 +90,7 @@ __global__ __launch_bounds__(256) void layernorm_kernel(const NormParams p) {
     for (int e = 0; e < 16; e++) v = add_sq(v, x[e] - mean);
     const float var = row_sum<TPR>(v, red, tid) * inv_n;
     const float rstd = 1.0f / sqrtf(var + p.eps);
+    if (LATE) gains();
 #pragma unroll
     for (int e = 0; e < 16; e++) y[e] = (x[e] - mean) * rstd * g[e] + bb[e];
     if (live) {
@@ -154,18 +155,22 @@ int launch_add_rmsnorm(bf16* x, const float* part, int splits, int64_t rows, con
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
 
+// Gains are asked for with the row while rows and results fit the memory-side cache (256 MiB), and behind the sums where rows come from memory: the row's loads are what counts then.  Us, behind / with:
+// 1025 rows of 1024 between products 4.90 / 4.68, 8192 and 12 288 rows of 4096 23.3 / 21.5 and 32.1 / 30.4, 65 600 of 1024 39.8 / 39.9; 98 400 72.1 / 74.6, 24 576 of 4096 72.6 / 78.8.  (Both in one kernel
+// hold 66 registers and lose a wave a SIMD.)
 int launch_layernorm(const NormParams& p, int n, int mode, hipStream_t stream) {
     if (p.rows <= 0) return CR_OK;
-    if (mode == 1) {
-        if (n != 4096) return CR_ERR_ARG;
-        hipLaunchKernelGGL((layernorm_kernel<256, 1>), dim3((unsigned)p.rows), dim3(256), 0, stream, p);
-    } else if (n == 1024) {
-        hipLaunchKernelGGL((layernorm_kernel<64, 0>), dim3((unsigned)((p.rows + 3) / 4)), dim3(256), 0, stream, p);
-    } else if (n == 4096) {
-        hipLaunchKernelGGL((layernorm_kernel<256, 0>), dim3((unsigned)p.rows), dim3(256), 0, stream, p);
-    } else {
-        return CR_ERR_ARG;
-    }
+    if ((n != 1024 && n != 4096) || (mode == 1 && n != 4096)) return CR_ERR_ARG;
+    const bool late = (int64_t)p.rows * n * 4 > (int64_t)256 << 20;
+    const dim3 grid((unsigned)(n == 1024 ? (p.rows + 3) / 4 : p.rows)), block(256);
+    auto launch = [&](auto l) {
+        constexpr bool LATE = decltype(l)::value;
+        if (mode == 1) hipLaunchKernelGGL((layernorm_kernel<256, 1, LATE>), grid, block, 0, stream, p);
+        else if (n == 1024) hipLaunchKernelGGL((layernorm_kernel<64, 0, LATE>), grid, block, 0, stream, p);
+        else hipLaunchKernelGGL((layernorm_kernel<256, 0, LATE>), grid, block, 0, stream, p);
+    };
+    if (late) launch(std::true_type{});
+    else launch(std::false_type{});
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
 

@@ -462,6 +462,16 @@ def test_layernorm(E, rows, n):
     torch.testing.assert_close(out.float(), ref, rtol=RTOL, atol=1e-2)
 
 
+@pytest.mark.parametrize('rows,n', [(65536, 1024), (65537, 1024), (16384, 4096), (16385, 4096)])
+def test_layernorm_of_many_rows_has_the_bits_of_few(E, rows, n):
+    """Past 256 MiB of rows and results the gains are loaded behind the sums: the last rows alone, and those of either side of that line, give one bit pattern."""
+    g = torch.Generator(device='cuda').manual_seed(rows)
+    x = torch.randn(rows, n, device='cuda', generator=g).to(torch.bfloat16)
+    gamma, beta = (torch.randn(n, device='cuda', generator=g).to(torch.bfloat16) for _ in range(2))
+    whole, last = E.op_layernorm(x, gamma, beta, 1e-6), E.op_layernorm(x[-37:].contiguous(), gamma, beta, 1e-6)
+    assert torch.isfinite(whole.float()).all() and torch.equal(whole[-37:], last)
+
+
 def test_layernorm_pixel_shuffle(E):
     from oracle import vision
     g = torch.Generator().manual_seed(6)
