@@ -493,8 +493,9 @@ __global__ __launch_bounds__(256, 4) void vit_attn_kernel(const AttnParams p) {
 // The same blocks for launches of few tiles, in halves of 64 queries under eight waves: four waves share 32 queries, so that the whole chip works on one tile (16 heads: 256 workgroups, where blocks of 128
 // left half the CUs idle and one wave a SIMD) and a wave's chain is a quarter as long.  Of a step of 128 keys each of the four takes 32: scores, softmax, its probabilities to LDS; a step later, under the
 // next softmax, two of them multiply all 128 by one half of V's columns each and a third adds the row sums.  Every accumulator sees the keys in the order it sees them above, so the bits are the same
-// whichever form a launch takes.  Bound by the instructions of a step (some 180 a wave, two waves a SIMD) and the launch's own ramps.  One tile of 16 heads and 1025 tokens: 20.7 us in blocks of 128, 15.7
-// with a barrier between probabilities and product, 13.8 with the product under the next softmax, the prologue's loads and a step's fragments asked for at once and running pointers for the tiles.
+// whichever form a launch takes.  Bound by the instructions of a step (some 180 a wave, two waves a SIMD) and the launch's own ramps.  One tile of 16 heads and 1025 tokens, this kernel alone in a
+// trace: 20.7 us in blocks of 128, 15.7 with a barrier between probabilities and product, 13.8 with the product under the next softmax, the prologue's loads and a step's fragments asked for at once and running
+// pointers for the tiles.
 constexpr int FEW_KV = 2 * TILE, FEW_STEP = 2 * FEW_KV, FEW_P = 3 * FEW_STEP, FEW_LDS = FEW_P + 2 * 2 * 4 * 2048;      // LDS: three steps of two tiles (K, V); then, for two steps, P[group][32 keys][k step][lane] x 16 bytes
 
 __global__ __launch_bounds__(512, 2) void vit_attn_few_kernel(const AttnParams p) {
@@ -818,9 +819,10 @@ int launch_vit_attn(const AttnParams& p, hipStream_t stream) {
     const char* e_nw = getenv("CR_VIT_ATTN_NW");                 // read per call (a bench flips it in one process)
     const bool two_waves = e_nw && e_nw[0] == '2';
     const int nb = (p.Sq - 1) / 128;
-    // Halves of blocks while they are all on the chip at once, a CU each.  Launches with their class rows' merge, 16 heads of 1025 tokens, blocks | halves: 1 tile 21.6 | 15.6 us, 2 tiles 22.5 | 24.2, 3 tiles
-    // 26.7 | 33.0, 11 tiles 66.7 | 114.8 (each key tile is staged twice as often).
-    const bool few = (int64_t)p.B * p.H * nb <= 128;
+    // Halves of blocks while they are all on the chip at once, a CU each.  Attention and its class rows' merge, us with blocks | halves: 16 heads of 1025 tokens, 1 tile 21.6 | 14.7, 2 tiles 22.5 | 24.2, 3 tiles
+    // 26.7 | 33.0, 11 tiles 66.7 | 114.8 (each key tile is staged twice as often); up to 128 blocks, 1 to 64 heads in 1 to 16 tiles: 257 tokens 15.5 | 13.7, 513 21 | 16.5, 1025 20.5 .. 22 | 13.1 .. 14.8,
+    // 1281 37.7 | 28.8, 2049 50 | 39, 4097 88 | 66.
+    const bool few = 2 * (int64_t)p.B * p.H * nb <= cr_device_cus();
     AttnParams q = p;
     q.part_o = p.part_ml + (size_t)p.B * p.H * (4 * nb + 1) * 2;       // one allocation: [m, l] pairs, then the O partials
     if (two_waves) hipLaunchKernelGGL(vit_attn2_kernel, dim3(nb, p.H, p.B), dim3(128), LDS, stream, q);
