@@ -52,7 +52,8 @@ constexpr int FOLD_MAX_SPLITS = 8;       // K-slices of the wqkv partial-sum GEM
 // slot are one DPP row); the six bf16 rows meet in 1.5 KiB of LDS behind one barrier.  q is read from there; the workgroup whose split holds the new position also
 // stores the K / V row to the cache and puts it into the registers of the lanes that would have loaded it (every lane at or past the new position: the cache row
 // itself is not written yet when they load it).  The same fp32 sums, the same roundings: a row's bits do not depend on which form its batch takes.
-template <bool DIV, bool FOLD = false>
+// AHEAD: workgroups past the rows bring the next product's weights into L2 (launch_decode_attn)
+template <bool DIV, bool FOLD, bool AHEAD>
 __global__ __launch_bounds__(256, 2) void decode_attn_kernel(const AttnParams p) {
     __shared__ __attribute__((aligned(16))) float s_o[16][NQ][HD];      // the workgroup's 16 partials: un-normalised O ...
     __shared__ float s_ml[16][NQ][2];                                   // ... maximum and row sum
@@ -60,7 +61,7 @@ __global__ __launch_bounds__(256, 2) void decode_attn_kernel(const AttnParams p)
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int split = blockIdx.x, head = blockIdx.y, batch = blockIdx.z;
-    if (batch >= p.B) {                                       // (uniform)
+    if (AHEAD && batch >= p.B) {                              // (uniform)
         const int plane = gridDim.x * gridDim.y, nth = (batch - p.B) * plane + head * gridDim.x + split;
         __builtin_amdgcn_s_sleep(48);                         // (about 1.3 us: the rows' own keys and values first.  Without it the launch takes 9.3 us for 7.7, with it 8.1)
         if (nth < L2_AHEAD_GROUPS) l2_ahead(p.ahead, p.B * plane + nth, nth);
@@ -93,7 +94,7 @@ __global__ __launch_bounds__(256, 2) void decode_attn_kernel(const AttnParams p)
         for (int h = 0; h < NQ; h++) q[h] = *(const bf16x8*)(qp + (int64_t)h * p.q_rs);
     } else if (fslot < 6) {
         const float* pp = p.qkv_part + (int64_t)batch * p.qkv_ld + (head * 6 + fslot) * HD + c * 8;
-        const int64_t sstep = (int64_t)p.B * p.qkv_ld;
+        const int64_t sstep = (int64_t)(AHEAD ? p.B : (int)gridDim.z) * p.qkv_ld;
 #pragma unroll
         for (int s = 0; s < FOLD_MAX_SPLITS; s++) {
             const f32x4* ps = (const f32x4*)(pp + (int64_t)min(s, p.qkv_splits - 1) * sstep);
@@ -259,14 +260,19 @@ bool decode_attn_fold_supported(const AttnParams& p, int head_dim) {
            (((uintptr_t)p.qkv_part | (uintptr_t)p.rope_cos | (uintptr_t)p.rope_sin) & 15) == 0;
 }
 
+// The weights go along only where the rows' own keys leave the caches room for them, in a kernel of its own: the branch alone costs the other one 2 % (64 rows of 3164 keys 146.1 us a launch, 149.1).
 int launch_decode_attn(const AttnParams& p, hipStream_t stream) {
-    const bool ahead = p.ahead.at && p.H * p.nsplit % 8 == 0;
-    const dim3 grid(p.nsplit, p.H, p.B + (ahead ? (L2_AHEAD_GROUPS + p.nsplit * p.H - 1) / (p.nsplit * p.H) : 0));
-    if (p.qkv_part) {
-        if (!decode_attn_fold_supported(p, HD)) return CR_ERR_ARG;
-        if (p.s_div != 1.0f) hipLaunchKernelGGL((decode_attn_kernel<true, true>), grid, dim3(256), 0, stream, p);
-        else hipLaunchKernelGGL((decode_attn_kernel<false, true>), grid, dim3(256), 0, stream, p);
-    } else if (p.s_div != 1.0f) hipLaunchKernelGGL((decode_attn_kernel<true, false>), grid, dim3(256), 0, stream, p);
-    else hipLaunchKernelGGL((decode_attn_kernel<false, false>), grid, dim3(256), 0, stream, p);
+    const int own = p.nsplit * p.H;
+    const bool ahead = p.ahead.at && own % 8 == 0 && l2_ahead_beside_attention((int64_t)own * p.B, cr_device_cus());
+    const dim3 grid(p.nsplit, p.H, p.B + (ahead ? (L2_AHEAD_GROUPS + own - 1) / own : 0));
+    if (p.qkv_part && !decode_attn_fold_supported(p, HD)) return CR_ERR_ARG;
+    auto launch = [&](auto div, auto fold, auto with) {
+        hipLaunchKernelGGL((decode_attn_kernel<decltype(div)::value, decltype(fold)::value, decltype(with)::value>), grid, dim3(256), 0, stream, p);
+    };
+    const std::true_type yes{};
+    const std::false_type no{};
+    auto with = [&](auto div, auto fold) { ahead ? launch(div, fold, yes) : launch(div, fold, no); };
+    auto folded = [&](auto div) { p.qkv_part ? with(div, yes) : with(div, no); };
+    p.s_div != 1.0f ? folded(yes) : folded(no);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }

@@ -20,6 +20,9 @@ inline L2Ahead l2_ahead_of(const void* at, int64_t bytes, int units) {
     return a;
 }
 inline int64_t l2_ahead_bytes(const L2Ahead& a) { return (int64_t)a.units * a.unit_bytes; }
+// Whether wo's 34 MB go beside `own` workgroups of 256 keys each of the chat model's attention.  A step of four layers and the head with fetching over one without: 72 .. 2560 own 1.02 .. 1.04, 4096 (64 rows of
+// 2000 keys) and 4608 1.01, 4992 and 5760 1.00, 6656 and 8192 (64 rows of 3164 and 3900) 0.99.
+inline bool l2_ahead_beside_attention(int64_t own, int cus) { return own <= 20 * cus; }
 // Most bytes that go beside `own` workgroups of latent attention.  What the caches do not hold is read twice, and where every second CU has a workgroup of its own the two share its load path.  A step with
 // fetching over one without, few experts, wo of 8 / 32 / 40 / 80 MiB: 1 .. 64 own 1.01 / 1.02 .. 1.05 / 1.04 / 0.98, 96 .. 128 1.01 / 1.00 / 1.02 / 0.96, 192 .. 256 1.00 / 0.98 / 0.99 / 0.94, 448 1.00 /
 // 0.99 / 0.97 / 0.88 (235 MB of 128 heads 0.85 throughout).

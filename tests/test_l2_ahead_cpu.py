@@ -18,6 +18,7 @@ WALK = r'''
 // units of a weight of N rows and K columns, `tiles` tiles of 16 rows a workgroup of its reader; own workgroups ahead of the fetching ones, `width` of them side by side
 int main(int n, char** v) {
     if (n == 3) return printf("%ld\n", (long)l2_ahead_beside_latent(atol(v[1]), atol(v[2]))), 0;
+    if (n == 4) return printf("%d\n", (int)l2_ahead_beside_attention(atol(v[1]) * atol(v[2]), atoi(v[3]))), 0;
     if (n == 5) {
         const L2AheadRoom r = l2_ahead_beside_mixer(atoi(v[1]), atol(v[2]), atoi(v[3]), atoi(v[4]));
         return printf("%ld %ld %d\n", (long)(r.most >> 20), (long)(r.least >> 20), r.products), 0;
@@ -78,6 +79,12 @@ def test_every_byte_once_in_16_byte_vectors_on_its_readers_xcd(walk, N, K, es, t
 def test_what_cannot_be_cut_is_left_alone(walk):
     assert walk(100, 64, 2, 1, 8, 8).stdout == 'nothing\n'             # 6 units, which do not divide 12 800 bytes
     assert walk(8, 64, 2, 1, 8, 8).stdout == 'nothing\n'               # none
+
+
+def test_beside_attention_until_its_keys_need_the_caches(walk):
+    takes = lambda rows, keys: walk(rows, 8 * -(-keys // 256), 256).stdout == '1\n'      # noqa: E731
+    assert takes(1, 77) and takes(13, 3164) and takes(64, 2000) and takes(32, 4500)
+    assert not takes(64, 3164) and not takes(64, 3900)
 
 
 def test_beside_latent_attention_as_much_as_the_caches_hold(walk):
