@@ -112,8 +112,9 @@ def test_decoded_state_steps_as_prompts_do(dim):
 @pytest.mark.parametrize('rows', [1, 3, 8])
 @pytest.mark.parametrize('width,ff,ret_heads', [(1024, 640, 1), (1152, 1152, 3), (2048, 4096, 4)])
 def test_weights_fetched_beside_a_mixer(width, ff, ret_heads, rows, dtype, monkeypatch):
-    """Behind a mixer's own workgroups others read the next products' weights: counts of workgroups and of weight tiles that eight does and does not divide, products that are left out of it, the
-    last layer of a span with the embedding's product next and the last of all with none.  The separate kernels fetch nothing: the same bits."""
+    """Behind a mixer's own workgroups others read the next products' weights: counts of own workgroups that eight does and does not divide, products of tiles that eight does not divide, which are left
+    out, the last layer of a span with the embedding's product next and the last of all with none.  The separate kernels fetch nothing: the same bits, for reading leaves nothing behind.  What is
+    read is tests/test_l2_ahead_cpu.py's to say."""
     from callireader_amd.modeling_decoder import LugasunForCausalLM
     layer = LC.layer(LC.heads(2, 1, 64, 64, 64), LC.ret(64, 64, (0.97,) * ret_heads), ff)
     cfg = LC.config(width, 90, [layer, layer, LC.layer(LC.heads(1, 1, 64, 40, 64), LC.ret(16, 16, (0.9,)), None)], side=24, loop=(1, 2, 2))

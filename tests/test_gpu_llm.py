@@ -340,6 +340,27 @@ def test_decode_layout_of_the_weights_gives_the_same_bits(rows):
     assert float(outs[0][6].abs().max()) > 0 and float(outs[0][1].abs().max()) > 0
 
 
+def test_decode_beside_fetched_weights_has_the_bits_of_the_plain_kernels(setup, monkeypatch):
+    """The attention of a decode step that brings wo into L2 beside it (up to 8 rows, and 9 to 64 with the rotation folded in; one and two key splits, a last plane of the grid that is not full) and that of
+    a context without decode-layout copies, which fetches nothing: the same bits."""
+    from callireader_amd.engine import Engine
+    monkeypatch.setenv('CR_DECODE_LAYOUT', '0')
+    plain = Engine(setup['dims'], max_pos=2048)
+    plain.load_state_dict(setup['sd']); plain.load_rope(); plain.finalize()
+    monkeypatch.delenv('CR_DECODE_LAYOUT')
+    for rows, S in ((1, 20), (5, 270), (9, 30), (33, 260)):
+        embs = [prompt(S + i % 3, 70 + i).cuda() for i in range(rows)]
+        given = torch.arange(3, 3 + rows)
+        got = []
+        for e in (setup['eng'], plain):
+            kv = e.kv_alloc(rows, S + 8)
+            e.prefill_batch(kv, list(range(rows)), embs)
+            got.append(torch.stack([e.decode(kv, list(range(rows)), force_tokens=given + t, want_logits=True) for t in range(3)]).cpu())
+            kv.free()
+        assert torch.isfinite(got[0]).all() and torch.equal(*got), (rows, S)
+    plain.close()
+
+
 def test_decode_graph_replay_equals_plain_launches(setup):
     """CR_DECODE_GRAPH=1 (opt-in): the decode step captured as a hipGraph and replayed -- across a change of the number
     of attention splits (a second capture) and with prefills in between -- generates exactly the plain path's ids."""
