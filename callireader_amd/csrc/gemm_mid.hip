@@ -1,11 +1,11 @@
 // bf16 MFMA GEMM for the row counts between decode (gemm_skinny.hip) and the persistent 256x256 kernel (gemm256.hip):  C = epi(A[M,K] . W[N,K]^T),  K % 64 == 0.
 //
-// What bounds these shapes is not arithmetic but how many bytes are under way: a 128x128 grid over M = 1025, N = 1024 is 72 workgroups, and a K loop that waits for each K-tile's
+// What bounds these shapes is neither arithmetic nor bytes but the chain of a K-tile's step: a 128x128 grid over M = 1025, N = 1024 is 72 workgroups, and a K loop that waits for each K-tile's
 // loads before it asks for the next-but-one pays a memory round trip per 64 of K.  So (a) the tile shape is a template and picked by the grid it gives (gemm_mid_cost below), down to
-// 16 x 32 for two waves, and (b) NBUF K-tiles live in LDS and NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles.
+// 16 x 32 for two waves, (b) NBUF K-tiles live in LDS and up to NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles, and (c) a step has no
+// branches and no address arithmetic.
 //   * one global_load_lds_dwordx4 brings eight rows x 64 k, whole 128-byte lines (pieces of 16 rows x 32 k reach 56 of the 69 GB/s per CU that these do on cold weights);
 //     LDS rows of 128 bytes, the 16-byte chunk XORed with (row >> 1) & 7 on both sides: a fragment's ds_read_b128 is free of bank conflicts;
-//   * the steps and their waits are k_ring.hpp's;
 //   * the weights are the MFMA's A operand: a lane's accumulator holds four consecutive columns of one row; what a column can do by itself happens there, and bf16 rows leave in whole
 //     16-byte chunks through a stage in the K-tile buffers (epilogue_staged; ragged edges and fp32 straight from the accumulators);
 //   * a row tile's fragments past M are neither read nor multiplied (M = 1025: the last row costs a sixteenth of a tile, not a tile);
@@ -206,15 +206,32 @@ __device__ __forceinline__ void epilogue(const GemmParams& p, const f32x4 (&acc)
     }
 }
 
+template <int N, int I = 0, typename F>
+__device__ __forceinline__ void constexpr_for(F f) {
+    if constexpr (I < N) { f(std::integral_constant<int, I>{}); constexpr_for<N, I + 1>(f); }
+}
+// the last J K-tiles after the one being multiplied: each has landed, for every wave, when f(even) reads it
+template <int J, int PER, bool EVEN = true, typename F>
+__device__ __forceinline__ void ring_tail(F f) {
+    if constexpr (J > 0) {
+        wait_vm<(J - 1) * PER>();
+        __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
+        f(std::integral_constant<bool, EVEN>{});
+        ring_tail<J - 1, PER, !EVEN>(f);
+    }
+}
+
 // WM x WN waves of FM x FN fragments of 16 x 16
 template <int WM, int WN, int FM, int FN, int NBUF>
 struct MidGeom {
-    static constexpr int BM = WM * FM * 16, BN = WN * FN * 16, WAVES = WM * WN, PIECES = (BM + BN) / 8, PER = (PIECES + WAVES - 1) / WAVES, STAGE = PIECES * 1024, LDS = NBUF * STAGE;
+    static constexpr int BM = WM * FM * 16, BN = WN * FN * 16, WAVES = WM * WN, PIECES = (BM + BN) / 8, PER = (PIECES + WAVES - 1) / WAVES, STAGE = PIECES * 1024, ROUND = NBUF % 2 ? 2 * NBUF : NBUF, PAD = (ROUND * 128 + 511) / 512 * 512, LDS = PAD + NBUF * STAGE;
     static_assert(WAVES * 32 * (FN * 32 + 16) <= LDS, "the epilogue's stage lies in the buffers");
-    static_assert((NBUF - 2) * PER <= 63 && NBUF >= 2 && LDS <= 160 * 1024, "vmcnt is six bits wide; a CU has 160 KiB");
+    static_assert((NBUF - 1) * PER <= 63 && NBUF >= 3 && LDS <= 160 * 1024, "vmcnt is six bits wide; a CU has 160 KiB");
 };
 
-template <int WM, int WN, int FM, int FN, int NBUF>
+template <int WM, int WN, int FM, int FN, int NBUF, bool FAR>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams p, const int epi, const int ntm) {
     typedef MidGeom<WM, WN, FM, FN, NBUF> G;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -237,24 +254,58 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
 
     // ---- this wave's pieces of a K-tile: eight rows of A or W, all 64 k (128 bytes a row); numbers past the last repeat it ----
     // (pieces of rows past the tile's move one lane's 16 bytes: the count of instructions under way stays a constant)
-    const bf16* src[G::PER];
-    int dst[G::PER];
-    bool dead[G::PER];
+    // A piece's first row is the same for all lanes, so its address is a scalar one; a lane's own row and chunk are 32 bits beyond it.
+    // (FAR: rows so far apart that eight of them span 4 GiB; a lane's address is 64 bits then.)
+    const char *src[G::PER], *lane_src[FAR ? G::PER : 1];
+    unsigned off[G::PER], dst[G::PER];
+    uint64_t lanes[G::PER];
+    const unsigned smem_base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
 #pragma unroll
     for (int i = 0; i < G::PER; i++) {
         const int piece = min(wave + i * G::WAVES, G::PIECES - 1), row = piece * 8 + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
-        const bf16* at = piece * 8 < G::BM ? p.A + (int64_t)min(m0 + row, p.M - 1) * p.lda : p.W + (int64_t)min(n0 + row - G::BM, p.N - 1) * p.ldw;
-        src[i] = at + chunk * 8 + (int64_t)blockIdx.y * nk * 64;
-        dst[i] = piece * 1024;
-        dead[i] = piece * 8 < G::BM && piece >= 2 * fn;
+        const bool a = piece * 8 < G::BM;
+        const int first = a ? min(m0 + piece * 8, p.M - 1) : min(n0 + piece * 8 - G::BM, p.N - 1), own = a ? min(m0 + row, p.M - 1) : min(n0 + row - G::BM, p.N - 1);
+        src[i] = (const char*)((a ? p.A + (int64_t)first * p.lda : p.W + (int64_t)first * p.ldw) + (int64_t)blockIdx.y * nk * 64);
+        if (FAR) lane_src[FAR ? i : 0] = src[i] + (int64_t)(own - first) * (a ? p.lda : p.ldw) * 2 + chunk * 16;
+        off[i] = (unsigned)((own - first) * (a ? p.lda : p.ldw) * 2) + chunk * 16;
+        dst[i] = smem_base + G::PAD + piece * 1024;
+        lanes[i] = a && piece >= 2 * fn ? 1 : ~0ull;
     }
-    auto ask = [&](int kt, int buf) {
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"               // (m0 is a reserved register: nothing else here uses it)
+    // LDS-DMA from inline asm (the compiler lets every LDS read wait for all others while one that it knows is under way); the loop below waits for its landing by hand.  The instruction's offset, K-tile
+    // U of an unrolled run, is added to both addresses: G::PAD keeps the LDS one positive.  All lanes are on here, before and after
+    auto ask1 = [&](auto i, auto u, unsigned at) __attribute__((always_inline)) {
+        constexpr int I = decltype(i)::value, O = decltype(u)::value * 128;
+        const unsigned o = off[I], d = dst[I], to = at - O;
+        const char* g = src[I];
+        if constexpr (FAR) {
+            const char* v = lane_src[I];
+            const uint64_t on = lanes[I];
+            asm volatile("s_add_u32 m0, %1, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, off offset:%4\n\ts_mov_b64 exec, -1" ::"v"(v), "s"(d), "s"(to), "s"(on), "n"(O) : "m0", "scc", "memory");
+        } else if constexpr (I * G::WAVES * 8 < G::BM) {
+            const uint64_t on = lanes[I];
+            asm volatile("s_add_u32 m0, %2, %3\n\ts_mov_b64 exec, %4\n\tglobal_load_lds_dwordx4 %0, %1 offset:%5\n\ts_mov_b64 exec, -1" ::"v"(o), "s"(g), "s"(d), "s"(to), "s"(on), "n"(O) : "m0", "scc", "memory");
+        } else asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%4" ::"v"(o), "s"(g), "s"(d), "s"(to), "n"(O) : "m0", "scc", "memory");
+    };
+#pragma clang diagnostic pop
+    // K-tile u of the run that `src` stands at, into buffer buf
+    auto ask = [&](auto u, int buf) __attribute__((always_inline)) {
+        constexpr_for<G::PER>([&](auto i) {
+            CR_DIAG_POISON(smem + G::PAD + buf * G::STAGE + (dst[decltype(i)::value] - smem_base - G::PAD))
+            ask1(i, u, buf * G::STAGE);
+        });
+    };
+    auto advance = [&](int tiles) {
 #pragma unroll
         for (int i = 0; i < G::PER; i++) {
-            CR_DIAG_POISON(smem + buf * G::STAGE + dst[i])
-            if (!dead[i] || lane == 0) __builtin_amdgcn_global_load_lds(CR_GLB(src[i] + (int64_t)kt * 64), CR_LDS(smem + buf * G::STAGE + dst[i]), 16, 0, 0);
+            if (FAR) lane_src[FAR ? i : 0] += tiles * 128;
+            else src[i] += tiles * 128;
         }
     };
+    constexpr std::integral_constant<int, 0> here{};
+
+    auto arrive = [&](int t) { ring_arrive<NBUF, G::PER>(nk, t); };
 
     f32x4 acc[FM][FN];
 #pragma unroll
@@ -267,7 +318,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
 
     struct Frags { bf16x8 a[2][FM], w[2][FN]; };
     auto read = [&](Frags& f, int buf, auto count) {
-        const char* s = smem + buf * G::STAGE;
+        const char* s = smem + G::PAD + buf * G::STAGE;
 #pragma unroll
         for (int h = 0; h < 2; h++) {
 #pragma unroll
@@ -287,36 +338,112 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
                     for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f.w[h][j], f.a[h][i], acc[i][j], 0, 0, 0);
                 }
     };
-    auto arrive = [&](int t) { ring_arrive<NBUF, G::PER>(nk, t); };
+    // Tile kt's fragments are read a step ahead.  With four buffers the tile asked for in step kt goes where tile kt lay, whose reads the step's barrier waits for; with more (LATE) where tile kt - 1 lay,
+    // which was multiplied before the barrier, so that no LDS read has to have come back by then.  These loops are not bound by bytes (64 x 64 tiles, K = 4096: 256 workgroups take little longer than one;
+    // a CU brings in 130 GB/s from its L2 and 480 from LDS) but by a step's chain -- branches, addresses, barrier, LDS reads -- and by how far ahead a K-tile is asked for.  So nothing in a step is
+    // conditional or computes an address (LEAN; three buffers are tiles so large that it spilled), and one workgroup a CU takes all the buffers there are.  1025 x 1024 x 4096 23.5 -> 18.7 us, 1025 x 1024 x
+    // 1024 9.0 -> 7.9, 1025 x 3072 x 1024 12.6 -> 11.5, 1531 x 2048 x 2048 20.5 -> 18.0; tiles of 16 x 32 and 32 x 64 on every CU 62 -> 42, 32.8 -> 27.8.
+    constexpr bool LATE = NBUF > 4, LEAN = NBUF > 3;
+    constexpr int AHEAD = LATE ? NBUF - 1 : NBUF;             // K-tiles asked for beyond the one being multiplied
     auto loop = [&](auto count) {
-        for (int t = 0; t < min(NBUF - 1, nk); t++) ask(t, t);
         Frags f0, f1;
-        arrive(0);
-        if (NBUF - 1 < nk) ask(NBUF - 1, NBUF - 1);
+        int kt = 0, buf = 0;                                  // buffer of tile kt
+        auto more = [&](int buf) { ask(here, buf); advance(1); };
+        if constexpr (!LEAN) {
+            for (int t = 0; t < min(NBUF - 1, nk); t++) more(t);
+            arrive(0);
+            if (NBUF - 1 < nk) more(NBUF - 1);
+            read(f0, 0, count);
+            auto step = [&](int kt, Frags& now, Frags& next) {
+                arrive(kt + 1);
+                if (kt + NBUF < nk) more(buf);                // the buffer that tile kt was read from
+                buf = buf + 1 == NBUF ? 0 : buf + 1;
+                read(next, buf, count);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(now, count);
+            };
+            for (; kt + 2 < nk; kt += 2) {                    // (no read of the loop is conditional: the compiler waited for it ahead of the multiplications then)
+                step(kt, f0, f1);
+                step(kt + 1, f1, f0);
+            }
+            if (kt + 1 < nk) {
+                step(kt, f0, f1);
+                multiply(f1, count);
+            } else multiply(f0, count);
+            return;
+        }
+        for (int t = 0; t < min(AHEAD, nk); t++) more(t);
+        if (nk < AHEAD) {                                     // all of K is under way at once
+            for (; kt < nk; kt++) {
+                wait_tail<AHEAD - 2, G::PER>(nk - 1 - kt);
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+                read(f0, kt, count);
+                multiply(f0, count);
+            }
+            return;
+        }
+        wait_vm<(AHEAD - 1) * G::PER>();
+        __builtin_amdgcn_s_waitcnt(0xC07F);                   // lgkmcnt(0): with a scalar load under way the loop's LDS reads could not be counted
+        __builtin_amdgcn_s_barrier();
+        __builtin_amdgcn_sched_barrier(0);
         read(f0, 0, count);
-        int buf = 0;                                          // buffer of tile kt
-        auto step = [&](int kt, Frags& now, Frags& next) {
-            arrive(kt + 1);
-            if (kt + NBUF < nk) ask(kt + NBUF, buf);          // the buffer that tile kt was read from
-            buf = buf + 1 == NBUF ? 0 : buf + 1;
-            read(next, buf, count);
+        // now in buffer b, next in the one behind; u: K-tiles since `src` was moved
+        auto step = [&](auto u, int b, Frags& now, Frags& next) __attribute__((always_inline)) {
+            wait_vm<(AHEAD - 2) * G::PER>();
+            if (!LATE) __builtin_amdgcn_s_waitcnt(0xC07F);
             __builtin_amdgcn_sched_barrier(0);
+            __builtin_amdgcn_s_barrier();
+            __builtin_amdgcn_sched_barrier(0);
+            ask(u, !LATE ? b : b == 0 ? NBUF - 1 : b - 1);
+            read(next, b + 1 == NBUF ? 0 : b + 1, count);
+            __builtin_amdgcn_sched_barrier(0);
+            if (LATE) {                                       // `now` has come, `next` is under way
+                __builtin_amdgcn_s_waitcnt(0xC07F | std::min(2 * (FN + decltype(count)::value), 15) << 8);
+                __builtin_amdgcn_sched_barrier(0);
+            }
             multiply(now, count);
         };
-        int kt = 0;
-        for (; kt + 2 < nk; kt += 2) {                        // (no read of the loop is conditional: the compiler waited for it ahead of the multiplications then)
-            step(kt, f0, f1);
-            step(kt + 1, f1, f0);
+        // a round of the buffers at a time, so that every address is a constant beside its base
+        constexpr int ROUND = G::ROUND;
+        for (; kt + ROUND + AHEAD <= nk; kt += ROUND) {
+            constexpr_for<ROUND / 2>([&](auto h) {
+                constexpr int U = 2 * decltype(h)::value;
+                step(std::integral_constant<int, U>{}, U % NBUF, f0, f1);
+                step(std::integral_constant<int, U + 1>{}, (U + 1) % NBUF, f1, f0);
+            });
+            advance(ROUND);
         }
-        if (kt + 1 < nk) {
-            step(kt, f0, f1);
-            multiply(f1, count);
-        } else multiply(f0, count);
+        auto one = [&](Frags& now, Frags& next) {
+            step(here, buf, now, next);
+            advance(1);
+            buf = buf + 1 == NBUF ? 0 : buf + 1;
+            kt++;
+        };
+        while (kt + 1 < nk - AHEAD) {
+            one(f0, f1);
+            one(f1, f0);
+        }
+        auto tail = [&](Frags& now, Frags& next) {
+            ring_tail<AHEAD - 1, G::PER>([&](auto even) {
+                constexpr bool E = decltype(even)::value;
+                buf = buf + 1 == NBUF ? 0 : buf + 1;
+                read(E ? next : now, buf, count);
+                __builtin_amdgcn_sched_barrier(0);
+                multiply(E ? now : next, count);
+            });
+            multiply((AHEAD - 1) & 1 ? next : now, count);
+        };
+        if (kt < nk - AHEAD) {
+            one(f0, f1);
+            tail(f1, f0);
+        } else tail(f0, f1);
     };
     if (live == FM) loop(std::integral_constant<int, FM>{});
     else if (FM > 1 && live == FM - 1) loop(std::integral_constant<int, FM - 1>{});
     else if (FM > 2 && live == FM - 2) loop(std::integral_constant<int, (FM > 2 ? FM - 2 : 0)>{});
     else if (FM > 3 && live == FM - 3) loop(std::integral_constant<int, (FM > 3 ? FM - 3 : 0)>{});
+    else if (FM > 4 && live == FM - 4) loop(std::integral_constant<int, (FM > 4 ? FM - 4 : 0)>{});
     else loop(std::integral_constant<int, 0>{});
 
     __builtin_amdgcn_s_waitcnt(0xC07F);
@@ -344,14 +471,22 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
     }
 }
 
-template <int WM, int WN, int FM, int FN, int NBUF>
+template <int WM, int WN, int FM, int FN, int NBUF, bool FAR = false>
 int launch_t(int epi, const GemmParams& p, int rt, hipStream_t stream) {
     typedef MidGeom<WM, WN, FM, FN, NBUF> G;
     static std::atomic<uint64_t> attr_done{0};
-    if (!cr_dyn_lds_once(attr_done, (const void*)gemm_mid_kernel<WM, WN, FM, FN, NBUF>, G::LDS)) return CR_ERR_HIP;
+    if (!cr_dyn_lds_once(attr_done, (const void*)gemm_mid_kernel<WM, WN, FM, FN, NBUF, FAR>, G::LDS)) return CR_ERR_HIP;
     const int ntm = std::max((p.M + G::BM - 1) / G::BM, rt), ntn = (p.N + G::BN - 1) / G::BN;
-    hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, FM, FN, NBUF>), dim3(ntm * ntn, epi == EPI_PARTIAL ? p.group : 1), dim3(64 * G::WAVES), G::LDS, stream, p, epi, ntm);
+    hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, FM, FN, NBUF, FAR>), dim3(ntm * ntn, epi == EPI_PARTIAL ? p.group : 1), dim3(64 * G::WAVES), G::LDS, stream, p, epi, ntm);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
+}
+// DEEP buffers where every workgroup has a CU to itself, as many as let two share one otherwise.  us, few / deep: 64 x 64 tiles (4 / 8 buffers) 1024 x 1024 x 4096 (256 workgroups) 19.8 / 16.1, 1025 x 1024 x 1024
+// (272) 9.7 / 12.3, 1025 x 4096 x 1024 (1088) 23.0 / 27.0; 128 x 64 (3 / 6) 1025 x 1024 x 4096 (144) 25.7 / 22.5, 1025 x 4096 x 1024 (576) 20.7 / 23.3; 64 x 128 (3 / 6) 23.6 / 20.7 and 20.3 / 23.6
+template <int WM, int WN, int FM, int FN, int FEW, int DEEP>
+int launch_two(int epi, const GemmParams& p, int rt, hipStream_t stream) {
+    typedef MidGeom<WM, WN, FM, FN, FEW> G;
+    const int64_t wgs = (int64_t)std::max((p.M + G::BM - 1) / G::BM, rt) * ((p.N + G::BN - 1) / G::BN) * (epi == EPI_PARTIAL ? p.group : 1);
+    return wgs <= cr_device_cus() ? launch_t<WM, WN, FM, FN, DEEP>(epi, p, rt, stream) : launch_t<WM, WN, FM, FN, FEW>(epi, p, rt, stream);
 }
 
 }  // namespace
@@ -361,17 +496,16 @@ namespace {
 // Tile shapes (launch_gemm_mid's `tile` = index + 1).  Eight waves where the tile is large enough to feed them: two waves a SIMD cover each other's LDS reads and barriers (64 x 64 at
 // M = 1025, N = 1024, K = 4096: four waves 27.5 us, eight 26.6, now 26.2; 128 x 128 at N = 3072, K = 1024: 20 and 13.4).
 struct MidShape { int bm, bn; };
-constexpr MidShape SHAPES[] = {{16, 32}, {16, 64}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {64, 128}, {96, 128}, {128, 128}, {96, 256}, {128, 256}};
+constexpr MidShape SHAPES[] = {{16, 32}, {16, 64}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {64, 128}, {96, 128}, {128, 128}, {96, 256}, {128, 256}, {160, 128}};
 constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 }  // namespace
 
-// A law to choose by, in us, and the tile shape (and number of row tiles) that takes least by it: a CU brings in its workgroups' operand bytes at 61 GB/s and does the rest under that, so
-// a K-tile (64) of a workgroup costs 0.05 us + 2.1 ns per row of A or W in it; a workgroup more on a CU costs its time again; launch, first fill and drain 3.5 us, the epilogue 0.1 ns
-// an element.  It is no prediction.  Measured / law on cold weights: one round of short tiles is up to a fifth faster (1025 x 3072 x 1024 12.4 / 13.8, 1025 x 1024 x 4096 21.1 / 26.6,
-// 77 x 4096 x 14336 44 / 53, 333 x 4096 x 14336 78 / 91), many rounds of large ones up to 8 % slower (8192 x 7168 x 2048 236 / 218, 6000 x 4096 x 14336 637 / 589), and no term stands for the
-// rate of HBM itself, which bounds wide weights at few rows (77 x 28672 x 4096 54 / 36).  At 22 products of M 77 .. 13325, N 1024 .. 28672, K 1024 .. 14336 the kernel that the two
-// laws (here and tile_us in gemm256.hip) choose was the fastest of gemm_mid, 256-row and 192-row tiles, or within 3 % of it.
+// A law to choose by, in us, and the tile shape (and number of row tiles) that takes least by it: launch and drain 2.5 us, a round of workgroups 1 us to its first K-tile, 1.9 ns per row of A or W in
+// each K-tile of 64 less 20 ns (the two shapes of three buffers 2.1 ns and 50 ns more), 0.1 ns an element in the epilogue; a workgroup more on a CU costs its time again.  It is no prediction.  Measured /
+// law, weights cold: 1025 x 1024 x 4096 18.7 / 20.2, 1025 x 1024 x 1024 7.9 / 8.1, 1025 x 3072 x 1024 11.5 / 11.9, 1025 x 4096 x 1024 14.9 / 13.3, 77 x 4096 x 4096 15.0 / 14.1, 333 x 4096 x 14336 81 / 69,
+// 1000 x 4096 x 14336 135 / 113; no term stands for the rate of HBM itself, which bounds wide weights at few rows (77 x 28672 x 4096 54 / 32).  At 37 products of M 77 .. 8200, N 1024 .. 28672,
+// K 512 .. 14336 the kernel that the two laws (here and tile_us in gemm256.hip) choose was the fastest of gemm_mid, 256-row and 192-row tiles, or within 4 % of it.
 double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
     const int nf = (p.M + 15) / 16, slices = epi == EPI_PARTIAL && p.group > 0 ? p.group : 1, nk = p.K / 64 / slices, cus = cr_device_cus();
     double best = 1e30;
@@ -384,7 +518,8 @@ double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
             if (want < least || want > nf || (per_cu && want > 2L * least)) continue;
             const int rows = 16 * ((nf + (int)want - 1) / (int)want);
             const double rounds = (double)((want * ntn + cus - 1) / cus);
-            const double c = 3.5 + rounds * (nk * (0.05 + 0.0021 * (rows + SHAPES[t].bn)) + 1e-4 * rows * SHAPES[t].bn);
+            const int side = rows + SHAPES[t].bn;
+            const double c = 2.5 + rounds * (1.0 + nk * (t == 10 || t == 11 ? 0.05 + 0.0021 * side : 0.0019 * side - 0.02) + 1e-4 * rows * SHAPES[t].bn);
             if (c < best - 1e-9) { best = c; *tile = t + 1; *row_tiles = (int)want; }
         }
     }
@@ -395,19 +530,21 @@ int launch_gemm_mid(int epi, const GemmParams& p, hipStream_t stream) {
     int tile = p.tile, rt = 0;
     if (!tile) gemm_mid_cost(epi, p, &tile, &rt);
     if (tile < 1 || tile > N_SHAPES || (epi == EPI_ARGMAX && SHAPES[tile - 1].bn != 256)) return CR_ERR_ARG;      // (a pin; a wave's columns have to be a partial's 64)
+    if (7 * 2 * std::max(p.lda, p.ldw) + 128 > (int64_t)UINT32_MAX) return launch_t<2, 4, 2, 4, 3, true>(epi, p, 0, stream);      // (whatever the epilogue; the same bits)
     switch (tile) {
         case 1: return launch_t<1, 2, 1, 1, 12>(epi, p, rt, stream);
         case 2: return launch_t<1, 4, 1, 1, 8>(epi, p, rt, stream);
         case 3: return launch_t<1, 4, 2, 1, 6>(epi, p, rt, stream);
         case 4: return launch_t<2, 2, 2, 1, 6>(epi, p, rt, stream);
-        case 5: return launch_t<2, 4, 2, 1, 4>(epi, p, rt, stream);
-        case 6: return launch_t<2, 4, 3, 1, 4>(epi, p, rt, stream);
-        case 7: return launch_t<2, 4, 4, 1, 3>(epi, p, rt, stream);
-        case 8: return launch_t<2, 4, 2, 2, 3>(epi, p, rt, stream);
+        case 5: return launch_two<2, 4, 2, 1, 4, 8>(epi, p, rt, stream);
+        case 6: return launch_t<2, 4, 3, 1, 6>(epi, p, rt, stream);
+        case 7: return launch_two<2, 4, 4, 1, 3, 6>(epi, p, rt, stream);
+        case 8: return launch_two<2, 4, 2, 2, 3, 6>(epi, p, rt, stream);
         case 9: return launch_t<2, 4, 3, 2, 5>(epi, p, rt, stream);
         case 10: return launch_t<2, 4, 4, 2, 4>(epi, p, rt, stream);
         case 11: return launch_t<2, 4, 3, 4, 3>(epi, p, rt, stream);
         case 12: return launch_t<2, 4, 4, 4, 3>(epi, p, rt, stream);
+        case 13: return launch_t<2, 4, 5, 2, 4>(epi, p, rt, stream);
     }
     return CR_ERR_ARG;
 }
