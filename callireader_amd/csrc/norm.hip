@@ -56,12 +56,19 @@ __device__ __forceinline__ void store_row_e4m3(const NormParams& p, int64_t orow
     }
 }
 
-// MODE 0: plain rows, 1: pixel-shuffle gather (N = 4096 from [T,1025,1024]).  LATE: the gains are asked for behind both sums instead of with the row (launch_layernorm)
-template <int TPR, int MODE, bool LATE>
+// AHEAD: workgroups past the rows read weights for a product behind.  MODE 0: plain rows, 1: pixel-shuffle gather (N = 4096 from [T,1025,1024]).  LATE: the gains are asked for behind both sums instead of with the row (launch_layernorm)
+template <int TPR, int MODE, bool LATE, bool AHEAD = false>
 __global__ __launch_bounds__(256) void layernorm_kernel(const NormParams p) {
     __shared__ float red[4];
     const int tid = threadIdx.x;
     constexpr int RPB = 256 / TPR;
+    if constexpr (AHEAD) {
+        const int own = (int)((p.rows + RPB - 1) / RPB), nth = l2_ahead_nth(blockIdx.x, own);
+        if ((int)blockIdx.x >= own) {                         // (uniform)
+            if (nth >= 0 && nth < L2_AHEAD_GROUPS) l2_ahead(p.ahead, blockIdx.x, nth);
+            return;
+        }
+    }
     const int64_t row = (int64_t)blockIdx.x * RPB + tid / TPR;
     const int t = tid % TPR;
     const bool live = row < p.rows;
@@ -162,7 +169,12 @@ int launch_layernorm(const NormParams& p, int n, int mode, hipStream_t stream) {
     if (p.rows <= 0) return CR_OK;
     if ((n != 1024 && n != 4096) || (mode == 1 && n != 4096)) return CR_ERR_ARG;
     const bool late = (int64_t)p.rows * n * 4 > (int64_t)256 << 20;
-    const dim3 grid((unsigned)(n == 1024 ? (p.rows + 3) / 4 : p.rows)), block(256);
+    const int own = (int)(n == 1024 ? (p.rows + 3) / 4 : p.rows);
+    const dim3 grid((unsigned)own), block(256);
+    if (p.ahead.at && n == 1024 && !late) {
+        hipLaunchKernelGGL((layernorm_kernel<64, 0, false, true>), dim3((unsigned)(own + l2_ahead_extra(own))), block, 0, stream, p);
+        return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
+    }
     auto launch = [&](auto l) {
         constexpr bool LATE = decltype(l)::value;
         if (mode == 1) hipLaunchKernelGGL((layernorm_kernel<256, 1, LATE>), grid, block, 0, stream, p);

@@ -1,5 +1,6 @@
 #pragma once
 #include "common.hpp"
+#include "l2_ahead.hpp"
 
 struct NormParams {
     const bf16* in; int64_t ld_in;
@@ -19,6 +20,7 @@ struct NormParams {
     // slack of both operands' e4m3 rounding, 1.0625^2) -- the e4m3 scale that linear's epilogue may use for ITS output row without
     // knowing the row's maximum (EPI_GELU_Q8)
     float* next_scale; const float* next_bound;
+    L2Ahead ahead;             // rows of 1024: weights that a product behind reads, brought nearer by workgroups past the rows (l2_ahead.hpp)
 };
 
 // mode 0: rows of n (1024 | 4096) bf16; mode 1: pixel-shuffle gather feeding mlp1's LayerNorm (n = 4096)

@@ -112,6 +112,10 @@ static int vit_chunk(cr_ctx* c, const bf16* px, int T, bf16* x, hipStream_t st) 
         CR_TRY(gemm(c, EPI_LS_RES, h, C1, pw, C1, x, C1, pb, ls1, x, C1, M, C1, C1, 0, st));
 
         np.gamma = n2w; np.beta = n2b;
+        // fc2's 8 MB come from HBM, 24 layers of weights being more than the memory-side cache holds, and a product of few rows waits for them (1025 x 1024 x 4096 23.3 us, 19.4 out of that cache): read
+        // beside the norm's 4.4 us, with fc1 between, they are there.  The whole tower, us without / with: 1 tile 2278 / 2184, 2 tiles 3083 / 3069, 3 tiles 3687 / 3669, 4 tiles 4533 / 4505, 6 tiles 6129 /
+        // 6161, 8 tiles 7362 / 7397, 11 tiles 8900 / 8922.  The other weights so, beside either norm, 0 to 10 us more or less: K = 1024 is over before it has to wait often
+        if (T <= 4 && !m8) np.ahead = l2_ahead_of(f2w, (int64_t)C1 * FF * 2, L2_AHEAD_GROUPS);
         if (m8all) { np.next_scale = fs; np.next_bound = (const float*)bnd->ptr; }
         CR_TRY(launch_layernorm(np, C1, 0, st));
         if (m8 && !m8all) {
