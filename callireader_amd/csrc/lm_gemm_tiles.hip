@@ -1,10 +1,12 @@
 // Prompt products of described decoders in true fp32: C = epi(A[M,K] . W[N,K]^T), K % 64 == 0, optionally batched over heads or grouped over experts with gathered rows and scattered
 // results.  (Decode batches: lm_gemm_rows.hip.)
 //
-// Bound by the matrix cores (v_mfma_f32_16x16x4_f32: 256 operations a clock and CU) where the grid fills the card, by what lies between K-tiles where it does not.  The form of
+// Bound by the matrix cores (v_mfma_f32_16x16x4_f32: 256 operations a clock and CU) where the grid fills the card, by what a K-tile asks for, reads and folds where it does not.  The form of
 // gemm_mid.hip: NBUF K-tiles in LDS, NBUF - 1 of them under way, one barrier a K-tile, eight rows of 128 bytes a load instruction; the tile shape is picked by the rounds it gives.
-// 402 rows, us: products of 1024 columns over K = 64, 1536 and 4096 49 on average -> 5, 22 and 49 (32 x 64 tiles, K-tiles of 64), 3584 x 1024 50 -> 42 and
-// 4096 x 1024 with the squared relu 51 -> 42 (112 x 64; 22 us of multiplications).  Before: 64 x 64 tiles, one K-tile of 32 in LDS, two barriers each.
+// 402 x 4096 x 1024, 40.5 us on 256 workgroups: multiplications and launch 30.6, folded chains 2.7, LDS reads 2 to 3, asking for K-tiles 4.5, the barriers nothing.  So asking takes a scalar address and three
+// other scalar instructions a piece, and both it and the reads go between the multiplications; every SIMD has all of a tile's rows in its two waves (with four wave rows a tile of six fragments left two SIMDs
+// with four of them and two with two).  402 rows, us: products of 1024 columns over K = 1536 22.2 -> 19.5, 3584 and 4096 x 1024 42.5 -> 37.3; 1600 x 4096 x 1024 142 -> 127, 800 x 4096 x 1024 77.6 -> 72.5,
+// 260 x 4096 x 1024 40.3 -> 31.5, experts of 1600 rows 154 and 85 -> 145 and 79.  (Tiles of half the size, two workgroups a CU: 45; K-tiles twice as deep, six buffers for three: no difference.)
 // A lane reads 16 bytes of its row, k = 16 h + 4 (lane >> 4) .. + 3; the four multiplications take one element of each, which permutes k inside 16 for both operands alike.  A row's
 // sum has the order of lm.hpp whatever the tile: an accumulator is a chain, and goes to the part's sum and that to the total when it ends.  That costs 1.6 us of the 22 where a chain is one block of 32 (two chains over all of K: 20), nothing on
 // the larger tiles, whose waves multiply under each other's additions.
@@ -73,7 +75,7 @@ struct Geom {
     static_assert((NBUF - 2) * PER <= 63 && NBUF >= 2 && LDS <= 160 * 1024, "vmcnt is six bits wide; a CU has 160 KiB");
 };
 
-template <int WM, int WN, int FM, int FN, int KB, int NBUF>
+template <int WM, int WN, int FM, int FN, int KB, int NBUF, bool FAR>
 __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmParams p, const int epi, const int ntm) {
     typedef Geom<WM, WN, FM, FN, KB, NBUF> G;
     extern __shared__ __attribute__((aligned(16))) char smem[];
@@ -97,25 +99,50 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
     }
     const int wf0 = fn * wm / WM, live = fn * (wm + 1) / WM - wf0;      // a tile's over its wave rows
 
-    const float* src[G::PER];
-    int dst[G::PER];
-    bool dead[G::PER];
+    // This wave's pieces of a K-tile: eight rows, 128 bytes each; numbers past the last repeat it, pieces past the tile's rows move one lane's 16 bytes (the count of instructions under way stays a
+    // constant).  A piece's first row is the same for all lanes, so its address is a scalar one and a lane's own row and chunk are 32 bits beyond it; FAR: gathered rows, and rows so far apart that eight of
+    // them span 4 GiB, have 64 bits a lane.  LDS-DMA from inline asm: from the builtin a piece came with 64-bit sums, a copy of m0 and a branch on the lanes.
+    const char *src[G::PER], *lane_src[FAR ? G::PER : 1];
+    unsigned off[G::PER], dst[G::PER];
+    uint64_t lanes[G::PER];
+    const unsigned smem_base = (unsigned)(size_t)(__attribute__((address_space(3))) char*)smem;
 #pragma unroll
-    for (int i = 0; i < G::PER; i++) {                        // this wave's pieces of a K-tile; numbers past the last repeat it, pieces past the tile's rows move one lane's 16 bytes
+    for (int i = 0; i < G::PER; i++) {
         const int at = min(wave + i * G::WAVES, G::PIECES - 1), kb = at / G::ROWS8, piece = at - kb * G::ROWS8, row = piece * 8 + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
-        const int m = pos0 + min(m0 + row, rows - 1);
-        const int64_t ar = piece * 8 < G::BM && p.perm && p.gather_div ? p.perm[m] / p.gather_div : m;
-        src[i] = (piece * 8 < G::BM ? A + ar * p.lda : W + (int64_t)min(n0 + row - G::BM, p.N - 1) * p.ldw) + kb * 32 + chunk * 4;
-        dst[i] = at * 1024;
-        dead[i] = piece * 8 < G::BM && piece >= 2 * fn;
+        const bool a = piece * 8 < G::BM;
+        const int first = a ? pos0 + min(m0 + piece * 8, rows - 1) : min(n0 + piece * 8 - G::BM, p.N - 1), own = a ? pos0 + min(m0 + row, rows - 1) : min(n0 + row - G::BM, p.N - 1);
+        src[i] = (const char*)((a ? A + (int64_t)first * p.lda : W + (int64_t)first * p.ldw) + kb * 32);
+        off[i] = (unsigned)((own - first) * (a ? p.lda : p.ldw) * 4) + chunk * 16;
+        if (FAR) {
+            const int64_t r = a && p.perm && p.gather_div ? p.perm[own] / p.gather_div : own;
+            lane_src[FAR ? i : 0] = (const char*)((a ? A + r * p.lda : W + r * p.ldw) + kb * 32 + chunk * 4);
+        }
+        dst[i] = smem_base + at * 1024;
+        lanes[i] = a && piece >= 2 * fn ? 1 : ~0ull;
     }
     const int nk = p.K / (32 * KB);
-    auto ask = [&](int kt, int buf) {
-#pragma unroll
-        for (int i = 0; i < G::PER; i++) {
-            CR_DIAG_POISON(smem + buf * G::STAGE + dst[i])
-            if (!dead[i] || lane == 0) __builtin_amdgcn_global_load_lds(CR_GLB(src[i] + (int64_t)kt * (32 * KB)), CR_LDS(smem + buf * G::STAGE + dst[i]), 16, 0, 0);
+#pragma clang diagnostic push
+#pragma clang diagnostic ignored "-Winline-asm"               // (m0 is a reserved register: nothing else here uses it)
+    // (all lanes are on here, before and after)
+    auto ask_piece = [&](int i, int buf) __attribute__((always_inline)) {
+        CR_DIAG_POISON(smem + buf * G::STAGE + (dst[i] - smem_base))
+        const unsigned to = buf * G::STAGE, d = dst[i], o = off[i];
+        const uint64_t on = lanes[i];
+        if constexpr (FAR) {
+            const char* v = lane_src[FAR ? i : 0];
+            asm volatile("s_add_u32 m0, %1, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, off\n\ts_mov_b64 exec, -1" ::"v"(v), "s"(d), "s"(to), "s"(on) : "m0", "scc", "memory");
+            lane_src[FAR ? i : 0] += KB * 128;
+        } else {
+            const char* g = src[i];
+            asm volatile("s_add_u32 m0, %2, %3\n\ts_mov_b64 exec, %4\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(o), "s"(g), "s"(d), "s"(to), "s"(on) : "m0", "scc", "memory");
+            src[i] += KB * 128;
         }
+    };
+#pragma clang diagnostic pop
+    // the K-tile that `src` stands at, into buffer buf
+    auto ask = [&](int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int i = 0; i < G::PER; i++) ask_piece(i, buf);
     };
     f32x4 acc[FM][FN], part[FM][FN], total[FM][FN];           // of the chain, of the part, of the whole sum
 #pragma unroll
@@ -128,17 +155,16 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
     const int c_off[2] = {((lane >> 4) ^ swz) * 16, ((4 + (lane >> 4)) ^ swz) * 16};
     const int a_off = (wf0 * 16 + (lane & 15)) * 128, w_off = (G::BM + wn * FN * 16 + (lane & 15)) * 128;
     struct Frags { f32x4 a[2 * KB][FM], w[2 * KB][FN]; };
-    auto read = [&](Frags& f, int buf, auto count) {
+    // fragment x of a K-tile's 2 * KB * (FN + FM): those of 16 k after each other, W's first
+    auto read_one = [&](Frags& f, int x, int buf, auto count) {
         const char* s = smem + buf * G::STAGE;
+        const int h = x / (FN + FM), c = x % (FN + FM), at = (h >> 1) * G::ROWS8 * 1024 + c_off[h & 1];
+        if (c < FN) f.w[h][c] = *(const f32x4*)(s + w_off + c * 2048 + at);
+        else if (c - FN < decltype(count)::value) f.a[h][c - FN] = *(const f32x4*)(s + a_off + (c - FN) * 2048 + at);
+    };
+    auto read = [&](Frags& f, int buf, auto count) {
 #pragma unroll
-        for (int h = 0; h < 2 * KB; h++) {
-            const int at = (h >> 1) * G::ROWS8 * 1024 + c_off[h & 1];
-#pragma unroll
-            for (int j = 0; j < FN; j++) f.w[h][j] = *(const f32x4*)(s + w_off + j * 2048 + at);
-#pragma unroll
-            for (int i = 0; i < FM; i++)
-                if (i < decltype(count)::value) f.a[h][i] = *(const f32x4*)(s + a_off + i * 2048 + at);
-        }
+        for (int x = 0; x < 2 * KB * (FN + FM); x++) read_one(f, x, buf, count);
     };
     auto fold = [&](f32x4 (&to)[FM][FN], f32x4 (&from)[FM][FN], auto count) {
 #pragma unroll
@@ -148,19 +174,22 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
                 for (int j = 0; j < FN; j++) { to[i][j] += from[i][j]; from[i][j] = f32x4{0.f, 0.f, 0.f, 0.f}; }
             }
     };
-    auto multiply = [&](const Frags& f, auto count) {
+    // beside(g): what is issued behind the multiplications g of 8 * KB
+    auto multiply = [&](const Frags& f, auto count, auto beside) {
 #pragma unroll
         for (int kb = 0; kb < KB; kb++) {
 #pragma unroll
             for (int h = 2 * kb; h < 2 * kb + 2; h++)
 #pragma unroll
-                for (int e = 0; e < 4; e++)
+                for (int e = 0; e < 4; e++) {
 #pragma unroll
                     for (int i = 0; i < FM; i++)
                         if (i < decltype(count)::value) {
 #pragma unroll
                             for (int j = 0; j < FN; j++) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.w[h][j][e], f.a[h][i][e], acc[i][j], 0, 0, 0);
                         }
+                    beside(4 * h + e);
+                }
             in_chain--; in_part--;
             if (in_chain == 0 || in_part == 0) {              // (uniform)
                 fold(part, acc, count);
@@ -169,34 +198,58 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
             }
         }
     };
+    auto nothing = [](int) {};
     auto arrive = [&](int t) { ring_arrive<NBUF, G::PER>(nk, t); };
     auto loop = [&](auto count) {
-        for (int t = 0; t < min(NBUF - 1, nk); t++) ask(t, t);
+        for (int t = 0; t < min(NBUF - 1, nk); t++) ask(t);
         Frags f0, f1;
         arrive(0);
-        if (NBUF - 1 < nk) ask(NBUF - 1, NBUF - 1);
+        if (NBUF - 1 < nk) ask(NBUF - 1);
         read(f0, 0, count);
         int buf = 0;                                          // buffer of K-tile kt
-        auto step = [&](int kt, Frags& now, Frags& next) {
-            arrive(kt + 1);
-            if (kt + NBUF < nk) ask(kt + NBUF, buf);
+        // What a step reads and asks for goes between its multiplications, which keep the matrix pipe busy for 32 clocks each
+        auto step = [&](int kt, Frags& now, Frags& next, auto all) {
+            if constexpr (decltype(all)::value) {
+                wait_vm<(NBUF - 2) * G::PER>();
+                __builtin_amdgcn_s_waitcnt(0xC07F);           // lgkmcnt(0)
+                __builtin_amdgcn_sched_barrier(0);
+                __builtin_amdgcn_s_barrier();
+                __builtin_amdgcn_sched_barrier(0);
+            } else arrive(kt + 1);
+            const int into = buf;
             buf = buf + 1 == NBUF ? 0 : buf + 1;
-            read(next, buf, count);
-            __builtin_amdgcn_sched_barrier(0);
-            multiply(now, count);
+            constexpr int READS = 2 * KB * (FN + FM), GROUPS = 8 * KB, EACH = (READS + G::PER + GROUPS - 2) / (GROUPS - 1);
+            multiply(now, count, [&](int g) {
+#pragma unroll
+                for (int x = g * EACH; x < (g + 1) * EACH; x++) {
+                    if (x < READS) read_one(next, x, buf, count);
+                    else if (x < READS + G::PER) {
+                        if (decltype(all)::value || kt + NBUF < nk) ask_piece(x - READS, into);
+                    }
+                }
+                __builtin_amdgcn_sched_barrier(0);
+            });
         };
+        constexpr std::true_type whole{};
+        constexpr std::false_type tail{};
         int kt = 0;
-        for (; kt + 2 < nk; kt += 2) {                        // (no step of the loop is conditional: the compiler waited for the reads ahead of the multiplications then)
-            step(kt, f0, f1);
-            step(kt + 1, f1, f0);
+        for (; kt + 1 + NBUF < nk; kt += 2) {                 // (no step of the loop is conditional: the compiler waited for the reads ahead of the multiplications then)
+            step(kt, f0, f1, whole);
+            step(kt + 1, f1, f0, whole);
+        }
+        for (; kt + 2 < nk; kt += 2) {
+            step(kt, f0, f1, tail);
+            step(kt + 1, f1, f0, tail);
         }
         if (kt + 1 < nk) {
-            step(kt, f0, f1);
-            multiply(f1, count);
-        } else multiply(f0, count);
+            step(kt, f0, f1, tail);
+            multiply(f1, count, nothing);
+        } else multiply(f0, count, nothing);
     };
+    // (fewer than FM - 1 live fragments: those past them multiply what an older K-tile left in LDS, and are not stored)
     if (live == FM) loop(std::integral_constant<int, FM>{});
     else if (FM > 1 && live == FM - 1) loop(std::integral_constant<int, FM - 1>{});
+    else if (FM > 2 && live > 0) loop(std::integral_constant<int, FM - 2>{});
     else loop(std::integral_constant<int, 0>{});
     const int row0 = m0 + wf0 * 16, col0 = n0 + wn * FN * 16;
     switch (epi) {                                            // (uniform)
@@ -209,14 +262,21 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
     }
 }
 
-template <int WM, int WN, int FM, int FN, int KB, int NBUF>
-int launch_t(int epi, const LmGemmParams& p, int ntm, hipStream_t st) {
+template <int WM, int WN, int FM, int FN, int KB, int NBUF, bool FAR>
+int launch_f(int epi, const LmGemmParams& p, int ntm, hipStream_t st) {
     typedef Geom<WM, WN, FM, FN, KB, NBUF> G;
     static std::atomic<uint64_t> attr_done{0};
-    if (!cr_dyn_lds_once(attr_done, (const void*)lm_tiles_kernel<WM, WN, FM, FN, KB, NBUF>, G::LDS)) return CR_ERR_HIP;
-    hipLaunchKernelGGL((lm_tiles_kernel<WM, WN, FM, FN, KB, NBUF>), dim3((p.N + G::BN - 1) / G::BN, ntm, p.batch > 0 ? p.batch : 1), dim3(64 * G::WAVES), G::LDS, st, p, epi, ntm);
+    if (!cr_dyn_lds_once(attr_done, (const void*)lm_tiles_kernel<WM, WN, FM, FN, KB, NBUF, FAR>, G::LDS)) return CR_ERR_HIP;
+    hipLaunchKernelGGL((lm_tiles_kernel<WM, WN, FM, FN, KB, NBUF, FAR>), dim3((p.N + G::BN - 1) / G::BN, ntm, p.batch > 0 ? p.batch : 1), dim3(64 * G::WAVES), G::LDS, st, p, epi, ntm);
     CR_HIP(hipGetLastError());
     return CR_OK;
+}
+
+template <int WM, int WN, int FM, int FN, int KB, int NBUF>
+int launch_t(int epi, const LmGemmParams& p, int ntm, hipStream_t st) {
+    // (eight rows of either operand, and an XOR that keeps to a row's 128 bytes, within 32 bits)
+    const bool far = p.tiles || 8 * std::max(p.lda, p.ldw) * 4 >= (1ll << 32);
+    return far ? launch_f<WM, WN, FM, FN, KB, NBUF, true>(epi, p, ntm, st) : launch_f<WM, WN, FM, FN, KB, NBUF, false>(epi, p, ntm, st);
 }
 
 struct Shape { int bm, bn; };
@@ -244,7 +304,7 @@ int launch_lm_gemm_tiles(int epi, const LmGemmParams& p, hipStream_t st) {      
         case 1: return launch_t<2, 2, 1, 1, 2, 4>(epi, p, ntm, st);
         case 2: return launch_t<2, 4, 1, 1, 2, 4>(epi, p, ntm, st);
         case 3: return launch_t<2, 4, 2, 1, 1, 4>(epi, p, ntm, st);
-        case 4: return launch_t<4, 2, 2, 2, 1, 3>(epi, p, ntm, st);
+        case 4: return launch_t<2, 4, 4, 1, 1, 3>(epi, p, ntm, st);
         case 5: return launch_t<2, 4, 2, 2, 1, 3>(epi, p, ntm, st);
     }
     return launch_t<4, 2, 2, 4, 1, 4>(epi, p, ntm, st);
