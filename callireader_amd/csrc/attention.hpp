@@ -48,7 +48,7 @@ struct AttnParams {
     int sk_mod;               // decode: > 0: a row sees the last sk_arr[slot] % sk_mod + sk_add keys, which start at its slot's first row
     int vdim;
     const bf16* gate; int64_t g_rs;
-    L2Ahead ahead;            // decode: weights of the product behind, brought into L2 beside (attention_decode.hip)
+    L2Ahead ahead;            // weights of the product behind, brought into L2 beside (decode: attention_decode.hip; vision: attention_vit.hip's last launch)
 };
 
 bool decode_attn_fold_supported(const AttnParams& p, int head_dim);

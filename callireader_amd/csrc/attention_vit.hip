@@ -789,8 +789,13 @@ __device__ __forceinline__ void vit_cls_combine_any(const AttnParams& p, int nsp
 }
 
 // Both in one launch: block 0 of a tile redoes what was flagged (patch rows), the others merge the class rows of four heads, a wave each.  (A launch of 4.8 us each, and a layer of one
-// tile has seven launches in all.)
+// tile has seven launches in all.  Workgroups past these read the output projection's weights, AttnParams::ahead.)
 __global__ __launch_bounds__(256) void vit_attn_finish_kernel(const AttnParams p, const int nb) {
+    if ((int)blockIdx.x > (p.H + 3) / 4) {                     // (uniform)
+        const int nth = l2_ahead_nth(blockIdx.x, 1 + (p.H + 3) / 4);
+        if (blockIdx.y == 0 && nth >= 0 && nth < L2_AHEAD_GROUPS) l2_ahead(p.ahead, blockIdx.x, nth);
+        return;
+    }
     const int batch = blockIdx.y, head = 4 * ((int)blockIdx.x - 1) + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
     if (blockIdx.x == 0) vit_attn_exact(p, batch, nb);
     else if (head >= p.H) return;
@@ -828,6 +833,7 @@ int launch_vit_attn(const AttnParams& p, hipStream_t stream) {
     if (two_waves) hipLaunchKernelGGL(vit_attn2_kernel, dim3(nb, p.H, p.B), dim3(128), LDS, stream, q);
     else if (few) hipLaunchKernelGGL(vit_attn_few_kernel, dim3(p.H, 2 * nb, p.B), dim3(512), FEW_LDS, stream, q);
     else hipLaunchKernelGGL(vit_attn_kernel, dim3(nb, p.H, p.B), dim3(256), LDS, stream, q);
-    hipLaunchKernelGGL(vit_attn_finish_kernel, dim3(1 + (p.H + 3) / 4, p.B), dim3(256), LDS, stream, q, nb);
+    const int own = 1 + (p.H + 3) / 4;
+    hipLaunchKernelGGL(vit_attn_finish_kernel, dim3(own + (p.ahead.at ? l2_ahead_extra(own) : 0), p.B), dim3(256), LDS, stream, q, nb);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
