@@ -132,6 +132,15 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 }
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + __expf(-x)); }
 
+// A launch's arguments: every 64-byte line of them is a round trip of its own, taken where the compiler places the first use.  All lines at once instead.
+template <int BYTES> __device__ __forceinline__ void touch_args() {
+    const __attribute__((address_space(4))) int* k = (const __attribute__((address_space(4))) int*)__builtin_amdgcn_kernarg_segment_ptr();
+    int x = 0;
+#pragma unroll
+    for (int i = 0; i < BYTES; i += 64) x ^= k[i / 4];
+    asm volatile("" ::"s"(x));
+}
+
 // Butterflies over the lane's bits from 32 down to 1, on the vector pipe: two swaps of halves and rows, two rotations of a row of 16 (its halves are equal by then, so rotating by 4 meets lane ^ 4's
 // value), two quad permutes.  Six LDS permutes of a round trip each before (us): layer norm of 1025 / 11 275 rows of 1024, two sums a row and its gains asked for with the row, 4.90 / 10.01 -> 4.68 / 9.80;
 // 402 rows of float32 attention 30.1 -> 29.3.

@@ -231,25 +231,41 @@ struct MidGeom {
     static_assert((NBUF - 1) * PER <= 63 && NBUF >= 3 && LDS <= 160 * 1024, "vmcnt is six bits wide; a CU has 160 KiB");
 };
 
+// What a launch's workgroups would divide for: the tiles' order, the fragments of a row tile, a slice's K-tiles
+struct MidGrid {
+    int epi, ntm, ntn, nk;                                    // epilogue; row and column tiles; K-tiles of a slice
+    int xq, xr;                                               // workgroups / 8 and % 8
+    int per_group, last;                                      // workgroups of a super-group of eight row tiles; row tiles of the last one
+    unsigned group_mul, last_mul;                             // ceil(2^32 / per_group), ceil(2^32 / last): exact where a workgroup's number times the divisor stays below 2^32 (group_mul 0: it does not)
+    int fq, fr;                                               // fragments / row tiles and % row tiles
+    unsigned rows_mul;                                        // ceil(2^32 / row tiles): exact for ntm^3 < 2^32 (0: it is not, or one row tile)
+};
+
 template <int WM, int WN, int FM, int FN, int NBUF, bool FAR>
-__global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams p, const int epi, const int ntm) {
+__global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const MidGrid g, const GemmParams p) {
     typedef MidGeom<WM, WN, FM, FN, NBUF> G;
     extern __shared__ __attribute__((aligned(16))) char smem[];
+    touch_args<(int)(sizeof(MidGrid) + sizeof(GemmParams))>();
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wm = wave / WN, wn = wave % WN;
+    const int wm = wave / WN, wn = wave % WN, epi = g.epi;
 
     // ---- workgroup -> tile: bijective XCD remap (an XCD's L2 gets a contiguous run of tiles), then super-groups of 8 row tiles ----
-    const int ntn = (p.N + G::BN - 1) / G::BN;
-    const int nwg = gridDim.x, orig = blockIdx.x;
-    const int nk = p.K / 64 / (int)gridDim.y;                 // K-tiles of this slice (EPI_PARTIAL: gridDim.y of them; one otherwise)
-    const int xcd = orig & 7, q = nwg >> 3, r = nwg & 7;
-    const int pid = (xcd < r ? xcd * (q + 1) : r * (q + 1) + (xcd - r) * q) + (orig >> 3);
+    // (no division: five of them, one in 64 bits, and the arguments' lines one after the other as they were come upon kept a workgroup from its first load for 2 us)
+    const int orig = blockIdx.x, nk = g.nk, xcd = orig & 7;
+    const int pid = (xcd < g.xr ? xcd * (g.xq + 1) : g.xr * (g.xq + 1) + (xcd - g.xr) * g.xq) + (orig >> 3);
     constexpr int GM = 8;
-    const int per_group = GM * ntn, grp = pid / per_group, first_m = grp * GM, gsz = min(ntm - first_m, GM), in_g = pid - grp * per_group;
-    const int tile_m = first_m + in_g % gsz, n0 = in_g / gsz * G::BN;
+    const int grp = g.group_mul ? (int)__umulhi((unsigned)pid, g.group_mul) : pid / g.per_group, first_m = grp * GM, in_g = pid - grp * g.per_group;
+    int col, in_col;
+    if (g.ntm - first_m >= GM) { col = in_g >> 3; in_col = in_g & 7; }
+    else {
+        col = g.last_mul ? (int)__umulhi((unsigned)in_g, g.last_mul) : in_g / g.last;
+        in_col = in_g - col * g.last;
+    }
+    const int tile_m = first_m + in_col, n0 = col * G::BN;
     // ---- the matrix's fragments of 16 rows dealt evenly over the row tiles (at most WM * FM each), a tile's over its wave rows ----
-    const int nf = (p.M + 15) >> 4, f0 = (int)((int64_t)tile_m * nf / ntm), fn = (int)((int64_t)(tile_m + 1) * nf / ntm) - f0;
+    auto dealt = [&](int t) { return t * g.fq + (g.rows_mul ? (int)__umulhi((unsigned)(t * g.fr), g.rows_mul) : (int)((int64_t)t * g.fr / g.ntm)); };
+    const int f0 = dealt(tile_m), fn = dealt(tile_m + 1) - f0;
     const int m0 = f0 * 16, wf0 = fn * wm / WM, live = fn * (wm + 1) / WM - wf0;
 
     // ---- this wave's pieces of a K-tile: eight rows of A or W, all 64 k (128 bytes a row); numbers past the last repeat it ----
@@ -265,9 +281,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const GemmParams
         const int piece = min(wave + i * G::WAVES, G::PIECES - 1), row = piece * 8 + (lane >> 3), chunk = (lane & 7) ^ ((row >> 1) & 7);
         const bool a = piece * 8 < G::BM;
         const int first = a ? min(m0 + piece * 8, p.M - 1) : min(n0 + piece * 8 - G::BM, p.N - 1), own = a ? min(m0 + row, p.M - 1) : min(n0 + row - G::BM, p.N - 1);
-        src[i] = (const char*)((a ? p.A + (int64_t)first * p.lda : p.W + (int64_t)first * p.ldw) + (int64_t)blockIdx.y * nk * 64);
-        if (FAR) lane_src[FAR ? i : 0] = src[i] + (int64_t)(own - first) * (a ? p.lda : p.ldw) * 2 + chunk * 16;
-        off[i] = (unsigned)((own - first) * (a ? p.lda : p.ldw) * 2) + chunk * 16;
+        if (FAR) {
+            src[i] = (const char*)((a ? p.A + (int64_t)first * p.lda : p.W + (int64_t)first * p.ldw) + (int64_t)blockIdx.y * nk * 64);
+            lane_src[FAR ? i : 0] = src[i] + (int64_t)(own - first) * (a ? p.lda : p.ldw) * 2 + chunk * 16;
+        } else {                                              // (rows are less than 2^28 elements apart)
+            const unsigned ld = (unsigned)(a ? p.lda : p.ldw);
+            src[i] = (const char*)((a ? p.A : p.W) + (uint64_t)(unsigned)first * ld + blockIdx.y * nk * 64);
+            off[i] = (unsigned)(own - first) * ld * 2 + chunk * 16;
+        }
         dst[i] = smem_base + G::PAD + piece * 1024;
         lanes[i] = a && piece >= 2 * fn ? 1 : ~0ull;
     }
@@ -477,7 +498,10 @@ int launch_t(int epi, const GemmParams& p, int rt, hipStream_t stream) {
     static std::atomic<uint64_t> attr_done{0};
     if (!cr_dyn_lds_once(attr_done, (const void*)gemm_mid_kernel<WM, WN, FM, FN, NBUF, FAR>, G::LDS)) return CR_ERR_HIP;
     const int ntm = std::max((p.M + G::BM - 1) / G::BM, rt), ntn = (p.N + G::BN - 1) / G::BN;
-    hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, FM, FN, NBUF, FAR>), dim3(ntm * ntn, epi == EPI_PARTIAL ? p.group : 1), dim3(64 * G::WAVES), G::LDS, stream, p, epi, ntm);
+    const int slices = epi == EPI_PARTIAL ? p.group : 1, nwg = ntm * ntn, nf = (p.M + 15) / 16, per_group = 8 * ntn, last = ntm % 8 ? ntm % 8 : 8;
+    auto mul = [&](int d) { return d > 1 && (int64_t)nwg * d < (1ll << 32) ? (unsigned)(((1ull << 32) + d - 1) / d) : 0u; };
+    const MidGrid g{epi, ntm, ntn, p.K / 64 / slices, nwg / 8, nwg % 8, per_group, last, mul(per_group), mul(last), nf / ntm, nf % ntm, ntm > 1 && ntm < 1600 ? (unsigned)(((1ull << 32) + ntm - 1) / ntm) : 0u};
+    hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, FM, FN, NBUF, FAR>), dim3(nwg, slices), dim3(64 * G::WAVES), G::LDS, stream, g, p);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
 // DEEP buffers where every workgroup has a CU to itself, as many as let two share one otherwise.  us, few / deep: 64 x 64 tiles (4 / 8 buffers) 1024 x 1024 x 4096 (256 workgroups) 19.8 / 16.1, 1025 x 1024 x 1024

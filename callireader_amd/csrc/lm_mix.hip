@@ -46,15 +46,6 @@ struct MixArgs {
 };
 __device__ __forceinline__ const float* mix_cos(const MixArgs& p, int row, int off) { return p.ang + (int64_t)row * p.ang_ld + off; }
 
-// A launch's arguments: every 64-byte line of them is a round trip of its own, taken where the compiler places the first use.  All lines at once instead.
-__device__ __forceinline__ void touch_args() {
-    const __attribute__((address_space(4))) int* k = (const __attribute__((address_space(4))) int*)__builtin_amdgcn_kernarg_segment_ptr();
-    int x = 0;
-#pragma unroll
-    for (int i = 0; i < (int)sizeof(MixArgs); i += 64) x ^= k[i / 4];
-    asm volatile("" ::"s"(x));
-}
-
 __device__ __forceinline__ void lds_barrier() {               // LDS writes are seen by all waves; loads from memory stay under way
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
@@ -365,7 +356,7 @@ __device__ __forceinline__ void mix_retain(const MixArgs& p, int h, int row, flo
 template <typename T, int D, int NR>
 __global__ __launch_bounds__(sizeof(T) == 4 ? MIX_THREADS32 : MIX_THREADS16, 4) void lm_mix_kernel(const MixArgs p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
-    touch_args();
+    touch_args<(int)sizeof(MixArgs)>();
     const int x = blockIdx.x, row = blockIdx.y, tid = threadIdx.x;
     if (row >= p.M) {                                          // (uniform)
         const int linear = x + (int)gridDim.x * row, nth = l2_ahead_nth(linear, (int)gridDim.x * p.M);
