@@ -55,6 +55,7 @@ constexpr int FOLD_MAX_SPLITS = 8;       // K-slices of the wqkv partial-sum GEM
 // AHEAD: workgroups past the rows bring the next product's weights into L2 (launch_decode_attn)
 template <bool DIV, bool FOLD, bool AHEAD>
 __global__ __launch_bounds__(256, 2) void decode_attn_kernel(const AttnParams p) {
+    touch_args<(int)(sizeof(AttnParams))>();
     __shared__ __attribute__((aligned(16))) float s_o[16][NQ][HD];      // the workgroup's 16 partials: un-normalised O ...
     __shared__ float s_ml[16][NQ][2];                                   // ... maximum and row sum
     __shared__ __attribute__((aligned(16))) bf16x8 s_qkv[FOLD ? 6 : 1][16];   // FOLD: the rotated q heads, the new K row, the new V row

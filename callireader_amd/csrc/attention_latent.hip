@@ -56,6 +56,7 @@ template <int HT> __device__ __forceinline__ float head_sum(float x) { return he
 // O^T += C^T . P^T: each wave owns a quarter of the latent columns, C^T by transposed LDS reads.  Three LDS-only barriers per tile.
 template <int R, int HT>
 __global__ __launch_bounds__(256, 2) void latent_decode_kernel(const LatentDecodeParams p) {
+    touch_args<(int)(sizeof(LatentDecodeParams))>();
     constexpr int KT = LATENT_TILE, CH = R / 8, KS = R / 64, DT = R / 64, SLD = KT + 4, PLD = KT + 8;
     extern __shared__ __attribute__((aligned(16))) char smem[];            // 2 key tiles | scores | weights | rescale factors
     float* sS = (float*)(smem + 2 * KT * R * 2);                           // [2][16 HT][SLD]
@@ -211,6 +212,7 @@ __global__ __launch_bounds__(256, 2) void latent_decode_kernel(const LatentDecod
 // of 512: 6.3 us with rows, weights first and gates last, 5.2 now; a step of 8 layers 953 / 948 / 944 us with 1 / 2 / 4 workgroups a row block.
 template <int R, int RW>
 __global__ __launch_bounds__(512) void latent_combine_kernel(const LatentDecodeParams p) {
+    touch_args<(int)(sizeof(LatentDecodeParams))>();
     __shared__ __attribute__((aligned(16))) bf16 sA[RW][R + 8];
     __shared__ float sO[RW == 1 ? 8 : 1][RW == 1 ? R : 1];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), H = p.a.H, head = blockIdx.x, m0 = blockIdx.y * RW;      // (head fastest: the row blocks of a head share an XCD's L2)
@@ -305,6 +307,7 @@ __global__ __launch_bounds__(512) void latent_combine_kernel(const LatentDecodeP
 // q'[m][h][:] = W_uk^T q[m][h] for 16 MT tokens of one head and 128 latent columns: the query's K-slices are added in slice order and rounded once on their way into LDS
 template <int MT>
 __global__ __launch_bounds__(256) void latent_absorb_kernel(const float* __restrict__ part, int slices, int M, int H, int Ap, int Rp, const bf16* __restrict__ ukT, int dl, bf16* __restrict__ out) {
+    touch_args<56>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     bf16* sq = (bf16*)smem;                            // [16 MT][Ap + 8]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, g = lane >> 4, li = lane & 15, head = blockIdx.y, ld = Ap + 8;

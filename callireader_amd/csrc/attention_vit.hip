@@ -500,6 +500,7 @@ constexpr int FEW_KV = 2 * TILE, FEW_STEP = 2 * FEW_KV, FEW_P = 3 * FEW_STEP, FE
 
 __global__ __launch_bounds__(512, 2) void vit_attn_few_kernel(const AttnParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
+    touch_args<(int)sizeof(AttnParams)>();
     // (the head is the fastest index: of 8, 16, ... heads each has its workgroups, hence its K and V, behind one L2)
     const int head = blockIdx.x, half = blockIdx.y & 1, qb = blockIdx.y >> 1, batch = blockIdx.z, gx = gridDim.y >> 1;
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), l31 = lane & 31, hh = lane >> 5;
@@ -791,6 +792,7 @@ __device__ __forceinline__ void vit_cls_combine_any(const AttnParams& p, int nsp
 // Both in one launch: block 0 of a tile redoes what was flagged (patch rows), the others merge the class rows of four heads, a wave each.  (A launch of 4.8 us each, and a layer of one
 // tile has seven launches in all.  Workgroups past these read the output projection's weights, AttnParams::ahead.)
 __global__ __launch_bounds__(256) void vit_attn_finish_kernel(const AttnParams p, const int nb) {
+    touch_args<(int)sizeof(AttnParams) + 4>();
     if ((int)blockIdx.x > (p.H + 3) / 4) {                     // (uniform)
         const int nth = l2_ahead_nth(blockIdx.x, 1 + (p.H + 3) / 4);
         if (blockIdx.y == 0 && nth >= 0 && nth < L2_AHEAD_GROUPS) l2_ahead(p.ahead, blockIdx.x, nth);

@@ -53,6 +53,7 @@ enum { DEPI_ROPE = 100 };
 //     spilled 16-24 and lost, profiles/round5/03_*), so these instances are built for two waves per SIMD -- which is all the w1|w3 / LM-head grids ever put on a CU.
 template <int EPI, int KW, int VS, int KPR, bool PRO, int TG = 1, bool ALIAS = false, bool SW = false, bool PROW = false>
 __global__ __launch_bounds__(TG * KW * 64, (PRO && !PROW) ? 4 : 2) void gemm_decode_kernel(const DecodeGemmParams p) {      // PRO forms: 128 registers, 16 waves per CU
+    touch_args<(int)(sizeof(DecodeGemmParams))>();
     extern __shared__ __attribute__((aligned(16))) char smem[];
     constexpr int T = VS * KPR;            // 32-deep k-steps per wave and tile
     constexpr int UB = 8;                  // k-steps per register batch; two batches of weight loads are in flight (batches of 16 in the 256-register forms: +-0, round 5)

@@ -47,6 +47,7 @@ constexpr bool skinny_two(int RT, int MT) { return RT == 1 || (RT == 2 && MT <= 
 
 template <int EPI, int WAVES, int MT, int RT = 1, bool W8 = false>
 __global__ __launch_bounds__(WAVES * 64, !W8 && skinny_two(RT, MT) ? 4 : 1) void gemm_skinny_kernel(const GemmParams p) {
+    touch_args<(int)(sizeof(GemmParams))>();
     // RT = 16-row weight tiles per wave: X fragments are loaded once per RT tiles (X re-reads through L2 are the
     // bottleneck once M > 16), used where N is large enough to still fill the chip
     __shared__ float red[WAVES][RT * MT][16][17];

@@ -13,6 +13,7 @@ namespace {
 // bf16: gemm_skinny_kernel's EPI_PARTIAL and EPI_RELU2 with one tile of rows, weights in the decode layout
 template <int EPI, int RT>
 __global__ __launch_bounds__(512) void ahead_skinny_kernel(const LmAhead a, const bf16* __restrict__ W, void* __restrict__ C, int N) {
+    touch_args<(int)(sizeof(LmAhead) + 20)>();
     extern __shared__ __attribute__((aligned(16))) bf16 hs[];  // [M][K + 8]
     __shared__ float red[8][RT][16][17], sums[AHEAD_SEGS];
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -68,6 +69,7 @@ __global__ __launch_bounds__(512) void ahead_skinny_kernel(const LmAhead a, cons
 template <int EPI>
 __global__ __launch_bounds__(512) void ahead_rows_kernel(const LmAhead a, const float* __restrict__ W, float* __restrict__ C, int N, const float* __restrict__ gate, int64_t ldg,
                                                          const int32_t* __restrict__ tok) {
+    touch_args<(int)(sizeof(LmAhead) + 48)>();
     constexpr int U = 8;
     extern __shared__ __attribute__((aligned(16))) float hf[];      // [M][K + 4]
     __shared__ __attribute__((aligned(16))) char sm[8 * U * 1024];

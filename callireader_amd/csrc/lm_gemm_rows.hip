@@ -17,6 +17,7 @@ constexpr int NW = LM_CHAINS;                // waves of a workgroup, one chain 
 
 template <int MT, int EPI>
 __global__ __launch_bounds__(64 * NW) void lm_rows_kernel(const LmGemmParams p) {
+    touch_args<(int)(sizeof(LmGemmParams))>();
     constexpr int U = MT == 4 ? 4 : 8;       // 16-deep steps whose loads are issued together
     constexpr int RED = NW * MT * 16 * 17 * 4, RING = NW * U * 1024;
     __shared__ __attribute__((aligned(16))) char sm[RED > RING ? RED : RING];      // the waves' U steps of W; after the products their partial tiles

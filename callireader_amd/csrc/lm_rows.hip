@@ -118,6 +118,7 @@ __global__ __launch_bounds__(TPB) void lm_embed_step_kernel(const T* __restrict_
 template <typename T, int TPB, int NV>
 __global__ __launch_bounds__(TPB) void lm_post_kernel(const LmPostIn in, int M, int Wp, int W, float eps, float* __restrict__ xio,
                                                       const float* __restrict__ gain_b, int replace, const LmSink to) {
+    touch_args<(int)(sizeof(LmPostIn) + 64)>();
     __shared__ float red[TPB / 64];
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x;
@@ -217,6 +218,7 @@ template <typename T>
 __global__ __launch_bounds__(256) void lm_latents_kernel(T* __restrict__ a, const float* __restrict__ part, int slices, int M, int Na, int q_rank, int Qp, int off_c, int kv_rank, int Rp,
                                                          int off_g, float eps, const float* __restrict__ nq, const float* __restrict__ nc, T* __restrict__ cq, T* __restrict__ c_dense,
                                                          T* __restrict__ cache, int max_tokens, const LmRowIndex ix, T* __restrict__ ao, int n_ao, int Gp) {
+    touch_args<(int)(100)>();
     __shared__ float red[4];
     const int tid = threadIdx.x;
     const int64_t row = blockIdx.x;
@@ -320,6 +322,7 @@ __global__ __launch_bounds__(256) void lm_side_act_kernel(const float* __restric
 // the same z for up to 16 rows, kept in LDS, and y = z . W^T behind it: a workgroup forms z for itself (a few KiB from L2) and multiplies 64 rows of W, 16 per wave
 __global__ __launch_bounds__(256) void lm_side_proj_kernel(const float* __restrict__ part, int slices, int M, int Sp, const bf16* __restrict__ side, int64_t lds, const int32_t* __restrict__ tok,
                                                            const bf16* __restrict__ W, int N, bf16* __restrict__ y) {
+    touch_args<(int)(64)>();
     extern __shared__ __attribute__((aligned(16))) bf16 sz[];              // [16][Sp + 8]
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, ld = Sp + 8, n0 = blockIdx.x * 64 + wave * 16;
     const bf16* w = W + (int64_t)min(n0 + (lane & 15), N - 1) * Sp + (lane >> 4) * 8;

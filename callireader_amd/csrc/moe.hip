@@ -220,6 +220,7 @@ __global__ __launch_bounds__(256) void lm_router_slice_kernel(const bf16* __rest
 constexpr int POST_COLS = 2048, POST_E = 64, POST_BATCH = 32, POST_COLS_TWO = 1536;      // columns and experts at most; experts of a batch of weights, columns at most with two batches
 __global__ __launch_bounds__(512) void lm_post_route_kernel(const LmAhead a, bf16* __restrict__ h, const bf16* __restrict__ Wr, int wsw, const float* __restrict__ corr, int E, int top, int groups,
                                                             int keep, int32_t* __restrict__ idx, float* __restrict__ wt) {
+    touch_args<(int)(sizeof(LmAhead) + 64)>();
     constexpr int SL = LM_ROUTER_SLICES / 8, MAX_PER = POST_COLS / 32 / LM_ROUTER_SLICES, PAIR = POST_BATCH / 16;      // slices a wave, k-steps a slice, blocks of 16 experts a batch
     __shared__ __attribute__((aligned(16))) bf16 hs[POST_COLS];
     __shared__ __attribute__((aligned(16))) float part[LM_ROUTER_SLICES][POST_E];

@@ -114,6 +114,7 @@ __global__ __launch_bounds__(256, 2) void moe_tiled_kernel(const MoeGemmParams p
 // SRC = true (gate | up): A rows are tokens; false (down): A rows are assignments.  C rows are assignments (token * top + slot) either way.
 template <bool GLU, int RT, int WAVES>
 __global__ __launch_bounds__(WAVES * 64) void moe_stream_kernel(const MoeGemmParams p) {
+    touch_args<(int)(sizeof(MoeGemmParams))>();
     __shared__ float red[WAVES][RT][16][17];
     __shared__ int list[64];
     __shared__ int s_count;

@@ -60,6 +60,7 @@ __device__ __forceinline__ void store_row_e4m3(const NormParams& p, int64_t orow
 template <int TPR, int MODE, bool LATE, bool AHEAD = false>
 __global__ __launch_bounds__(256) void layernorm_kernel(const NormParams p) {
     __shared__ float red[4];
+    touch_args<(int)sizeof(NormParams)>();
     const int tid = threadIdx.x;
     constexpr int RPB = 256 / TPR;
     if constexpr (AHEAD) {
