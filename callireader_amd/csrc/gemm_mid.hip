@@ -223,10 +223,18 @@ __device__ __forceinline__ void ring_tail(F f) {
     }
 }
 
+// K-tile u of an unrolled round goes to buffer u (of four) or to the one before it (of more: the kernel's loop), by an instruction offset of 128 u that is taken off the LDS address again: bytes ahead of the
+// first buffer that keep that address from being negative (none with four buffers: two workgroups of 96 x 64 fill a CU's LDS to the byte)
+constexpr int mid_pad(int nbuf, int round, int stage) {
+    int pad = 0;
+    for (int u = 0; nbuf > 3 && u < round; u++) pad = std::max(pad, u * 128 - (nbuf > 4 ? (u + nbuf - 1) % nbuf : u % nbuf) * stage);
+    return (pad + 511) / 512 * 512;
+}
 // WM x WN waves of FM x FN fragments of 16 x 16
 template <int WM, int WN, int FM, int FN, int NBUF>
 struct MidGeom {
-    static constexpr int BM = WM * FM * 16, BN = WN * FN * 16, WAVES = WM * WN, PIECES = (BM + BN) / 8, PER = (PIECES + WAVES - 1) / WAVES, STAGE = PIECES * 1024, ROUND = NBUF % 2 ? 2 * NBUF : NBUF, PAD = (ROUND * 128 + 511) / 512 * 512, LDS = PAD + NBUF * STAGE;
+    static constexpr int BM = WM * FM * 16, BN = WN * FN * 16, WAVES = WM * WN, PIECES = (BM + BN) / 8, PER = (PIECES + WAVES - 1) / WAVES, STAGE = PIECES * 1024, ROUND = NBUF % 2 ? 2 * NBUF : NBUF, PAD = mid_pad(NBUF, ROUND, STAGE), LDS = PAD + NBUF * STAGE;
+    static constexpr bool TWO_A_CU = 2 * LDS <= 160 * 1024;
     static_assert(WAVES * 32 * (FN * 32 + 16) <= LDS, "the epilogue's stage lies in the buffers");
     static_assert((NBUF - 1) * PER <= 63 && NBUF >= 3 && LDS <= 160 * 1024, "vmcnt is six bits wide; a CU has 160 KiB");
 };
@@ -504,11 +512,15 @@ int launch_t(int epi, const GemmParams& p, int rt, hipStream_t stream) {
     hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, FM, FN, NBUF, FAR>), dim3(nwg, slices), dim3(64 * G::WAVES), G::LDS, stream, g, p);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
-// DEEP buffers where every workgroup has a CU to itself, as many as let two share one otherwise.  us, few / deep: 64 x 64 tiles (4 / 8 buffers) 1024 x 1024 x 4096 (256 workgroups) 19.8 / 16.1, 1025 x 1024 x 1024
-// (272) 9.7 / 12.3, 1025 x 4096 x 1024 (1088) 23.0 / 27.0; 128 x 64 (3 / 6) 1025 x 1024 x 4096 (144) 25.7 / 22.5, 1025 x 4096 x 1024 (576) 20.7 / 23.3; 64 x 128 (3 / 6) 23.6 / 20.7 and 20.3 / 23.6
+// DEEP buffers where every workgroup has a CU to itself, as many as let two share one otherwise (by LDS and by registers).  us, few / deep: 16 x 64 tiles (7 / 8 buffers)
+// 1025 x 1024 x 1024 (1040 workgroups) 13.9 / 17.6; 64 x 64 (4 / 8) 1024 x 1024 x 4096 (256) 19.8 / 16.1, 1025 x 1024 x 1024 (272) 9.7 / 12.3, 1025 x 4096 x 1024 (1088) 23.0 / 27.0; 96 x 64 (3 / 6) 25000 x 64 x
+// 512 (261) 7.8 / 9.5, 1500 x 2048 x 1024 (512) 13.6 / 15.8, 3000 x 2048 x 4096 (1024) 79.5 / 88.8; 128 x 64 (3 / 6) 1025 x 1024 x 4096 (144) 25.7 / 22.5, 1025 x 4096 x 1024 (576) 20.7 / 23.3; 64 x 128 (3 / 6)
+// 23.6 / 20.7 and 20.3 / 23.6.  The law below gives these shapes more workgroups than CUs only at the ends of the range: 64 columns or fewer in more than 24 000 rows (96 and 128 x 64), fewer than 65 rows of a K that
+// the weight-streaming kernels do not take (16 and 64 x 64, 64 x 128).
 template <int WM, int WN, int FM, int FN, int FEW, int DEEP>
 int launch_two(int epi, const GemmParams& p, int rt, hipStream_t stream) {
     typedef MidGeom<WM, WN, FM, FN, FEW> G;
+    static_assert(G::TWO_A_CU);
     const int64_t wgs = (int64_t)std::max((p.M + G::BM - 1) / G::BM, rt) * ((p.N + G::BN - 1) / G::BN) * (epi == EPI_PARTIAL ? p.group : 1);
     return wgs <= cr_device_cus() ? launch_t<WM, WN, FM, FN, DEEP>(epi, p, rt, stream) : launch_t<WM, WN, FM, FN, FEW>(epi, p, rt, stream);
 }
@@ -557,11 +569,11 @@ int launch_gemm_mid(int epi, const GemmParams& p, hipStream_t stream) {
     if (7 * 2 * std::max(p.lda, p.ldw) + 128 > (int64_t)UINT32_MAX) return launch_t<2, 4, 2, 4, 3, true>(epi, p, 0, stream);      // (whatever the epilogue; the same bits)
     switch (tile) {
         case 1: return launch_t<1, 2, 1, 1, 12>(epi, p, rt, stream);
-        case 2: return launch_t<1, 4, 1, 1, 8>(epi, p, rt, stream);
+        case 2: return launch_two<1, 4, 1, 1, 7, 8>(epi, p, rt, stream);
         case 3: return launch_t<1, 4, 2, 1, 6>(epi, p, rt, stream);
         case 4: return launch_t<2, 2, 2, 1, 6>(epi, p, rt, stream);
         case 5: return launch_two<2, 4, 2, 1, 4, 8>(epi, p, rt, stream);
-        case 6: return launch_t<2, 4, 3, 1, 6>(epi, p, rt, stream);
+        case 6: return launch_two<2, 4, 3, 1, 3, 6>(epi, p, rt, stream);
         case 7: return launch_two<2, 4, 4, 1, 3, 6>(epi, p, rt, stream);
         case 8: return launch_two<2, 4, 2, 2, 3, 6>(epi, p, rt, stream);
         case 9: return launch_t<2, 4, 3, 2, 5>(epi, p, rt, stream);

@@ -11,8 +11,10 @@ def operands(M, N, K):
     return [torch.randn(*s, generator=g).bfloat16().cuda() for s in ((M, K), (N, K), (N,), (M, N))]
 
 
-@pytest.mark.parametrize('K', [64, 192, 320, 448, 704, 960, 1024, 1088, 1216])
-@pytest.mark.parametrize('M,N', [(150, 136), (145, 512), (1111, 1111)])
+# K-tiles: fewer than the buffers, then none, one and two rounds and a rest of each depth (a round of 3 to 12 K-tiles, 14 of seven buffers, and as many again asked for ahead; K = 2304 is two rounds of twelve);
+# workgroups: at most one a CU, or several (1500 x 1500: 288 to 8 836 of every shape up to 128 x 64 and 64 x 128)
+@pytest.mark.parametrize('K', [64, 192, 320, 448, 704, 960, 1024, 1088, 1216, 1472, 1536, 1792, 2304])
+@pytest.mark.parametrize('M,N', [(150, 136), (145, 512), (1111, 1111), (1500, 1500)])
 def test_depths_of_buffers(M, N, K):
     from callireader_amd import engine as E
     A, W, bias, res = operands(M, N, K)
