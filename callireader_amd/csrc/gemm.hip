@@ -15,7 +15,27 @@ int launch_gemm256(int epi, const GemmParams& p, hipStream_t stream);
 int launch_gemm256_f8(int epi, const GemmParams& p, hipStream_t stream);
 bool gemm_skinny_supported(int epi, const GemmParams& p);
 int launch_gemm_skinny(int epi, const GemmParams& p, hipStream_t stream);
-double gemm256_cost(const GemmParams& p);
+double gemm256_cost(const GemmParams& p, double full);
+
+// Rows of a product that the 256x256 kernel takes, the others go to gemm_mid: all, none, or those up to a multiple of 256, as a few rows past it can cost the persistent kernel a round of tiles (32 ViT tiles are
+// 128 x 256 + 32 rows: three rounds for two rounds' work at N = 1024).  Apart only where the laws see 3 % in it, also with rounds that fill the card (what is cut off leaves mostly those) priced FULL above
+// the others.  us, whole | apart: 3162 x 4096 x 4096 (208 tiles of 256 rows; 256 of 192) 80.3 | 85.6, 3162 x 4096 x 14336 270 | 285, 6145 x 2048 x 2048 43.1 | 45.6, 696 x 28672 x 8192 278 | 325; 4100 x 4096 x
+// 4096 126 | 99.7, 6145 x 4096 x 4096 157 | 149, 6145 x 6144 x 4096 241 | 219.  Of 421 sizes with rows past a multiple of 256 it is the slower choice by more than 2 % at three (at most 3 %), without
+// either rule at sixteen.
+int gemm_tiled_rows(int epi, const GemmParams& p) {
+    constexpr double APART = 1.03, FULL = 0.08;
+    int tile, rt;
+    const int r = p.M % 256;
+    const double whole = gemm256_cost(p, 0.0), mid = gemm_mid_cost(epi, p, &tile, &rt);
+    if (r > 0 && p.M > r && epi != EPI_PATCH && epi != EPI_ARGMAX) {
+        GemmParams a = p, b = p;
+        a.M = p.M - r;
+        b.M = r;
+        const double rest = gemm_mid_cost(epi, b, &tile, &rt), cut = gemm256_cost(a, 0.0) + rest;
+        if (APART * cut < whole && gemm256_cost(a, FULL) + rest < gemm256_cost(p, FULL)) return mid < cut ? 0 : a.M;
+    }
+    return mid < whole ? 0 : p.M;
+}
 
 int launch_gemm(int epi, const GemmParams& p, hipStream_t stream) {
     if (p.M <= 0 || p.N <= 0 || p.K <= 0 || (p.K % 64) != 0) return CR_ERR_ARG;
@@ -42,22 +62,15 @@ int launch_gemm(int epi, const GemmParams& p, hipStream_t stream) {
         default: return CR_ERR_ARG;
     }
     if (force == 128 || !gemm256_supported(epi, p)) return launch_gemm_mid(epi, p, stream);
-    // Whole on either kernel, or the rows past a multiple of 256 on their own: a few of them can cost the persistent kernel a round of tiles (32 ViT tiles are 128 x 256 + 32 rows:
-    // three rounds for two rounds' work at N = 1024).
-    int tile, rt;
-    const int r = p.M % 256;
-    double whole = gemm256_cost(p), mid = gemm_mid_cost(epi, p, &tile, &rt), cut = 1e30;
+    const int rows = gemm_tiled_rows(epi, p);
+    if (rows == 0) return launch_gemm_mid(epi, p, stream);
+    if (rows == p.M) return launch_gemm256(epi, p, stream);
     GemmParams a = p, b = p;
-    if (r > 0 && p.M > r && epi != EPI_PATCH && epi != EPI_ARGMAX) {
-        a.M = p.M - r;
-        b.M = r;
-        b.A = p.A + (int64_t)a.M * p.lda;
-        b.C = (char*)p.C + (int64_t)a.M * p.ldc * (epi == EPI_F32 ? 4 : 2);
-        if (p.res) b.res = p.res + (int64_t)a.M * p.ldr;
-        cut = gemm256_cost(a) + gemm_mid_cost(epi, b, &tile, &rt);
-    }
-    if (mid < whole && mid < cut) return launch_gemm_mid(epi, p, stream);
-    if (whole <= cut) return launch_gemm256(epi, p, stream);
+    a.M = rows;
+    b.M = p.M - rows;
+    b.A = p.A + (int64_t)rows * p.lda;
+    b.C = (char*)p.C + (int64_t)rows * p.ldc * (epi == EPI_F32 ? 4 : 2);
+    if (p.res) b.res = p.res + (int64_t)rows * p.ldr;
     const int rc = launch_gemm256(epi, a, stream);
     return rc != CR_OK ? rc : launch_gemm_mid(epi, b, stream);
 }

@@ -531,17 +531,20 @@ namespace {
 
 // Tile shapes (launch_gemm_mid's `tile` = index + 1).  Eight waves where the tile is large enough to feed them: two waves a SIMD cover each other's LDS reads and barriers (64 x 64 at
 // M = 1025, N = 1024, K = 4096: four waves 27.5 us, eight 26.6, now 26.2; 128 x 128 at N = 3072, K = 1024: 20 and 13.4).
-struct MidShape { int bm, bn; };
-constexpr MidShape SHAPES[] = {{16, 32}, {16, 64}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {64, 128}, {96, 128}, {128, 128}, {96, 256}, {128, 256}, {160, 128}};
+struct MidShape { int bm, bn; double launch = 2.5, row = 1.9e-3, step = -0.02; };      // (the law's: us a launch, a row of A or W in a K-tile, a K-tile)
+constexpr MidShape SHAPES[] = {{16, 32}, {16, 64}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {64, 128}, {96, 128}, {128, 128}, {96, 256, 2.5, 2e-3, 0.0}, {128, 256, 3.0, 2e-3, 0.02}, {160, 128, 2.5, 1.9e-3, 0.03}};
 constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 
 }  // namespace
 
 // A law to choose by, in us, and the tile shape (and number of row tiles) that takes least by it: launch and drain 2.5 us, a round of workgroups 1 us to its first K-tile, 1.9 ns per row of A or W in
-// each K-tile of 64 less 20 ns (the two shapes of three buffers 2.1 ns and 50 ns more), 0.1 ns an element in the epilogue; a workgroup more on a CU costs its time again.  It is no prediction.  Measured /
-// law, weights cold: 1025 x 1024 x 4096 18.7 / 20.2, 1025 x 1024 x 1024 7.9 / 8.1, 1025 x 3072 x 1024 11.5 / 11.9, 1025 x 4096 x 1024 14.9 / 13.3, 77 x 4096 x 4096 15.0 / 14.1, 333 x 4096 x 14336 81 / 69,
-// 1000 x 4096 x 14336 135 / 113; no term stands for the rate of HBM itself, which bounds wide weights at few rows (77 x 28672 x 4096 54 / 32).  At 37 products of M 77 .. 8200, N 1024 .. 28672,
-// K 512 .. 14336 the kernel that the two laws (here and tile_us in gemm256.hip) choose was the fastest of gemm_mid, 256-row and 192-row tiles, or within 4 % of it.
+// each K-tile of 64 less 20 ns (the three largest shapes more: SHAPES), 0.1 ns an element in the epilogue; a workgroup more on a CU costs its time again (two shallow ones to a CU take 0.8 of that).  It is no
+// prediction.  Measured / law, weights cold: 1025 x 1024 x 4096 18.7 / 20.2, 1025 x 1024 x 1024 7.9 / 8.1, 1025 x 3072 x 1024 11.5 / 11.9, 1025 x 4096 x 1024 14.4 / 14.1, 77 x 4096 x 4096 15.0 / 12.1, 333 x
+// 4096 x 14336 81 / 68, 1000 x 4096 x 14336 135 / 110, 13325 x 5120 x 1344 199 / 190; no term stands for the rate of HBM itself, which bounds wide weights at few rows (77 x 28672 x 4096 54 / 29).
+// Against every way there is, 500 sizes drawn over M 65 .. 16000, N 512 .. 28672, K 256 .. 14336 (profiles/tiled_products/choice.txt): 1.006 times the fastest in geometric mean, above 1.05 at 15 of them.
+// The largest shapes' terms decide where a product takes several rounds of one and fewer of the other, above all where K leaves 64 modulo 128, which the 256x256 kernel does not take.  us, 160 x 128 | 128 x
+// 256: 3075 x 9216 x 448 48.3 | 39.9, 6124 x 9216 x 2240 260 | 228, 13325 x 5120 x 1344 212 | 199, and one round either way 2050 x 2048 x 2048 24.2 | 29.4; 96 x 128 | 96 x 256: 356 x 12800 x 14336 215 | 177,
+// 1923 x 2560 x 14336 186 | 162.
 double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
     const int nf = (p.M + 15) / 16, slices = epi == EPI_PARTIAL && p.group > 0 ? p.group : 1, nk = p.K / 64 / slices, cus = cr_device_cus();
     double best = 1e30;
@@ -554,8 +557,7 @@ double gemm_mid_cost(int epi, const GemmParams& p, int* tile, int* row_tiles) {
             if (want < least || want > nf || (per_cu && want > 2L * least)) continue;
             const int rows = 16 * ((nf + (int)want - 1) / (int)want);
             const double rounds = (double)((want * ntn + cus - 1) / cus);
-            const int side = rows + SHAPES[t].bn;
-            const double c = 2.5 + rounds * (1.0 + nk * (t == 10 || t == 11 ? 0.05 + 0.0021 * side : 0.0019 * side - 0.02) + 1e-4 * rows * SHAPES[t].bn);
+            const double c = SHAPES[t].launch + rounds * (1.0 + nk * (SHAPES[t].row * (rows + SHAPES[t].bn) + SHAPES[t].step) + 1e-4 * rows * SHAPES[t].bn);
             if (c < best - 1e-9) { best = c; *tile = t + 1; *row_tiles = (int)want; }
         }
     }
