@@ -31,9 +31,12 @@ inline int64_t l2_ahead_beside_latent(int64_t own, int cus) { return (int64_t)(2
 //   bf16, one key split: up to 256 own 0.98 .. 1.07; 288 .. 960 0.95 .. 1.05 with 34 MiB, 0.97 .. 1.05 with 26; where all that there is are 7 MiB, 320 .. 512 0.97 .. 0.99.
 //   Several splits (retention then streams its states through the caches before the weights' reader starts): up to 256 0.97 .. 1.05, 320 0.98 .. 1.04, 384 .. 1024 0.93 .. 1.03, mostly below one.
 //   float32, whose workgroups have a CU each: up to 128 0.99 .. 1.04; 144 .. 192 0.95 .. 1.03, the first product alone 1.00 .. 1.03 (of 32 MiB 0.99 .. 1.02); 200 .. 256 0.95 .. 1.03 and 0.98 .. 1.03.
+//   float32 with heads of 128 and more, by the bytes of keys and values that its workgroups read (profiles/read_ahead/float32_keys.txt): 2048 wide up to 26 MB 0.99 .. 1.03, 33 .. 164 (5 rows of 400 keys, 4 of 520
+//   and more) 0.98 .. 1.00; 1024 wide, 14 passes, up to 26 MB 1.00 .. 1.05, 34 .. 131 0.99 .. 1.00.  Heads of 64 lose nothing by 98 MB (0.99 .. 1.06).
 struct L2AheadRoom { int64_t most, least; int products; };
-inline L2AheadRoom l2_ahead_beside_mixer(bool f32, int64_t own, int splits, int cus) {
+inline L2AheadRoom l2_ahead_beside_mixer(bool f32, int64_t own, int splits, int cus, int dim = 0, int64_t key_bytes = 0) {
     constexpr int64_t MiB = 1 << 20;
+    if (f32 && dim >= 128 && key_bytes > 30 * MiB) return {};
     if (f32) return 2 * own <= cus ? L2AheadRoom{34 * MiB, 0, L2_AHEAD_MOST} : 4 * own <= 3 * cus ? L2AheadRoom{16 * MiB, 0, 1} : L2AheadRoom{};
     if (own <= cus) return {34 * MiB, 0, L2_AHEAD_MOST};
     return splits > 1 && 4 * own > 5 * cus ? L2AheadRoom{} : L2AheadRoom{26 * MiB, 8 * MiB, L2_AHEAD_MOST};

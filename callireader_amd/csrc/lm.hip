@@ -260,6 +260,7 @@ struct Step {
     int nsplit, split;              // decode, latent attention: splits of the longest sequence, keys per split
     std::vector<KeyPlan> plans;     // prefill, one per distinct chunk size
     std::vector<int> hsplit;        // decode: attention splits per distinct chunk size
+    std::vector<int64_t> hkeys;     // decode: keys that the rows see together, per distinct chunk size
     const int32_t *d_rseg, *d_snap0, *d_chunks;      // prefill: {first row, rows, first position, sequence} per segment, its first retention chunk; {first row, rows} per chunk
     int snaps, longest;
 };
@@ -472,9 +473,9 @@ int latent_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer
 // out, the first that is too large ends the list.  The token side's small products (0.3 MB and two launches that wait for each other) are not fetched.  float32 leaves the next projection out as well: 512 wide,
 // 2 rows 204 us a step without any fetching, 205 without it, 214 with it; 1024 wide it does not fit anyway.  Us a step with nothing / the output projection alone / all that fits (delay in lm_mix.hip): 1024 wide, 14
 // passes, 1 row 469 / 471 / 443; float32 2 rows 725 / 726 / 708, 8 rows 820 / 817 / 795; 2048 wide, 8 layers, whose up projection no longer fits, 1 row 453 / 447, 4 rows 487 / 482, 32 rows 720 / 710.
-L2AheadList behind_mixer(const Lm& lm, int M, const LmLayer& L, size_t r, int unit, int splits) {
+L2AheadList behind_mixer(const Lm& lm, int M, const LmLayer& L, size_t r, int unit, int splits, int64_t keys) {
     const int64_t own = (L.heads() ? (int64_t)M * (L.s.attn.heads / unit) * (lm.f32 ? 1 : splits) : 0) + (L.retention() && (lm.f32 || splits == 1) ? (int64_t)M * L.s.ret.heads : 0);
-    const L2AheadRoom room = l2_ahead_beside_mixer(lm.f32, own, splits, cr_device_cus());
+    const L2AheadRoom room = l2_ahead_beside_mixer(lm.f32, own, splits, cr_device_cus(), L.Ap, L.heads() ? keys * L.s.attn.heads * 2 * L.Ap * (int64_t)lm.esz() : 0);
     L2AheadList l{};
     int64_t bytes = 0;
     bool full = false;
@@ -520,7 +521,7 @@ int heads_mixer(cr_ctx* c, cr_kv* kv, const Step& sp, Buffers& b, const LmLayer&
         in.M = M; in.part = b.sl; in.slices = s_a; in.where = b.where; in.ang = b.ang; in.ao = b.ao; in.cache_k = ck; in.cache_v = cv; in.ring = ring; in.chunk = chunk; in.rows = unit; in.nsplit = split ? splits : 1;
         in.state = state;
         if (split) { in.part_o = b.part; in.part_ml = b.part + (size_t)M * a.heads * splits * L.Ap; }
-        const L2AheadList ahead = behind_mixer(lm, M, L, r, unit, splits);
+        const L2AheadList ahead = behind_mixer(lm, M, L, r, unit, splits, L.heads() ? sp.hkeys[L.chunk_ix] : 0);
         in.ahead = &ahead;
         return launch_lm_mix(lm.f32, lm, L, in, st);
     }
@@ -799,8 +800,10 @@ int lm_decode_step(cr_ctx* c, cr_kv* kv, int n, const int64_t* force_tokens, flo
     sp.split = latent_split_keys(heads, keys); sp.nsplit = (longest + sp.split - 1) / sp.split;
     for (int chunk : lm.chunks) {
         int most = 0;
-        for (int32_t s : kv->seqs_on_device) most = std::max(most, kv->len[s] % chunk + 1);
+        int64_t all = 0;
+        for (int32_t s : kv->seqs_on_device) { most = std::max(most, kv->len[s] % chunk + 1); all += kv->len[s] % chunk + 1; }
         sp.hsplit.push_back((most + HEADS_SPLIT - 1) / HEADS_SPLIT);
+        sp.hkeys.push_back(all);
     }
     const size_t cb = carve_bytes(lm, sp);
     CR_TRY(ws_ensure(c, cb + (size_t)n * lm.Wp * lm.esz() + (size_t)n * lm.d.vocab * 4 + 1024));

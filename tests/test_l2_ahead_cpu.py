@@ -23,6 +23,10 @@ int main(int n, char** v) {
         const L2AheadRoom r = l2_ahead_beside_mixer(atoi(v[1]), atol(v[2]), atoi(v[3]), atoi(v[4]));
         return printf("%ld %ld %d\n", (long)(r.most >> 20), (long)(r.least >> 20), r.products), 0;
     }
+    if (n == 6) {
+        const L2AheadRoom r = l2_ahead_beside_mixer(true, atol(v[1]), atoi(v[2]), 256, atoi(v[3]), atol(v[4]) * atol(v[5]));
+        return printf("%ld %ld %d\n", (long)(r.most >> 20), (long)(r.least >> 20), r.products), 0;
+    }
     const long N = atol(v[1]), K = atol(v[2]), es = atol(v[3]), tiles = atol(v[4]), own = atol(v[5]), width = atol(v[6]);
     static char base;
     const L2Ahead a = l2_ahead_of(&base, N * K * es, (int)(N / (16 * tiles)));
@@ -98,3 +102,11 @@ def test_beside_a_mixer_less_where_the_chip_is_full(walk):
     assert room(0, 10, 1) == room(0, 256, 4) == (34, 0, 5)
     assert room(0, 257, 1) == room(0, 320, 2) == (26, 8, 5) and room(0, 321, 2) == (0, 0, 0)
     assert room(1, 128, 1) == (34, 0, 5) and room(1, 129, 1) == room(1, 192, 1) == (16, 0, 1) and room(1, 193, 1) == (0, 0, 0)
+
+
+def test_beside_a_float32_mixer_until_its_keys_need_the_caches(walk):
+    # rows of 2048 wide, 16 heads of 128 and 8 of retention; heads of 64, 768 wide
+    wide = lambda rows, keys: walk(24 * rows, -(-keys // 256), 128, 16 * 2 * 128 * 4, rows * keys).stdout      # noqa: E731
+    assert wide(1, 40) == wide(1, 1200) == wide(4, 400) == wide(5, 300) == '34 0 5\n'
+    assert wide(1, 2000) == wide(4, 520) == wide(5, 400) == '0 0 0\n'
+    assert walk(128, 8, 64, 12 * 2 * 64 * 4, 8 * 2000).stdout == '34 0 5\n'
