@@ -264,7 +264,7 @@ bool decode_attn_fold_supported(const AttnParams& p, int head_dim) {
 // The weights go along only where the rows' own keys leave the caches room for them, in a kernel of its own: the branch alone costs the other one 2 % (64 rows of 3164 keys 146.1 us a launch, 149.1).
 int launch_decode_attn(const AttnParams& p, hipStream_t stream) {
     const int own = p.nsplit * p.H;
-    const bool ahead = p.ahead.at && own % 8 == 0 && l2_ahead_beside_attention((int64_t)own * p.B, cr_device_cus());
+    const bool ahead = p.ahead.at && p.s_div != 1.0f && own % 8 == 0 && l2_ahead_beside_attention((int64_t)own * p.B, cr_device_cus());
     const dim3 grid(p.nsplit, p.H, p.B + (ahead ? (L2_AHEAD_GROUPS + own - 1) / own : 0));
     if (p.qkv_part && !decode_attn_fold_supported(p, HD)) return CR_ERR_ARG;
     auto launch = [&](auto div, auto fold, auto with) {
@@ -272,8 +272,8 @@ int launch_decode_attn(const AttnParams& p, hipStream_t stream) {
     };
     const std::true_type yes{};
     const std::false_type no{};
-    auto with = [&](auto div, auto fold) { ahead ? launch(div, fold, yes) : launch(div, fold, no); };
-    auto folded = [&](auto div) { p.qkv_part ? with(div, yes) : with(div, no); };
-    p.s_div != 1.0f ? folded(yes) : folded(no);
+    auto folded = [&](auto div, auto with) { p.qkv_part ? launch(div, yes, with) : launch(div, no, with); };
+    if (p.s_div == 1.0f) folded(no, no);                      // (scores that are not divided: no caller of these has weights to bring along)
+    else ahead ? folded(yes, yes) : folded(yes, no);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
