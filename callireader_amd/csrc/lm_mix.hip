@@ -414,13 +414,13 @@ bool lm_mix_supported(bool f32, const LmLayer& L) {
 //   40 x 2500 (400) -5.  Two a CU: heads of 128 gain throughout (16 on 16, 64 x 2500 +20); of 64, whose cache rows of 128 bytes come in pieces of 32, up to four rounds: 32 on 32,
 //   9 x 900 (1152) +1.7, 64 x 200 (2048) +4.5, 9 x 2500 (2880) -1.4, 64 x 900 (8192) -15; 32 on 2 (groups of 16), 64 x 900 (512) +0.6, 64 x 2500 (1280) -2.
 bool lm_mix_pays(bool f32, const LmLayer& L, int M, int rows, int splits) {
-    constexpr int64_t CUS = 256;
+    const int64_t cus = cr_device_cus();
     const int64_t att = L.heads() ? (int64_t)M * (L.s.attn.heads / rows) * (f32 ? 1 : splits) : 0, ret = L.retention() ? (int64_t)M * L.s.ret.heads : 0;
-    if (f32) return att + ret <= (!L.heads() || L.Ap <= 64 || splits <= 1 ? CUS : CUS * ((L.Ap <= 128 ? 4 : 3) - (splits > 4)) / 4);
+    if (f32) return att + ret <= (!L.heads() || L.Ap <= 64 || splits <= 1 ? cus : cus * ((L.Ap <= 128 ? 4 : 3) - (splits > 4)) / 4);
     if (!L.heads()) return true;
     const int lds = L.Ap == 64 ? mix_lds16<64>(rows) : mix_lds16<128>(rows);
-    if (2 * lds > 160 * 1024) return att <= CUS;
-    return L.Ap == 128 || att <= (rows > 8 ? 4 : 8) * CUS;
+    if (2 * lds > 160 * 1024) return att <= cus;
+    return L.Ap == 128 || att <= (rows > 8 ? 4 : 8) * cus;
 }
 
 int launch_lm_mix(bool f32, const Lm& lm, const LmLayer& L, const LmMixIn& in, hipStream_t st) {
