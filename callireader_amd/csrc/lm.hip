@@ -488,7 +488,7 @@ L2AheadList behind_mixer(const Lm& lm, int M, const LmLayer& L, size_t r, int un
         bytes += l2_ahead_bytes(w);
     };
     add(L.wo, L.wo_dl, lm.Wp, L.Gp, true);
-    if (L.s.ff == CR_FF_MOE) return l;
+    if (L.s.ff == CR_FF_MOE) return l;                        // (`least` or not: 3 MiB of wo beside 280 .. 600 workgroups ahead of experts, 1024 wide, 6 layers, us a step with / without: 28 rows 344 / 350, 48 402 / 416, 60 454 / 464)
     if (L.s.ff == CR_FF_DENSE) {
         add(L.wgu, L.wgu_dl, L.ffp, lm.Wp, false);
         add(L.wdn, L.wdn_dl, lm.Wp, L.ffp, true);
