@@ -262,21 +262,14 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
     }
 }
 
-template <int WM, int WN, int FM, int FN, int KB, int NBUF, bool FAR>
-int launch_f(int epi, const LmGemmParams& p, int ntm, hipStream_t st) {
+template <int WM, int WN, int FM, int FN, int KB, int NBUF, bool FAR = false>
+int launch_t(int epi, const LmGemmParams& p, int ntm, hipStream_t st) {
     typedef Geom<WM, WN, FM, FN, KB, NBUF> G;
     static std::atomic<uint64_t> attr_done{0};
     if (!cr_dyn_lds_once(attr_done, (const void*)lm_tiles_kernel<WM, WN, FM, FN, KB, NBUF, FAR>, G::LDS)) return CR_ERR_HIP;
     hipLaunchKernelGGL((lm_tiles_kernel<WM, WN, FM, FN, KB, NBUF, FAR>), dim3((p.N + G::BN - 1) / G::BN, ntm, p.batch > 0 ? p.batch : 1), dim3(64 * G::WAVES), G::LDS, st, p, epi, ntm);
     CR_HIP(hipGetLastError());
     return CR_OK;
-}
-
-template <int WM, int WN, int FM, int FN, int KB, int NBUF>
-int launch_t(int epi, const LmGemmParams& p, int ntm, hipStream_t st) {
-    // (eight rows of either operand, and an XOR that keeps to a row's 128 bytes, within 32 bits)
-    const bool far = p.tiles || 8 * std::max(p.lda, p.ldw) * 4 >= (1ll << 32);
-    return far ? launch_f<WM, WN, FM, FN, KB, NBUF, true>(epi, p, ntm, st) : launch_f<WM, WN, FM, FN, KB, NBUF, false>(epi, p, ntm, st);
 }
 
 struct Shape { int bm, bn; };
@@ -289,8 +282,9 @@ constexpr Shape SHAPES[] = {{16, 32}, {32, 32}, {32, 64}, {64, 64}, {128, 64}, {
 int launch_lm_gemm_tiles(int epi, const LmGemmParams& p, hipStream_t st) {      // (checked by launch_lm_gemm)
     static_assert(LM_TILE_M == 64, "an expert's list of rows is one row tile");
     if (epi < LM_STORE || epi > LM_SIDE) return cr_fail(CR_ERR_ARG, "lm_gemm: epilogue %d", epi);
-    if (p.tiles) return launch_t<2, 4, 2, 1, 1, 4>(epi, p, p.max_tiles, st);
     const int nf = (p.M + 15) / 16, batch = std::max(p.batch, 1), nk = p.K / 32, cus = cr_device_cus();
+    // 64 bits a lane, whatever the epilogue and with the same bits: rows that a list names, and operands eight of whose rows (and an XOR that keeps to a row's 128 bytes) are not within 32 bits of each other
+    if (p.tiles || (p.perm && p.gather_div) || 8 * std::max(p.lda, p.ldw) * 4 >= (1ll << 32)) return launch_t<2, 4, 2, 1, 1, 4, true>(epi, p, p.tiles ? p.max_tiles : (nf + 3) / 4, st);
     int tile = 0, ntm = 0;
     double best = 1e30;
     for (int t = 0; t < (int)(sizeof(SHAPES) / sizeof(SHAPES[0])); t++) {
