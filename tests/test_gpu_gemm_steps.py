@@ -42,13 +42,15 @@ def test_the_largest_shapes_row_tiles(M):
 
 
 @pytest.mark.parametrize('far', ['activations', 'weights'])
-def test_rows_that_span_4_gib_between_eight(far):
+@pytest.mark.parametrize('ld', [2 ** 31 // 14 * 2 // 8 * 8 - 16, 2 ** 31 // 14 * 2 // 8 * 8 + 8])   # seven rows of bf16 just within 4 GiB (offsets of 32 bits, the last above 2^31), and past it
+def test_rows_that_span_4_gib_between_eight(far, ld):
     from callireader_amd import engine as E
-    ld = (2 ** 31 // 7 // 8 + 2) * 8
-    M, N, K = (3, 64, 192) if far == 'activations' else (70, 3, 192)
+    assert (7 * 2 * ld + 128 < 2 ** 32) == (ld < 2 ** 31 // 7)
+    M, N, K = (20, 64, 192) if far == 'activations' else (70, 20, 192)
     A, W, bias, _ = operands(M, N, K)
     rows = M if far == 'activations' else N
     wide = torch.empty((rows - 1) * ld + K, device='cuda', dtype=torch.bfloat16).as_strided((rows, K), (ld, 1))
     wide.copy_(A if far == 'activations' else W)
-    got = E.op_gemm(0, *((wide, W) if far == 'activations' else (A, wide)), bias=bias, kernel=1)
-    assert torch.equal(got, E.op_gemm(0, A, W, bias=bias, kernel=1))
+    args = (wide, W) if far == 'activations' else (A, wide)
+    for tile in (1, 16, 20, 25, 27, 28):                 # (the dispatcher's choice, and shapes with four to eight rows of both operands to a wave's piece)
+        assert torch.equal(E.op_gemm(0, *args, bias=bias, kernel=tile), E.op_gemm(0, A, W, bias=bias, kernel=tile)), tile
