@@ -26,7 +26,8 @@ def test_kernel_tests_pass_on_the_poisoned_build():
     assert os.path.exists(lib)
     sel = 'gemm256 or gemm_epilogues or gelu or both_schedules or back_to_back or attention_vit or patch_rows or swiglu or argmax or tail_rows'
     files = {'test_gpu_gemm192.py': 'same_bits', 'test_gpu_gemm_mid.py': 'every_shape or patches', 'test_gpu_few_rows.py': 'fp32_decode_rows or prompt_rows or among_64', 'test_gpu_grouped.py': 'many_tiles',
-             'test_gpu_decode_mixer.py': 'one_launch or residual_updates', 'test_gpu_routing.py': 'many_tokens'}
+             'test_gpu_decode_mixer.py': 'one_launch or residual_updates', 'test_gpu_routing.py': 'many_tokens', 'test_gpu_gemm_steps.py': 'depths_of_buffers or largest_shapes',
+             'test_gpu_fp32_tiles.py': 'prompt_tiles', 'test_gpu_lm_gemm.py': 'named_by_a_list'}
     sel += ' or ' + ' or '.join(files.values())
     r = subprocess.run([sys.executable, '-m', 'pytest', *(os.path.join(ROOT, 'tests', f) for f in ('test_gpu_ops.py', *files)), '-x', '-q', '-m', 'gpu', '-k', sel],
                        capture_output=True, text=True, env=dict(env, CR_HIP_LIB=lib), cwd=ROOT, timeout=900)
