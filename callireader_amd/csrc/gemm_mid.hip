@@ -2,8 +2,8 @@
 //
 // What bounds these shapes is neither arithmetic nor bytes but the chain of a K-tile's step: a 128x128 grid over M = 1025, N = 1024 is 72 workgroups, and a K loop that waits for each K-tile's
 // loads before it asks for the next-but-one pays a memory round trip per 64 of K.  So (a) the tile shape is a template and picked by the grid it gives (gemm_mid_cost below), down to
-// 16 x 32 for two waves, (b) NBUF K-tiles live in LDS and up to NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles, and (c) a step has no
-// branches and no address arithmetic.
+// 16 x 32 for two waves, (b) NBUF K-tiles live in LDS and up to NBUF - 1 of them are in flight: one barrier per K-tile, counted vmcnt, never a drain before the last tiles, and (c) with four
+// buffers and more a step has no branches and no address arithmetic.
 //   * one global_load_lds_dwordx4 brings eight rows x 64 k, whole 128-byte lines (pieces of 16 rows x 32 k reach 56 of the 69 GB/s per CU that these do on cold weights);
 //     LDS rows of 128 bytes, the 16-byte chunk XORed with (row >> 1) & 7 on both sides: a fragment's ds_read_b128 is free of bank conflicts;
 //   * the weights are the MFMA's A operand: a lane's accumulator holds four consecutive columns of one row; what a column can do by itself happens there, and bf16 rows leave in whole
@@ -370,7 +370,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const MidGrid g,
     // Tile kt's fragments are read a step ahead.  With four buffers the tile asked for in step kt goes where tile kt lay, whose reads the step's barrier waits for; with more (LATE) where tile kt - 1 lay,
     // which was multiplied before the barrier, so that no LDS read has to have come back by then.  These loops are not bound by bytes (64 x 64 tiles, K = 4096: 256 workgroups take little longer than one;
     // a CU brings in 130 GB/s from its L2 and 480 from LDS) but by a step's chain -- branches, addresses, barrier, LDS reads -- and by how far ahead a K-tile is asked for.  So nothing in a step is
-    // conditional or computes an address (LEAN; three buffers are tiles so large that it spilled), and one workgroup a CU takes all the buffers there are.  1025 x 1024 x 4096 23.5 -> 18.7 us, 1025 x 1024 x
+    // conditional or computes an address (LEAN; three buffers keep the loop with its conditions), and one workgroup a CU takes all the buffers there are.  1025 x 1024 x 4096 23.5 -> 18.7 us, 1025 x 1024 x
     // 1024 9.0 -> 7.9, 1025 x 3072 x 1024 12.6 -> 11.5, 1531 x 2048 x 2048 20.5 -> 18.0; tiles of 16 x 32 and 32 x 64 on every CU 62 -> 42, 32.8 -> 27.8.
     constexpr bool LATE = NBUF > 4, LEAN = NBUF > 3;
     constexpr int AHEAD = LATE ? NBUF - 1 : NBUF;             // K-tiles asked for beyond the one being multiplied
@@ -463,10 +463,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const MidGrid g,
             });
             multiply((AHEAD - 1) & 1 ? next : now, count);
         };
+        // (an odd K-tile is copied: with a tail for either order of the two sets the compiler joined the tails and held a third set for it, 256 registers and a spill in 160 x 128 where there are 176 now.  us,
+        // two tails / one: 160 x 128 1025 x 4096 x 1024 15.8 / 14.7, 2050 x 2048 x 2048 24.7 / 23.5, 4100 x 2048 x 2240 47.7 / 48.0; 128 x 128 1025 x 3072 x 1024 13.0 / 12.9, of 1088 13.9 / 13.9)
         if (kt < nk - AHEAD) {
             one(f0, f1);
-            tail(f1, f0);
-        } else tail(f0, f1);
+            f0 = f1;
+        }
+        tail(f0, f1);
     };
     if (live == FM) loop(std::integral_constant<int, FM>{});
     else if (FM > 1 && live == FM - 1) loop(std::integral_constant<int, FM - 1>{});

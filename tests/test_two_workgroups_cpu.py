@@ -1,5 +1,5 @@
-"""gemm_mid.hip's shallow forms, taken where there are more workgroups than compute units, leave a CU room for a second workgroup: eight waves of 128 registers at most each (their LDS is asserted in the source).
-Read from the notes of the library's own object file."""
+"""gemm_mid.hip's shallow forms, taken where there are more workgroups than compute units, leave a CU room for a second workgroup: eight waves of 128 registers at most each (their LDS is asserted in the source); and no
+shape's fragments spill.  Read from the notes of the library's own object file."""
 import os
 import re
 import shutil
@@ -34,3 +34,7 @@ def kernels(tmp_path_factory):
 def test_registers_of_the_shallow_forms(kernels, shape):
     vgpr, spill = kernels[shape]
     assert vgpr <= 128 and spill == 0
+
+
+def test_no_shape_spills(kernels):
+    assert len(kernels) >= 13 and not {k: v for k, v in kernels.items() if v[1]}
