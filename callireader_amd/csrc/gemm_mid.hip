@@ -241,7 +241,7 @@ struct MidGeom {
 
 // What a launch's workgroups would divide for: the tiles' order, the fragments of a row tile, a slice's K-tiles
 struct MidGrid {
-    int epi, ntm, ntn, nk;                                    // epilogue; row and column tiles; K-tiles of a slice
+    int epi, ntm, nk;                                         // epilogue; row tiles; K-tiles of a slice
     int xq, xr;                                               // workgroups / 8 and % 8
     int per_group, last;                                      // workgroups of a super-group of eight row tiles; row tiles of the last one
     unsigned group_mul, last_mul;                             // ceil(2^32 / per_group), ceil(2^32 / last): exact where a workgroup's number times the divisor stays below 2^32 (group_mul 0: it does not)
@@ -292,7 +292,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const MidGrid g,
         if (FAR) {
             src[i] = (const char*)((a ? p.A + (int64_t)first * p.lda : p.W + (int64_t)first * p.ldw) + (int64_t)blockIdx.y * nk * 64);
             lane_src[FAR ? i : 0] = src[i] + (int64_t)(own - first) * (a ? p.lda : p.ldw) * 2 + chunk * 16;
-        } else {                                              // (rows are less than 2^28 elements apart)
+        } else {                                              // (eight rows lie within 4 GiB: less than 306 783 370 elements apart, launch_gemm_mid)
             const unsigned ld = (unsigned)(a ? p.lda : p.ldw);
             src[i] = (const char*)((a ? p.A : p.W) + (uint64_t)(unsigned)first * ld + blockIdx.y * nk * 64);
             off[i] = (unsigned)(own - first) * ld * 2 + chunk * 16;
@@ -300,24 +300,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_mid_kernel(const MidGrid g,
         dst[i] = smem_base + G::PAD + piece * 1024;
         lanes[i] = a && piece >= 2 * fn ? 1 : ~0ull;
     }
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"               // (m0 is a reserved register: nothing else here uses it)
-    // LDS-DMA from inline asm (the compiler lets every LDS read wait for all others while one that it knows is under way); the loop below waits for its landing by hand.  The instruction's offset, K-tile
-    // U of an unrolled run, is added to both addresses: G::PAD keeps the LDS one positive.  All lanes are on here, before and after
-    auto ask1 = [&](auto i, auto u, unsigned at) __attribute__((always_inline)) {
+    // (u is a K-tile of an unrolled run: G::PAD keeps the LDS address positive)
+    auto ask1 = [&](auto i, auto u, unsigned to) __attribute__((always_inline)) {
         constexpr int I = decltype(i)::value, O = decltype(u)::value * 128;
-        const unsigned o = off[I], d = dst[I], to = at - O;
-        const char* g = src[I];
-        if constexpr (FAR) {
-            const char* v = lane_src[I];
-            const uint64_t on = lanes[I];
-            asm volatile("s_add_u32 m0, %1, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, off offset:%4\n\ts_mov_b64 exec, -1" ::"v"(v), "s"(d), "s"(to), "s"(on), "n"(O) : "m0", "scc", "memory");
-        } else if constexpr (I * G::WAVES * 8 < G::BM) {
-            const uint64_t on = lanes[I];
-            asm volatile("s_add_u32 m0, %2, %3\n\ts_mov_b64 exec, %4\n\tglobal_load_lds_dwordx4 %0, %1 offset:%5\n\ts_mov_b64 exec, -1" ::"v"(o), "s"(g), "s"(d), "s"(to), "s"(on), "n"(O) : "m0", "scc", "memory");
-        } else asm volatile("s_add_u32 m0, %2, %3\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1 offset:%4" ::"v"(o), "s"(g), "s"(d), "s"(to), "n"(O) : "m0", "scc", "memory");
+        if constexpr (FAR) ring_ask_far<O>(lane_src[I], dst[I], to, lanes[I]);
+        else if constexpr (I * G::WAVES * 8 < G::BM) ring_ask<O>(src[I], off[I], dst[I], to, lanes[I]);
+        else ring_ask<O>(src[I], off[I], dst[I], to);
     };
-#pragma clang diagnostic pop
     // K-tile u of the run that `src` stands at, into buffer buf
     auto ask = [&](auto u, int buf) __attribute__((always_inline)) {
         constexpr_for<G::PER>([&](auto i) {
@@ -511,7 +500,7 @@ int launch_t(int epi, const GemmParams& p, int rt, hipStream_t stream) {
     const int ntm = std::max((p.M + G::BM - 1) / G::BM, rt), ntn = (p.N + G::BN - 1) / G::BN;
     const int slices = epi == EPI_PARTIAL ? p.group : 1, nwg = ntm * ntn, nf = (p.M + 15) / 16, per_group = 8 * ntn, last = ntm % 8 ? ntm % 8 : 8;
     auto mul = [&](int d) { return d > 1 && (int64_t)nwg * d < (1ll << 32) ? (unsigned)(((1ull << 32) + d - 1) / d) : 0u; };
-    const MidGrid g{epi, ntm, ntn, p.K / 64 / slices, nwg / 8, nwg % 8, per_group, last, mul(per_group), mul(last), nf / ntm, nf % ntm, ntm > 1 && ntm < 1600 ? (unsigned)(((1ull << 32) + ntm - 1) / ntm) : 0u};
+    const MidGrid g{epi, ntm, p.K / 64 / slices, nwg / 8, nwg % 8, per_group, last, mul(per_group), mul(last), nf / ntm, nf % ntm, ntm > 1 && ntm < 1600 ? (unsigned)(((1ull << 32) + ntm - 1) / ntm) : 0u};
     hipLaunchKernelGGL((gemm_mid_kernel<WM, WN, FM, FN, NBUF, FAR>), dim3(nwg, slices), dim3(64 * G::WAVES), G::LDS, stream, g, p);
     return hipGetLastError() == hipSuccess ? CR_OK : CR_ERR_HIP;
 }
@@ -533,7 +522,7 @@ int launch_two(int epi, const GemmParams& p, int rt, hipStream_t stream) {
 namespace {
 
 // Tile shapes (launch_gemm_mid's `tile` = index + 1).  Eight waves where the tile is large enough to feed them: two waves a SIMD cover each other's LDS reads and barriers (64 x 64 at
-// M = 1025, N = 1024, K = 4096: four waves 27.5 us, eight 26.6, now 26.2; 128 x 128 at N = 3072, K = 1024: 20 and 13.4).
+// M = 1025, N = 1024, K = 4096: four waves 27.5 us, eight 26.6, before the loop that is there now; 128 x 128 at N = 3072, K = 1024: 20 and 13.4).
 struct MidShape { int bm, bn; double launch = 2.5, row = 1.9e-3, step = -0.02; };      // (the law's: us a launch, a row of A or W in a K-tile, a K-tile)
 constexpr MidShape SHAPES[] = {{16, 32}, {16, 64}, {32, 64}, {64, 32}, {64, 64}, {96, 64}, {128, 64}, {64, 128}, {96, 128}, {128, 128}, {96, 256, 2.5, 2e-3, 0.0}, {128, 256, 3.0, 2e-3, 0.02}, {160, 128, 2.5, 1.9e-3, 0.03}};
 constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);

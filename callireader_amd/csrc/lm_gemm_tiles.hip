@@ -101,7 +101,7 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
 
     // This wave's pieces of a K-tile: eight rows, 128 bytes each; numbers past the last repeat it, pieces past the tile's rows move one lane's 16 bytes (the count of instructions under way stays a
     // constant).  A piece's first row is the same for all lanes, so its address is a scalar one and a lane's own row and chunk are 32 bits beyond it; FAR: gathered rows, and rows so far apart that eight of
-    // them span 4 GiB, have 64 bits a lane.  LDS-DMA from inline asm: from the builtin a piece came with 64-bit sums, a copy of m0 and a branch on the lanes.
+    // them span 4 GiB, have 64 bits a lane.
     const char *src[G::PER], *lane_src[FAR ? G::PER : 1];
     unsigned off[G::PER], dst[G::PER];
     uint64_t lanes[G::PER];
@@ -121,24 +121,16 @@ __global__ __launch_bounds__(64 * WM * WN) void lm_tiles_kernel(const LmGemmPara
         lanes[i] = a && piece >= 2 * fn ? 1 : ~0ull;
     }
     const int nk = p.K / (32 * KB);
-#pragma clang diagnostic push
-#pragma clang diagnostic ignored "-Winline-asm"               // (m0 is a reserved register: nothing else here uses it)
-    // (all lanes are on here, before and after)
     auto ask_piece = [&](int i, int buf) __attribute__((always_inline)) {
         CR_DIAG_POISON(smem + buf * G::STAGE + (dst[i] - smem_base))
-        const unsigned to = buf * G::STAGE, d = dst[i], o = off[i];
-        const uint64_t on = lanes[i];
         if constexpr (FAR) {
-            const char* v = lane_src[FAR ? i : 0];
-            asm volatile("s_add_u32 m0, %1, %2\n\ts_mov_b64 exec, %3\n\tglobal_load_lds_dwordx4 %0, off\n\ts_mov_b64 exec, -1" ::"v"(v), "s"(d), "s"(to), "s"(on) : "m0", "scc", "memory");
+            ring_ask_far<0>(lane_src[FAR ? i : 0], dst[i], buf * G::STAGE, lanes[i]);
             lane_src[FAR ? i : 0] += KB * 128;
         } else {
-            const char* g = src[i];
-            asm volatile("s_add_u32 m0, %2, %3\n\ts_mov_b64 exec, %4\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(o), "s"(g), "s"(d), "s"(to), "s"(on) : "m0", "scc", "memory");
+            ring_ask<0>(src[i], off[i], dst[i], buf * G::STAGE, lanes[i]);
             src[i] += KB * 128;
         }
     };
-#pragma clang diagnostic pop
     // the K-tile that `src` stands at, into buffer buf
     auto ask = [&](int buf) __attribute__((always_inline)) {
 #pragma unroll
