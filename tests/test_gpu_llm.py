@@ -341,14 +341,14 @@ def test_decode_layout_of_the_weights_gives_the_same_bits(rows):
 
 
 def test_decode_beside_fetched_weights_has_the_bits_of_the_plain_kernels(setup, monkeypatch):
-    """The attention of a decode step that brings wo into L2 beside it (up to 8 rows, and 9 to 64 with the rotation folded in; one and two key splits, a last plane of the grid that is not full) and that of
+    """The attention of a decode step that brings wo into L2 beside it (up to 8 rows, and 9 to 64 with the rotation folded in; one to three key splits, of which three leave the grid's last plane not full) and that of
     a context without decode-layout copies, which fetches nothing: the same bits."""
     from callireader_amd.engine import Engine
     monkeypatch.setenv('CR_DECODE_LAYOUT', '0')
     plain = Engine(setup['dims'], max_pos=2048)
     plain.load_state_dict(setup['sd']); plain.load_rope(); plain.finalize()
     monkeypatch.delenv('CR_DECODE_LAYOUT')
-    for rows, S in ((1, 20), (5, 270), (9, 30), (33, 260)):
+    for rows, S in ((1, 20), (5, 270), (3, 530), (9, 30), (33, 260), (10, 600)):
         embs = [prompt(S + i % 3, 70 + i).cuda() for i in range(rows)]
         given = torch.arange(3, 3 + rows)
         got = []
@@ -359,6 +359,23 @@ def test_decode_beside_fetched_weights_has_the_bits_of_the_plain_kernels(setup, 
             kv.free()
         assert torch.isfinite(got[0]).all() and torch.equal(*got), (rows, S)
     plain.close()
+
+
+def test_decode_of_more_keys_than_leave_the_caches_room(setup, monkeypatch):
+    """64 rows of eleven key splits: 5632 workgroups of keys, beside which wo is left where it is (from 5121 on, on 256 compute units).  The bits of a context that never fetches."""
+    from callireader_amd.engine import Engine
+    rows, S = 64, 2570
+    embs, given, got = prompt(S, 91).cuda(), torch.arange(3, 3 + rows), []
+    for layout in ('1', '0'):
+        monkeypatch.setenv('CR_DECODE_LAYOUT', layout)
+        e = Engine(setup['dims'], max_pos=3072)
+        e.load_state_dict(setup['sd']); e.load_rope(); e.finalize()
+        kv = e.kv_alloc(rows, S + 8)
+        for i in range(rows):
+            e.prefill(kv, i, embs[:, :S - i % 5].contiguous())
+        got.append(torch.stack([e.decode(kv, list(range(rows)), force_tokens=given + t, want_logits=True) for t in range(2)]).cpu())
+        kv.free(); e.close()
+    assert torch.isfinite(got[0]).all() and torch.equal(*got)
 
 
 def test_decode_graph_replay_equals_plain_launches(setup):

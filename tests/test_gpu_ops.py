@@ -487,6 +487,15 @@ def test_layernorm_pixel_shuffle(E):
     torch.testing.assert_close(out.float().cpu(), ref, rtol=RTOL, atol=1e-2)
 
 
+def test_layernorm_pixel_shuffle_of_many_tiles_has_the_bits_of_few(E):
+    """64 tiles are the last whose gains are loaded with the row, 65 the first behind the sums."""
+    g = torch.Generator(device='cuda').manual_seed(8)
+    v, gamma, beta = (torch.randn(*s, device='cuda', generator=g).to(torch.bfloat16) for s in ((65, 1025, 1024), (4096,), (4096,)))
+    of = lambda x: E.op_layernorm(x.contiguous(), gamma, beta, 1e-5, pixel_shuffle=True)      # noqa: E731
+    whole = of(v)
+    assert torch.isfinite(whole.float()).all() and torch.equal(whole[:64 * 256], of(v[:64])) and torch.equal(whole[-256:], of(v[-1:]))
+
+
 def test_rmsnorm(E):
     g = torch.Generator().manual_seed(7)
     x = bf(_rand((333, 4096), g) * 3).to(dev())
