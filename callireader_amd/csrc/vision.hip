@@ -73,6 +73,8 @@ static int vit_chunk(cr_ctx* c, const bf16* px, int T, bf16* x, hipStream_t st) 
     CR_TRY(gemm(c, EPI_PATCH, col, KPAD, patch_w, KPAD, x, C1, patch_b, nullptr, pos, C1, T * 1024, C1, KPAD, 1024, st));
     CR_TRY(launch_cls_rows(cls, pos, x, T, C1, TOK, st));
 
+    // tiles up to which weights are read ahead beside the norms and the merge (figures below, of 256 compute units): their own rows keep memory busy for longer the fewer units share them
+    const int cus = cr_device_cus(), one = cus / 256, few = cus / 64;
     for (int l = 0; l < c->d.vit_layers; l++) {
         const std::string p = "vision_model.encoder.layers." + std::to_string(l) + ".";
         const bf16 *n1w = W(c, p + "norm1.weight"), *n1b = W(c, p + "norm1.bias");
@@ -97,7 +99,7 @@ static int vit_chunk(cr_ctx* c, const bf16* px, int T, bf16* x, hipStream_t st) 
         np.in = x; np.ld_in = C1; np.out = h; np.ld_out = C1; np.rows = M; np.eps = c->d.vit_ln_eps;
         np.gamma = n1w; np.beta = n1b;
         // (one tile: 2158 / 2137 us the whole tower without / with; 2 tiles 3041 / 3057, 4 tiles 4409 / 4421)
-        if (T == 1 && !m8) np.ahead = l2_ahead_of(qkvw, (int64_t)C1 * C3 * 2, L2_AHEAD_GROUPS);
+        if (T <= one && !m8) np.ahead = l2_ahead_of(qkvw, (int64_t)C1 * C3 * 2, L2_AHEAD_GROUPS);
         if (m8) { np.out8 = (unsigned char*)h; np.out8_scale = hs; }
         CR_TRY(launch_layernorm(np, C1, 0, st));
         if (m8) CR_TRY(ctx_gemm_f8(c, EPI_STORE, h, hs, q_qkv, s_qkv, qkv, C3, qkvb, M, C3, C1, st));
@@ -112,7 +114,7 @@ static int vit_chunk(cr_ctx* c, const bf16* px, int T, bf16* x, hipStream_t st) 
         ap.part_ml = apart;
         // beside the class rows' merge, five workgroups a tile that leave memory idle for 4 us: 1 tile 2178 / 2159 us, 2 tiles 3064 / 3041, 4 tiles 4424 / 4409, from 6 on nothing (fc1's 8 MB there, alone or
         // behind these: 5 to 10 us less, 5 more)
-        if (T <= 4 && !m8) ap.ahead = l2_ahead_of(pw, (int64_t)C1 * C1 * 2, L2_AHEAD_GROUPS);
+        if (T <= few && !m8) ap.ahead = l2_ahead_of(pw, (int64_t)C1 * C1 * 2, L2_AHEAD_GROUPS);
         if (launch_flash_attn(ap, 64, false, st) != CR_OK) return cr_fail(CR_ERR_HIP, "vit attention launch failed");
         CR_TRY(gemm(c, EPI_LS_RES, h, C1, pw, C1, x, C1, pb, ls1, x, C1, M, C1, C1, 0, st));
 
@@ -120,7 +122,7 @@ static int vit_chunk(cr_ctx* c, const bf16* px, int T, bf16* x, hipStream_t st) 
         // fc2's 8 MB come from HBM, 24 layers of weights being more than the memory-side cache holds, and a product of few rows waits for them (1025 x 1024 x 4096 23.3 us, 19.4 out of that cache): read
         // beside the norm's 4.4 us, with fc1 between, they are there.  The whole tower, us without / with: 1 tile 2278 / 2184, 2 tiles 3083 / 3069, 3 tiles 3687 / 3669, 4 tiles 4533 / 4505, 6 tiles 6129 /
         // 6161, 8 tiles 7362 / 7397, 11 tiles 8900 / 8922.  fc1's weights so, beside either norm, 0 to 10 us more or less
-        if (T <= 4 && !m8) np.ahead = l2_ahead_of(f2w, (int64_t)C1 * FF * 2, L2_AHEAD_GROUPS);
+        if (T <= few && !m8) np.ahead = l2_ahead_of(f2w, (int64_t)C1 * FF * 2, L2_AHEAD_GROUPS);
         if (m8all) { np.next_scale = fs; np.next_bound = (const float*)bnd->ptr; }
         CR_TRY(launch_layernorm(np, C1, 0, st));
         if (m8 && !m8all) {
