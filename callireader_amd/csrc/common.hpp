@@ -133,8 +133,10 @@ __device__ __forceinline__ float gelu_tanh(float x) {
 __device__ __forceinline__ float silu(float x) { return x / (1.0f + __expf(-x)); }
 
 // A launch's arguments: every 64-byte line of them is a round trip of its own, taken where the compiler places the first use.  All lines at once instead.  The kernels of a decode step and of few tiles, us
-// without / with: 24 latent requests of 32 steps 33 210 / 32 940, a float32 request's 12 steps 11 640 / 11 420, a page's answer 19 428 / 19 323, one and two tiles 2032 / 2029 and 3015 / 3006; prompts' attention
-// and the streaming products, which live longer, 0 to 0.3 % slower and go without.
+// without / with, two measurements each (profiles/main_paths/arguments.txt): a float32 request's 12 steps 11 658 / 11 389 and 11 622 / 11 386, a request of 32 steps of 14 passes 15 401 / 15 291 and 15 451 /
+// 15 158, 24 latent requests of 32 steps 33 703 / 33 523 and 33 551 / 33 367, a page's answer 19 717 / 19 605 and 19 708 / 19 593, a question 7876 / 7830 and 7876 / 7836, one tile 2113 / 2097 and 2122 / 2111
+// (within what its runs differ by); what is larger 0 to 0.2 % faster, layer norm and the updates of prompts included.  A trace of single kernels shows nothing of it beside its own 3 to 6 %.  Prompts' attention and the
+// streaming products, which live longer, were 0 to 0.3 % slower and go without.
 template <int BYTES> __device__ __forceinline__ void touch_args() {
     const __attribute__((address_space(4))) int* k = (const __attribute__((address_space(4))) int*)__builtin_amdgcn_kernarg_segment_ptr();
     int x = 0;
