@@ -15,24 +15,25 @@ int launch_gemm256(int epi, const GemmParams& p, hipStream_t stream);
 int launch_gemm256_f8(int epi, const GemmParams& p, hipStream_t stream);
 bool gemm_skinny_supported(int epi, const GemmParams& p);
 int launch_gemm_skinny(int epi, const GemmParams& p, hipStream_t stream);
-double gemm256_cost(const GemmParams& p, double full);
+double gemm256_cost(const GemmParams& p);
+double gemm256_round_us(const GemmParams& p);
 
 // Rows of a product that the 256x256 kernel takes, the others go to gemm_mid: all, none, or those up to a multiple of 256, as a few rows past it can cost the persistent kernel a round of tiles (32 ViT tiles are
-// 128 x 256 + 32 rows: three rounds for two rounds' work at N = 1024).  Apart only where the laws see 3 % in it, also with rounds that fill the card (what is cut off leaves mostly those) priced FULL above
-// the others.  us, whole | apart: 3162 x 4096 x 4096 (208 tiles of 256 rows; 256 of 192) 80.3 | 85.6, 3162 x 4096 x 14336 270 | 285, 6145 x 2048 x 2048 43.1 | 45.6, 696 x 28672 x 8192 278 | 325; 4100 x 4096 x
-// 4096 126 | 99.7, 6145 x 4096 x 4096 157 | 149, 6145 x 6144 x 4096 241 | 219.  Of 421 sizes with rows past a multiple of 256 it is the slower choice by more than 2 % at three (at most 3 %), without
-// either rule at sixteen.
+// 128 x 256 + 32 rows: three rounds for two rounds' work at N = 1024).  Apart only where the laws see a fifth of a round in it: what is cut off leaves mostly rounds that fill the card, which the law prices too
+// low.  541 sizes of 300 .. 99 000 rows, us whole | apart, by the saving that the laws see in rounds: 0.00 .. 0.18 800 x 16384 x 14336 315 | 361, 787 x 28672 x 4096 172 | 185, 3162 x 4096 x 4096 80.3 | 85.6, 4180 x
+// 8192 x 1024 63.8 | 69.5; 0.20 .. 0.40 632 x 28672 x 4096 143 | 135, 12373 x 2048 x 4096 157 | 152, 41132 x 28672 x 4096 6539 | 6354, 1170 x 16384 x 4096 138 | 125; above 4100 x 4096 x 4096 126 | 99.7, 98400 x 4096 x
+// 1024 640 | 627.  By this line the slower one is taken by more than 2 % at ten of the 423 sizes that gemm_mid does not take whole; by the sign of the saving, or by 3 % of the whole, at eighteen (profiles/tiled_products/last_rows.txt).
 int gemm_tiled_rows(int epi, const GemmParams& p) {
-    constexpr double APART = 1.03, FULL = 0.08;
+    constexpr double APART = 0.19;
     int tile, rt;
     const int r = p.M % 256;
-    const double whole = gemm256_cost(p, 0.0), mid = gemm_mid_cost(epi, p, &tile, &rt);
+    const double whole = gemm256_cost(p), mid = gemm_mid_cost(epi, p, &tile, &rt);
     if (r > 0 && p.M > r && epi != EPI_PATCH && epi != EPI_ARGMAX) {
         GemmParams a = p, b = p;
         a.M = p.M - r;
         b.M = r;
-        const double rest = gemm_mid_cost(epi, b, &tile, &rt), cut = gemm256_cost(a, 0.0) + rest;
-        if (APART * cut < whole && gemm256_cost(a, FULL) + rest < gemm256_cost(p, FULL)) return mid < cut ? 0 : a.M;
+        const double cut = gemm256_cost(a) + gemm_mid_cost(epi, b, &tile, &rt);
+        if (whole - cut > APART * gemm256_round_us(p)) return mid < cut ? 0 : a.M;
     }
     return mid < whole ? 0 : p.M;
 }

@@ -882,12 +882,12 @@ int launch_s(const GemmParams& p, hipStream_t stream) {
 // (1000 x 4096 x 14336 takes 251 us), of 192 rows 0.93 (203 us).  One round is up to 14 % faster than that (1025 x 3072 x 1024 21.2 measured / 24.4, 77 x 4096 x 14336 238 / 257), rounds
 // that fill the card 5 to 16 % slower, as its clock falls (11275 x 4096 x 1024 76.7 / 66.3, 3164 x 28672 x 4096 527 / 452, 6000 x 4096 x 14336 559 / 511).  The shorter tile wins where it takes no more rounds (x 256 rows / 192 rows, us): 11275 x 3072 x 1024 (540 / 708 tiles) 73.7 / 62.8,
 // 11275 x 1024 x 4096 (180 / 236) 82.5 / 74.8, 8200 x 4096 x 1024 (528 / 688) 83.3 / 71.0, 6000 x 4096 x 14336 (384 / 512) 587 / 495; it loses where it takes one more:
-// 13325 x 1024 x 4096 (212 / 280) 91 / 130, 11275 x 4096 x 1024 (720 / 944) 89 / 94, 4700 x 28672 x 4096 (2128 / 2800) 799 / 811.  full: what a round that fills the card costs beyond
-// the others, as a share (gemm.hip, where a product loses its last rows).
-double tile_us(const GemmParams& p, int f1, double full = 0.0) {
+// 13325 x 1024 x 4096 (212 / 280) 91 / 130, 11275 x 4096 x 1024 (720 / 944) 89 / 94, 4700 x 28672 x 4096 (2128 / 2800) 799 / 811.
+double round_us(const GemmParams& p, int f1) { return f1 == 4 ? p.K / BK2 * 1.12 + 3.0 : p.K / BK2 * 0.93 + 2.6; }
+double tile_us(const GemmParams& p, int f1) {
     const int tm = 128 + 32 * f1;
     const long tiles = (long)((p.M + tm - 1) / tm) * ((p.N + BN2 - 1) / BN2), cus = cr_device_cus();
-    return 3.5 + ((double)((tiles + cus - 1) / cus) + full * (double)(tiles / cus)) * (f1 == 4 ? p.K / BK2 * 1.12 + 3.0 : p.K / BK2 * 0.93 + 2.6);
+    return 3.5 + (double)((tiles + cus - 1) / cus) * round_us(p, f1);
 }
 
 // Two schedules of the same sums (bit-identical results): 32-MFMA matrix slots measured 2-5 % faster on the wide outputs at K <= 4096 (ViT QKV
@@ -915,7 +915,8 @@ static bool rows_within_4g(const GemmParams& p) {
 
 bool gemm256_supported(int epi, const GemmParams& p) { return epi != EPI_PARTIAL && p.N >= 64 && p.K % 128 == 0 && !p.raw32 && rows_within_4g(p); }
 
-double gemm256_cost(const GemmParams& p, double full) { const double a = tile_us(p, 4, full), b = tile_us(p, 2, full); return a < b ? a : b; }
+double gemm256_cost(const GemmParams& p) { const double a = tile_us(p, 4), b = tile_us(p, 2); return a < b ? a : b; }
+double gemm256_round_us(const GemmParams& p) { return round_us(p, 4); }
 
 int launch_gemm256_grouped(int epi, const GemmParams& p, hipStream_t stream) {
     if (p.K <= 0 || p.K % 128 || p.N < 64 || p.N % 64 || (p.lda & 7) || (p.ldc & 7) || !p.tiles || !p.n_tiles || p.max_tiles <= 0 || ((p.gather_div || p.scatter) && !p.perm) ||

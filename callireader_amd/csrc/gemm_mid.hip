@@ -533,7 +533,7 @@ constexpr int N_SHAPES = sizeof(SHAPES) / sizeof(SHAPES[0]);
 // each K-tile of 64 less 20 ns (the three largest shapes more: SHAPES), 0.1 ns an element in the epilogue; a workgroup more on a CU costs its time again (two shallow ones to a CU take 0.8 of that).  It is no
 // prediction.  Measured / law, weights cold: 1025 x 1024 x 4096 18.7 / 20.2, 1025 x 1024 x 1024 7.9 / 8.1, 1025 x 3072 x 1024 11.5 / 11.9, 1025 x 4096 x 1024 14.4 / 14.1, 77 x 4096 x 4096 15.0 / 12.1, 333 x
 // 4096 x 14336 81 / 68, 1000 x 4096 x 14336 135 / 110, 13325 x 5120 x 1344 199 / 190; no term stands for the rate of HBM itself, which bounds wide weights at few rows (77 x 28672 x 4096 54 / 29).
-// Against every way there is, 500 sizes drawn over M 65 .. 16000, N 512 .. 28672, K 256 .. 14336 (profiles/tiled_products/choice.txt): 1.007 times the fastest in geometric mean, above 1.05 at 14 of them.
+// Against every way there is, 500 sizes drawn over M 65 .. 16000, N 512 .. 28672, K 256 .. 14336 (profiles/tiled_products/choice.txt): 1.007 times the fastest in geometric mean, above 1.05 at 21 of them.
 // The largest shapes' terms decide where a product takes several rounds of one and fewer of the other, above all where K leaves 64 modulo 128, which the 256x256 kernel does not take.  us, 160 x 128 | 128 x
 // 256: 3075 x 9216 x 448 48.3 | 39.9, 6124 x 9216 x 2240 260 | 228, 13325 x 5120 x 1344 212 | 199, and one round either way 2050 x 2048 x 2048 24.2 | 29.4; 96 x 128 | 96 x 256: 356 x 12800 x 14336 215 | 177,
 // 1923 x 2560 x 14336 186 | 162.

@@ -66,6 +66,12 @@ def test_tile_shape(ask, M, N, K, tile):
     (4100, 4096, 4096, 4096),     # 126, 99.7
     (6145, 4096, 4096, 6144),     # 157, 149
     (6145, 6144, 4096, 6144),     # 241, 219
+    (98400, 4096, 1024, 98304),   # 640, 627
+    (41132, 28672, 4096, 40960),  # 6539, 6354
+    (632, 28672, 4096, 512),      # 143, 135
+    (12373, 2048, 4096, 12288),   # 157, 152
+    (4180, 8192, 1024, 4180),     # 63.8, 69.5
+    (800, 16384, 14336, 800),     # 315, 361
     (11275, 4096, 1024, 11275), (1025, 4096, 1024, 0), (77, 4096, 4096, 0)])
 def test_rows_apart(ask, M, N, K, rows):
     assert ask(M, N, K)[0] == rows
