@@ -22,12 +22,14 @@ inline L2Ahead l2_ahead_of(const void* at, int64_t bytes, int units) {
 inline int64_t l2_ahead_bytes(const L2Ahead& a) { return (int64_t)a.units * a.unit_bytes; }
 // Whether wo's 34 MB go beside `own` workgroups of 256 keys each of the chat model's attention.  A step of four layers and the head with fetching over one without: 72 .. 2560 own 1.02 .. 1.04, 4096 (64 rows of
 // 2000 keys) and 4608 1.01, 4992 and 5760 1.00, 6656 and 8192 (64 rows of 3164 and 3900) 0.99.
+// Measured again, with rows of unequal length: profiles/read_ahead/chat.txt (up to 4608 1.01 .. 1.04, 5632 and 6656 1.01; 64 rows of 100 to 3164 keys, 6656 launched, 1.01).
 inline bool l2_ahead_beside_attention(int64_t own, int cus) { return own <= 20 * cus; }
 // Most bytes that go beside `own` workgroups of latent attention.  What the caches do not hold is read twice, and where every second CU has a workgroup of its own the two share its load path.  A step with
 // fetching over one without, few experts, wo of 8 / 32 / 40 / 80 MiB: 1 .. 64 own 1.01 / 1.02 .. 1.05 / 1.04 / 0.98, 96 .. 128 1.01 / 1.00 / 1.02 / 0.96, 192 .. 256 1.00 / 0.98 / 0.99 / 0.94, 448 1.00 /
-// 0.99 / 0.97 / 0.88 (235 MB of 128 heads 0.85 throughout).
+// 0.99 / 0.97 / 0.88 (235 MB of 128 heads 0.85 throughout).  Again, with rows of unequal length: profiles/read_ahead/latent.txt.
 inline int64_t l2_ahead_beside_latent(int64_t own, int cus) { return (int64_t)(2 * own <= cus ? 40 : 8) << 20; }
-// The same beside `own` workgroups of a decode mixer (lm_mix.hip), with how little it must be to go at all and how many products it may be.  A step with all that fits over one without:
+// The same beside `own` workgroups of a decode mixer (lm_mix.hip), with how little it must be to go at all and how many products it may be.  A step with all that fits over one without (bf16 again, with rows of
+// unequal length: profiles/read_ahead/mixer.txt):
 //   bf16, one key split: up to 256 own 0.98 .. 1.07; 288 .. 960 0.95 .. 1.05 with 34 MiB, 0.97 .. 1.05 with 26; where all that there is are 7 MiB, 320 .. 512 0.97 .. 0.99.
 //   Several splits (retention then streams its states through the caches before the weights' reader starts): up to 256 0.97 .. 1.05, 320 0.98 .. 1.04, 384 .. 1024 0.93 .. 1.03, mostly below one.
 //   float32, whose workgroups have a CU each: up to 128 0.99 .. 1.04; 144 .. 192 0.95 .. 1.03, the first product alone 1.00 .. 1.03 (of 32 MiB 0.99 .. 1.02); 200 .. 256 0.95 .. 1.03 and 0.98 .. 1.03.

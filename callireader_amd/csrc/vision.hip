@@ -73,7 +73,7 @@ static int vit_chunk(cr_ctx* c, const bf16* px, int T, bf16* x, hipStream_t st) 
     CR_TRY(gemm(c, EPI_PATCH, col, KPAD, patch_w, KPAD, x, C1, patch_b, nullptr, pos, C1, T * 1024, C1, KPAD, 1024, st));
     CR_TRY(launch_cls_rows(cls, pos, x, T, C1, TOK, st));
 
-    // tiles up to which weights are read ahead beside the norms and the merge (figures below, of 256 compute units): their own rows keep memory busy for longer the fewer units share them
+    // tiles up to which weights are read ahead beside the norms and the merge (figures below and in profiles/read_ahead/vision.txt, of 256 compute units): their own rows keep memory busy for longer the fewer units share them
     const int cus = cr_device_cus(), one = cus / 256, few = cus / 64;
     for (int l = 0; l < c->d.vit_layers; l++) {
         const std::string p = "vision_model.encoder.layers." + std::to_string(l) + ".";
