@@ -6,12 +6,13 @@ import torch
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize('tile,bm,bn', [(0, 16, 32), (4, 64, 64), (9, 128, 128), (12, 160, 128)])
-@pytest.mark.parametrize('rows,cols', [(1, 1), (7, 3), (8, 1), (9, 5), (15, 7), (17, 11), (1599, 1), (1601, 2)])
+TILES, GRIDS = [(0, 16, 32), (4, 64, 64), (9, 128, 128), (12, 160, 128)], [(1, 1), (7, 3), (8, 1), (9, 5), (15, 7), (17, 11)]
+
+
+# (as many row tiles as 1600 with the smallest tile alone)
+@pytest.mark.parametrize('tile,bm,bn,rows,cols', [(*t, *g) for g in GRIDS for t in TILES] + [(*TILES[0], *g) for g in ((1599, 1), (1601, 2))])
 def test_every_tile_once(tile, bm, bn, rows, cols):
     from callireader_amd import engine as E
-    if rows > 100 and tile:
-        pytest.skip('as many row tiles with the smallest tile alone')
     g = torch.Generator().manual_seed(rows + cols)
     M, N, K = rows * bm - bm // 2 + 3, cols * bn - 8, 128
     A, W = (torch.randint(-3, 4, s, generator=g).to(torch.bfloat16).cuda() for s in ((M, K), (N, K)))
